@@ -228,7 +228,7 @@ SMLM_API int smlm_lora_fwd_multi(int n_proj, void* const* y, const void* const* 
  *   a_ptrs, b_ptrs, da_ptrs, db_ptrs: device arrays of NA device addresses.
  *   v: NULL (recomputed from x and A) or [n_rows, r].
  *   part_scale: NULL or float [P] (device), the forward's seg_scale.
- * Needs n_rows >= 1, P >= 1, NA >= 1 and r <= 64.
+ * Needs n_rows >= 1, P >= 1 and NA >= 1.
  */
 SMLM_API int smlm_lora_bwd_workspace_size(int n_rows, int P, int NA, int h_in, int h_out, int r,
                                           size_t* bytes);
@@ -302,8 +302,8 @@ typedef struct smlm_dropout {
  *                  get the plan launch first.  Adapter ids must lie below n_weights (negative:
  *                  no adapter, see the tile plan above); stages must include SMLM_STAGE_SHRINK.
  *                  smlm_lora_bwd_ex takes the pair (part_indptr, part_adapter) the same way and
- *                  builds its plan inside the dV launch when r <= 64, P <= 512,
- *                  n_rows / 16 + P < 1024, v is given and there is no dropout.
+ *                  builds its plan inside the dV launch when P <= 512, n_rows / 16 + P < 1024,
+ *                  v is given and there is no dropout.
  *   build_seg_key_a, build_seg_key_b (both or neither, with build_seg_indptr, instead of
  *                  build_seg_adapter; smlm_lora_fwd_multi_ex only):
  *                  the plan to build is the one smlm_plan_build2 builds from these two arrays of S

@@ -53,9 +53,9 @@ inline int tiles_per_wave(int T, int r) {
   const int from = r <= 16 ? 2048 : (r <= 32 ? 768 : (r <= 48 ? 512 : (r <= 64 ? 128 : 1024)));
   return T >= from ? kBlkTiles : 1;
 }
-// The backward runs on tile blocks at every size up to rank 64: its single-tile route needs transposed copies
-// of the weights first (64 rows at rank 64: 25.0 / 18.8 us; 1024 rows at rank 16: 28.3 / 25.3 us).
-inline int bwd_tiles_per_wave(int n_rows, int r) { return (r <= 64 || n_rows >= 1024) ? kBlkTiles : 1; }
+// (The backward runs on tile blocks at every size and rank: they read the weights the other way round as they lie
+// in memory, where single tiles would need transposed copies of them first.  64 rows at rank 64, single tiles / tile
+// blocks: 25.0 / 18.8 us; 1024 rows at rank 16: 28.3 / 25.3 us.)
 
 // Upper bound of the number of work units along the tile axis.  `groups` bounds
 // the number of distinct plan keys (adapters): every group ends in at most one
@@ -187,12 +187,12 @@ inline dim3 item_grid(const ItemSpace& sp, long items) {
   return dim3((unsigned)rows, (unsigned)sp.units_max, (unsigned)sp.nproj);
 }
 
-template <int DT, int NW, bool RM, bool DIRECT, bool DROP = false>
+template <int DT, int NW, bool DIRECT, bool DROP = false>
 int launch_shrink_nb(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
   const dim3 block(NW * kWaveSize);  // U must match shrink_cfg
-  if (NB == 1) return launch(shrink_kernel<DT, 1, 4, NW, RM, DIRECT, DROP>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_kernel<DT, 2, 4, NW, RM, DIRECT, DROP>, grid, block, st, a);
-  return launch(shrink_kernel<DT, 4, 2, NW, RM, DIRECT, DROP>, grid, block, st, a);
+  if (NB == 1) return launch(shrink_kernel<DT, 1, 4, NW, DIRECT, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_kernel<DT, 2, 4, NW, DIRECT, DROP>, grid, block, st, a);
+  return launch(shrink_kernel<DT, 4, 2, NW, DIRECT, DROP>, grid, block, st, a);
 }
 
 template <int DT, bool DIRECT, bool WKN, bool DROP = false>
@@ -204,27 +204,25 @@ int launch_shrink_block(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) 
 }
 
 template <int DT, bool DIRECT>
-int launch_shrink_dt(bool row_major, int NB, int MT, int NW, dim3 grid, hipStream_t st,
+int launch_shrink_dt(int NB, int MT, int NW, dim3 grid, hipStream_t st,
                      const ShrinkArgs& a) {
-  if (row_major)  // the slow layout
-    return launch_shrink_nb<DT, kFwdWaves, true, DIRECT>(NB, grid, st, a);
   if (a.drop.seg_p) {  // dropout of the training rows: x in the usual layout, weights [n][k]
     if (MT == 1)
-      return NW == kDecodeWaves ? launch_shrink_nb<DT, kDecodeWaves, false, DIRECT, true>(NB, grid, st, a)
-                                : launch_shrink_nb<DT, kFwdWaves, false, DIRECT, true>(NB, grid, st, a);
+      return NW == kDecodeWaves ? launch_shrink_nb<DT, kDecodeWaves, DIRECT, true>(NB, grid, st, a)
+                                : launch_shrink_nb<DT, kFwdWaves, DIRECT, true>(NB, grid, st, a);
     return launch_shrink_block<DT, DIRECT, false, true>(NB, grid, st, a);
   }
   if (MT == 1)
-    return NW == kDecodeWaves ? launch_shrink_nb<DT, kDecodeWaves, false, DIRECT>(NB, grid, st, a)
-                              : launch_shrink_nb<DT, kFwdWaves, false, DIRECT>(NB, grid, st, a);
+    return NW == kDecodeWaves ? launch_shrink_nb<DT, kDecodeWaves, DIRECT>(NB, grid, st, a)
+                              : launch_shrink_nb<DT, kFwdWaves, DIRECT>(NB, grid, st, a);
   return a.w_kn ? launch_shrink_block<DT, DIRECT, true>(NB, grid, st, a)
                 : launch_shrink_block<DT, DIRECT, false>(NB, grid, st, a);
 }
 
 // all projections of one launch share NB / U / MT / NW (same rank, same T)
-int launch_shrink(int dtype, bool row_major, const ShrinkCfg& c, int S, int groups, hipStream_t st,
+int launch_shrink(int dtype, const ShrinkCfg& c, int S, int groups, hipStream_t st,
                   ShrinkArgs& a) {
-  const int MT = row_major ? 1 : c.MT;
+  const int MT = c.MT;
   a.items.interleave = 1;
   const int units = tile_units_max(a.T, S, groups, MT);
   const long items = (long)units * a.items.row_start[a.items.nproj];
@@ -232,10 +230,10 @@ int launch_shrink(int dtype, bool row_major, const ShrinkCfg& c, int S, int grou
   const dim3 grid = item_grid(a.items, items);
   const bool f16 = dtype == SMLM_DTYPE_F16;
   if (a.items.units_max)
-    return f16 ? launch_shrink_dt<SMLM_DTYPE_F16, true>(row_major, c.NB, MT, c.NW, grid, st, a)
-               : launch_shrink_dt<SMLM_DTYPE_BF16, true>(row_major, c.NB, MT, c.NW, grid, st, a);
-  return f16 ? launch_shrink_dt<SMLM_DTYPE_F16, false>(row_major, c.NB, MT, c.NW, grid, st, a)
-             : launch_shrink_dt<SMLM_DTYPE_BF16, false>(row_major, c.NB, MT, c.NW, grid, st, a);
+    return f16 ? launch_shrink_dt<SMLM_DTYPE_F16, true>(c.NB, MT, c.NW, grid, st, a)
+               : launch_shrink_dt<SMLM_DTYPE_BF16, true>(c.NB, MT, c.NW, grid, st, a);
+  return f16 ? launch_shrink_dt<SMLM_DTYPE_F16, false>(c.NB, MT, c.NW, grid, st, a)
+             : launch_shrink_dt<SMLM_DTYPE_BF16, false>(c.NB, MT, c.NW, grid, st, a);
 }
 
 template <int DT, int THREADS, bool PAIRS>
@@ -345,34 +343,27 @@ template <int DT, int NQ, bool DIRECT>
 int launch_expand_wave(int KS, bool vfold, dim3 grid, hipStream_t st, const ExpandArgs& a) {
   const dim3 block(kFwdThreads);
   if (vfold) {
-    if (KS == 1) return launch(expand_wave_kernel<DT, NQ, 1, false, DIRECT, true>, grid, block, st, a);
-    if (KS == 2) return launch(expand_wave_kernel<DT, NQ, 2, false, DIRECT, true>, grid, block, st, a);
-    return launch(expand_wave_kernel<DT, NQ, 0, false, DIRECT, true>, grid, block, st, a);
+    if (KS == 1) return launch(expand_wave_kernel<DT, NQ, 1, DIRECT, true>, grid, block, st, a);
+    if (KS == 2) return launch(expand_wave_kernel<DT, NQ, 2, DIRECT, true>, grid, block, st, a);
+    return launch(expand_wave_kernel<DT, NQ, 0, DIRECT, true>, grid, block, st, a);
   }
-  if (KS == 1) return launch(expand_wave_kernel<DT, NQ, 1, false, DIRECT, false>, grid, block, st, a);
-  if (KS == 2) return launch(expand_wave_kernel<DT, NQ, 2, false, DIRECT, false>, grid, block, st, a);
-  return launch(expand_wave_kernel<DT, NQ, 0, false, DIRECT, false>, grid, block, st, a);
+  if (KS == 1) return launch(expand_wave_kernel<DT, NQ, 1, DIRECT, false>, grid, block, st, a);
+  if (KS == 2) return launch(expand_wave_kernel<DT, NQ, 2, DIRECT, false>, grid, block, st, a);
+  return launch(expand_wave_kernel<DT, NQ, 0, DIRECT, false>, grid, block, st, a);
 }
 
 template <int DT, bool DIRECT>
-int launch_expand_dt(bool row_major, bool block, int nq, int KS, dim3 grid, hipStream_t st,
+int launch_expand_dt(bool block, int nq, int KS, dim3 grid, hipStream_t st,
                      const ExpandArgs& a) {
-  if (row_major)
-    return launch(expand_wave_kernel<DT, 2, 0, true, DIRECT, false>, grid, dim3(kFwdThreads), st, a);
   if (a.drop.seg_p) {  // the backward's dX with the dropout of x undone: no fold
-    const dim3 bl(kFwdThreads);
-    if (block)  // launch_expand admits only [k][n] weights here
-      return KS == 1 ? launch(expand_block_kernel<DT, 4, 1, DIRECT, true, true>, grid, bl, st, a)
-                     : launch(expand_block_kernel<DT, 4, 2, DIRECT, true, true>, grid, bl, st, a);
-    if (KS == 0)  // ranks above 64: the general loop over k
-      return nq == 4 ? launch(expand_wave_kernel<DT, 4, 0, false, DIRECT, false, true>, grid, bl, st, a)
-                     : launch(expand_wave_kernel<DT, 2, 0, false, DIRECT, false, true>, grid, bl, st, a);
-    if (nq == 4)
-      return KS == 1 ? launch(expand_wave_kernel<DT, 4, 1, false, DIRECT, false, true>, grid, bl, st, a)
-                     : launch(expand_wave_kernel<DT, 4, 2, false, DIRECT, false, true>, grid, bl, st, a);
-    return KS == 1 ? launch(expand_wave_kernel<DT, 2, 1, false, DIRECT, false, true>, grid, bl, st, a)
-                   : launch(expand_wave_kernel<DT, 2, 2, false, DIRECT, false, true>, grid, bl, st, a);
+    const dim3 bl(kFwdThreads);  // (launch_expand admits only tile blocks with [k][n] weights here)
+    if (KS == 4) return launch(expand_block_kernel<DT, 4, 4, DIRECT, true, true>, grid, bl, st, a);
+    return KS == 1 ? launch(expand_block_kernel<DT, 4, 1, DIRECT, true, true>, grid, bl, st, a)
+                   : launch(expand_block_kernel<DT, 4, 2, DIRECT, true, true>, grid, bl, st, a);
   }
+  if (block && KS == 4)
+    return a.w_kn ? launch(expand_block_kernel<DT, 4, 4, DIRECT, true>, grid, dim3(kFwdThreads), st, a)
+                  : launch(expand_block_kernel<DT, 4, 4, DIRECT, false>, grid, dim3(kFwdThreads), st, a);
   if (block && a.w_kn)
     return KS == 1 ? launch(expand_block_kernel<DT, 4, 1, DIRECT, true>, grid, dim3(kFwdThreads), st, a)
                    : launch(expand_block_kernel<DT, 4, 2, DIRECT, true>, grid, dim3(kFwdThreads), st, a);
@@ -388,12 +379,13 @@ int launch_expand_dt(bool row_major, bool block, int nq, int KS, dim3 grid, hipS
 }
 
 // all projections of one launch share the rank (d_in); d_out may differ
-int launch_expand(int dtype, bool row_major, int nq, int MT, int S, int groups, int nproj, int max_d_in,
+int launch_expand(int dtype, int nq, int MT, int S, int groups, int nproj, int max_d_in,
                   hipStream_t st, ExpandArgs& a) {
-  const int KS = max_d_in <= 32 ? 1 : (max_d_in <= 64 ? 2 : 0);
-  const bool block = !row_major && MT > 1 && KS > 0;  // tile blocks with the weights staged in LDS
-  if (a.drop.seg_p && (row_major || a.p[0].vsplit > 0 || (block && !a.w_kn))) return SMLM_ERR_ARG;
-  if (row_major) nq = 2;
+  const bool block = MT > 1;  // tile blocks with the weights staged in LDS
+  // (ranks above 64: 128 of k at a time on tile blocks, the general loop over k on single tiles)
+  const int KS = max_d_in <= 32 ? 1 : (max_d_in <= 64 ? 2 : (block ? 4 : 0));
+  if (a.drop.seg_p && !(block && a.w_kn)) return SMLM_ERR_ARG;
+  if (a.w_kn && !block) return SMLM_ERR_ARG;  // (no caller: the single-tile kernel reads [n][k] weights)
   // Tile blocks: 128 columns a workgroup, or 256 where measured better (rank 64, 8192 rows: 5-13 % at every
   // width; a row stride that is a multiple of 4 KiB, e.g. h_out = 14336, from 4096 rows on at every rank:
   // the 64 rows of a tile block then meet in few HBM channels and pieces of 512 bytes spread them over
@@ -405,7 +397,7 @@ int launch_expand(int dtype, bool row_major, int nq, int MT, int S, int groups, 
     const bool aligned = (wide * 2) % 4096 == 0;
     const bool wider = !a.w_kn && !a.drop.seg_p &&
                        ((KS == 2 && a.T >= 8192) || (aligned && wide >= 8192 && a.T >= 4096));
-    nq = wider ? 8 : 4;
+    nq = wider && KS <= 2 ? 8 : 4;
   }
   const int chunk = block ? 32 * nq : kFwdWaves * 32 * nq;  // columns per workgroup
   a.items.nproj = nproj;
@@ -433,10 +425,10 @@ int launch_expand(int dtype, bool row_major, int nq, int MT, int S, int groups, 
   const dim3 grid = item_grid(a.items, items);
   const bool f16 = dtype == SMLM_DTYPE_F16;
   if (a.items.units_max)
-    return f16 ? launch_expand_dt<SMLM_DTYPE_F16, true>(row_major, block, nq, KS, grid, st, a)
-               : launch_expand_dt<SMLM_DTYPE_BF16, true>(row_major, block, nq, KS, grid, st, a);
-  return f16 ? launch_expand_dt<SMLM_DTYPE_F16, false>(row_major, block, nq, KS, grid, st, a)
-             : launch_expand_dt<SMLM_DTYPE_BF16, false>(row_major, block, nq, KS, grid, st, a);
+    return f16 ? launch_expand_dt<SMLM_DTYPE_F16, true>(block, nq, KS, grid, st, a)
+               : launch_expand_dt<SMLM_DTYPE_BF16, true>(block, nq, KS, grid, st, a);
+  return f16 ? launch_expand_dt<SMLM_DTYPE_F16, false>(block, nq, KS, grid, st, a)
+             : launch_expand_dt<SMLM_DTYPE_BF16, false>(block, nq, KS, grid, st, a);
 }
 
 int check_common(int T, int S, int dtype) {
@@ -475,14 +467,14 @@ struct SideOut {
   ZeroSpans zero;  // memory the fold's launch is to clear as well (n = 0: none)
 };
 
-int run_shrink(int dtype, bool row_major, const PlanView& pv, int T, int S, int groups, int nproj,
+int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int nproj,
                const void* const* x, const void* const* const* w_ptrs, float* const* partial,
                void* const* out, const int* d_in, int d_out, const int* ldw, float beta,
                const float* seg_scale, int mt, hipStream_t st, bool fold = true, bool w_kn = false,
                const DropArgs* drop = nullptr, const int32_t* w_rank = nullptr, int packed = 0,
                const PlanSortArgs* build = nullptr, bool solo = false, const SideOut* side = nullptr,
                bool* side_done = nullptr) {
-  if (drop && drop->seg_p && (row_major || w_kn)) return SMLM_ERR_ARG;
+  if (drop && drop->seg_p && w_kn) return SMLM_ERR_ARG;
   if (side_done) *side_done = false;
   ShrinkArgs a{};
   if (drop) a.drop = *drop;
@@ -499,7 +491,7 @@ int run_shrink(int dtype, bool row_major, const PlanView& pv, int T, int S, int 
   bool need_reduce = false, all_reduce = true;
   ShrinkCfg c0{};
   size_t bits_off = 0;
-  const int nw = row_major ? kFwdWaves : shrink_waves(mt, nproj, d_in, d_out);
+  const int nw = shrink_waves(mt, nproj, d_in, d_out);
   for (int i = 0; i < nproj; ++i) {
     const ShrinkCfg c = shrink_cfg(T, d_in[i], d_out, nw, solo, mt);
     if (i == 0) c0 = c;
@@ -534,7 +526,7 @@ int run_shrink(int dtype, bool row_major, const PlanView& pv, int T, int S, int 
   // `build`: the plan does not exist yet -- the decode shrink whose workgroups find their
   // own tile, with one more workgroup that builds the plan (the caller has checked the limits)
   int rc = build ? launch_shrink_self_planned(dtype, c0, S, groups, *build, st, a)
-                 : launch_shrink(dtype, row_major, c0, S, groups, st, a);
+                 : launch_shrink(dtype, c0, S, groups, st, a);
   if (rc || !need_reduce || !fold) return rc;
   ra.plan = a.plan;
   ra.seg_scale = seg_scale;
@@ -574,7 +566,7 @@ int launch_wgrad(int nbj, bool split, dim3 grid, hipStream_t st, const WgradArgs
 }
 
 struct BwdProjLayout {
-  size_t at, bt, at_ptrs, bt_ptrs, partial, dv16, v16, pt_a, pt_b, bits;
+  size_t partial, dv16, v16, pt_a, pt_b, bits;
 };
 struct BwdLayout {
   BwdProjLayout p[kMaxProj];
@@ -596,10 +588,6 @@ BwdLayout bwd_layout(int n_proj, int n_rows, int P, int NA, const int* h_in, con
     BwdProjLayout& Q = L.p[i];
     const int ks_dv = fwd_ksplit_bound(n_rows, h_out[i], r), ks_v = fwd_ksplit_bound(n_rows, h_in[i], r);
     const int ks = ks_dv > ks_v ? ks_dv : ks_v;
-    Q.at = take((size_t)NA * h_in[i] * r * 2);
-    Q.bt = take((size_t)NA * h_out[i] * r * 2);
-    Q.at_ptrs = take((size_t)NA * 8);
-    Q.bt_ptrs = take((size_t)NA * 8);
     Q.partial = take((size_t)ks * n_rows * r * 4);
     Q.dv16 = take((size_t)n_rows * r * 2);
     Q.v16 = take((size_t)n_rows * r * 2);
@@ -735,20 +723,19 @@ SMLM_API int smlm_gemm_planned(void* y, const void* x, const void* const* w_ptrs
     P.w_ptrs = w_ptrs;
     P.d_in = d_in; P.d_out = d_out; P.ldw = w_ld;
     // Row-major weights (element (k, n) at w[k * w_ld + n]) are the [k][n] layout the tile-block kernels read
-    // as it lies (as the backward's dX = dV A does): up to a contraction of 64 they run at every size, as
-    // they do for the backward; longer ones keep the one-tile kernel's strided reads.
-    if (w_row_major && d_in <= 64) {
+    // as it lies (as the backward's dX = dV A does): they run at every size, as they do for the backward.
+    if (w_row_major) {
       a.w_kn = 1;
-      return launch_expand(dtype, false, expand_nq(T, d_out), kBlkTiles, S, n_weights, 1, d_in, st, a);
+      return launch_expand(dtype, expand_nq(T, d_out), kBlkTiles, S, n_weights, 1, d_in, st, a);
     }
-    return launch_expand(dtype, w_row_major != 0, expand_nq(T, d_out), tiles_per_wave(T, d_in), S, n_weights,
+    return launch_expand(dtype, expand_nq(T, d_out), tiles_per_wave(T, d_in), S, n_weights,
                          1, d_in, st, a);
   }
   float* partial = reinterpret_cast<float*>(workspace);
   if (w_row_major)  // the tile-block shrink stages [k][n] weights as they lie (as the backward's dV = dY B does)
-    return run_shrink(dtype, false, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
+    return run_shrink(dtype, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
                       seg_scale, kBlkTiles, st, true, true);
-  return run_shrink(dtype, false, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in,
+  return run_shrink(dtype, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in,
                     d_out, &w_ld, beta, seg_scale, tiles_per_wave(T, d_out), st);
 }
 
@@ -796,7 +783,7 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
     if (!aligned16(y) || !aligned16(x)) return SMLM_ERR_ALIGN;
     const PlanSortArgs build{pv, seg_indptr, w_ptrs, SMLM_KEY_PTR2, S, next_pow2(S), w_ptrs};
     float* partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + plan_bytes);
-    return run_shrink(dtype, false, pv, T, S, S, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
+    return run_shrink(dtype, pv, T, S, S, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
                       seg_scale, mt, st, true, false, nullptr, nullptr, 0, &build);
   }
   rc = plan_build_impl(pv, seg_indptr, w_ptrs, SMLM_KEY_PTR, S, st);
@@ -947,7 +934,7 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
                                                    : (expand_folds && (S <= kSelfPlanThreads || even_splits)));
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, build_kind, S, st, build_k2))) return rc;
   if (stages & SMLM_STAGE_SHRINK) {
-    rc = run_shrink(dtype, false, pv, T, S, n_weights, n_proj, x, a_ptrs, partial, v16, h_in, r, h_in,
+    rc = run_shrink(dtype, pv, T, S, n_weights, n_proj, x, a_ptrs, partial, v16, h_in, r, h_in,
                     0.0f, nullptr, mt, st, !expand_folds, false, &drop, w_rank, packed,
                     self_planned ? &build : nullptr);
     if (rc) return rc;
@@ -978,7 +965,7 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
     }
   }
   if (n_exp == 0) return SMLM_OK;
-  return launch_expand(dtype, false, expand_nq(T, exp_h_out), mt, S, n_weights, n_exp, r, st, ea);
+  return launch_expand(dtype, expand_nq(T, exp_h_out), mt, S, n_weights, n_exp, r, st, ea);
 }
 
 SMLM_API int smlm_lora_fwd_workspace_size(int T, int S, int h_in, int h_out, int r, size_t* bytes) {
@@ -1033,10 +1020,8 @@ SMLM_API int smlm_lora_bwd_ex(void* dx, void* const* da_ptrs, void* const* db_pt
 
 // every projection's dV product is folded from k-split partials: the fold then writes what the weight gradients read
 static bool bwd_all_folded(int n_proj, int n_rows, const int* h_out, int r) {
-  const int mt = bwd_tiles_per_wave(n_rows, r);
-  const int nw = shrink_waves(mt, n_proj, h_out, r);
   for (int i = 0; i < n_proj; ++i)
-    if (shrink_cfg(n_rows, h_out[i], r, nw, true, mt).ksplit <= 1) return false;
+    if (shrink_cfg(n_rows, h_out[i], r, kFwdWaves, true, kBlkTiles).ksplit <= 1) return false;
   return true;
 }
 
@@ -1090,35 +1075,18 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   if ((build_s != nullptr) != (build_k != nullptr)) return SMLM_ERR_ARG;
   if (build_s && !(stages & SMLM_BWD_PRODUCTS)) return SMLM_ERR_ARG;  // the plan is built with the first stage
   PlanSortArgs build{pv, build_s, build_k, SMLM_KEY_I32, P, next_pow2(P)};
-  const int mt = bwd_tiles_per_wave(n_rows, r);
+  constexpr int mt = kBlkTiles;
   bool even_dv = true;  // (k slices in pairs beyond 256 partitions)
   for (int i = 0; i < n_proj; ++i) even_dv = even_dv && shrink_cfg(n_rows, h_out[i], r, kFwdWaves, true, mt).ksplit % 2 == 0;
-  const bool self_planned = build_s && have_v && !drop.seg_p && mt > 1 && r <= 64 &&
+  const bool self_planned = build_s && have_v && !drop.seg_p &&
                             self_planned_ok(n_rows, P, NA, pv.nt_max, mt) && (P <= kFwdThreads || even_dv);
   const bool products = (stages & SMLM_BWD_PRODUCTS) != 0;
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, SMLM_KEY_I32, P, st))) return rc;
 
   // 1. The backward multiplies by B and A where the forward multiplies by A^T and B^T.  The
-  // tile-block kernels read the weights as they lie in memory; ranks above 64 take the one-tile
-  // expand kernel's general k loop, which reads [n][k] weights: transposed copies At [h_in, r],
-  // Bt [r, h_out] made here.
-  // (The row-major layout needs no copies at any rank: dV = dY B^T and dX = dV A^T read B [r, h_out] and
-  // A [h_in, r] the way the forward reads A [r, h_in] and B [h_out, r], and v = x A reads A as [k][n].)
-  const bool in_place = rm || (mt > 1 && r <= 64);
-  if (!in_place && products) {
-    for (int i = 0; i < n_proj; ++i) {
-      TransposeArgs ta{};
-      ta.set[0] = TransposeSet{a_ptrs[i], reinterpret_cast<uint16_t*>(ws + L.p[i].at),
-                               reinterpret_cast<const void**>(ws + L.p[i].at_ptrs), (long)h_in[i] * r, r, h_in[i]};
-      ta.set[1] = TransposeSet{b_ptrs[i], reinterpret_cast<uint16_t*>(ws + L.p[i].bt),
-                               reinterpret_cast<const void**>(ws + L.p[i].bt_ptrs), (long)h_out[i] * r, h_out[i], r};
-      ta.NA = NA;
-      ta.w_rank = w_rank;
-      ta.packed = packed;
-      const int gx = ceil_div(h_in[i] > h_out[i] ? h_in[i] : h_out[i], 64), gy = ceil_div(r, 64);
-      if ((rc = launch(transpose_kernel, dim3(gx, gy, 2 * NA), dim3(256), st, ta))) return rc;
-    }
-  }
+  // tile-block kernels read the weights as they lie in memory: B [h_out, r] and A [r, h_in] as [k][n].
+  // (In the row-major layout dV = dY B^T and dX = dV A^T read B [r, h_out] and A [h_in, r] the way the
+  // forward reads A [r, h_in] and B [h_out, r], and v = x A reads A as [k][n].)
 
   // The keep bits of x's dropout mask (projection i: the stream offset + i; the caller's bits of the
   // projections lie end to end): the forward's when the caller kept them, else made here (same stream,
@@ -1161,21 +1129,17 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
     if (rm) {  // A [h_in, r] is [k][n]: the tile-block shrink at every size
       int a_ld[kMaxProj];
       for (int i = 0; i < n_proj; ++i) a_ld[i] = r;
-      if ((rc = run_shrink(dtype, false, pv, n_rows, P, NA, n_proj, x, a_ptrs, partial, v16, h_in, r, a_ld, 0.0f,
+      if ((rc = run_shrink(dtype, pv, n_rows, P, NA, n_proj, x, a_ptrs, partial, v16, h_in, r, a_ld, 0.0f,
                            nullptr, kBlkTiles, st, true, true, nullptr, w_rank, 0, nullptr, true)))
         return rc;
-    } else if ((rc = run_shrink(dtype, false, pv, n_rows, P, NA, n_proj, x, a_ptrs, partial, v16, h_in, r, h_in,
+    } else if ((rc = run_shrink(dtype, pv, n_rows, P, NA, n_proj, x, a_ptrs, partial, v16, h_in, r, h_in,
                                 0.0f, nullptr, mt, st, true, false, &vdrop, w_rank, 0, nullptr, true)))  // v of the dropped x, as the forward made it
       return rc;
   }
 
   // 3. dV = round16(dY B)
-  const void* const* btp[kMaxProj];
   int b_ld[kMaxProj];
-  for (int i = 0; i < n_proj; ++i) {
-    btp[i] = in_place ? b_ptrs[i] : reinterpret_cast<const void* const*>(ws + L.p[i].bt_ptrs);
-    b_ld[i] = (in_place && !rm) ? r : h_out[i];  // B [h_out, r] read as [k][n]; B [r, h_out] and the copies as [n][k]
-  }
+  for (int i = 0; i < n_proj; ++i) b_ld[i] = rm ? h_out[i] : r;  // B [h_out, r] read as [k][n]; B [r, h_out] as [n][k]
   // The weight gradients read s*dV and s*v by tile slot, transposed.  The fold of dV leaves them behind when there is
   // one for every projection (cheaper there than among dX's stores: cfg4-like batch dV 12.5 -> 13.5, dX 10.8 -> 8.2 us;
   // ragged 32-row partitions over six projections dV 84 -> 91, dX 90 -> 74 us); else dX's launch writes them.
@@ -1208,10 +1172,10 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
            (rc = launch(zero_spans_kernel, dim3((unsigned)tail.first[tail.n]), dim3(256), st, tail)))
     return rc;
   bool side_done = false;
-  if (products && (rc = run_shrink(dtype, false, pv, n_rows, P, NA, n_proj, dy, btp, partial, dv16, h_out, r, b_ld,
-                                   0.0f, nullptr, mt, st, true, in_place && !rm, nullptr, w_rank, in_place ? packed : 0,
+  if (products && (rc = run_shrink(dtype, pv, n_rows, P, NA, n_proj, dy, b_ptrs, partial, dv16, h_out, r, b_ld,
+                                   0.0f, nullptr, mt, st, true, !rm, nullptr, w_rank, packed,
                                    self_planned ? &build : nullptr, true, side_in_fold ? &side : nullptr, &side_done)))
-    return rc;  // (B in place is read at its stored rank; the transposed copies keep the full-rank strides)
+    return rc;
   if (products && side_done != side_in_fold) return SMLM_ERR_ARG;  // (cannot happen: both follow shrink_cfg)
 
   // 4. dX = s dV A, and the slot-ordered transposed s*dV, s*v for step 5
@@ -1226,8 +1190,8 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
     ExpandProj& E = ea.p[i];
     E.y = reinterpret_cast<uint16_t*>(dx[i]);
     E.v = reinterpret_cast<const uint16_t*>(dv16[i]);
-    E.w_ptrs = in_place ? a_ptrs[i] : reinterpret_cast<const void* const*>(ws + L.p[i].at_ptrs);
-    E.d_in = r; E.d_out = h_in[i]; E.ldw = (in_place && !rm) ? h_in[i] : r;  // A [r, h_in] as [k][n]; A [h_in, r] as [n][k]
+    E.w_ptrs = a_ptrs[i];
+    E.d_in = r; E.d_out = h_in[i]; E.ldw = rm ? r : h_in[i];  // A [r, h_in] as [k][n]; A [h_in, r] as [n][k]
     E.pt_a = side_in_fold ? nullptr : side.pt_a[i];
     E.pt_b = side_in_fold ? nullptr : side.pt_b[i];
     E.v2 = side.v2[i];
@@ -1235,9 +1199,9 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
     E.drop_pitch = h_in[i] / 8;
     if (h_in[i] > widest) widest = h_in[i];
   }
-  ea.w_kn = (in_place && !rm) ? 1 : 0;
+  ea.w_kn = rm ? 0 : 1;
   ea.drop = drop;  // dX is the gradient with respect to x before its dropout
-  if ((stages & SMLM_BWD_DX) && (rc = launch_expand(dtype, false, expand_nq(n_rows, widest), mt, P, NA, n_proj, r, st, ea)))
+  if ((stages & SMLM_BWD_DX) && (rc = launch_expand(dtype, expand_nq(n_rows, widest), mt, P, NA, n_proj, r, st, ea)))
     return rc;
   if (!(stages & SMLM_BWD_WGRAD)) return SMLM_OK;
 

@@ -1,4 +1,4 @@
-// Backward-only kernels: weight transposes and the per-adapter token
+// Backward-only kernel: the per-adapter token
 // reductions dA_a = sum_t dV[t,:]^T x[t,:], dB_a = sum_t dY[t,:]^T v[t,:].
 //
 // The reference computes these with one torch matmul per train partition
@@ -9,74 +9,6 @@
 #include "smlm_common.hpp"
 
 namespace smlm {
-
-struct TransposeSet {
-  const void* const* src_ptrs;  // [NA] matrices [rows, cols] row-major
-  uint16_t* dst_base;           // NA matrices [cols, rows], `stride` elements apart
-  const void** dst_ptrs;        // [NA] receives the address of each transposed matrix
-  long stride;
-  int rows, cols;
-};
-
-struct TransposeArgs {
-  TransposeSet set[2];  // A [r, h_in] -> At [h_in, r] and B [h_out, r] -> Bt [r, h_out]
-  int NA;
-  const int32_t* w_rank;  // optional [NA] with packed: the sources are stored at their true rank (rounded up
-  int packed;             //   to 8), A_a [r_a, h_in], B_a [h_out, r_a]; the copies keep the full-rank strides
-};
-
-constexpr int kTrPitch = 80;  // LDS row pitch in 16-bit elements (40 banks: see kWgPitch)
-
-// 64x64 tiles through LDS, 16-byte global accesses on both sides: rows of the
-// source tile are written to LDS as they are and read back down the columns
-// with the transposing LDS read.  grid (tiles along the hidden dimension, tiles
-// along the rank, 2*NA), block 256: x walks the columns of A and the rows of B.
-// Rows and columns are multiples of 8.
-__global__ __launch_bounds__(256) void transpose_kernel(TransposeArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t t[64 * kTrPitch];
-  const int which = blockIdx.z / a.NA, ad = blockIdx.z - which * a.NA;
-  TransposeSet S = a.set[which];
-  if (a.w_rank && a.packed) {  // the rank is A's row count and B's column count
-    const int full = which == 0 ? S.rows : S.cols;
-    const int r8 = (uload(a.w_rank, ad) + 7) & ~7;
-    const int ra = r8 < full ? r8 : full;
-    if (which == 0) S.rows = ra; else S.cols = ra;
-  }
-  const int c0 = (which == 0 ? blockIdx.x : blockIdx.y) * 64;
-  const int r0 = (which == 0 ? blockIdx.y : blockIdx.x) * 64;
-  if (c0 >= S.cols || r0 >= S.rows) return;  // uniform over the workgroup
-  const uint16_t* src = reinterpret_cast<const uint16_t*>(S.src_ptrs[ad]);
-  uint16_t* dst = S.dst_base + (long)ad * S.stride;
-  const int dst_pitch = a.set[which].rows;  // the copy is [cols, rows] of the full-rank shape
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) S.dst_ptrs[ad] = dst;
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  // in: lane -> (row = tid / 8 (+32), 8 columns at (tid % 8) * 8)
-  const int ir = threadIdx.x >> 3, ic = (threadIdx.x & 7) * 8;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int r = r0 + ir + 32 * h, c = c0 + ic;
-    const u32x4 v = (r < S.rows && c < S.cols) ? ldg16(src + (long)r * S.cols + c) : zero;
-    *reinterpret_cast<u32x4*>(&t[(ir + 32 * h) * kTrPitch + ic]) = v;
-  }
-  __syncthreads();
-  // out: thread -> output row (source column) oc = tid / 8 (+32), 8 source rows at 8 * (tid % 8).
-  // Within 16 lanes (two output rows... ) the transposing read wants lane i to name source row
-  // (i / 4) and four columns at 4 * (i % 4); lane 4a+b then holds column 4*... of rows a, a+4, ...
-  // so a wave covers 16 source columns x 16 source rows per read: organise the 256 threads as
-  // (column block cb = tid / 64 -> 16 columns, wave-lane l): g = l / 16 picks 16 of the 64 rows.
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int g = lane >> 4, i = lane & 15;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    // rows 16g + 8h + {0..7} of the tile: two reads of four rows each; lane i = 4a+b names row
-    // (base + i/4), columns 16*wave + 4*(i%4) .. +3 and receives column 16*wave + i, rows base + {0..3}
-    const int rb = 16 * g + 8 * h;
-    const uint16_t* p0 = &t[(rb + (i >> 2)) * kTrPitch + 16 * wave + 4 * (i & 3)];
-    const u32x2 q0 = lds_read_tr16(p0), q1 = lds_read_tr16(p0 + 4 * kTrPitch);
-    const int oc = c0 + 16 * wave + i, orow = r0 + rb;
-    if (oc < S.cols && orow < S.rows) stg16(dst + (long)oc * dst_pitch + orow, u32x4{q0[0], q0[1], q1[0], q1[1]});
-  }
-}
 
 constexpr int kWgMaxProj = 8;  // projections one weight-gradient launch can serve (as the forward's launches)
 

@@ -153,20 +153,6 @@ __device__ __forceinline__ const uint16_t* uload_ptr(const void* const* tab, int
   return reinterpret_cast<const uint16_t*>(v);
 }
 
-// Eight 16-bit elements with a stride (the slow gather used for the weight
-// layout the reference never passes).
-__device__ __forceinline__ u32x4 ldg_strided8(const uint16_t* p, long stride) {
-  const SMLM_GLOBAL uint16_t* q = (const SMLM_GLOBAL uint16_t*)p;
-  u32x4 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t a = q[(2 * i) * stride];
-    uint32_t b = q[(2 * i + 1) * stride];
-    r[i] = a | (b << 16);
-  }
-  return r;
-}
-
 // Views into a plan buffer (all int32).  Sizes are functions of (T, S) only.
 struct PlanView {
   int32_t* hdr;         // [16]: 0 n_tiles, 1 n_groups, 2 rows covered, 3 key kind used, 4 n_blocks,

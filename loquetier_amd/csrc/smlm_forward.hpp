@@ -166,17 +166,6 @@ __device__ __forceinline__ void pick_tiles(const TileArgs& p, int tb, int* t0, i
   }
 }
 
-// eight consecutive-k elements of weight column n (zeros when !ok)
-template <bool ROWMAJOR>
-__device__ __forceinline__ u32x4 load_w8(const uint16_t* W, int n, int k, int ldw, bool ok,
-                                         const uint16_t* zeros) {
-  if (ROWMAJOR) {
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-    return ok ? ldg_strided8(W + (long)k * ldw + n, ldw) : zero;
-  }
-  return ldg16_or(W + (long)n * ldw + k, ok, zeros);
-}
-
 // out = beta*old + scale*acc for four consecutive columns of one row
 template <int DT>
 __device__ __forceinline__ void store4(uint16_t* dst, f32x4 a, float scale, float beta) {
@@ -219,7 +208,7 @@ struct ShrinkArgs {
 // ranges; their accumulators are summed through LDS in wave order and written
 // either as an fp32 partial (k split over workgroups, or a consumer that folds)
 // or as the final 16-bit value.  NW = 8 is for decode batches: few tiles, long k.
-template <int DT, int NB, int U, int NW, bool ROWMAJOR, bool DIRECT, bool DROP = false>
+template <int DT, int NB, int U, int NW, bool DIRECT, bool DROP = false>
 __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
   __shared__ f32x4 red[NW][NB][kWaveSize];
   const int units = DIRECT ? 0 : tile_units<1>(a.plan, 0);
@@ -261,7 +250,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
           const int n = n0 + 16 * nb + c;
-          wf[nb][u] = load_w8<ROWMAJOR>(W, n, kk, P.ldw, kin && n < nlim, zeros);
+          wf[nb][u] = ldg16_or(W + (long)n * P.ldw + kk, kin && n < nlim, zeros);
         }
       }
     };
@@ -595,11 +584,11 @@ struct ExpandProj {
   uint16_t* y;                // [T, d_out]
   const uint16_t* v;          // [T, d_in]
   const void* const* w_ptrs;  // indexed by the plan's tile_wid
-  uint16_t* v_out;            // optional [T, d_in]: copy of v, by row
+  uint16_t* v_out;            // wave kernels, optional [T, d_in]: copy of v, by row
   const float* vpart;         // VFOLD wave kernels: v arrives as vsplit (1..4) fp32 k-split partials
   int vsplit;                 //   [vsplit, T, d_in], summed here in split order and rounded
   int d_in, d_out, ldw;
-  uint16_t* pt_a;             // optional [d_in, nt_max*16]: scale*v by tile slot, transposed
+  uint16_t* pt_a;             // block kernels, optional [d_in, nt_max*16]: scale*v by tile slot, transposed
   uint16_t* pt_b;             // optional: same treatment of v2 (a second [T, d_in] matrix)
   const uint16_t* v2;
   const uint8_t* drop_bits;   // DROP kernels: keep bits of this projection's mask, [rows, drop_pitch]
@@ -620,26 +609,22 @@ struct ExpandArgs {
                              //   (probabilities and row count; the keep bits are each projection's own)
 };
 
-// by-products one wave per tile writes while it holds the token fragment: the
-// rounded v by row, and scale*v / scale*v2 by tile slot, transposed ([k][slot]),
+// by-products one wave per tile writes: scale*v / scale*v2 by tile slot, transposed ([k][slot]),
 // which the weight-gradient kernel reads with the token index innermost
 template <int DT>
 __device__ __forceinline__ void write_side(const ExpandArgs& a, const ExpandProj& P, int slot, int row,
                                            int kk, u32x4 vf, float scale) {
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  if (P.v_out && row >= 0) stg16(P.v_out + (long)row * P.d_in + kk, vf);
-  if (P.pt_a) {
-    const long pitch = (long)a.nt_max * kTileRows;
-    u32x4 v2f = zero;
-    if (P.pt_b && row >= 0) v2f = ldg16(P.v2 + (long)row * P.d_in + kk);
+  const long pitch = (long)a.nt_max * kTileRows;
+  u32x4 v2f = zero;
+  if (P.pt_b && row >= 0) v2f = ldg16(P.v2 + (long)row * P.d_in + kk);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      P.pt_a[(kk + 2 * e) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(vf[e]));
-      P.pt_a[(kk + 2 * e + 1) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(vf[e]));
-      if (P.pt_b) {
-        P.pt_b[(kk + 2 * e) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(v2f[e]));
-        P.pt_b[(kk + 2 * e + 1) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(v2f[e]));
-      }
+  for (int e = 0; e < 4; ++e) {
+    P.pt_a[(kk + 2 * e) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(vf[e]));
+    P.pt_a[(kk + 2 * e + 1) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(vf[e]));
+    if (P.pt_b) {
+      P.pt_b[(kk + 2 * e) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(v2f[e]));
+      P.pt_b[(kk + 2 * e + 1) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(v2f[e]));
     }
   }
 }
@@ -746,7 +731,7 @@ __device__ __forceinline__ void store_y_lines(float* stg, const f32x4 (&acc)[NQ]
 // short: KS > 0 unrolls KS 32-wide k steps, KS == 0 is the general loop over k.
 // MFMA row m of column block (q,p) is output column 32q + 8(m/4) + 4p + m%4, so
 // that a lane's eight accumulators for one q are eight consecutive columns.
-template <int DT, int NQ, int KS, bool ROWMAJOR, bool DIRECT, bool VFOLD, bool DROP = false>
+template <int DT, int NQ, int KS, bool DIRECT, bool VFOLD>
 __global__ __launch_bounds__(kFwdThreads) void expand_wave_kernel(ExpandArgs a) {
   __shared__ __attribute__((aligned(16))) float olds[kFwdWaves][kTileRows * kOPitch];
   const int units = DIRECT ? 0 : tile_units<1>(a.plan, 0);
@@ -767,11 +752,10 @@ __global__ __launch_bounds__(kFwdThreads) void expand_wave_kernel(ExpandArgs a) 
     if (!wid_ok(a.plan, wid)) continue;  // past the last tile (direct mode), or no such adapter
     const uint16_t* W = uload_ptr(P.w_ptrs, wid);
     const int klim = rank_limit(a.plan, wid, P.d_in);  // k at or past it: zero padding of v and the weights
-    const int ldw = ROWMAJOR ? P.ldw : rank_ld(a.plan, P.ldw, klim);
+    const int ldw = rank_ld(a.plan, P.ldw, klim);
     const int slot = tile * kTileRows + c;
     const int row = a.plan.tile_row[slot];
-    const int rseg = a.seg_scale ? a.plan.tile_rseg[slot] : -1;  // -1 on empty slots too
-    const bool side = (yy == 0 && wave == 0);  // the one wave per tile that writes by-products
+    const bool side = (yy == 0 && wave == 0);  // the one wave per tile that writes the caller's copy of v
     const uint16_t* zeros = reinterpret_cast<const uint16_t*>(a.plan.hdr + kHdrZeros);
 
     // Every load of the item is issued before anything waits for one: the old values of the
@@ -786,15 +770,11 @@ __global__ __launch_bounds__(kFwdThreads) void expand_wave_kernel(ExpandArgs a) 
       L.srow[j] = a.plan.tile_row[tile * kTileRows + L.orow + 8 * j];
       sseg[j] = a.seg_scale ? a.plan.tile_rseg[tile * kTileRows + L.orow + 8 * j] : -1;
       L.yrow[j] = P.y + (long)(L.srow[j] < 0 ? 0 : L.srow[j]) * P.d_out + ncol0 + L.ocol;
-      if (DROP) L.drop[j] = drop_row(a.drop, L.srow[j], a.plan.tile_rseg, tile * kTileRows + L.orow + 8 * j);
     }
     u32x4 yold[NQ / 2][2];
     load_y_lines<NQ>(yold, L, ncol0, P.d_out, a.beta != 0.0f, zeros);
-    if (DROP) load_keep_bits<NQ>(L, a.drop, P.drop_bits, P.drop_pitch, ncol0, P.d_out, zeros);
 #pragma unroll
     for (int j = 0; j < 2; ++j) L.scale[j] = sseg[j] >= 0 ? a.seg_scale[sseg[j]] : 1.0f;
-
-    const float scale = (side && P.pt_a && rseg >= 0) ? a.seg_scale[rseg] : 1.0f;  // for the by-products
 
     f32x4 acc[NQ][2];
 #pragma unroll
@@ -811,7 +791,7 @@ __global__ __launch_bounds__(kFwdThreads) void expand_wave_kernel(ExpandArgs a) 
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           const int n = ncol0 + 32 * q + 4 * p + mrow;
-          wf[q][p] = load_w8<ROWMAJOR>(W, n, kk, ldw, kreal && n < P.d_out, zeros);
+          wf[q][p] = ldg16_or(W + (long)n * ldw + kk, kreal && n < P.d_out, zeros);
         }
       u32x4 vf;
       const bool vok = kreal && row >= 0;
@@ -833,13 +813,13 @@ __global__ __launch_bounds__(kFwdThreads) void expand_wave_kernel(ExpandArgs a) 
       } else {
         vf = ldg16_or(P.v + (long)row * P.d_in + kk, vok, zeros);
       }
-      if (side && kin) write_side<DT>(a, P, slot, row, kk, vf, scale);
+      if (side && kin && P.v_out && row >= 0) stg16(P.v_out + (long)row * P.d_in + kk, vf);
 #pragma unroll
       for (int q = 0; q < NQ; ++q)
 #pragma unroll
         for (int p = 0; p < 2; ++p) acc[q][p] = Num<DT>::mfma(wf[q][p], vf, acc[q][p]);
     }
-    store_y_lines<DT, NQ, DROP>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
+    store_y_lines<DT, NQ>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
   }
 }
 
@@ -850,10 +830,16 @@ __global__ __launch_bounds__(kFwdThreads) void expand_wave_kernel(ExpandArgs a) 
 // tiles instead of once per tile.
 // WKN: weights stored [k][n] (A [r, h_in] for the backward's dX = dV A): the chunk is staged
 // as it lies in memory and read out of LDS with the transposing read.
+// K (= LoRA rank): up to 32*KS in one piece; KS = 4 serves every rank above 64, 128 of k at a time, the
+// next piece on its way while one is multiplied.
 template <int DT, int NQ, int KS, bool DIRECT, bool WKN, bool DROP = false>
 // (five workgroups a CU instead of the four the compiler's own register budget gives: more y
 // lines in flight per CU; worth 2 % on the prefill launch and 6 % on the fine-tune one)
-__global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(DIRECT ? (NQ > 4 ? 3 : 5) : 1)))
+// KS = 4: bound by HBM like the others (2064 rows, two projections 4096 -> 4096 at rank 128: 21.6 us for 80 MB, and
+// the backward's dX 17.9 us for 46 MB, where the one-tile kernel's loop over k took 50.8 and 43.5 us: it fetched the
+// weights once per 16 rows).  Four waves a SIMD spill (37.1 / 20.6 us), 64 columns a workgroup 24.0 / 18.0.
+__global__ __launch_bounds__(kFwdThreads)
+__attribute__((amdgpu_waves_per_eu(DIRECT ? ((KS > 2 || NQ > 4) ? 3 : 5) : 1)))
 void expand_block_kernel(ExpandArgs a) {
   static_assert(NQ % 2 == 0, "the output is written 64 columns at a time");
   constexpr int kPitch = WKN ? 32 * NQ + 8 : 32 * KS + 8;  // LDS row pitch in 16-bit elements
@@ -900,7 +886,6 @@ void expand_block_kernel(ExpandArgs a) {
       L.yrow[j] = P.y + (long)(L.srow[j] < 0 ? 0 : L.srow[j]) * P.d_out + ncol0 + L.ocol;
       if (DROP) L.drop[j] = drop_row(a.drop, L.srow[j], a.plan.tile_rseg, tslot + L.orow + 8 * j);
     }
-    const int rseg = (P.pt_a && a.seg_scale && active) ? a.plan.tile_rseg[slot] : -1;
     const uint16_t* zeros = reinterpret_cast<const uint16_t*>(a.plan.hdr + kHdrZeros);
 
     // Every load of the item is issued before anything waits for one (predicated-off loads
@@ -908,76 +893,94 @@ void expand_block_kernel(ExpandArgs a) {
     // weight chunk -> registers (written to LDS below): 32*NQ rows of 4*KS 16-byte pieces
     constexpr int kPieces = 32 * NQ * 4 * KS;
     constexpr int kPer = (kPieces + kFwdThreads - 1) / kFwdThreads;
-    u32x4 stage[kPer];
+    constexpr int kK = 32 * KS;  // k of one piece
+    constexpr bool kLoop = KS > 2;
+    u32x4 stage[kPer], vf[KS];
+    auto load_stage = [&](int k0) {
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int idx = threadIdx.x + j * kFwdThreads;
-      if (WKN) {
-        const int kl = idx / (4 * NQ), n8 = (idx % (4 * NQ)) * 8;
-        stage[j] = ldg16_or(W + (long)kl * ldw + ncol0 + n8,
-                            idx < kPieces && ncol0 + n8 < P.d_out && kl < klim, zeros);
-      } else {
-        const int nl = idx / (4 * KS), k8 = (idx % (4 * KS)) * 8;
-        stage[j] = ldg16_or(W + (long)(ncol0 + nl) * ldw + k8,
-                            idx < kPieces && ncol0 + nl < P.d_out && k8 < klim, zeros);
+      for (int j = 0; j < kPer; ++j) {
+        const int idx = threadIdx.x + j * kFwdThreads;
+        if (WKN) {
+          const int kl = k0 + idx / (4 * NQ), n8 = (idx % (4 * NQ)) * 8;
+          stage[j] = ldg16_or(W + (long)kl * ldw + ncol0 + n8,
+                              idx < kPieces && ncol0 + n8 < P.d_out && kl < klim, zeros);
+        } else {
+          const int nl = idx / (4 * KS), k8 = k0 + (idx % (4 * KS)) * 8;
+          stage[j] = ldg16_or(W + (long)(ncol0 + nl) * ldw + k8,
+                              idx < kPieces && ncol0 + nl < P.d_out && k8 < klim, zeros);
+        }
       }
-    }
+    };
+    auto load_v = [&](int k0) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int kk = k0 + 32 * ks + 8 * g;
+        vf[ks] = ldg16_or(P.v + (long)row * P.d_in + kk, kk < klim && row >= 0, zeros);
+      }
+    };
+    load_stage(0);
     const bool read_y = a.beta != 0.0f;
     u32x4 yold[NQ / 2][2];
     load_y_lines<NQ>(yold, L, ncol0, P.d_out, read_y, zeros);
     if (DROP) load_keep_bits<NQ>(L, a.drop, P.drop_bits, P.drop_pitch, ncol0, P.d_out, zeros);
-    u32x4 vf[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int kk = 32 * ks + 8 * g;
-      vf[ks] = ldg16_or(P.v + (long)row * P.d_in + kk, kk < klim && row >= 0, zeros);
-    }
+    load_v(0);
 #pragma unroll
     for (int j = 0; j < 2; ++j) L.scale[j] = (sseg[j] >= 0 && L.srow[j] >= 0) ? a.seg_scale[sseg[j]] : 1.0f;
-    if (yy == 0 && active) {  // by-products for the backward (v copy, transposed scaled copies)
-      const float sc = (rseg >= 0 && row >= 0) ? a.seg_scale[rseg] : 1.0f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int kk = 32 * ks + 8 * g;
-        if (kk < P.d_in) write_side<DT>(a, P, slot, row, kk, vf[ks], sc);
-      }
-    }
 
-    __syncthreads();  // every wave is done reading the previous item's weights
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int idx = threadIdx.x + j * kFwdThreads;
-      const int r_ = WKN ? idx / (4 * NQ) : idx / (4 * KS);
-      const int c_ = WKN ? (idx % (4 * NQ)) * 8 : (idx % (4 * KS)) * 8;
-      if (idx < kPieces) *reinterpret_cast<u32x4*>(&wlds[r_ * kPitch + c_]) = stage[j];
-    }
-    __syncthreads();
     f32x4 acc[NQ][2];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[q][0] = acc[q][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // (waves without a tile multiply zeros: whole waves only, MFMA runs with every lane, and every
-    // wave reaches the barrier below)
+#pragma unroll 1
+    for (int k0 = 0;; k0 += kK) {
+      // (opaque: the compiler otherwise keeps an induction register pair for each of a hundred addresses)
+      if (kLoop) asm volatile("" : "+s"(k0));
+      __syncthreads();  // every wave is done reading the previous piece's (or item's) weights
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+      for (int j = 0; j < kPer; ++j) {
+        const int idx = threadIdx.x + j * kFwdThreads;
+        const int r_ = WKN ? idx / (4 * NQ) : idx / (4 * KS);
+        const int c_ = WKN ? (idx % (4 * NQ)) * 8 : (idx % (4 * KS)) * 8;
+        if (idx < kPieces) *reinterpret_cast<u32x4*>(&wlds[r_ * kPitch + c_]) = stage[j];
+      }
+      __syncthreads();
+      // (waves without a tile multiply zeros: whole waves only, MFMA runs with every lane, and every
+      // wave reaches the barriers)
 #pragma unroll
-      for (int q = 0; q < NQ; ++q)
+      for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          u32x4 wf;
-          if (WKN) {
-            // lane c names k row 32ks + 8g (+4) + c/4 and columns 32q + 4p + 8(c%4) .. +3; it
-            // receives column 32q + 4p + 8(c/4) + c%4 (its MFMA row's column) of four k rows
-            const uint16_t* base = &wlds[(32 * ks + 8 * g + (c >> 2)) * kPitch + 32 * q + 4 * p + 8 * (c & 3)];
-            const u32x2 q0 = lds_read_tr16(base), q1 = lds_read_tr16(base + 4 * kPitch);
-            wf = u32x4{q0[0], q0[1], q1[0], q1[1]};
-          } else {
-            wf = *reinterpret_cast<const u32x4*>(&wlds[(32 * q + 4 * p + mrow) * kPitch + 32 * ks + 8 * g]);
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            u32x4 wf;
+            if (WKN) {
+              // lane c names k row 32ks + 8g (+4) + c/4 and columns 32q + 4p + 8(c%4) .. +3; it
+              // receives column 32q + 4p + 8(c/4) + c%4 (its MFMA row's column) of four k rows
+              const uint16_t* base = &wlds[(32 * ks + 8 * g + (c >> 2)) * kPitch + 32 * q + 4 * p + 8 * (c & 3)];
+              const u32x2 q0 = lds_read_tr16(base), q1 = lds_read_tr16(base + 4 * kPitch);
+              wf = u32x4{q0[0], q0[1], q1[0], q1[1]};
+            } else {
+              wf = *reinterpret_cast<const u32x4*>(&wlds[(32 * q + 4 * p + mrow) * kPitch + 32 * ks + 8 * g]);
+            }
+            acc[q][p] = Num<DT>::mfma(wf, vf[ks], acc[q][p]);
           }
-          acc[q][p] = Num<DT>::mfma(wf, vf[ks], acc[q][p]);
-        }
+        // (the weight fragments of one k step at a time: all of them at once do not fit the registers)
+        if (kLoop) __builtin_amdgcn_sched_barrier(0);
+      }
+      if (!kLoop || k0 + kK >= P.d_in) break;  // uniform over the workgroup
+      load_stage(k0 + kK);
+      load_v(k0 + kK);
+    }
 
     __syncthreads();  // every wave has read its weights: the area is free for the accumulators
     if (active) store_y_lines<DT, NQ, DROP>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
+    if (P.pt_a && yy == 0 && active) {  // by-products for the backward, when no fold has written them
+      const int rseg = a.seg_scale ? a.plan.tile_rseg[slot] : -1;
+      const float side_scale = (rseg >= 0 && row >= 0) ? a.seg_scale[rseg] : 1.0f;
+#pragma unroll 1
+      for (int kk = 8 * g; kk < P.d_in; kk += 32)
+        write_side<DT>(a, P, slot, row, kk, ldg16_or(P.v + (long)row * P.d_in + kk, kk < klim && row >= 0, zeros),
+                       side_scale);
+    }
   }
 }
 

@@ -1,0 +1,89 @@
+"""Ranks above 64: the kernels walk the rank 128 at a time.  Edges of those pieces (72, 128, 136, 256), ragged
+widths, single rows to several tile blocks, adapters stored at their own rank; exact (dyadic) inputs against the
+oracle, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_parity import TDT, K, _ragged_segments, dev_t, dyadic, ptrs, to_np  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # T, S, NA, h_in, h_out, r, ranks of the adapters (None: all r)
+    (3, 2, 2, 64, 72, 128, None),
+    (150, 7, 3, 264, 200, 72, None),
+    (1100, 9, 3, 2048, 1160, 128, None),
+    (1040, 5, 2, 136, 88, 136, None),
+    (1030, 6, 2, 328, 264, 256, None),
+    (1200, 9, 3, 256, 520, 128, [8, 72, 128]),
+]
+IDS = ["3-rows", "rank72", "rank128", "rank136", "rank256", "packed"]
+
+
+def _inputs(case, dt, d, seed):
+    T, S, NA, h_in, h_out, r, ranks = case
+    rng = np.random.default_rng(seed)
+    seg = _ragged_segments(rng, T, S)
+    ids = [int(i) for i in rng.integers(0, NA, S)]
+    ranks = ranks or [r] * NA
+    A = [dyadic(rng, (q, h_in), 8, 64) for q in ranks]
+    B = [dyadic(rng, (h_out, q), 8, 8) for q in ranks]
+    rank_t = torch.tensor(ranks, dtype=torch.int32, device=d) if min(ranks) < r else None
+    pad = lambda w, axis: np.pad(w, [(0, r - w.shape[i]) if i == axis else (0, 0) for i in range(2)])
+    return (rng, seg, ids, A, B, [pad(a, 0) for a in A], [pad(b, 1) for b in B], [dev_t(a, dt, d) for a in A],
+            [dev_t(b, dt, d) for b in B], rank_t)
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("case", SHAPES, ids=IDS)
+def test_forward_dyadic_bit_exact(K, oracle, gpu_device, case, dt):
+    T, S, NA, h_in, h_out, r, _ = case
+    d = gpu_device
+    rng, seg, ids, _, _, Ap, Bp, Ad, Bd, rank_t = _inputs(case, dt, d, 31)
+    x, y0 = dyadic(rng, (T, h_in), 16, 8), dyadic(rng, (T, h_out), 16, 8)
+    scale = (rng.integers(1, 5, S) / 2.0).astype(np.float32)
+    plan = K.SegmentPlan(torch.tensor(seg, dtype=torch.int32, device=d),
+                         torch.tensor(ids, dtype=torch.int32, device=d), T, defer=True)
+    y, v = dev_t(y0, dt, d), torch.zeros(T, r, dtype=TDT[dt], device=d)
+    K.smlm_lora_forward(y, dev_t(x, dt, d), ptrs(Ad, d), ptrs(Bd, d), plan, r, beta=1.0, v_out=v,
+                        seg_scale=torch.from_numpy(scale).to(d), adapter_rank=rank_t, packed_ranks=rank_t is not None)
+    yo, vo = oracle.lora_fused(y0, x, [Ap[i] for i in ids], [Bp[i] for i in ids], seg, scale.tolist(), 1.0, dt)
+    covered = np.zeros(T, bool)
+    covered[seg[0]:seg[-1]] = True
+    assert np.array_equal(to_np(v)[covered], vo[covered]), "v"
+    assert np.array_equal(to_np(y), yo), "y"
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("drop", [False, True], ids=["plain", "dropout"])
+@pytest.mark.parametrize("case", SHAPES, ids=IDS)
+def test_backward_dyadic_bit_exact(K, oracle, gpu_device, case, drop, dt):
+    T, S, NA, h_in, h_out, r, _ = case
+    d = gpu_device
+    rng, seg, ids, A, B, Ap, Bp, Ad, Bd, rank_t = _inputs(case, dt, d, 32)
+    tp = [c - seg[0] for c in seg]
+    n = tp[-1]
+    x, g = dyadic(rng, (n, h_in), 16, 8), dyadic(rng, (n, h_out), 16, 8)
+    seg_p = np.array([0.5 if a % 2 == 0 else 0.0 for a in ids], np.float32)
+    spec = K.DropoutSpec(torch.from_numpy(seg_p).to(d), n, 7, 11) if drop else None
+    dA, dB = [torch.full_like(a, 9.0) for a in Ad], [torch.full_like(b, 9.0) for b in Bd]
+    dx = torch.empty(n, h_in, dtype=TDT[dt], device=d)
+    plan = K.SegmentPlan(torch.tensor(tp, dtype=torch.int32, device=d),
+                         torch.tensor(ids, dtype=torch.int32, device=d), n, defer=True)
+    xo = x
+    if drop:
+        rp = np.zeros(n, np.float32)
+        for i in range(S):
+            rp[tp[i]:tp[i + 1]] = seg_p[i]
+        xo = oracle.dropout_rows(x, rp, 7, 11, dt)
+    _, vo = oracle.add_lora_forward(xo, [Ap[i] for i in ids], [Bp[i] for i in ids], tp, h_out, dt)
+    K.smlm_lora_backward(dx, ptrs(dA, d), ptrs(dB, d), dev_t(g, dt, d), dev_t(x, dt, d), dev_t(vo, dt, d), ptrs(Ad, d),
+                         ptrs(Bd, d), plan, r, dropout=spec, adapter_rank=rank_t, packed_ranks=rank_t is not None)
+    gx, ga, gb = oracle.add_lora_backward(g, xo, Ap, Bp, tp, ids, dt)
+    if drop:
+        gx = oracle.dropout_rows(gx, rp, 7, 11, dt)
+    assert np.array_equal(to_np(dx), gx), "dX"
+    for a in range(NA):
+        assert np.array_equal(to_np(dA[a]), ga[a][:A[a].shape[0]]), f"dA[{a}]"
+        assert np.array_equal(to_np(dB[a]), gb[a][:, :B[a].shape[1]]), f"dB[{a}]"
