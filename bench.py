@@ -106,7 +106,7 @@ def single_tiles(T: int, r: int) -> bool:
     """Whether the forward of a batch of T rows at rank r runs on single 16-row tiles (the decode route)
     or on tile blocks: the library's rule, loquetier_amd/csrc/smlm_api.hip (tiles_per_wave); only used
     here to say in the output how the step's plan is built."""
-    return T < (2048 if r <= 16 else 768 if r <= 32 else 512 if r <= 48 else 128 if r <= 64 else 1024)
+    return T < (2048 if r <= 16 else 768 if r <= 32 else 512 if r <= 48 or r > 64 else 128)
 
 
 def algorithmic_bytes(w, h_in, h_out, accumulate=True, own_x=True):

@@ -47,10 +47,12 @@ int launch(void (*kernel)(A), dim3 grid, dim3 block, hipStream_t st, const A& a)
 // 15.6 / 17.8, at 1536 rows 21.7 / 19.2; rank 64 at 256 rows 17.0 / 16.3, at 1000 rows 22.9 / 18.8.  A launch of
 // several projections, whose workgroups fill the chip together, would change over earlier (q/k/v/o: rank 16 at
 // 1024 rows 30.9 / 30.9, at 2048 rows 53.1 / 47.5; rank 32 at 384 rows 24.5 / 25.3, at 768 rows 34.6 / 30.7;
-// rank 64 at 128 rows 27.6 / 24.7); the rule lies between the two and does not look at the number of
+// rank 64 at 128 rows 27.6 / 24.7).  Rank 128, forward of one projection 4096 -> 4096: 256 rows over 32 adapters
+// 25.5 / 29.7, 512 rows 29.2 / 31.5, 1000 rows over 16 adapters 42.3 / 33.0; q/k/v/o at 128 rows 74.2 / 70.6, at 512
+// rows 86.7 / 78.9.  The rule lies between the two and does not look at the number of
 // projections, so that a launch of several gives the bits that launches of one give.
 inline int tiles_per_wave(int T, int r) {
-  const int from = r <= 16 ? 2048 : (r <= 32 ? 768 : (r <= 48 ? 512 : (r <= 64 ? 128 : 1024)));
+  const int from = r <= 16 ? 2048 : (r <= 32 ? 768 : (r <= 48 || r > 64 ? 512 : 128));
   return T >= from ? kBlkTiles : 1;
 }
 // (The backward runs on tile blocks at every size and rank: they read the weights the other way round as they lie
@@ -104,12 +106,14 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
 // whether they are launched alone or together, so that either way gives the same bits
 ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
   ShrinkCfg c;
-  c.zblocks = ceil_div(d_out, 64);
-  const int cols = d_out >= 64 ? 64 : d_out;
-  c.NB = cols <= 16 ? 1 : (cols <= 32 ? 2 : 4);
   c.MT = mt;
-  // 32-wide k steps per load batch (the tile-block kernel stages four per batch in LDS)
-  c.U = c.MT > 1 ? 4 : (c.NB == 4 ? 2 : 4);
+  c.NB = d_out <= 16 ? 1 : (d_out <= 32 ? 2 : (d_out <= 64 || mt == 1 ? 4 : 8));
+  c.zblocks = ceil_div(d_out, c.NB == 8 ? 128 : 64);
+  // 32-wide k steps per load batch (the tile-block kernel stages four per batch in LDS, two of 128 weight rows).
+  // (Ranks above 64 take 128 columns a workgroup and read x once for them; with 64, twice: 2064 rows, two projections
+  // 4096 -> 4096 at rank 128, shrink 25.5 -> 20.7 us, the backward's dV 23.8 -> 18.1; four steps a batch 27.5 / 22.2,
+  // whose 70 KB of LDS leave two workgroups a CU.)
+  c.U = c.NB == 8 ? 2 : (c.MT > 1 ? 4 : (c.NB == 4 ? 2 : 4));
   const int kq = 32 * c.U;
   c.NW = nw;
   const int units = ceil_div(T > 0 ? T : 1, kTileRows * c.MT);
@@ -200,6 +204,7 @@ int launch_shrink_block(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) 
   const dim3 block(kFwdThreads);
   if (NB == 1) return launch(shrink_block_kernel<DT, 1, 4, DIRECT, WKN, DROP>, grid, block, st, a);
   if (NB == 2) return launch(shrink_block_kernel<DT, 2, 4, DIRECT, WKN, DROP>, grid, block, st, a);
+  if (NB == 8) return launch(shrink_block_kernel<DT, 8, 2, DIRECT, WKN, DROP>, grid, block, st, a);
   return launch(shrink_block_kernel<DT, 4, 4, DIRECT, WKN, DROP>, grid, block, st, a);
 }
 
@@ -249,6 +254,7 @@ int launch_self_planned_block_nb(int NB, dim3 grid, hipStream_t st, const SelfPl
   const dim3 block(THREADS);  // U must match shrink_cfg
   if (NB == 1) return launch(shrink_block_self_planned_kernel<DT, 1, 4, WKN, THREADS, PAIRS>, grid, block, st, a);
   if (NB == 2) return launch(shrink_block_self_planned_kernel<DT, 2, 4, WKN, THREADS, PAIRS>, grid, block, st, a);
+  if (NB == 8) return launch(shrink_block_self_planned_kernel<DT, 8, 2, WKN, THREADS, PAIRS>, grid, block, st, a);
   return launch(shrink_block_self_planned_kernel<DT, 4, 4, WKN, THREADS, PAIRS>, grid, block, st, a);
 }
 template <int DT, bool WKN, bool PAIRS>

@@ -405,7 +405,7 @@ __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(Self
   const int c = lane & 15, g = lane >> 4;
   const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
   const int kz = yy % P.ksplit, zb = yy / P.ksplit;
-  const int n0 = zb * 64;
+  const int n0 = zb * 16 * NB;  // (several column blocks only where NB = 4 or 8)
   const int kbeg = kz * kFwdWaves * P.k_per_wave;
   const int kend = min(kbeg + kFwdWaves * P.k_per_wave, P.d_in);
   const int kstop = GROUPS > 1 ? kbeg + kFwdWaves * P.k_per_wave : kend;  // the same number of batches for both groups

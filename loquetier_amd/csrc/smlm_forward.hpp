@@ -345,7 +345,7 @@ __global__ __launch_bounds__(kFwdThreads) void shrink_block_kernel(ShrinkArgs a)
     int t0, cnt, wid;
     pick_tiles<kBlkTiles>(a.plan, tb, &t0, &cnt, &wid);
     if (cnt == 0) continue;  // uniform over the workgroup
-    const int n0 = zb * 64;
+    const int n0 = zb * 16 * NB;  // (several column blocks only where NB = 4 or 8)
     const bool active = wave < cnt;
     const int slot = (t0 + (active ? wave : 0)) * kTileRows + c;
     const int row = active ? a.plan.tile_row[slot] : -1;

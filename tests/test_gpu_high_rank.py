@@ -14,11 +14,13 @@ SHAPES = [
     (3, 2, 2, 64, 72, 128, None),
     (150, 7, 3, 264, 200, 72, None),
     (1100, 9, 3, 2048, 1160, 128, None),
+    (511, 4, 2, 2048, 72, 128, None),       # single tiles forward, the row below tile blocks
+    (512, 4, 2, 2048, 72, 128, None),
     (1040, 5, 2, 136, 88, 136, None),
     (1030, 6, 2, 328, 264, 256, None),
     (1200, 9, 3, 256, 520, 128, [8, 72, 128]),
 ]
-IDS = ["3-rows", "rank72", "rank128", "rank136", "rank256", "packed"]
+IDS = ["3-rows", "rank72", "rank128", "511-rows", "512-rows", "rank136", "rank256", "packed"]
 
 
 def _inputs(case, dt, d, seed):
