@@ -549,26 +549,20 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
   return launch_reduce(dtype, S, groups, st, ra, with_side);
 }
 
-template <int DT>
+template <int DT, bool DROP>
 int launch_wgrad(int nbj, bool split, dim3 grid, hipStream_t st, const WgradArgs& wa) {
-  if (wa.drop.seg_p) {
-    if (split) {
-      if (nbj == 1) return launch(wgrad_kernel<DT, 1, 4, true>, grid, dim3(256), st, wa);
-      if (nbj == 2) return launch(wgrad_kernel<DT, 2, 4, true>, grid, dim3(256), st, wa);
-      return launch(wgrad_kernel<DT, 4, 4, true>, grid, dim3(256), st, wa);
-    }
-    if (nbj == 1) return launch(wgrad_kernel<DT, 1, 1, true>, grid, dim3(64), st, wa);
-    if (nbj == 2) return launch(wgrad_kernel<DT, 2, 1, true>, grid, dim3(64), st, wa);
-    return launch(wgrad_kernel<DT, 4, 1, true>, grid, dim3(64), st, wa);
-  }
+  const dim3 bl(split ? 256 : 64);
+  if (wa.zcount > 1)  // several workgroups along the rank: NBJ = 4
+    return split ? launch(wgrad_kernel<DT, 4, 4, DROP, true>, grid, bl, st, wa)
+                 : launch(wgrad_kernel<DT, 4, 1, DROP, true>, grid, bl, st, wa);
   if (split) {
-    if (nbj == 1) return launch(wgrad_kernel<DT, 1, 4>, grid, dim3(256), st, wa);
-    if (nbj == 2) return launch(wgrad_kernel<DT, 2, 4>, grid, dim3(256), st, wa);
-    return launch(wgrad_kernel<DT, 4, 4>, grid, dim3(256), st, wa);
+    if (nbj == 1) return launch(wgrad_kernel<DT, 1, 4, DROP, false>, grid, bl, st, wa);
+    if (nbj == 2) return launch(wgrad_kernel<DT, 2, 4, DROP, false>, grid, bl, st, wa);
+    return launch(wgrad_kernel<DT, 4, 4, DROP, false>, grid, bl, st, wa);
   }
-  if (nbj == 1) return launch(wgrad_kernel<DT, 1, 1>, grid, dim3(64), st, wa);
-  if (nbj == 2) return launch(wgrad_kernel<DT, 2, 1>, grid, dim3(64), st, wa);
-  return launch(wgrad_kernel<DT, 4, 1>, grid, dim3(64), st, wa);
+  if (nbj == 1) return launch(wgrad_kernel<DT, 1, 1, DROP, false>, grid, bl, st, wa);
+  if (nbj == 2) return launch(wgrad_kernel<DT, 2, 1, DROP, false>, grid, bl, st, wa);
+  return launch(wgrad_kernel<DT, 4, 1, DROP, false>, grid, bl, st, wa);
 }
 
 struct BwdProjLayout {
@@ -1267,13 +1261,18 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   wa.w_rank = w_rank;
   wa.packed = packed;
   wa.drop = drop;  // dA against the dropped x
-  // ranks above 64 are covered 64 at a time along the grid's z axis
+  // ranks above 64 are covered 64 at a time by workgroups of their own
   const int nbj = r > 64 ? 4 : ceil_div(r, 16);
-  // (along z: 64 ranks a workgroup, or what a dA workgroup of the launched kernel takes when that is less)
+  // (64 ranks a workgroup, or what a dA workgroup of the launched kernel takes when that is less)
   const int z_per_64 = nbj / wgrad_nbj_a(nbj, split ? 4 : 1, drop.seg_p != nullptr);
-  dim3 grid(units, NA, ceil_div(r, 64) * z_per_64);
-  return dtype == SMLM_DTYPE_F16 ? launch_wgrad<SMLM_DTYPE_F16>(nbj, split, grid, st, wa)
-                                 : launch_wgrad<SMLM_DTYPE_BF16>(nbj, split, grid, st, wa);
+  wa.units = units;
+  wa.zcount = ceil_div(r, 64) * z_per_64;
+  dim3 grid(wa.zcount > 1 ? round_up(units, kWgXcd) * wa.zcount : units, NA);
+  if (drop.seg_p)
+    return dtype == SMLM_DTYPE_F16 ? launch_wgrad<SMLM_DTYPE_F16, true>(nbj, split, grid, st, wa)
+                                   : launch_wgrad<SMLM_DTYPE_BF16, true>(nbj, split, grid, st, wa);
+  return dtype == SMLM_DTYPE_F16 ? launch_wgrad<SMLM_DTYPE_F16, false>(nbj, split, grid, st, wa)
+                                 : launch_wgrad<SMLM_DTYPE_BF16, false>(nbj, split, grid, st, wa);
 }
 
 // workgroups of the RMSNorm backward: enough to fill the chip, each with several rows so that

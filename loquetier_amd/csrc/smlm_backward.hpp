@@ -33,6 +33,8 @@ struct WgradArgs {
   const int32_t* tile_row;
   WgradProj p[kWgMaxProj];
   int nproj;
+  int units;               // units of all projections
+  int zcount;              // workgroups along the rank, see wgrad_kernel
   int walk;                // chunks a one-wave workgroup takes in turn (NW = 1 kernels; else 1)
   long pitch;
   int r;
@@ -47,6 +49,7 @@ struct WgradArgs {
 constexpr int kWgCols = 64;     // columns of x / dY per workgroup
 constexpr int kWgPitch = 80;    // LDS row pitch in 16-bit elements: 40 banks, so any eight
                                 // consecutive rows start 8 banks apart and tile the 64 banks
+constexpr int kWgXcd = 8;       // XCDs workgroups go to in turn
 constexpr int kWgSlots = 64;    // gathered rows (four tiles) per wave and loop step
 
 // LDS row of gathered-row slot s of a step: bits 2 and 3 of s change places, so
@@ -56,8 +59,8 @@ __device__ __forceinline__ int wg_lds_row(int s) {
   return (s & ~12) | ((s & 4) << 1) | ((s & 8) >> 1);
 }
 
-// grid: (sum over the projections of their dA and dB units, NA, ceil(r/64) -- twice that for the kernel named at
-// wgrad_nbj_a), block 64*NW; a unit is
+// grid: (sum over the projections of their dA and dB units, NA), block 64*NW; with ZSPLIT ceil(r/64) workgroups per
+// unit -- twice that for the kernel named at wgrad_nbj_a.  A unit is
 // `walk` neighbouring 64-column chunks of one projection's dA or dB.  A workgroup owns the unit's columns (and
 // up to 64 ranks) of one adapter's gradient and walks all of that adapter's tiles once per chunk, 64
 // gathered rows (four tiles, two MFMA k steps) per wave and loop step.  With
@@ -77,7 +80,7 @@ __device__ __forceinline__ int wg_lds_row(int s) {
 // bits (one byte per eight columns, the projection's drop_bits) travel with the rows and are applied while the
 // rows are staged; every row of the workgroup belongs to one adapter, whose probability is read
 // once from the group's first segment.
-template <int DT, int NBJ, int NW, bool IS_A, bool DROP = false>
+template <int DT, int NBJ, int NW, bool IS_A, bool DROP, bool ZSPLIT>
 __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& P, int chunk_first, int n_chunks,
                                            int j0, char* smem) {
   constexpr int kWgWaves = NW;
@@ -155,8 +158,10 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const bool ok = row[u] >= 0 && col_ok;
-      // x and dY are read here for the last time in the backward: non-temporal
-      val[u] = ldg16_or_nt(Q + (long)row[u] * h + n0 + lcol, ok, zeros);
+      // x and dY are read here for the last time in the backward: non-temporal, unless the workgroup next door
+      // reads the same lines for other ranks
+      const uint16_t* q = Q + (long)row[u] * h + n0 + lcol;
+      val[u] = ZSPLIT ? ldg16_or(q, ok, zeros) : ldg16_or_nt(q, ok, zeros);
       if (DROP) {  // rows at or past drop.rows keep everything: their byte is never applied
         const bool dropped = ok && row[u] < a.drop.rows;
         keep[u] = *(const SMLM_GLOBAL uint8_t*)(dropped ? P.drop_bits + (long)row[u] * P.drop_pitch + ((n0 + lcol) >> 3)
@@ -354,30 +359,42 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
 // rank blocks of 16 a dA workgroup takes (a dB workgroup: NBJ)
 constexpr int wgrad_nbj_a(int nbj, int nw, bool drop) { return (drop && nw == 1 && nbj == 4) ? 2 : nbj; }
 
-template <int DT, int NBJ, int NW, bool DROP = false>
+// ZSPLIT: several workgroups share a unit, each taking other ranks (a.zcount of them: ranks above 64).  They are
+// numbered eight apart, so that they run at about the same time on one XCD (workgroup number modulo eight) and the
+// rows of x and dY, which all of them read, come out of its L2 for the second (2048 rows, two projections
+// 4096 -> 4096 at rank 128: 40.2 us with the ranks along the grid's z axis, 37.4 eight apart, 32.9 with loads that
+// are not marked non-temporal as well).
+template <int DT, int NBJ, int NW, bool DROP, bool ZSPLIT>
 // (two waves a SIMD at every rank: the one-wave kernels hide their latencies through occupancy)
 __global__ __launch_bounds__(NW * kWaveSize) __attribute__((amdgpu_waves_per_eu(2))) void wgrad_kernel(WgradArgs a) {
   constexpr int kStageBytes = NW * kWgSlots * kWgPitch * 2;
   constexpr int kTailBytes = (NW > 1 ? NW * 4 * kWaveSize * 16 : 0) + 16 * (64 + 4) * 4;  // red + store staging
   __shared__ __attribute__((aligned(16))) char smem[kStageBytes > kTailBytes ? kStageBytes : kTailBytes];
+  int zi = 0, u = (int)blockIdx.x;
+  if (ZSPLIT) {
+    const int per = kWgXcd * a.zcount, in = u % per;
+    zi = in / kWgXcd;
+    u = u / per * kWgXcd + in % kWgXcd;
+    if (u >= a.units) return;
+  }
   int pj = 0;
 #pragma unroll
-  for (int i = 1; i < kWgMaxProj; ++i) pj += (i < a.nproj && (int)blockIdx.x >= a.p[i].unit0) ? 1 : 0;
+  for (int i = 1; i < kWgMaxProj; ++i) pj += (i < a.nproj && u >= a.p[i].unit0) ? 1 : 0;
   const WgradProj& P = a.p[pj];
-  const int unit = (int)blockIdx.x - P.unit0;
+  const int unit = u - P.unit0;
   const int walk = NW > 1 ? 1 : a.walk;
   // The one-wave kernel that applies dropout to 64 ranks at a time does not fit the registers of a lane
   // (200 bytes of spills, and twice the time of the kernel without dropout): its dA workgroups take 32 ranks
-  // each, two along z where the others have one; dB, which no dropout touches, keeps 64.
+  // each, two per unit where the others have one; dB, which no dropout touches, keeps 64.
   constexpr int NBJ_A = wgrad_nbj_a(NBJ, NW, DROP), ZA = NBJ / NBJ_A;
   if (unit < P.units_a) {  // uniform over the workgroup
     const int first = unit * walk, left = P.chunks_a - first;
-    wgrad_body<DT, NBJ_A, NW, true, DROP>(a, P, first, left < walk ? left : walk, 16 * NBJ_A * (int)blockIdx.z, smem);
+    wgrad_body<DT, NBJ_A, NW, true, DROP, ZSPLIT>(a, P, first, left < walk ? left : walk, 16 * NBJ_A * zi, smem);
   } else {
-    if (blockIdx.z % ZA) return;
+    if (zi % ZA) return;
     const int chunks_b = (P.h_out + kWgCols - 1) / kWgCols;
     const int first = (unit - P.units_a) * walk, left = chunks_b - first;
-    wgrad_body<DT, NBJ, NW, false>(a, P, first, left < walk ? left : walk, 16 * NBJ * (int)(blockIdx.z / ZA), smem);
+    wgrad_body<DT, NBJ, NW, false, false, ZSPLIT>(a, P, first, left < walk ? left : walk, 16 * NBJ * (zi / ZA), smem);
   }
 }
 
