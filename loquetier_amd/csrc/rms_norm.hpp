@@ -22,7 +22,8 @@ namespace smlm {
 constexpr int kRmsChunks = 8;                       // 512-element chunks a wave keeps in registers
 constexpr int kRmsWaveCols = 512 * kRmsChunks;      // columns one wave covers
 constexpr int kRmsMaxCols = 4 * kRmsWaveCols;       // four waves per row at most
-constexpr int kRmsFoldRows = 16;                    // partial rows summed side by side in the fold
+constexpr int kRmsFoldRows = 64;                    // partial rows summed side by side in the fold ...
+constexpr int kRmsFoldCols = 16;                    // ... whose workgroups take this many columns
 
 // Sum over the wave with DPP adds (shifts inside rows of 16 lanes, then the
 // row totals); every lane returns the total.
@@ -63,9 +64,7 @@ struct RmsFwdArgs {
 // + gridDim.x * (4 / WPR), ...  Chunk i of wave v covers the 512 columns starting
 // at (i * WPR + v) * 512, eight per lane.  When a workgroup has more than one
 // turn, the next row is on its way from memory while the current one is
-// reduced, scaled and stored.  (Measured: one turn per workgroup is fastest for
-// the forward, four for the backward, whose per-workgroup dw partials cost
-// traffic of their own.)
+// reduced, scaled and stored.  (Measured: one turn per workgroup is fastest.)
 // x is read and the output written non-temporally: both are touched once per launch (the next
 // reader of x is the backward, much later; a reader of the output that follows at once still
 // finds it in the caches when it fits them).
@@ -155,130 +154,116 @@ struct RmsBwdArgs {
   int rows, cols;
 };
 
-// A workgroup walks rows blockIdx.x, blockIdx.x + gridDim.x, ... (WPR == 4: one
-// row at a time, a quarter of the columns per wave; WPR == 1: four rows at a
-// time, one per wave) and keeps its share of dw in registers.
-template <int DT, int WPR>
-__global__ __launch_bounds__(256) void rms_bwd_kernel(RmsBwdArgs a) {
-  __shared__ float part[2][4];
-  __shared__ __attribute__((aligned(16))) float dwred[WPR == 1 ? 4 * (kRmsWaveCols / 2) : 4];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int sub = wave % WPR;
-  const u32x4 zero = {0u, 0u, 0u, 0u};
+// A workgroup takes a contiguous share of the rows, R at a time, a thread 8 columns (CH = 1, up to 8192 columns: as
+// many threads as a row has pieces of 8, in whole waves) or 16 (CH = 2, 1024 threads), and keeps its columns of w and
+// its share of dw in registers.  The dots of the R rows cross the waves through LDS together, one barrier for them;
+// the next rows are on their way meanwhile.
+// Bound by HBM: three passes of 2 bytes an element.  A thread per column piece keeps a lane's registers few (dw is
+// eight floats) and the rows in flight many.  4224 x 4096, bf16: 23.3 us and 3.9 us for the fold of 256 partial rows
+// (a wave to a row, 64 columns a lane, 208 registers: 31.9 + 4.1); four rows at a time without the rows ahead
+// 30.3 us, two 25.6 with 512 workgroups, whose fold then takes longer.  2000 x 8192: 31.9 -> 24.7 us, 300 x 1024
+// 9.9 -> 3.5, 4000 x 2048 equal.
+template <int DT, int CH, int R>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void rms_bwd_kernel(RmsBwdArgs a) {
+  typedef float dots_t __attribute__((ext_vector_type(R)));
+  __shared__ dots_t part[2][16];  // the rows' dots by wave, two halves in turn
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = (int)blockDim.x >> 6;
   const float inv_n = 1.0f / (float)a.cols;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  const int row0 = (int)((long)blockIdx.x * a.rows / gridDim.x), row1 = (int)((long)(blockIdx.x + 1) * a.rows / gridDim.x);
 
-  u32x4 wv[kRmsChunks];
+  int col[CH];
+  bool ok[CH];
+  u32x4 wv[CH];
+  float dw[CH][8];
 #pragma unroll
-  for (int i = 0; i < kRmsChunks; ++i) {
-    const int col = ((i * WPR + sub) * 64 + lane) * 8;
-    wv[i] = col < a.cols ? ldg16(a.w + col) : zero;
-  }
-  float dw[kRmsChunks][8];
-#pragma unroll
-  for (int i = 0; i < kRmsChunks; ++i)
+  for (int i = 0; i < CH; ++i) {
+    col[i] = ((int)threadIdx.x + i * (int)blockDim.x) * 8;
+    ok[i] = col[i] < a.cols;
+    if (!ok[i]) col[i] = 0;
+    wv[i] = ldg16(a.w + col[i]);
+    if (!ok[i]) wv[i] = zero;  // (the columns past the row then add nothing to a dot)
 #pragma unroll
     for (int e = 0; e < 8; ++e) dw[i][e] = 0.0f;
-
-  constexpr int kRows = 4 / WPR;
-  bool ok[kRmsChunks];
+  }
+  // rows past the workgroup's share re-read its last row and are not used
+  auto load = [&](int row, u32x4 (&xr)[R][CH], u32x4 (&gr)[R][CH], float (&r)[R]) {
 #pragma unroll
-  for (int i = 0; i < kRmsChunks; ++i) ok[i] = ((i * WPR + sub) * 64 + lane) * 8 < a.cols;
-  auto load_row = [&](int row, u32x4 (&xr)[kRmsChunks], u32x4 (&gr)[kRmsChunks], float& r) {
-    const long off = (long)(row < a.rows ? row : 0) * a.cols;
+    for (int t = 0; t < R; ++t) {
+      const int rr = row + t < row1 ? row + t : row1 - 1;
 #pragma unroll
-    for (int i = 0; i < kRmsChunks; ++i) {
-      const int col = ((i * WPR + sub) * 64 + lane) * 8;
-      xr[i] = ldg16_nt(a.x + off + (ok[i] ? col : 0));
-      gr[i] = ldg16_nt(a.g + off + (ok[i] ? col : 0));
+      for (int i = 0; i < CH; ++i) {
+        xr[t][i] = ldg16_nt(a.x + (long)rr * a.cols + col[i]);
+        gr[t][i] = ldg16_nt(a.g + (long)rr * a.cols + col[i]);
+      }
+      r[t] = uload(a.rms, rr);
     }
-    r = a.rms[row < a.rows ? row : 0];
   };
-  const int step = (int)gridDim.x * kRows;
-  int row = (int)blockIdx.x * kRows + wave / WPR;
-  u32x4 xv[kRmsChunks], gv[kRmsChunks];
-  float rms;
-  load_row(row, xv, gv, rms);
+  u32x4 xv[R][CH], gv[R][CH];
+  float rms[R];
+  load(row0, xv, gv, rms);
   int parity = 0;
-  // WPR == 4: `row` is uniform over the workgroup, so every wave reaches the barrier
-  for (; row < a.rows; row += step) {
-    const long off = (long)row * a.cols;
-    u32x4 xn[kRmsChunks], gn[kRmsChunks];
-    float rms_n = 0.0f;
-    // unconditional (past the last row it re-reads row 0): a branch around the loads would make
-    // the wave wait for everything in flight where the paths join
-    load_row(row + step, xn, gn, rms_n);
-    __builtin_amdgcn_sched_barrier(0);  // the next row's loads are issued before this row is used
-    float dot = 0.0f;
+  for (int row = row0; row < row1; row += R) {  // uniform over the workgroup
+    u32x4 xn[R][CH], gn[R][CH];
+    float rn[R];
+    // unconditional (past the end it re-reads the last row): a branch around the loads would make the wave wait
+    // for everything in flight where the paths join
+    load(row + R, xn, gn, rn);
+    __builtin_amdgcn_sched_barrier(0);  // the next rows' loads are issued before these rows are used
+    dots_t dots;
 #pragma unroll
-    for (int i = 0; i < kRmsChunks; ++i) {
-      if (!ok[i]) xv[i] = gv[i] = zero;
-      float xf[8], gf[8], wf[8];
-      unpack8<DT>(xv[i], xf);
-      unpack8<DT>(gv[i], gf);
-      unpack8<DT>(wv[i], wf);
+    for (int t = 0; t < R; ++t) {
+      float dot = 0.0f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dot += gf[e] * wf[e] * xf[e];
+      for (int i = 0; i < CH; ++i) {
+        float xf[8], gf[8], wf[8];
+        unpack8<DT>(xv[t][i], xf);
+        unpack8<DT>(gv[t][i], gf);
+        unpack8<DT>(wv[i], wf);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot += gf[e] * wf[e] * xf[e];
+      }
+      dots[t] = wave_sum_f32(dot);
     }
-    dot = wave_sum_f32(dot);
-    if (WPR > 1) {
-      if (lane == 0) part[parity][wave] = dot;
-      __syncthreads();  // one barrier a row: the two halves of `part` alternate
-      dot = (part[parity][0] + part[parity][1]) + (part[parity][2] + part[parity][3]);
-      parity ^= 1;
+    if (lane == 0) part[parity][wave] = dots;
+    __syncthreads();
+    dots = part[parity][0];
+    for (int v = 1; v < nw; ++v) dots += part[parity][v];
+    parity ^= 1;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      if (row + t >= row1) break;  // uniform over the workgroup
+      const float coef = dots[t] * rms[t] * rms[t] * inv_n;
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        float xf[8], gf[8], wf[8];
+        unpack8<DT>(xv[t][i], xf);
+        unpack8<DT>(gv[t][i], gf);
+        unpack8<DT>(wv[i], wf);
+        u32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          o[e] = pack2<DT>((gf[2 * e] * wf[2 * e] - xf[2 * e] * coef) * rms[t],
+                           (gf[2 * e + 1] * wf[2 * e + 1] - xf[2 * e + 1] * coef) * rms[t]);
+        if (ok[i]) stg16_nt(a.dx + (long)(row + t) * a.cols + col[i], o);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dw[i][e] += xf[e] * rms[t] * gf[e];
+      }
     }
-    const float coef = dot * rms * rms * inv_n;
 #pragma unroll
-    for (int i = 0; i < kRmsChunks; ++i) {
-      const int col = ((i * WPR + sub) * 64 + lane) * 8;
-      if (!ok[i]) continue;
-      float xf[8], gf[8], wf[8];
-      unpack8<DT>(xv[i], xf);
-      unpack8<DT>(gv[i], gf);
-      unpack8<DT>(wv[i], wf);
-      u32x4 o;
+    for (int t = 0; t < R; ++t) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        o[e] = pack2<DT>((gf[2 * e] * wf[2 * e] - xf[2 * e] * coef) * rms,
-                         (gf[2 * e + 1] * wf[2 * e + 1] - xf[2 * e + 1] * coef) * rms);
-      stg16_nt(a.dx + off + col, o);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) dw[i][e] += xf[e] * rms * gf[e];
+      for (int i = 0; i < CH; ++i) xv[t][i] = xn[t][i], gv[t][i] = gn[t][i];
+      rms[t] = rn[t];
     }
-#pragma unroll
-    for (int i = 0; i < kRmsChunks; ++i) xv[i] = xn[i], gv[i] = gn[i];
-    rms = rms_n;
   }
 
   float* prow = a.partial + (long)blockIdx.x * a.cols;
-  if (WPR == 1) {
-    // the four waves hold sums over different rows of the same columns: add them in wave
-    // order through LDS, half of the columns at a time
-    constexpr int kHalf = kRmsWaveCols / 2;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int i = 0; i < kRmsChunks / 2; ++i) {
-        const int ci = h * (kRmsChunks / 2) + i, lc = (i * 64 + lane) * 8;
-        *reinterpret_cast<f32x4*>(&dwred[wave * kHalf + lc]) = f32x4{dw[ci][0], dw[ci][1], dw[ci][2], dw[ci][3]};
-        *reinterpret_cast<f32x4*>(&dwred[wave * kHalf + lc + 4]) = f32x4{dw[ci][4], dw[ci][5], dw[ci][6], dw[ci][7]};
-      }
-      __syncthreads();
-      for (int lc = threadIdx.x * 4; lc < kHalf && h * kHalf + lc < a.cols; lc += 256 * 4) {
-        f32x4 s = *reinterpret_cast<const f32x4*>(&dwred[lc]);
-#pragma unroll
-        for (int v = 1; v < 4; ++v) s += *reinterpret_cast<const f32x4*>(&dwred[v * kHalf + lc]);
-        *(SMLM_GLOBAL f32x4*)(prow + h * kHalf + lc) = s;
-      }
-      __syncthreads();
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < kRmsChunks; ++i) {
-      const int col = ((i * WPR + sub) * 64 + lane) * 8;
-      if (col >= a.cols) continue;
-      *(SMLM_GLOBAL f32x4*)(prow + col) = f32x4{dw[i][0], dw[i][1], dw[i][2], dw[i][3]};
-      *(SMLM_GLOBAL f32x4*)(prow + col + 4) = f32x4{dw[i][4], dw[i][5], dw[i][6], dw[i][7]};
-    }
+  for (int i = 0; i < CH; ++i) {
+    if (!ok[i]) continue;
+    *(SMLM_GLOBAL f32x4*)(prow + col[i]) = f32x4{dw[i][0], dw[i][1], dw[i][2], dw[i][3]};
+    *(SMLM_GLOBAL f32x4*)(prow + col[i] + 4) = f32x4{dw[i][4], dw[i][5], dw[i][6], dw[i][7]};
   }
 }
 
@@ -373,16 +358,17 @@ struct RmsFoldArgs {
   int n_part, cols;
 };
 
-// grid: ceil(cols / 64), block 256: thread (rg = tid / 16, c4 = tid % 16) adds
-// partial rows rg, rg + 16, ... of four columns; the sixteen row groups are then
-// added in order through LDS.
+// grid: ceil(cols / 16), block 256: thread (rg = tid / 4, c4 = tid % 4) adds partial rows rg, rg + 64, ... of four
+// columns; the 64 row groups are then added across the lanes of each wave and the four waves through LDS, always in
+// the same order.  (Sixteen columns a workgroup: a row of 4096 columns keeps every CU busy; with 64 columns a
+// workgroup only a quarter of them worked.)
 template <int DT>
 __global__ __launch_bounds__(256) void rms_fold_kernel(RmsFoldArgs a) {
-  __shared__ f32x4 red[kRmsFoldRows][16];
-  const int rg = threadIdx.x >> 4, c4 = threadIdx.x & 15;
-  const int col = (int)blockIdx.x * 64 + c4 * 4;
+  __shared__ f32x4 red[4][4];
+  const int rg = threadIdx.x >> 2, c4 = threadIdx.x & 3, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int col = (int)blockIdx.x * kRmsFoldCols + c4 * 4;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
-  if (col < a.cols) {
+  if (col < a.cols && rg < a.n_part) {
     // eight partial rows are requested at a time; rows past the end re-read row rg and are dropped
     for (int p0 = rg; p0 < a.n_part; p0 += 8 * kRmsFoldRows) {
       f32x4 v[8];
@@ -397,12 +383,14 @@ __global__ __launch_bounds__(256) void rms_fold_kernel(RmsFoldArgs a) {
         if (p0 + j * kRmsFoldRows < a.n_part) s += v[j];
     }
   }
-  red[rg][c4] = s;
-  __syncthreads();
-  if (rg == 0 && col < a.cols) {
-    f32x4 t = red[0][c4];
 #pragma unroll
-    for (int v = 1; v < kRmsFoldRows; ++v) t += red[v][c4];
+  for (int d = 4; d < kWaveSize; d *= 2)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] += __shfl_xor(s[e], d, kWaveSize);
+  if (lane < 4) red[wave][c4] = s;
+  __syncthreads();
+  if (threadIdx.x < 4 && col < a.cols) {
+    const f32x4 t = (red[0][c4] + red[1][c4]) + (red[2][c4] + red[3][c4]);
     u32x2 o;
     o[0] = pack2<DT>(t[0], t[1]);
     o[1] = pack2<DT>(t[2], t[3]);

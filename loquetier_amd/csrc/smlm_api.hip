@@ -1275,19 +1275,24 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
                                  : launch_wgrad<SMLM_DTYPE_BF16, false>(nbj, split, grid, st, wa);
 }
 
-// workgroups of the RMSNorm backward: enough to fill the chip, each with several rows so that
-// the partial sums of dw stay small next to x and g
-// workgroups of the RMSNorm kernels: the forward gives every row group its own workgroup; the
-// backward walks four turns per workgroup (the next rows are fetched while the current ones are
-// worked on), so that its partial sums of dw stay small next to x and g
+static int rms_bwd_threads(int cols) {
+  const int pieces = cols / 8;
+  return pieces >= 1024 ? 1024 : round_up(pieces, kWaveSize);
+}
+// workgroups of the RMSNorm kernels: the forward gives every row group its own workgroup; the backward's fill the
+// chip once (512 threads a CU) with two rows each or more, so that the partial sums of dw stay small next to x and g
 static int rms_blocks(int rows, int cols, bool backward) {
+  int nb, cap = 1 << 22;
   if (cols > kRmsMaxCols) {  // wide rows: a workgroup per row; the backward's partial rows are whole rows of floats
-    const int cap = backward ? 128 : (1 << 22);
-    return rows < 1 ? 1 : (rows < cap ? rows : cap);
+    nb = rows;
+    if (backward) cap = 128;
+  } else if (backward) {
+    const int threads = rms_bwd_threads(cols);
+    nb = ceil_div(rows, 2);
+    cap = threads >= 512 ? 256 : 256 * 512 / threads;
+  } else {
+    nb = ceil_div(rows, cols <= kRmsWaveCols ? 4 : 1);
   }
-  const int rows_per_step = cols <= kRmsWaveCols ? 4 : 1;
-  int nb = ceil_div(rows, rows_per_step * (backward ? 4 : 1));
-  const int cap = backward ? 512 : (1 << 22);
   if (nb > cap) nb = cap;
   return nb < 1 ? 1 : nb;
 }
@@ -1360,19 +1365,18 @@ SMLM_API int smlm_rms_norm_bwd(void* dx, void* dw, const void* g, const void* x,
                      reinterpret_cast<const uint16_t*>(g), reinterpret_cast<const uint16_t*>(x),
                      reinterpret_cast<const uint16_t*>(w), rms, rows, cols};
   const dim3 grid((unsigned)nb);
-  const dim3 bl(256);
   if (cols > kRmsMaxCols)
-    rc = f16 ? launch(rms_bwd_wide_kernel<SMLM_DTYPE_F16>, grid, bl, st, a)
-             : launch(rms_bwd_wide_kernel<SMLM_DTYPE_BF16>, grid, bl, st, a);
-  else if (cols <= kRmsWaveCols)
-    rc = f16 ? launch(rms_bwd_kernel<SMLM_DTYPE_F16, 1>, grid, bl, st, a)
-             : launch(rms_bwd_kernel<SMLM_DTYPE_BF16, 1>, grid, bl, st, a);
+    rc = f16 ? launch(rms_bwd_wide_kernel<SMLM_DTYPE_F16>, grid, dim3(256), st, a)
+             : launch(rms_bwd_wide_kernel<SMLM_DTYPE_BF16>, grid, dim3(256), st, a);
+  else if (cols <= 8192)
+    rc = f16 ? launch(rms_bwd_kernel<SMLM_DTYPE_F16, 1, 2>, grid, dim3(rms_bwd_threads(cols)), st, a)
+             : launch(rms_bwd_kernel<SMLM_DTYPE_BF16, 1, 2>, grid, dim3(rms_bwd_threads(cols)), st, a);
   else
-    rc = f16 ? launch(rms_bwd_kernel<SMLM_DTYPE_F16, 4>, grid, bl, st, a)
-             : launch(rms_bwd_kernel<SMLM_DTYPE_BF16, 4>, grid, bl, st, a);
+    rc = f16 ? launch(rms_bwd_kernel<SMLM_DTYPE_F16, 2, 1>, grid, dim3(1024), st, a)
+             : launch(rms_bwd_kernel<SMLM_DTYPE_BF16, 2, 1>, grid, dim3(1024), st, a);
   if (rc) return rc;
   const RmsFoldArgs fa{reinterpret_cast<uint16_t*>(dw), reinterpret_cast<const float*>(workspace), nb, cols};
-  const dim3 fgrid((unsigned)ceil_div(cols, 64));
+  const dim3 fgrid((unsigned)ceil_div(cols, kRmsFoldCols));
   return f16 ? launch(rms_fold_kernel<SMLM_DTYPE_F16>, fgrid, dim3(256), st, fa)
              : launch(rms_fold_kernel<SMLM_DTYPE_BF16>, fgrid, dim3(256), st, fa);
 }
