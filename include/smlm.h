@@ -293,7 +293,7 @@ typedef struct smlm_dropout {
  *                  for every later call on the stream) and uses it.  The reference sets its
  *                  problems up inside every call as well (precompute_smlm_forward_args,
  *                  kernel_src/csrc/smlm_forward/smlm_forward_cutlass.cuh:31-46,76-79).  With
- *                  n_weights <= 1024, no dropout and either a batch of few rows (the single-tile
+ *                  n_weights <= 1024 and either a batch of few rows (the single-tile
  *                  kernels: below 2048 rows at rank <= 16, 768 at rank <= 32, 512 at rank <= 48,
  *                  128 at rank <= 64, 512 above), S <= 1024 and every h_in >= 2048, or a
  *                  larger batch with S <= 512 and T / 16 + S < 1024, this costs no
@@ -303,11 +303,11 @@ typedef struct smlm_dropout {
  *                  no adapter, see the tile plan above); stages must include SMLM_STAGE_SHRINK.
  *                  smlm_lora_bwd_ex takes the pair (part_indptr, part_adapter) the same way and
  *                  builds its plan inside the dV launch when P <= 512, n_rows / 16 + P < 1024,
- *                  v is given and there is no dropout.
+ *                  v is given and so are, under dropout, the mask's keep bits.
  *   build_seg_key_a, build_seg_key_b (both or neither, with build_seg_indptr, instead of
  *                  build_seg_adapter; smlm_lora_fwd_multi_ex only):
  *                  the plan to build is the one smlm_plan_build2 builds from these two arrays of S
- *                  addresses; with S <= 1024 (and the other limits above) inside the shrink launch.
+ *                  addresses; with S <= 1024 (and the other limits above) and no dropout inside the shrink launch.
  *                  The weight tables of the call have one entry per segment (n_weights = S).
  *   bwd_stages   : (backward entry points) 0 = the whole backward; else a set of SMLM_BWD_* bits: the
  *                  stages of one backward may be issued as separate calls with the same arguments,

@@ -241,29 +241,29 @@ int launch_shrink(int dtype, const ShrinkCfg& c, int S, int groups, hipStream_t 
              : launch_shrink_dt<SMLM_DTYPE_BF16, false>(c.NB, MT, c.NW, grid, st, a);
 }
 
-template <int DT, int THREADS, bool PAIRS>
+template <int DT, int THREADS, bool PAIRS, bool DROP = false>
 int launch_self_planned_nb(int NB, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
   const dim3 block(THREADS);  // U must match shrink_cfg
-  if (NB == 1) return launch(shrink_self_planned_kernel<DT, 1, 4, THREADS, PAIRS>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_self_planned_kernel<DT, 2, 4, THREADS, PAIRS>, grid, block, st, a);
-  return launch(shrink_self_planned_kernel<DT, 4, 2, THREADS, PAIRS>, grid, block, st, a);
+  if (NB == 1) return launch(shrink_self_planned_kernel<DT, 1, 4, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_self_planned_kernel<DT, 2, 4, THREADS, PAIRS, DROP>, grid, block, st, a);
+  return launch(shrink_self_planned_kernel<DT, 4, 2, THREADS, PAIRS, DROP>, grid, block, st, a);
 }
 
-template <int DT, bool WKN, int THREADS, bool PAIRS>
+template <int DT, bool WKN, int THREADS, bool PAIRS, bool DROP = false>
 int launch_self_planned_block_nb(int NB, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
   const dim3 block(THREADS);  // U must match shrink_cfg
-  if (NB == 1) return launch(shrink_block_self_planned_kernel<DT, 1, 4, WKN, THREADS, PAIRS>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_block_self_planned_kernel<DT, 2, 4, WKN, THREADS, PAIRS>, grid, block, st, a);
-  if (NB == 8) return launch(shrink_block_self_planned_kernel<DT, 8, 2, WKN, THREADS, PAIRS>, grid, block, st, a);
-  return launch(shrink_block_self_planned_kernel<DT, 4, 4, WKN, THREADS, PAIRS>, grid, block, st, a);
+  if (NB == 1) return launch(shrink_block_self_planned_kernel<DT, 1, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_block_self_planned_kernel<DT, 2, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 8) return launch(shrink_block_self_planned_kernel<DT, 8, 2, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  return launch(shrink_block_self_planned_kernel<DT, 4, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
 }
-template <int DT, bool WKN, bool PAIRS>
+template <int DT, bool WKN, bool PAIRS, bool DROP = false>
 int launch_self_planned_block(int NB, int S, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
-  if (S <= kFwdThreads) return launch_self_planned_block_nb<DT, WKN, kFwdThreads, PAIRS>(NB, grid, st, a);
+  if (S <= kFwdThreads) return launch_self_planned_block_nb<DT, WKN, kFwdThreads, PAIRS, DROP>(NB, grid, st, a);
   // more segments than the four-wave workgroup has threads: two such groups a workgroup, each
   // taking one of two neighbouring k slices (the caller has checked that the splits are even)
   grid.x = (grid.x + 1) / 2;
-  return launch_self_planned_block_nb<DT, WKN, 2 * kFwdThreads, PAIRS>(NB, grid, st, a);
+  return launch_self_planned_block_nb<DT, WKN, 2 * kFwdThreads, PAIRS, DROP>(NB, grid, st, a);
 }
 
 // batches this route takes: few enough segments for the plan-building workgroups of the launch
@@ -278,17 +278,22 @@ bool self_planned_ok(int T, int S, int n_weights, int nt_max, int mt) {
 
 template <int DT>
 int launch_self_planned_dt(bool pairs, const ShrinkCfg& c, int S, dim3 grid, hipStream_t st, const SelfPlanArgs& sp) {
+  const bool drop = sp.sh.drop.seg_p != nullptr;
+  if (drop && (pairs || sp.sh.w_kn)) return SMLM_ERR_ARG;  // (no caller: their plans are built with a launch)
   if (c.MT == 1 && S > kSelfPlanThreads) {
     // more segments than the eight-wave workgroup has threads: workgroups of two such groups of
     // waves, each taking two neighbouring k slices (the caller has checked that the splits are even)
     grid.x = (grid.x + 1) / 2;
+    if (drop) return launch_self_planned_nb<DT, 2 * kSelfPlanThreads, false, true>(c.NB, grid, st, sp);
     return pairs ? launch_self_planned_nb<DT, 2 * kSelfPlanThreads, true>(c.NB, grid, st, sp)
                  : launch_self_planned_nb<DT, 2 * kSelfPlanThreads, false>(c.NB, grid, st, sp);
   }
   if (c.MT > 1 && sp.sh.w_kn) return launch_self_planned_block<DT, true, false>(c.NB, S, grid, st, sp);
+  if (c.MT > 1 && drop) return launch_self_planned_block<DT, false, false, true>(c.NB, S, grid, st, sp);
   if (c.MT > 1)
     return pairs ? launch_self_planned_block<DT, false, true>(c.NB, S, grid, st, sp)
                  : launch_self_planned_block<DT, false, false>(c.NB, S, grid, st, sp);
+  if (drop) return launch_self_planned_nb<DT, kSelfPlanThreads, false, true>(c.NB, grid, st, sp);
   return pairs ? launch_self_planned_nb<DT, kSelfPlanThreads, true>(c.NB, grid, st, sp)
                : launch_self_planned_nb<DT, kSelfPlanThreads, false>(c.NB, grid, st, sp);
 }
@@ -923,13 +928,16 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
       w += align_up((size_t)T * r * 2, 256);
     }
   }
-  // A plan still to be built (opts->build_*): decode batches build it inside the shrink launch,
-  // every other batch with the plan launch first.
+  // A plan still to be built (opts->build_*): inside the shrink launch where the batch is within its limits, else
+  // with the plan launch first -- as under dropout with plans keyed by pairs of addresses, which no kernel of that
+  // kind takes.  (2786 rows, two projections 4096 -> 4096 and 1024 at rank 32, dropout: forward + backward with two
+  // plan launches of 5.6 us 116.0 us, both plans built in the shrinks 106.0 us.)
   PlanSortArgs build{pv, build_s, build_k, build_kind, S, next_pow2(S), build_k2};
   bool even_splits = true;  // (the decode route pairs k slices up beyond 512 segments)
   for (int i = 0; i < n_proj; ++i) even_splits = even_splits && (vsplit[i] % 2 == 0);
   // (both routes pair k slices up in one workgroup beyond 512 / 256 segments)
-  const bool self_planned = build_s && !drop.seg_p && self_planned_ok(T, S, n_weights, pv.nt_max, mt) &&
+  const bool self_planned = build_s && (!drop.seg_p || build_kind == SMLM_KEY_I32) &&
+                            self_planned_ok(T, S, n_weights, pv.nt_max, mt) &&
                             (mt > 1 ? (S <= kFwdThreads || even_splits)
                                                    : (expand_folds && (S <= kSelfPlanThreads || even_splits)));
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, build_kind, S, st, build_k2))) return rc;
@@ -1069,7 +1077,8 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   plan_carve(const_cast<void*>(plan), n_rows, P, &pv);
 
   // A plan still to be built (opts->build_*): the dV shrink builds it inside its launch when it is
-  // the first launch to use it (tile-block route, v given, no dropout); else the plan launch first.
+  // the first launch to use it (tile-block route, v given, the mask's keep bits given under dropout); else the
+  // plan launch first.
   const int32_t* build_s = opts ? opts->build_seg_indptr : nullptr;
   const int32_t* build_k = opts ? opts->build_seg_adapter : nullptr;
   if ((build_s != nullptr) != (build_k != nullptr)) return SMLM_ERR_ARG;
@@ -1078,7 +1087,7 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   constexpr int mt = kBlkTiles;
   bool even_dv = true;  // (k slices in pairs beyond 256 partitions)
   for (int i = 0; i < n_proj; ++i) even_dv = even_dv && shrink_cfg(n_rows, h_out[i], r, kFwdWaves, true, mt).ksplit % 2 == 0;
-  const bool self_planned = build_s && have_v && !drop.seg_p &&
+  const bool self_planned = build_s && have_v && (!drop.seg_p || drop.bits) &&
                             self_planned_ok(n_rows, P, NA, pv.nt_max, mt) && (P <= kFwdThreads || even_dv);
   const bool products = (stages & SMLM_BWD_PRODUCTS) != 0;
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, SMLM_KEY_I32, P, st))) return rc;

@@ -244,7 +244,8 @@ union SelfPlanLds {
   f32x4 red[THREADS / kWaveSize][NB][kWaveSize];    // ... which reuse the finder's memory when the two do not fit side by side
 };
 
-template <int DT, int NB, int U, int THREADS, bool PAIRS = false>
+// DROP (plans keyed by ids): dropout of the training rows of x, as shrink_kernel applies it.
+template <int DT, int NB, int U, int THREADS, bool PAIRS = false, bool DROP = false>
 __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanArgs a) {
   static_assert(THREADS == kSelfPlanThreads || THREADS == 2 * kSelfPlanThreads, "one or two groups of eight waves");
   __shared__ SelfPlanLds<NB, THREADS, PAIRS> sm;
@@ -307,6 +308,9 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   find_rows<THREADS, 1, PAIRS>(F, seg, un);
   const int row = F.rows[c], rseg = F.rseg[c];
   if (kOverlay) __syncthreads();  // every wave holds its tile: the finder's LDS turns into the sum's staging area
+  DropRow dr{};
+  DropArgs dp{};
+  if (DROP) dp = drop_proj(a.sh.drop, pj), dr = drop_row_of(dp, row, rseg);
 
   // ---- the product, as the eight-wave shrink_kernel does it
   f32x4 acc[NB];
@@ -322,9 +326,12 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
     }
     if (k != kbeg) load_w(k, wf);  // uniform over the wave (k is usually one batch)
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      const int kk = k + 32 * u + 8 * g;
+      const u32x4 xu = DROP ? drop8<DT>(xf[u], dp, dr, row, kk >> 3, P.drop_bits, P.d_in >> 3, zb == 0 && kk < kend) : xf[u];
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(wf[nb][u], xf[u], acc[nb]);
+      for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(wf[nb][u], xu, acc[nb]);
+    }
   }
 
   // decided at compile time; every group of eight waves has its own part of the area
@@ -379,7 +386,7 @@ union SelfPlanBlockLds {
   SelfPlanBlockStage<NB, U, WKN, THREADS / kFwdThreads> stage;  // ... then the staged weight batches
 };
 
-template <int DT, int NB, int U, bool WKN, int THREADS, bool PAIRS = false>
+template <int DT, int NB, int U, bool WKN, int THREADS, bool PAIRS = false, bool DROP = false>
 __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(SelfPlanArgs a) {
   static_assert(THREADS == kFwdThreads || THREADS == 2 * kFwdThreads, "one or two groups of four waves");
   constexpr int GROUPS = THREADS / kFwdThreads;
@@ -465,6 +472,9 @@ __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(Self
   const int row = active ? sm.find.rows[wave * kTileRows + c] : -1;
   const int rseg = active ? sm.find.rseg[wave * kTileRows + c] : -1;
   const uint16_t* xrow = P.x + (long)(row < 0 ? 0 : row) * P.d_in;
+  DropRow dr{};
+  DropArgs dp{};
+  if (DROP) dp = drop_proj(a.sh.drop, pj), dr = drop_row_of(dp, row, rseg);
   auto load_x = [&](int kb, u32x4 (&xf)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -492,8 +502,10 @@ __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(Self
     if (active) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        const int kk = kb + 32 * u + 8 * g;
+        const u32x4 xu = DROP ? drop8<DT>(xf[u], dp, dr, row, kk >> 3, P.drop_bits, P.d_in >> 3, zb == 0 && kk < kend) : xf[u];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(weight_frag(buf, u, nb), xf[u], acc[nb]);
+        for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(weight_frag(buf, u, nb), xu, acc[nb]);
       }
     }
     stage_w(buf ^ 1, wn);

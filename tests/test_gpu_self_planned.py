@@ -385,3 +385,59 @@ def test_deferred_plans_with_true_ranks(K, gpu_device, rows, packed):
     for a, b in zip(*outs):
         assert torch.equal(a, b)
     assert not torch.isnan(outs[1][2].float()).any()
+
+
+# name, h_in, rank, lengths of the training segments, of the others; adapters
+DROP_CASES = [
+    ("single-tiles", 2048, 16, [20, 17, 1, 33], [1] * 40, 5),
+    ("single-tiles-600-segments", 4096, 32, [3] * 30, [1] * 570, 7),
+    ("tile-blocks", 1024, 32, [300, 257, 15], [1] * 30 + [200], 5),
+    ("tile-blocks-400-segments", 1024, 64, [3] * 60, [2] * 340, 9),
+    ("tile-blocks-rank-128", 512, 128, [300, 1], [1] * 20 + [250], 4),
+    ("odd-width", 1160, 24, [700, 30], [1] * 20 + [60], 6),
+]
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("case", DROP_CASES, ids=[c[0] for c in DROP_CASES])
+def test_deferred_plans_under_dropout(K, gpu_device, case, dt):
+    """Outputs, v, the mask's keep bits, the plans' bytes and the gradients equal those over plans built beforehand,
+    bit for bit; probabilities include 0, one below the mask's resolution and 1."""
+    name, h_in, r, train, serve, NA = case
+    d, tdt, h_out = gpu_device, TDT[dt], 192
+    lens = train + serve
+    seg = [0]
+    for l in lens:
+        seg.append(seg[-1] + l)
+    T, P = seg[-1], len(train)
+    n = seg[P]
+    ids = [i % NA for i in range(len(lens))]
+    gen = torch.Generator().manual_seed(5)
+    A = [(torch.randn(r, h_in, generator=gen) / h_in ** 0.5).to(tdt).to(d) for _ in range(NA)]
+    B = [(torch.randn(h_out, r, generator=gen) / r ** 0.5).to(tdt).to(d) for _ in range(NA)]
+    x, y0 = torch.randn(T, h_in, generator=gen).to(tdt).to(d), torch.randn(T, h_out, generator=gen).to(tdt).to(d)
+    g = torch.randn(n, h_out, generator=gen).to(tdt).to(d)
+    int32 = lambda v: torch.tensor(v, dtype=torch.int32, device=d)
+    ad_p = [(0.1, 0.5, 1.0, 0.0, 1e-6)[a % 5] for a in range(NA)]
+    seg_p = torch.tensor([ad_p[a] if i < P else 0.0 for i, a in enumerate(ids)], device=d)
+    scale = torch.full((len(lens),), 1.5, device=d)
+    seg_t, ids_t, parts, part_ad = int32(seg), int32(ids), int32(seg[:P + 1]), int32(ids[:P])
+    ta, tb = ptrs(A, d), ptrs(B, d)
+
+    def run(defer):
+        bits = torch.zeros(K.DropoutSpec.mask_nbytes(n, [h_in]), dtype=torch.uint8, device=d)
+        new_plan = lambda *a: K.SegmentPlan(*a, buf=torch.full((max(K.SegmentPlan.nbytes(a[2], a[0].numel() - 1), 64),), 0xA5,
+                                                               dtype=torch.uint8, device=d), defer=defer)
+        plan, bplan = new_plan(seg_t, ids_t, T), new_plan(parts, part_ad, n)
+        y, v = y0.clone(), torch.zeros(T, r, dtype=tdt, device=d)
+        K.smlm_lora_forward_multi([y], [x], [ta], [tb], plan, r, seg_scale=scale, beta=1.0, v_out=[v],
+                                  dropout=K.DropoutSpec(seg_p, n, 17, 3, bits))
+        dA, dB = [torch.full_like(a, 5.0) for a in A], [torch.full_like(b, 5.0) for b in B]
+        dx = torch.full((n, h_in), 5.0, dtype=tdt, device=d)
+        K.smlm_lora_backward_multi([dx], [ptrs(dA, d)], [ptrs(dB, d)], [g], [x], [v], [ta], [tb], bplan, r, scale[:P].contiguous(),
+                                   dropout=K.DropoutSpec(seg_p[:P].contiguous(), n, 17, 3, bits))
+        torch.cuda.synchronize()
+        return [y, v, bits, plan.buf, bplan.buf, dx] + dA + dB
+
+    for a, b in zip(run(False), run(True)):
+        assert torch.equal(a, b)
