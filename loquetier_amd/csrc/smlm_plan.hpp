@@ -163,7 +163,8 @@ __device__ __forceinline__ int usable_kind(const void* key, int key_kind, int S,
 // owns (pair i of a wave's 64 pairs lies in keys [128 w, 128 w + 128), in every pass of the loop over i), and
 // a wave's LDS accesses complete in order: between two such stages the waves need not meet, which takes the
 // barriers of 56 of the 66 stages of a 2048-key sort away (1075 segments: the launch 27.1 -> 25.6 us; placing every
-// key by counting the keys below it instead, all lanes reading one LDS address at a time: 38.5 us).
+// key by counting the keys below it instead, all lanes reading one LDS address at a time: 38.5 us).  It serves plans
+// keyed by addresses; ids are sorted by radix_sort_ids.
 template <bool IN_LDS = false, typename KeyArray>
 __device__ __forceinline__ void bitonic_sort(KeyArray K, int N) {
   bool own = false;  // the stage before this one was one of those
@@ -189,6 +190,90 @@ __device__ __forceinline__ void bitonic_sort(KeyArray K, int N) {
     }
   }
   __syncthreads();
+}
+
+// Sort keys of the S <= kPlanLdsKeys segments of a plan keyed by ids, ascending, into K: counting passes over eight
+// bits of the id, as many as the largest id needs (one for ids below 256).  Keys of equal id keep their order, so
+// the segment index in a key's low bits takes no pass.  A wave owns a run of segments and numbers the equal digits
+// of 64 of them at a time by ballots; `hist` holds the counts by (digit, wave), whose running sum is where a wave's
+// first key of a digit goes.
+// Bound by the round trips between the barriers of one workgroup: 1075 segments over 64 adapters, the launch 28.2 us
+// with the bitonic sort (66 stages) and a scan for tiles and one for blocks, 10.3 us with this and one scan for both.
+constexpr int kRadix = 256, kPlanWaves = kPlanThreads / kWaveSize;
+constexpr int kRadixKeys = kPlanLdsKeys / kPlanThreads;  // keys a thread holds
+__device__ __forceinline__ void radix_sort_ids(const int32_t* ids, int S, uint64_t (&K)[kPlanLdsKeys],
+                                               uint32_t (&hist)[kRadix * kPlanWaves], uint64_t* wave_tot, int* wide) {
+  static_assert(kPlanLdsKeys % kPlanThreads == 0 && kRadix * kPlanWaves == 4 * kPlanThreads, "whole shares a thread");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int run = ((S + kPlanThreads - 1) / kPlanThreads) * kWaveSize;  // segments of a wave, whole steps of 64
+  uint64_t key[kRadixKeys];
+  uint32_t top = 0;
+#pragma unroll
+  for (int j = 0; j < kRadixKeys; ++j) {
+    const int i = wave * run + kWaveSize * j + lane;
+    key[j] = ~0ull;
+    if (kWaveSize * j < run && i < S) {
+      const uint32_t id = (uint32_t)ids[i];
+      top |= id;
+      key[j] = ((uint64_t)id << kSegBits) | (uint32_t)i;
+    }
+  }
+  if (tid < 4) wide[tid] = 0;
+  __syncthreads();
+  for (int q = 1; q < 4; ++q)
+    if (top >> (8 * q)) wide[q] = 1;  // (every store writes the same value)
+  __syncthreads();
+  const int passes = wide[3] ? 4 : (wide[2] ? 3 : (wide[1] ? 2 : 1));
+
+  for (int pass = 0; pass < passes; ++pass) {  // uniform over the workgroup
+    if (pass) {
+#pragma unroll
+      for (int j = 0; j < kRadixKeys; ++j) {
+        const int i = wave * run + kWaveSize * j + lane;
+        if (kWaveSize * j < run && i < S) key[j] = K[i];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) hist[tid + kPlanThreads * e] = 0;
+    __syncthreads();
+    int at[kRadixKeys];
+#pragma unroll
+    for (int j = 0; j < kRadixKeys; ++j) {
+      at[j] = 0;
+      if (kWaveSize * j >= run) continue;  // uniform over the workgroup
+      const bool valid = wave * run + kWaveSize * j + lane < S;
+      const int digit = (int)(key[j] >> (kSegBits + 8 * pass)) & (kRadix - 1);
+      uint64_t same = __ballot(valid);
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const uint64_t set = __ballot((digit >> b) & 1);
+        same &= ((digit >> b) & 1) ? set : ~set;
+      }
+      const int before = __popcll(same & ((1ull << lane) - 1));
+      if (valid) at[j] = (int)hist[digit * kPlanWaves + wave] + before;
+      // (a wave's LDS accesses are served in order: all its lanes have read the count before one raises it)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (valid && before == 0) hist[digit * kPlanWaves + wave] += (uint32_t)__popcll(same);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint32_t n[4], sum = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) n[e] = hist[4 * tid + e], sum += n[e];
+    uint32_t first = (uint32_t)block_scan_incl(sum, wave_tot) - sum;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) hist[4 * tid + e] = first, first += n[e];
+    __syncthreads();  // (every thread has read its keys of this pass by now: K may be written)
+#pragma unroll
+    for (int j = 0; j < kRadixKeys; ++j) {
+      if (kWaveSize * j >= run || wave * run + kWaveSize * j + lane >= S) continue;
+      const int digit = (int)(key[j] >> (kSegBits + 8 * pass)) & (kRadix - 1);
+      K[hist[digit * kPlanWaves + wave] + at[j]] = key[j];
+    }
+    __syncthreads();
+  }
 }
 
 // last index i in [0, n) with a[i] <= q, given a[0] <= q < a[n]
@@ -445,6 +530,8 @@ __global__ __launch_bounds__(kPlanThreads) void plan_sort_kernel(PlanSortArgs ar
   __shared__ uint64_t wave_tot[17];
   __shared__ int bad_key;
   __shared__ uint64_t carry;
+  __shared__ uint32_t hist[USE_LDS ? kRadix * kPlanWaves : 1];
+  __shared__ int wide[4];
   const PlanView pv = args.pv;
   const int32_t* __restrict__ s = args.s;
   const int S = args.S, N = args.N, tid = threadIdx.x;
@@ -454,10 +541,14 @@ __global__ __launch_bounds__(kPlanThreads) void plan_sort_kernel(PlanSortArgs ar
   const uint64_t* key2 = (args.key_kind == SMLM_KEY_PTR2 && kind == SMLM_KEY_PTR)
                              ? reinterpret_cast<const uint64_t*>(args.key2) : nullptr;
 
-  if (USE_LDS) {
-    for (int i = tid; i < N; i += kPlanThreads) lds_keys[i] = i < S ? make_key(args.key, kind, i) : ~0ull;
-    __syncthreads();
-    if (kind != SMLM_KEY_NONE) bitonic_sort<true>(lds_keys, N);
+  if constexpr (USE_LDS) {
+    if (kind == SMLM_KEY_I32) {
+      radix_sort_ids(reinterpret_cast<const int32_t*>(args.key), S, lds_keys, hist, wave_tot, wide);
+    } else {
+      for (int i = tid; i < N; i += kPlanThreads) lds_keys[i] = i < S ? make_key(args.key, kind, i) : ~0ull;
+      __syncthreads();
+      if (kind != SMLM_KEY_NONE) bitonic_sort<true>(lds_keys, N);
+    }
     for (int i = tid; i < S; i += kPlanThreads) pv.sort_keys[i] = lds_keys[i];
   } else {
     for (int i = tid; i < N; i += kPlanThreads) pv.sort_keys[i] = i < S ? make_key(args.key, kind, i) : ~0ull;
@@ -465,7 +556,10 @@ __global__ __launch_bounds__(kPlanThreads) void plan_sort_kernel(PlanSortArgs ar
     if (kind != SMLM_KEY_NONE) bitonic_sort(pv.sort_keys, N);
   }
   __syncthreads();
-  const uint64_t* K = pv.sort_keys;  // global from here on
+  auto sorted_key = [&](int p) -> uint64_t {
+    if constexpr (USE_LDS) return lds_keys[p];
+    else return pv.sort_keys[p];
+  };
 
   // Pass A: gathered-row position of every sorted segment, group heads.
   if (tid == 0) carry = 0;
@@ -478,15 +572,16 @@ __global__ __launch_bounds__(kPlanThreads) void plan_sort_kernel(PlanSortArgs ar
     uint64_t gk = 0;
     bool head = false;
     if (valid) {
-      const uint64_t k = K[p];
+      const uint64_t k = sorted_key(p);
       seg = (int)(k & (kMaxSegments - 1));
       gk = k >> kSegBits;
       len = s[seg + 1] - s[seg];
       if (len < 0) len = 0;
       head = true;
       if (p > 0) {
-        head = (K[p - 1] >> kSegBits) != gk;
-        if (!head && key2) head = key2[(int)(K[p - 1] & (kMaxSegments - 1))] != key2[seg];
+        const uint64_t prev = sorted_key(p - 1);
+        head = (prev >> kSegBits) != gk;
+        if (!head && key2) head = key2[(int)(prev & (kMaxSegments - 1))] != key2[seg];
       }
     }
     const uint64_t v = (uint64_t)len | ((uint64_t)(head ? 1 : 0) << 32);
@@ -521,41 +616,29 @@ __global__ __launch_bounds__(kPlanThreads) void plan_sort_kernel(PlanSortArgs ar
   }
   __syncthreads();
 
-  // Pass B: tiles per group -> first tile of each group.
+  // Pass B: tiles and tile blocks per group -> first tile and first block of each group (one scan: tiles in the low
+  // half, blocks in the high half).
   if (tid == 0) carry = 0;
   __syncthreads();
   for (int base = 0; base < NG; base += kPlanThreads) {
     const int G = base + tid;
     uint64_t nt = 0;
     if (G < NG) nt = (uint64_t)((pv.grp_row[G + 1] - pv.grp_row[G] + kTileRows - 1) / kTileRows);
-    const uint64_t incl = block_scan_incl(nt, wave_tot) + carry;
-    if (G < NG) pv.grp_tile[G] = (int)(incl - nt);
+    const uint64_t both = nt | ((nt + kBlkTiles - 1) / kBlkTiles) << 32;
+    const uint64_t excl = block_scan_incl(both, wave_tot) + carry - both;
+    if (G < NG) {
+      pv.grp_tile[G] = (int)(uint32_t)excl;
+      pv.grp_blk[G] = (int)(excl >> 32);
+    }
     __syncthreads();
     if (tid == 0) carry += wave_tot[16];
     __syncthreads();
   }
   if (tid == 0) {
-    pv.grp_tile[NG] = (int)carry;
-    pv.hdr[0] = (int)carry;
-  }
-  __syncthreads();
-
-  // Pass C: tile blocks per group -> first block of each group.
-  if (tid == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < NG; base += kPlanThreads) {
-    const int G = base + tid;
-    uint64_t nb = 0;
-    if (G < NG) nb = (uint64_t)((pv.grp_tile[G + 1] - pv.grp_tile[G] + kBlkTiles - 1) / kBlkTiles);
-    const uint64_t incl = block_scan_incl(nb, wave_tot) + carry;
-    if (G < NG) pv.grp_blk[G] = (int)(incl - nb);
-    __syncthreads();
-    if (tid == 0) carry += wave_tot[16];
-    __syncthreads();
-  }
-  if (tid == 0) {
-    pv.grp_blk[NG] = (int)carry;
-    pv.hdr[4] = (int)carry;
+    pv.grp_tile[NG] = (int)(uint32_t)carry;
+    pv.hdr[0] = (int)(uint32_t)carry;
+    pv.grp_blk[NG] = (int)(carry >> 32);
+    pv.hdr[4] = (int)(carry >> 32);
   }
 }
 

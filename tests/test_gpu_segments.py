@@ -135,3 +135,46 @@ def test_layer_from_device_built_segments(K, oracle, gpu_device):
         with torch.no_grad():
             outs.append(layer(x))
     assert torch.equal(outs[0], outs[1])
+
+
+ID_PATTERNS = {
+    "few": lambda rng, n: rng.integers(0, 64, n),
+    "one": lambda rng, n: np.full(n, 255),
+    "distinct": lambda rng, n: rng.permutation(n),
+    "three-bytes": lambda rng, n: rng.integers(0, 200000, n),
+    "negative": lambda rng, n: rng.integers(-5, 5, n),
+}
+
+
+@pytest.mark.parametrize("S", [1025, 2047, 2048, 2049, 4095, 4096])
+@pytest.mark.parametrize("pattern", list(ID_PATTERNS))
+def test_plans_of_many_segments(gpu_device, S, pattern):
+    """The tables of a plan of 1025 to 4096 segments (sorted by counting passes over the ids, as many as the largest
+    takes) equal those made on the host; ids sort as unsigned numbers, equal ones keep their order."""
+    from loquetier_amd.ops import _kernels as K
+    rng = np.random.default_rng(S)
+    ids = ID_PATTERNS[pattern](rng, S).astype(np.int32)
+    lens = rng.integers(0, 4, S)
+    lens[rng.integers(0, S, 3)] = 150
+    seg = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(seg[-1])
+    plan = K.SegmentPlan(torch.from_numpy(seg).to(gpu_device), torch.from_numpy(ids).to(gpu_device), T)
+    buf = plan.buf.cpu().numpy()
+    align = lambda n: (n + 255) // 256 * 256
+    tables = [buf[256 + i * align(4 * (S + 1)):][:4 * (S + 1)].view(np.int32) for i in range(7)]
+    sorted_seg, rowpos, grp_tile, grp_row, grp_seg, grp_id, grp_blk = tables
+
+    order = np.argsort(ids.view(np.uint32), kind="stable")
+    rows = np.concatenate([[0], np.cumsum(lens[order])])
+    heads = np.flatnonzero(np.concatenate([[True], np.diff(ids[order]) != 0]))
+    grp_rows = np.concatenate([rows[heads], [T]])
+    tiles = (np.diff(grp_rows) + 15) // 16
+    NG = len(heads)
+    assert np.array_equal(sorted_seg[:S], order)
+    assert np.array_equal(rowpos, rows)
+    assert np.array_equal(grp_row[:NG + 1], grp_rows)
+    assert np.array_equal(grp_seg[:NG], order[heads])
+    assert np.array_equal(grp_id[:NG], ids[order][heads])
+    assert np.array_equal(grp_tile[:NG + 1], np.concatenate([[0], np.cumsum(tiles)]))
+    assert np.array_equal(grp_blk[:NG + 1], np.concatenate([[0], np.cumsum((tiles + 3) // 4)]))
+    assert list(plan.header()) == [int(tiles.sum()), NG, T, 1]
