@@ -169,7 +169,6 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
   __shared__ dots_t part[2][16];  // the rows' dots by wave, two halves in turn
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = (int)blockDim.x >> 6;
   const float inv_n = 1.0f / (float)a.cols;
-  const u32x4 zero = {0u, 0u, 0u, 0u};
   const int row0 = (int)((long)blockIdx.x * a.rows / gridDim.x), row1 = (int)((long)(blockIdx.x + 1) * a.rows / gridDim.x);
 
   int col[CH];
@@ -182,7 +181,6 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     ok[i] = col[i] < a.cols;
     if (!ok[i]) col[i] = 0;
     wv[i] = ldg16(a.w + col[i]);
-    if (!ok[i]) wv[i] = zero;  // (the columns past the row then add nothing to a dot)
 #pragma unroll
     for (int e = 0; e < 8; ++e) dw[i][e] = 0.0f;
   }
@@ -220,8 +218,10 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
         unpack8<DT>(xv[t][i], xf);
         unpack8<DT>(gv[t][i], gf);
         unpack8<DT>(wv[i], wf);
+        float d = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) dot += gf[e] * wf[e] * xf[e];
+        for (int e = 0; e < 8; ++e) d += gf[e] * wf[e] * xf[e];
+        dot += ok[i] ? d : 0.0f;  // (a column read past the row is column 0, whose g or x may be infinite or NaN)
       }
       dots[t] = wave_sum_f32(dot);
     }

@@ -34,3 +34,20 @@ def test_backward(K, oracle, gpu_device, dt, rows, cols):
         assert within_ulps(to_np(dx), want_dx, dt, 2)
         # dw sums `rows` terms in float in another order than the oracle's double
         assert np.all(np.abs(to_np(dw) - want_dw) <= 1.5 * ULP[dt] * np.maximum(np.abs(want_dw), np.sqrt(rows) * 2.0 ** -6))
+
+
+@pytest.mark.parametrize("cols", [72, 512, 3000, 8200])
+def test_backward_infinite_gradient(K, gpu_device, cols):
+    # an infinite g in the first column makes every dx of its row infinite, with the sign the formula gives it, and its
+    # own NaN; threads beyond the row's last column add nothing to the dot
+    x = torch.ones(3, cols)
+    g = torch.full((3, cols), 0.5)
+    g[1, 0] = float("inf")
+    xd, gd = (t.to(torch.bfloat16).to(gpu_device) for t in (x, g))
+    w, rms = torch.ones(cols, dtype=torch.bfloat16, device=gpu_device), torch.ones(3, device=gpu_device)
+    dx, dw = torch.empty_like(xd), torch.empty_like(w)
+    K.rms_norm_backward(dx, dw, gd, xd, w, rms)
+    got = dx.float().cpu()
+    assert torch.isnan(got[1, 0]) and (got[1, 1:] == float("-inf")).all()
+    assert (got[[0, 2]].abs() < 2.0 ** -20).all()  # g - x * mean(g * x), 1 / cols rounded to float
+    assert dw[0].item() == float("inf") and (dw[1:].float() == 1.5).all()
