@@ -1271,7 +1271,7 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   wa.packed = packed;
   wa.drop = drop;  // dA against the dropped x
   // ranks above 64 are covered 64 at a time by workgroups of their own
-  const int nbj = r > 64 ? 4 : ceil_div(r, 16);
+  const int nbj = r <= 16 ? 1 : (r <= 32 ? 2 : 4);  // what launch_wgrad has kernels for
   // (64 ranks a workgroup, or what a dA workgroup of the launched kernel takes when that is less)
   const int z_per_64 = nbj / wgrad_nbj_a(nbj, split ? 4 : 1, drop.seg_p != nullptr);
   wa.units = units;

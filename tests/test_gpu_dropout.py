@@ -164,17 +164,19 @@ BWD_CASES = [
 ]
 
 
-def run_backward(K, d, dt, x, A, B, g, tp, part_ad, r, spec, v=None):
+def run_backward(K, d, dt, x, A, B, g, tp, part_ad, r, spec, v=None, ranks=None):
+    # ranks: the adapters are handed over stored at their own ranks
     n_rows = tp[-1]
     xd, gd = dev_t(x, dt, d), dev_t(g, dt, d)
     Ad, Bd = [dev_t(a, dt, d) for a in A], [dev_t(b, dt, d) for b in B]
-    dA, dB = [torch.empty_like(a) for a in Ad], [torch.empty_like(b) for b in Bd]
+    dA, dB = [torch.full_like(a, 9.0) for a in Ad], [torch.full_like(b, 9.0) for b in Bd]
     dx = torch.full((n_rows + 3, x.shape[1]), 9.0, dtype=TDT[dt], device=d)
     pi = torch.tensor(tp, dtype=torch.int32, device=d)
     pa = torch.tensor(part_ad, dtype=torch.int32, device=d)
     plan = K.SegmentPlan(pi, pa, n_rows)
+    rank_t = None if ranks is None else torch.tensor(ranks, dtype=torch.int32, device=d)
     K.smlm_lora_backward(dx, ptrs(dA, d), ptrs(dB, d), gd, xd, v, ptrs(Ad, d), ptrs(Bd, d), plan, r,
-                         dropout=spec)
+                         dropout=spec, adapter_rank=rank_t, packed_ranks=ranks is not None)
     return to_np(dx), [to_np(t) for t in dA], [to_np(t) for t in dB]
 
 
@@ -228,6 +230,35 @@ def test_backward_dropout_exact(K, oracle, gpu_device, case, dt, with_v, with_bi
         rows = sum(tp[i + 1] - tp[i] for i in range(len(part_ad)) if part_ad[i] == a)
         if rows:
             assert np.array_equal(dA_plain[a], dA[a]) == (ad_p[a] == 0.0)
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("packed", [False, True], ids=["padded", "packed"])
+@pytest.mark.parametrize("tp", [[0, 33, 90], [0, 1100, 2300]], ids=["one-wave", "four-waves"])
+@pytest.mark.parametrize("r", [40, 48, 56])
+def test_backward_dropout_ranks_between_32_and_64(K, oracle, gpu_device, r, tp, packed, dt):
+    """Ranks of three and four blocks of 16: the weight gradient's dA workgroups take 32 ranks each under dropout
+    when an adapter has few rows (one-wave workgroups), 64 when it has many."""
+    d = gpu_device
+    part_ad, h_in, h_out, n_rows = [0, 1], 192, 136, tp[-1]
+    ranks = [r, 8 if r == 48 else 32] if packed else [r, r]
+    rng = np.random.default_rng(33)
+    x = dyadic(rng, (n_rows, h_in), 16, 8)
+    A = [dyadic(rng, (q, h_in), 8, 64) for q in ranks]
+    B = [dyadic(rng, (h_out, q), 8, 8) for q in ranks]
+    Ap = [np.pad(a, [(0, r - a.shape[0]), (0, 0)]) for a in A]
+    Bp = [np.pad(b, [(0, 0), (0, r - b.shape[1])]) for b in B]
+    g = dyadic(rng, (n_rows, h_out), 16, 8)
+    seg_p = np.array([0.5, 0.5], np.float32)
+    spec = K.DropoutSpec(torch.from_numpy(seg_p).to(d), n_rows, 7, 3)
+    rp = row_probs(tp, seg_p, n_rows, n_rows)
+    xdrop = oracle.dropout_rows(x, rp, 7, 3, dt)
+    dx, dA, dB = run_backward(K, d, dt, x, A, B, g, tp, part_ad, r, spec, ranks=ranks if packed else None)
+    gx, ga, gb = oracle.add_lora_backward(g, xdrop, Ap, Bp, tp, part_ad, dt)
+    assert np.array_equal(dx[:n_rows], oracle.dropout_rows(gx, rp, 7, 3, dt))
+    for a in range(2):
+        assert np.array_equal(dA[a], ga[a][:ranks[a]]), f"dA[{a}]"
+        assert np.array_equal(dB[a], gb[a][:, :ranks[a]]), f"dB[{a}]"
 
 
 @pytest.mark.parametrize("dt", ["fp16", "bf16"])

@@ -117,8 +117,8 @@ def test_random_backward(K, oracle, gpu_device, seed):
     seg_p = ad_p[part_ad]
     xd, gd = dev_t(x, dt, d), dev_t(g, dt, d)
     Ad, Bd = [dev_t(a, dt, d) for a in A], [dev_t(b, dt, d) for b in B]
-    dA, dB = [torch.empty_like(a) for a in Ad], [torch.empty_like(b) for b in Bd]
-    dx = torch.empty(n_rows, h_in, dtype=TDT[dt], device=d)
+    dA, dB = [torch.full_like(a, 9.0) for a in Ad], [torch.full_like(b, 9.0) for b in Bd]
+    dx = torch.full((n_rows, h_in), 9.0, dtype=TDT[dt], device=d)
     plan = K.SegmentPlan(torch.tensor(tp, dtype=torch.int32, device=d),
                          torch.tensor(part_ad, dtype=torch.int32, device=d), n_rows)
     spec = K.DropoutSpec(torch.from_numpy(seg_p).to(d), n_rows, 7, seed) if use_drop else None
