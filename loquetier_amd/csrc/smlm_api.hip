@@ -114,7 +114,10 @@ ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
   // 4096 -> 4096 at rank 128, shrink 25.5 -> 20.7 us, the backward's dV 23.8 -> 18.1; four steps a batch 27.5 / 22.2,
   // whose 70 KB of LDS leave two workgroups a CU.)
   c.U = c.NB == 8 ? 2 : (c.MT > 1 ? 4 : (c.NB == 4 ? 2 : 4));
-  const int kq = 32 * c.U;
+  // k of a load batch of one wave, the unit the split is made in.  (Tile blocks: four steps, also where a batch is two:
+  // slices of 256 of k instead of 512 double the partial sums, past smlm_gemm_static's scratch at 1024 rows and 128
+  // columns.)
+  const int kq = c.MT > 1 ? 128 : 32 * c.U;
   c.NW = nw;
   const int units = ceil_div(T > 0 ? T : 1, kTileRows * c.MT);
   // k split over workgroups: enough of them to fill the chip, but every split writes and

@@ -94,6 +94,17 @@ def test_argument_validation_codes(lib):
                            None, None) == -4
 
 
+@pytest.mark.parametrize("T,d_in,d_out", [(512, 4096, 256), (600, 4096, 256), (1000, 5120, 128), (1024, 4096, 128),
+                                           (300, 4096, 512)])
+def test_products_wider_than_64_columns_fit_the_static_scratch(lib, T, d_in, d_out):
+    """The k split of tile blocks stops at pieces of 512, also where a workgroup stages 256 of k at a time for 128
+    output columns: the partial sums of these products are at most 6.3 MB, within smlm_gemm_static's scratch."""
+    need = lib.size_query("smlm_gemm_workspace_size", T, 16, d_in, d_out)
+    partials = (d_in // 512) * T * d_out * 4
+    assert need <= partials + lib.size_query("smlm_plan_size", T, 16) + 256
+    assert need <= lib.SMLM_STATIC_SCRATCH_BYTES
+
+
 def test_plan_on_first_use_argument_validation(lib):
     """smlm_lora_opts.build_seg_indptr / build_seg_adapter: both or neither, and only with the shrink stage."""
     L = lib.load()
