@@ -107,16 +107,13 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
 ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
   ShrinkCfg c;
   c.MT = mt;
-  c.NB = d_out <= 16 ? 1 : (d_out <= 32 ? 2 : (d_out <= 64 || mt == 1 ? 4 : 8));
-  c.zblocks = ceil_div(d_out, c.NB == 8 ? 128 : 64);
-  // 32-wide k steps per load batch (the tile-block kernel stages four per batch in LDS, two of 128 weight rows).
-  // (Ranks above 64 take 128 columns a workgroup and read x once for them; with 64, twice: 2064 rows, two projections
-  // 4096 -> 4096 at rank 128, shrink 25.5 -> 20.7 us, the backward's dV 23.8 -> 18.1; four steps a batch 27.5 / 22.2,
-  // whose 70 KB of LDS leave two workgroups a CU.)
-  c.U = c.NB == 8 ? 2 : (c.MT > 1 ? 4 : (c.NB == 4 ? 2 : 4));
-  // k of a load batch of one wave, the unit the split is made in.  (Tile blocks: four steps, also where a batch is two:
-  // slices of 256 of k instead of 512 double the partial sums, past smlm_gemm_static's scratch at 1024 rows and 128
-  // columns.)
+  c.NB = d_out <= 16 ? 1 : (d_out <= 32 ? 2 : 4);  // (run_shrink may turn 4 into 8: shrink_wide)
+  c.zblocks = ceil_div(d_out, 64);
+  // 32-wide k steps per load batch (the tile-block kernel stages four per batch in LDS)
+  c.U = c.MT > 1 ? 4 : (c.NB == 4 ? 2 : 4);
+  // k of a load batch of one wave, the unit the split is made in.  (Tile blocks: four steps, also for 128 columns a
+  // workgroup, whose batches are two: slices of 256 of k instead of 512 double the partial sums, past
+  // smlm_gemm_static's scratch at 1024 rows and 128 columns.)
   const int kq = c.MT > 1 ? 128 : 32 * c.U;
   c.NW = nw;
   const int units = ceil_div(T > 0 ? T : 1, kTileRows * c.MT);
@@ -154,6 +151,20 @@ ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
       }
   }
   return c;
+}
+
+// Tile-block shrinks of more than 64 columns: 128 columns a workgroup, which then reads x once for them, instead of
+// 64 -- when that leaves workgroups enough (`wgs`, of 128 columns, over all projections of the launch).  The batches
+// are two k steps then (four would take 70 KB of LDS, two workgroups a CU: 27.5 us instead of 20.7 in the first line).
+// The choice does not touch the order of any sum.  64 / 128 columns, us (forward: the whole call; [k][n]: the product):
+//   forward, 2064 rows, two projections 4096 -> 4096 at rank 128 (528 workgroups): the shrink 25.5 / 20.7
+//   forward at rank 128, 4096 -> 4096: 512 rows (64) 20.2 / 23.0, 1024 rows (128) 23.0 / 25.7, 1500 rows (192)
+//     28.6 / 29.3, 2048 rows (256) 31.7 / 32.2, 3000 rows (282) 43.7 / 40.8; 11008 -> 4096: 512 rows (128) 25.5 / 27.8,
+//     640 rows (160) 30.8 / 29.2, 1024 rows (256) 34.4 / 31.5; q/k/v/o: 512 rows (256) 38.7 / 34.5
+//   weights [k][n], 4096 -> 128: 16 rows (8) 10.3 / 13.8, 1024 rows (128) 14.4 / 17.5, 4096 rows (256) 22.6 / 24.6;
+//     4096 -> 1024: 128 rows (128) 32.7 / 34.6, 512 rows (512) 41.2 / 39.4, 4096 rows (2048) 107.7 / 87.1
+inline bool shrink_wide(int mt, int d_out, bool w_kn, long wgs) {
+  return mt > 1 && d_out > 64 && (w_kn ? wgs > 256 : wgs >= 160);
 }
 
 // most k-split partials a shrink of this shape can leave behind, whichever wave count it runs with
@@ -506,8 +517,13 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
   ShrinkCfg c0{};
   size_t bits_off = 0;
   const int nw = shrink_waves(mt, nproj, d_in, d_out);
+  long wgs = 0;
+  for (int i = 0; i < nproj; ++i)
+    wgs += (long)ceil_div(T, kTileRows * mt) * shrink_cfg(T, d_in[i], d_out, nw, solo, mt).ksplit * ceil_div(d_out, 128);
+  const bool wide = shrink_wide(mt, d_out, w_kn, wgs);
   for (int i = 0; i < nproj; ++i) {
-    const ShrinkCfg c = shrink_cfg(T, d_in[i], d_out, nw, solo, mt);
+    ShrinkCfg c = shrink_cfg(T, d_in[i], d_out, nw, solo, mt);
+    if (wide) c.NB = 8, c.U = 2, c.zblocks = ceil_div(d_out, 128);
     if (i == 0) c0 = c;
     ShrinkProj& P = a.p[i];
     P.x = reinterpret_cast<const uint16_t*>(x[i]);

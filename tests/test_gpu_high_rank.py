@@ -1,4 +1,5 @@
-"""Ranks above 64: the kernels walk the rank 128 at a time.  Edges of those pieces (72, 128, 136, 256), ragged
+"""Ranks above 64: the kernels walk the rank 128 at a time (the tile-block shrinks 64 at a time in launches of few
+workgroups).  Edges of those pieces (72, 128, 136, 256), ragged
 widths, single rows to several tile blocks, adapters stored at their own rank; exact (dyadic) inputs against the
 oracle, bit for bit."""
 import numpy as np
@@ -19,8 +20,9 @@ SHAPES = [
     (1040, 5, 2, 136, 88, 136, None),
     (1030, 6, 2, 328, 264, 256, None),
     (1200, 9, 3, 256, 520, 128, [8, 72, 128]),
+    (1100, 9, 3, 4096, 4096, 200, [200, 72, 136]),   # 288 workgroups of 128 columns: shrinks 128 columns wide, both ways
 ]
-IDS = ["3-rows", "rank72", "rank128", "511-rows", "512-rows", "rank136", "rank256", "packed"]
+IDS = ["3-rows", "rank72", "rank128", "511-rows", "512-rows", "rank136", "rank256", "packed", "wide-shrinks"]
 
 
 def _inputs(case, dt, d, seed):
@@ -89,3 +91,42 @@ def test_backward_dyadic_bit_exact(K, oracle, gpu_device, case, drop, dt):
     for a in range(NA):
         assert np.array_equal(to_np(dA[a]), ga[a][:A[a].shape[0]]), f"dA[{a}]"
         assert np.array_equal(to_np(dB[a]), gb[a][:, :B[a].shape[1]]), f"dB[{a}]"
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("drop", [False, True], ids=["plain", "dropout"])
+@pytest.mark.parametrize("packed", [False, True], ids=["padded", "packed"])
+@pytest.mark.parametrize("k", [1024, 4096, 2560], ids=["64-columns", "128-columns", "odd-split-falls-back"])
+def test_plans_of_300_segments_built_in_the_shrinks(K, gpu_device, k, packed, drop, dt):
+    """More segments than a four-wave workgroup has threads: the shrinks of both directions run two groups of waves a
+    workgroup, 64 or 128 columns wide.  Everything they leave equals what plans built beforehand give, bit for bit."""
+    d, tdt, r, NA, S = gpu_device, TDT[dt], 200, 9, 300
+    T = 5 * S
+    ranks = [(8, 72, 200)[a % 3] for a in range(NA)] if packed else [r] * NA
+    gen = torch.Generator().manual_seed(7)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).to(tdt).to(d)
+    A, B = [rand(q, k) / k ** 0.5 for q in ranks], [rand(k, q) / q ** 0.5 for q in ranks]
+    x, y0, g = rand(T, k), rand(T, k), rand(T, k)
+    int32 = lambda v: torch.tensor(v, dtype=torch.int32, device=d)
+    seg, ids = int32(list(range(0, T + 1, 5))), int32([(i * 7) % NA for i in range(S)])
+    rank = dict(adapter_rank=int32(ranks) if packed else None, packed_ranks=packed)
+    scale = torch.full((S,), 1.5, device=d)
+    seg_p = torch.tensor([0.5 if i % 7 else 0.0 for i in range(S)], device=d)
+    nbytes = K.SegmentPlan.nbytes(T, S)
+
+    def run(defer):
+        plan, bplan = (K.SegmentPlan(seg, ids, T, buf=torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=d), defer=defer)
+                       for _ in range(2))
+        bits = torch.zeros(K.DropoutSpec.mask_nbytes(T, [k]), dtype=torch.uint8, device=d)
+        spec = K.DropoutSpec(seg_p, T, 17, 3, bits) if drop else None
+        y, v = y0.clone(), torch.zeros(T, r, dtype=tdt, device=d)
+        K.smlm_lora_forward(y, x, ptrs(A, d), ptrs(B, d), plan, r, seg_scale=scale, beta=1.0, v_out=v, dropout=spec, **rank)
+        dA, dB = [torch.full_like(a, 9.0) for a in A], [torch.full_like(b, 9.0) for b in B]
+        dx = torch.full((T, k), 9.0, dtype=tdt, device=d)
+        K.smlm_lora_backward(dx, ptrs(dA, d), ptrs(dB, d), g, x, v, ptrs(A, d), ptrs(B, d), bplan, r, scale, dropout=spec,
+                             **rank)
+        torch.cuda.synchronize()
+        return [y, v, bits, plan.buf, bplan.buf, dx] + dA + dB
+
+    for a, b in zip(run(False), run(True)):
+        assert torch.equal(a, b)

@@ -26,6 +26,11 @@ CASES = [
      2048, 128, 16),
     ("80-distinct-pairs-tile-blocks-two-rounds", list(range(0, 644, 4)), [i % 10 for i in range(160)],
      [(i // 10) % 8 for i in range(160)], 2048, 192, 64),
+    # ranks above 64 on tile blocks: 64 columns a workgroup, 128, and 128 with two groups of waves a workgroup
+    ("tile-blocks-rank-72", [0, 700, 1100, 1101, 1500], [0, 1, 0, 1], [2, 1, 2, 0], 512, 200, 72),
+    ("tile-blocks-rank-200", [0, 700, 1100, 1101, 1500, 2300], [0, 1, 0, 1, 0], [2, 1, 2, 0, 2], 2048, 320, 200),
+    ("tile-blocks-rank-128-300-segments", list(range(0, 1501, 5)), [i % 3 for i in range(300)], [i % 4 for i in range(300)],
+     4096, 128, 128),
     ("1500-segments-two-launch-plan", list(range(1501)), [(i * 7) % 9 for i in range(1500)],
      [(i * 5) % 6 for i in range(1500)], 256, 128, 8),
 ]

@@ -294,7 +294,7 @@ BWD_CASES = [
     ("300-partitions", [0] + [7 * i + 100 for i in range(1, 301)], [i % 9 for i in range(300)], 9, 256, 2048, 16, True),
     ("v-recomputed-falls-back", [0, 700, 1400], [0, 1], 2, 256, 128, 32, False),
     ("few-rows", [0, 35, 90], [0, 1], 2, 192, 320, 16, True),
-    ("rank72-single-tiles-fall-back", [0, 35, 90], [0, 1], 2, 192, 320, 72, True),
+    ("rank72-few-rows", [0, 35, 90], [0, 1], 2, 192, 320, 72, True),
 ]
 
 
@@ -302,7 +302,7 @@ BWD_CASES = [
 @pytest.mark.parametrize("case", BWD_CASES, ids=[c[0] for c in BWD_CASES])
 def test_backward_deferred_plan_equals_built_plan(K, gpu_device, case, dt):
     """The backward builds a deferred plan too -- inside its dV shrink when that is the first launch to
-    need it (ranks up to 64, v given, no dropout), with the plan launch otherwise."""
+    need it (v given), with the plan launch otherwise."""
     name, tp, part_ad, NA, h_in, h_out, r, with_v = case
     d, tdt = gpu_device, TDT[dt]
     n_rows = tp[-1]
