@@ -737,7 +737,12 @@ __device__ __forceinline__ void store_y_lines(float* stg, const f32x4 (&acc)[NQ]
 // MFMA row m of column block (q,p) is output column 32q + 8(m/4) + 4p + m%4, so
 // that a lane's eight accumulators for one q are eight consecutive columns.
 template <int DT, int NQ, int KS, bool DIRECT, bool VFOLD>
-__global__ __launch_bounds__(kFwdThreads) void expand_wave_kernel(ExpandArgs a) {
+// KS == 0 with the fold: two workgroups a CU at most.  Its registers would allow three, and launches of up to two
+// workgroups a CU then come to lie three on some CUs and one on others (512 workgroups, q/k/v/o of 256 rows in two
+// segments: rank 72 28.7 -> 25.9 us, rank 128 41.6 -> 34.8, rank 256 71.7 -> 58.4; 1024 workgroups, 256 decoded rows:
+// 51.8 -> 52.6, 66.7 -> 68.6, 133.2 -> 133.0).
+__global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(1, KS == 0 && VFOLD ? 2 : 8)))
+void expand_wave_kernel(ExpandArgs a) {
   __shared__ __attribute__((aligned(16))) float olds[kFwdWaves][kTileRows * kOPitch];
   const int units = DIRECT ? 0 : tile_units<1>(a.plan, 0);
   const WorkRange wr = item_range<DIRECT>(a.items, units);
