@@ -47,12 +47,22 @@ int launch(void (*kernel)(A), dim3 grid, dim3 block, hipStream_t st, const A& a)
 // 15.6 / 17.8, at 1536 rows 21.7 / 19.2; rank 64 at 256 rows 17.0 / 16.3, at 1000 rows 22.9 / 18.8.  A launch of
 // several projections, whose workgroups fill the chip together, would change over earlier (q/k/v/o: rank 16 at
 // 1024 rows 30.9 / 30.9, at 2048 rows 53.1 / 47.5; rank 32 at 384 rows 24.5 / 25.3, at 768 rows 34.6 / 30.7;
-// rank 64 at 128 rows 27.6 / 24.7).  Rank 128, forward of one projection 4096 -> 4096: 256 rows over 32 adapters
-// 25.5 / 29.7, 512 rows 29.2 / 31.5, 1000 rows over 16 adapters 42.3 / 33.0; q/k/v/o at 128 rows 74.2 / 70.6, at 512
-// rows 86.7 / 78.9.  The rule lies between the two and does not look at the number of
+// rank 64 at 128 rows 27.6 / 24.7); the rule lies between the two and does not look at the number of
 // projections, so that a launch of several gives the bits that launches of one give.
-inline int tiles_per_wave(int T, int r) {
-  const int from = r <= 16 ? 2048 : (r <= 32 ? 768 : (r <= 48 || r > 64 ? 512 : 128));
+// Ranks above 64: rank 128, 4096 -> 4096, prompts of 512 rows 22.9 / 20.2, of 640 rows 34.7 / 21.7, q/k/v/o at 512
+// rows 62.3 / 34.5, 1024 -> 4096 at 768 rows 23.6 / 18.8; the tile blocks lose where more than 512 segments take their
+// plan out of the launch and k is short (1024 -> 4096, 768 decoded rows 37.5 / 43.0) and where an odd split does (11008
+// -> 4096, 512 decoded rows 36.7 / 50.5).  Up to rank 96 the second block of 64 columns is at most half full, and the
+// line also looks at the shortest k of the launch (h_in; projections of one input, as a group's, share it): rank 72,
+// 4096 -> 4096, 512 rows 17.0 / 18.3, 512 decoded rows 29.3 / 32.1, 640 rows 24.4 / 20.4; 2048 -> 2048, 768 rows
+// 16.3 / 17.5; 1024 -> 4096, 1000 rows 17.0 / 20.0.
+constexpr int kNoShrink = 1 << 30;  // k of an expand by itself
+inline int tiles_per_wave(int T, int r, int k) {
+  int from;
+  if (r <= 32) from = r <= 16 ? 2048 : 768;
+  else if (r <= 64) from = r <= 48 ? 512 : 128;
+  else if (r <= 96) from = k >= 4096 ? 640 : 1024;
+  else from = 512;
   return T >= from ? kBlkTiles : 1;
 }
 // (The backward runs on tile blocks at every size and rank: they read the weights the other way round as they lie
@@ -752,7 +762,7 @@ SMLM_API int smlm_gemm_planned(void* y, const void* x, const void* const* w_ptrs
       a.w_kn = 1;
       return launch_expand(dtype, expand_nq(T, d_out), kBlkTiles, S, n_weights, 1, d_in, st, a);
     }
-    return launch_expand(dtype, expand_nq(T, d_out), tiles_per_wave(T, d_in), S, n_weights,
+    return launch_expand(dtype, expand_nq(T, d_out), tiles_per_wave(T, d_in, kNoShrink), S, n_weights,
                          1, d_in, st, a);
   }
   float* partial = reinterpret_cast<float*>(workspace);
@@ -760,7 +770,7 @@ SMLM_API int smlm_gemm_planned(void* y, const void* x, const void* const* w_ptrs
     return run_shrink(dtype, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
                       seg_scale, kBlkTiles, st, true, true);
   return run_shrink(dtype, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in,
-                    d_out, &w_ld, beta, seg_scale, tiles_per_wave(T, d_out), st);
+                    d_out, &w_ld, beta, seg_scale, tiles_per_wave(T, d_out, d_in), st);
 }
 
 SMLM_API int smlm_gemm_workspace_size(int T, int S, int d_in, int d_out, size_t* bytes) {
@@ -797,7 +807,7 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
   // (d_in >= d_out, weights [n][k]) over few enough segments builds it inside its own launch: every
   // workgroup numbers the addresses by their first occurrence and finds its tile itself, a few more
   // write the plan for the fold launch behind it (as the fused forward does with adapter ids).
-  const int mt = tiles_per_wave(T, d_out);
+  const int mt = tiles_per_wave(T, d_out, d_in);
   const int nw = shrink_waves(mt, 1, &d_in, d_out);
   const int ks = shrink_cfg(T, d_in, d_out, nw, false, mt).ksplit;
   const bool in_launch = d_in >= d_out && !w_row_major && self_planned_ok(T, S, S, pv.nt_max, mt) &&
@@ -933,7 +943,9 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
   float* partial[kMaxProj];
   void* v16[kMaxProj];
   int vsplit[kMaxProj];
-  const int mt = tiles_per_wave(T, r);
+  int k_min = h_in[0];
+  for (int i = 1; i < n_proj; ++i) k_min = h_in[i] < k_min ? h_in[i] : k_min;
+  const int mt = tiles_per_wave(T, r, k_min);
   const int nw = shrink_waves(mt, n_proj, h_in, r);
   bool expand_folds = nw == kDecodeWaves && mt == 1;
   {

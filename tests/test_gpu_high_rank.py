@@ -17,12 +17,16 @@ SHAPES = [
     (1100, 9, 3, 2048, 1160, 128, None),
     (511, 4, 2, 2048, 72, 128, None),       # single tiles forward, the row below tile blocks
     (512, 4, 2, 2048, 72, 128, None),
+    (639, 5, 2, 4096, 72, 72, None),        # ... at ranks up to 96 and k of 4096
+    (640, 5, 2, 4096, 72, 96, None),
+    (1023, 5, 2, 264, 88, 72, None),        # ... and at shorter k
+    (1024, 5, 2, 264, 88, 96, None),
     (1040, 5, 2, 136, 88, 136, None),
     (1030, 6, 2, 328, 264, 256, None),
     (1200, 9, 3, 256, 520, 128, [8, 72, 128]),
     (1100, 9, 3, 4096, 4096, 200, [200, 72, 136]),   # 288 workgroups of 128 columns: shrinks 128 columns wide, both ways
 ]
-IDS = ["3-rows", "rank72", "rank128", "511-rows", "512-rows", "rank136", "rank256", "packed", "wide-shrinks"]
+IDS = ["3-rows", "rank72", "rank128", "511-rows", "512-rows", "639-rows", "640-rows", "1023-rows", "1024-rows", "rank136", "rank256", "packed", "wide-shrinks"]
 
 
 def _inputs(case, dt, d, seed):
