@@ -22,8 +22,6 @@ namespace smlm {
 constexpr int kRmsChunks = 8;                       // 512-element chunks a wave keeps in registers
 constexpr int kRmsWaveCols = 512 * kRmsChunks;      // columns one wave covers
 constexpr int kRmsMaxCols = 4 * kRmsWaveCols;       // four waves per row at most
-constexpr int kRmsFoldRows = 64;                    // partial rows summed side by side in the fold ...
-constexpr int kRmsFoldCols = 16;                    // ... whose workgroups take this many columns
 
 // Sum over the wave with DPP adds (shifts inside rows of 16 lanes, then the
 // row totals); every lane returns the total.
@@ -358,15 +356,15 @@ struct RmsFoldArgs {
   int n_part, cols;
 };
 
-// grid: ceil(cols / 16), block 256: thread (rg = tid / 4, c4 = tid % 4) adds partial rows rg, rg + 64, ... of four
-// columns; the 64 row groups are then added across the lanes of each wave and the four waves through LDS, always in
-// the same order.  (Sixteen columns a workgroup: a row of 4096 columns keeps every CU busy; with 64 columns a
-// workgroup only a quarter of them worked.)
-template <int DT>
+// grid: ceil(cols / (4 * C4)), block 256: thread (rg = tid / C4, c4 = tid % C4) adds partial rows rg, rg + 256 / C4, ...
+// of four columns; the row groups are then added across the lanes of each wave and the four waves through LDS, always
+// in the same order.
+template <int DT, int C4>
 __global__ __launch_bounds__(256) void rms_fold_kernel(RmsFoldArgs a) {
-  __shared__ f32x4 red[4][4];
-  const int rg = threadIdx.x >> 2, c4 = threadIdx.x & 3, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int col = (int)blockIdx.x * kRmsFoldCols + c4 * 4;
+  constexpr int kRmsFoldRows = 256 / C4;
+  __shared__ f32x4 red[4][C4];
+  const int rg = threadIdx.x / C4, c4 = threadIdx.x % C4, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int col = (int)blockIdx.x * 4 * C4 + c4 * 4;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
   if (col < a.cols && rg < a.n_part) {
     // eight partial rows are requested at a time; rows past the end re-read row rg and are dropped
@@ -384,12 +382,12 @@ __global__ __launch_bounds__(256) void rms_fold_kernel(RmsFoldArgs a) {
     }
   }
 #pragma unroll
-  for (int d = 4; d < kWaveSize; d *= 2)
+  for (int d = C4; d < kWaveSize; d *= 2)
 #pragma unroll
     for (int e = 0; e < 4; ++e) s[e] += __shfl_xor(s[e], d, kWaveSize);
-  if (lane < 4) red[wave][c4] = s;
+  if (lane < C4) red[wave][c4] = s;
   __syncthreads();
-  if (threadIdx.x < 4 && col < a.cols) {
+  if (threadIdx.x < C4 && col < a.cols) {
     const f32x4 t = (red[0][c4] + red[1][c4]) + (red[2][c4] + red[3][c4]);
     u32x2 o;
     o[0] = pack2<DT>(t[0], t[1]);

@@ -651,6 +651,18 @@ void* static_scratch() {
   return p;
 }
 
+// Columns a workgroup of the RMSNorm backward's fold takes: 16 where a row is short, so that its workgroups fill the
+// chip; of wider rows 32 and 64, as the pieces of 64 bytes that 16 columns read of every partial row fetch the lines
+// twice.  Whole backward, us, 16 / 32 / 64 columns: 4096 x 2048 16.9 / 16.9 / -, 1000 x 4096 12.4 / 11.0 / -,
+// 1000 x 8192 21.8 / 18.8 / 18.6, 1000 x 11008 28.7 / 25.1 / 24.8, 64 x 20480 16.9 / - / 14.5.
+template <int DT>
+int launch_rms_fold(hipStream_t st, const RmsFoldArgs& a) {
+  const dim3 bl(256);
+  if (a.cols <= 2048) return launch(rms_fold_kernel<DT, 4>, dim3((unsigned)ceil_div(a.cols, 16)), bl, st, a);
+  if (a.cols <= 4096) return launch(rms_fold_kernel<DT, 8>, dim3((unsigned)ceil_div(a.cols, 32)), bl, st, a);
+  return launch(rms_fold_kernel<DT, 16>, dim3((unsigned)ceil_div(a.cols, 64)), bl, st, a);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1416,9 +1428,7 @@ SMLM_API int smlm_rms_norm_bwd(void* dx, void* dw, const void* g, const void* x,
              : launch(rms_bwd_kernel<SMLM_DTYPE_BF16, 2, 1>, grid, dim3(1024), st, a);
   if (rc) return rc;
   const RmsFoldArgs fa{reinterpret_cast<uint16_t*>(dw), reinterpret_cast<const float*>(workspace), nb, cols};
-  const dim3 fgrid((unsigned)ceil_div(cols, kRmsFoldCols));
-  return f16 ? launch(rms_fold_kernel<SMLM_DTYPE_F16>, fgrid, dim3(256), st, fa)
-             : launch(rms_fold_kernel<SMLM_DTYPE_BF16>, fgrid, dim3(256), st, fa);
+  return f16 ? launch_rms_fold<SMLM_DTYPE_F16>(st, fa) : launch_rms_fold<SMLM_DTYPE_BF16>(st, fa);
 }
 
 SMLM_API int smlm_segments_build(const int32_t* req_adapter, const int32_t* req_len, int R,
