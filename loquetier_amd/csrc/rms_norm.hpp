@@ -152,22 +152,24 @@ struct RmsBwdArgs {
   int rows, cols;
 };
 
-// A workgroup takes a contiguous share of the rows, R at a time, a thread 8 columns (CH = 1, up to 8192 columns: as
-// many threads as a row has pieces of 8, in whole waves) or 16 (CH = 2, 1024 threads), and keeps its columns of w and
-// its share of dw in registers.  The dots of the R rows cross the waves through LDS together, one barrier for them;
-// the next rows are on their way meanwhile.
+// A workgroup walks the rows R at a time, blockIdx.x * R, + gridDim.x * R, ...; a thread takes 8 columns (CH = 1, up to
+// 8192 columns: as many threads as a row has pieces of 8, in whole waves) or 16 (CH = 2: half as many threads) and
+// keeps its columns of w and its share of dw in registers.  The dots of the R rows cross the waves through LDS
+// together, one barrier for them; the next rows are on their way meanwhile.
 // Bound by HBM: three passes of 2 bytes an element.  A thread per column piece keeps a lane's registers few (dw is
-// eight floats) and the rows in flight many.  4224 x 4096, bf16: 23.3 us and 3.9 us for the fold of 256 partial rows
-// (a wave to a row, 64 columns a lane, 208 registers: 31.9 + 4.1); four rows at a time without the rows ahead
-// 30.3 us, two 25.6 with 512 workgroups, whose fold then takes longer.  2000 x 8192: 31.9 -> 24.7 us, 300 x 1024
-// 9.9 -> 3.5, 4000 x 2048 equal.
+// eight floats) and the rows in flight many.  Neighbouring workgroups work on neighbouring rows: with a contiguous
+// share each, all of them stand at the same place modulo the share and meet in few HBM channels.  Whole backward with
+// its fold, bf16, us, a wave to a row of up to 4096 columns (64 columns a lane, 208 registers) and four waves to a
+// wider one / contiguous shares / interleaved: 4096 x 4096 26.0 / 24.3 / 23.2, 8192 x 4096 46.4 / 41.0 / 38.0,
+// 8192 x 6144 80.6 / 67.2 / 55.0, 4096 x 12288 66.7 / 70.1 / 57.6, 1000 x 16384 30.4 / 31.1 / 29.8,
+// 4096 x 16384 85.6 / 83.0 / 76.7, 300 x 1024 12.0 / 6.5 / 6.3, 4096 x 2048 17.4 / 17.1 / 16.5.
 template <int DT, int CH, int R>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void rms_bwd_kernel(RmsBwdArgs a) {
   typedef float dots_t __attribute__((ext_vector_type(R)));
   __shared__ dots_t part[2][16];  // the rows' dots by wave, two halves in turn
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = (int)blockDim.x >> 6;
   const float inv_n = 1.0f / (float)a.cols;
-  const int row0 = (int)((long)blockIdx.x * a.rows / gridDim.x), row1 = (int)((long)(blockIdx.x + 1) * a.rows / gridDim.x);
+  const int step = (int)gridDim.x * R;
 
   int col[CH];
   bool ok[CH];
@@ -182,11 +184,11 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
 #pragma unroll
     for (int e = 0; e < 8; ++e) dw[i][e] = 0.0f;
   }
-  // rows past the workgroup's share re-read its last row and are not used
+  // rows past the last re-read it and are not used
   auto load = [&](int row, u32x4 (&xr)[R][CH], u32x4 (&gr)[R][CH], float (&r)[R]) {
 #pragma unroll
     for (int t = 0; t < R; ++t) {
-      const int rr = row + t < row1 ? row + t : row1 - 1;
+      const int rr = row + t < a.rows ? row + t : a.rows - 1;
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
         xr[t][i] = ldg16_nt(a.x + (long)rr * a.cols + col[i]);
@@ -197,14 +199,14 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
   };
   u32x4 xv[R][CH], gv[R][CH];
   float rms[R];
-  load(row0, xv, gv, rms);
+  load((int)blockIdx.x * R, xv, gv, rms);
   int parity = 0;
-  for (int row = row0; row < row1; row += R) {  // uniform over the workgroup
+  for (int row = (int)blockIdx.x * R; row < a.rows; row += step) {  // uniform over the workgroup
     u32x4 xn[R][CH], gn[R][CH];
     float rn[R];
-    // unconditional (past the end it re-reads the last row): a branch around the loads would make the wave wait
+    // unconditional (past the end it re-reads these rows): a branch around the loads would make the wave wait
     // for everything in flight where the paths join
-    load(row + R, xn, gn, rn);
+    load(row + step < a.rows ? row + step : row, xn, gn, rn);
     __builtin_amdgcn_sched_barrier(0);  // the next rows' loads are issued before these rows are used
     dots_t dots;
 #pragma unroll
@@ -230,7 +232,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     parity ^= 1;
 #pragma unroll
     for (int t = 0; t < R; ++t) {
-      if (row + t >= row1) break;  // uniform over the workgroup
+      if (row + t >= a.rows) break;  // uniform over the workgroup
       const float coef = dots[t] * rms[t] * rms[t] * inv_n;
 #pragma unroll
       for (int i = 0; i < CH; ++i) {

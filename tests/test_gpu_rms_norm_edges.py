@@ -1,7 +1,7 @@
 """Backward of RMSNorm at the edges of its launch: rows of one wave's pieces and of 1024 threads', the change to two
-pieces a thread (8200 columns), row counts around a workgroup's share, the fold's 16, 32 and 64 columns a workgroup.  Exact inputs (unit-magnitude rows, dyadic w and
-g, power-of-two widths: every term is exact in float) equal the oracle; other widths within the bars of the RMSNorm
-parity tests."""
+pieces a thread (8200 columns), row counts around the workgroups' turns, the fold's 16, 32 and 64 columns a
+workgroup.  Exact inputs (unit-magnitude rows, dyadic w and g, power-of-two widths: every term is exact in float) equal
+the oracle; other widths within the bars of the RMSNorm parity tests."""
 import numpy as np
 import pytest
 import torch
@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dt", ["fp16", "bf16"])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (2, 64), (513, 64), (1025, 512), (5, 8192), (515, 16384), (6, 8200), (515, 72), (40, 2048),
-                                       (40, 2056), (40, 4096), (40, 4104), (1300, 12288)])
+                                       (40, 2056), (40, 4096), (40, 4104), (1300, 12288),
+                                       (511, 8192), (512, 8192), (1023, 4096), (1025, 3072), (257, 8208)])
 def test_backward(K, oracle, gpu_device, dt, rows, cols):
     exact = cols & (cols - 1) == 0
     rng = np.random.default_rng(rows * 31 + cols)
