@@ -166,6 +166,13 @@ __device__ __forceinline__ void pick_tiles(const TileArgs& p, int tb, int* t0, i
   }
 }
 
+// eight consecutive-k elements of weight column n (zeros when !ok).  A function of its own for the order it gives the
+// single-tile shrink's loads: with the address written out at the call, q/k/v/o of 256 rows at rank 16 take 9.2 us
+// instead of 9.0, of 1000 rows 15.2 instead of 14.8, 11008 -> 16 of 256 rows 9.5 instead of 9.3.
+__device__ __forceinline__ u32x4 load_w8(const uint16_t* W, int n, int k, int ldw, bool ok, const uint16_t* zeros) {
+  return ldg16_or(W + (long)n * ldw + k, ok, zeros);
+}
+
 // out = beta*old + scale*acc for four consecutive columns of one row
 template <int DT>
 __device__ __forceinline__ void store4(uint16_t* dst, f32x4 a, float scale, float beta) {
@@ -250,7 +257,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
           const int n = n0 + 16 * nb + c;
-          wf[nb][u] = ldg16_or(W + (long)n * P.ldw + kk, kin && n < nlim, zeros);
+          wf[nb][u] = load_w8(W, n, kk, P.ldw, kin && n < nlim, zeros);
         }
       }
     };
@@ -311,7 +318,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
 }
 
 // Shrink for tile blocks (larger batches, and the backward).  Work item -> (projection, k
-// slice, 64-column block, tile block) as above, but here wave w owns tile w of the block
+// slice, column block of 16 * NB, tile block) as above, but here wave w owns tile w of the block
 // and all four waves walk the whole k slice together: each 32*U-wide batch of the weight
 // rows is staged once in LDS (two buffers in turn, one barrier a batch) and shared by the
 // four tiles, while every wave loads the x fragments of its own tile straight into
