@@ -737,10 +737,11 @@ __device__ __forceinline__ void store_y_lines(float* stg, const f32x4 (&acc)[NQ]
 // loads its weight fragments straight into registers.  K (= LoRA rank) is
 // short: KS > 0 unrolls KS 32-wide k steps, KS == 0 is the general loop over k.
 // Bound by the chain of dependent loads (tile -> adapter and row numbers -> y, v, weights): the weights need the
-// adapter alone and are requested first, ahead of the row numbers' arrival (KS > 0).  Whole forward, us, weights after
-// the row numbers / before: six times q/k/v/o of 256 decoded rows at rank 16 from a graph 114.1 / 111.1, one
-// projection of 64 decoded rows 10.0 / 9.0, 600 rows in four segments 10.8 / 10.0, rank 64 and 16 rows over 16
-// adapters, q/k/v/o 26.7 / 23.9.  At ranks above 64 the same for the loop's first step gained nothing (13.3 / 13.8).
+// adapter alone and up to rank 32 (KS = 1) are requested ahead of the row numbers' arrival.  Whole forward, us, weights
+// after the row numbers / before: six times q/k/v/o of 256 decoded rows at rank 16 from a graph 114.1 / 111.1, one
+// projection of 64 decoded rows 10.0 / 9.0, 600 rows in four segments 10.8 / 10.0.  At KS = 2 the registers cost more
+// than it gains where there are many workgroups (rank 40, twice 4096 -> 11008, 200 decoded rows: 28.1, the first step
+// ahead 29.3, both 29.2), and above rank 64 the loop's first step ahead gained nothing (13.3 / 13.8).
 // MFMA row m of column block (q,p) is output column 32q + 8(m/4) + 4p + m%4, so
 // that a lane's eight accumulators for one q are eight consecutive columns.
 template <int DT, int NQ, int KS, bool DIRECT, bool VFOLD>
@@ -787,20 +788,19 @@ void expand_wave_kernel(ExpandArgs a) {
       L.srow[j] = a.plan.tile_row[tile * kTileRows + L.orow + 8 * j];
       sseg[j] = a.seg_scale ? a.plan.tile_rseg[tile * kTileRows + L.orow + 8 * j] : -1;
     }
-    u32x4 wf[KSU][NQ][2];
-    auto load_w = [&](int ks, u32x4 (&w)[NQ][2]) {
+    u32x4 wf[NQ][2];
+    auto load_w = [&](int ks) {
       const int kk = 32 * ks + 8 * g;
 #pragma unroll
       for (int q = 0; q < NQ; ++q)
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           const int n = ncol0 + 32 * q + 4 * p + mrow;
-          w[q][p] = ldg16_or(W + (long)n * ldw + kk, kk < klim && n < P.d_out, zeros);
+          wf[q][p] = ldg16_or(W + (long)n * ldw + kk, kk < klim && n < P.d_out, zeros);
         }
     };
-    if (KS > 0) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) load_w(ks, wf[ks]);
+    if (KS == 1) {
+      load_w(0);
       __builtin_amdgcn_sched_barrier(0);  // the weights are on their way before the row numbers are waited for
     }
 #pragma unroll
@@ -821,7 +821,7 @@ void expand_wave_kernel(ExpandArgs a) {
     for (int ks = 0; ks < nks; ++ks) {
       const int kk = 32 * ks + 8 * g;
       const bool kin = kk < P.d_in, kreal = kk < klim;
-      if (KS == 0) load_w(ks, wf[0]);
+      if (KS != 1) load_w(ks);
       u32x4 vf;
       const bool vok = kreal && row >= 0;
       if (VFOLD) {  // fold (and round) the shrink's fp32 partial sums as its fold launch would
@@ -846,7 +846,7 @@ void expand_wave_kernel(ExpandArgs a) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q)
 #pragma unroll
-        for (int p = 0; p < 2; ++p) acc[q][p] = Num<DT>::mfma(wf[KS > 0 ? ks : 0][q][p], vf, acc[q][p]);
+        for (int p = 0; p < 2; ++p) acc[q][p] = Num<DT>::mfma(wf[q][p], vf, acc[q][p]);
     }
     store_y_lines<DT, NQ>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
   }
