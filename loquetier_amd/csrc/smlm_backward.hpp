@@ -59,8 +59,8 @@ __device__ __forceinline__ int wg_lds_row(int s) {
   return (s & ~12) | ((s & 4) << 1) | ((s & 8) >> 1);
 }
 
-// grid: (sum over the projections of their dA and dB units, NA), block 64*NW; with ZSPLIT ceil(r/64) workgroups per
-// unit -- twice that for the kernel named at wgrad_nbj_a.  A unit is
+// grid: (sum over the projections of their dA and dB units, NA), block 64*NW; with ZSPLIT several workgroups per unit,
+// one for every 64 ranks -- twice that for the kernel named at wgrad_nbj_a.  A unit is
 // `walk` neighbouring 64-column chunks of one projection's dA or dB.  A workgroup owns the unit's columns (and
 // up to 64 ranks) of one adapter's gradient and walks all of that adapter's tiles once per chunk, 64
 // gathered rows (four tiles, two MFMA k steps) per wave and loop step.  With
@@ -88,7 +88,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   constexpr int kRedBytes = NW > 1 ? NW * 4 * kWaveSize * 16 : 0;
 
   const int ad = blockIdx.y;
-  // j0: first rank of this workgroup (16 * NBJ ranks per workgroup along the grid's z axis)
+  // j0: first rank of this workgroup, which takes 16 * NBJ
   constexpr bool is_a = IS_A;
   const int h = is_a ? P.h_in : P.h_out;
   const uint16_t* Q = is_a ? P.q_a : P.q_b;
@@ -359,7 +359,8 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
 // rank blocks of 16 a dA workgroup takes (a dB workgroup: NBJ)
 constexpr int wgrad_nbj_a(int nbj, int nw, bool drop) { return (drop && nw == 1 && nbj == 4) ? 2 : nbj; }
 
-// ZSPLIT: several workgroups share a unit, each taking other ranks (a.zcount of them: ranks above 64).  They are
+// ZSPLIT: several workgroups share a unit, each taking other ranks (a.zcount of them: ranks above 64, and those above
+// 32 in the one-wave kernel under dropout, whose dA workgroups take 32 each).  They are
 // numbered eight apart, so that they run at about the same time on one XCD (workgroup number modulo eight) and the
 // rows of x and dY, which all of them read, come out of its L2 for the second (2048 rows, two projections
 // 4096 -> 4096 at rank 128: 40.2 us with the ranks along the grid's z axis, 37.4 eight apart, 32.9 with loads that

@@ -401,7 +401,7 @@ __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(Self
     if (part < kSelfPlanBuilders) plan_small_body(a.plan, sm.plan, part, all < kSelfPlanBuilders ? all : kSelfPlanBuilders);
     return;
   }
-  // grid x: (k slice, 64-column block) of the projection, k slices fastest -- in pairs when a
+  // grid x: (k slice, column block of 16 * NB) of the projection, k slices fastest -- in pairs when a
   // workgroup takes two (the host launches that kind only when every k split is even)
   const int pj = blockIdx.z;
   if ((int)blockIdx.x * GROUPS >= a.sh.items.row_start[pj + 1] - a.sh.items.row_start[pj]) return;

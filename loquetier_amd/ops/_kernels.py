@@ -18,7 +18,8 @@ from .. import _lib
 _DTYPE_CODE = {torch.float16: _lib.SMLM_DTYPE_F16, torch.bfloat16: _lib.SMLM_DTYPE_BF16}
 
 class Workspace:
-    """Scratch memory for the kernels (k-split partial sums, the rounded v, transposed weights).
+    """Scratch memory for the kernels (plans of unplanned calls, k-split partial sums, the rounded v and
+    dV, and their transposed copies for the weight gradients).
 
     The C ABI allocates nothing: every call is handed a buffer at least as large as its
     `*_workspace_size` query says.  A Workspace owns such a buffer.  It only ever grows, a

@@ -90,7 +90,7 @@ FWD_CASES = [
     ("many-segments-offset", 1600, list(range(7, 1508)), [i % 5 for i in range(1500)], 5, 2048, 64, 16),
     ("rank64", 45, [0, 20, 45], [0, 1], 2, 512, 256, 64),
     ("rank24", 33, [0, 33], [0], 1, 96, 136, 24),
-    ("rank128", 45, [0, 20, 45], [0, 1], 2, 512, 256, 128),   # ranks above 64: general k loop in the expand
+    ("rank128", 45, [0, 20, 45], [0, 1], 2, 512, 256, 128),   # ranks above 64: single tiles' loop over the rank
     ("rank72", 33, [0, 33], [0], 1, 96, 136, 72),
     ("decode", 64, list(range(65)), [i % 5 for i in range(64)], 5, 512, 512, 16),
 ]
@@ -581,8 +581,8 @@ BWD_CASES = [
     ("empty-part", [0, 17, 17, 50], [0, 1, 2], 3, 0, 256, 128, 32),
     ("rank64", [0, 33, 90], [0, 1], 2, 4, 192, 320, 64),
     ("long", [0, 300, 700], [1, 0], 2, 20, 512, 384, 16),
-    # ranks above 64 (PEFT ranks 128 / 256 are ordinary): general k loop in the dX expand, the weight
-    # gradient covers the rank 64 at a time
+    # ranks above 64 (PEFT ranks 128 / 256 are ordinary): dX walks the rank 128 at a time, the weight
+    # gradient covers it 64 at a time
     ("rank128", [0, 33, 90], [0, 1], 2, 4, 192, 320, 128),
     ("rank72", [0, 50], [0], 1, 0, 128, 136, 72),
     ("rank256-blocks", [0, 600, 1100], [1, 0], 2, 3, 256, 192, 256),

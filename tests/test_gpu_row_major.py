@@ -20,9 +20,12 @@ pytestmark = pytest.mark.gpu
     (700, 40, 5, 1024, 64),     # shrink, 64 output columns
     (700, 40, 5, 64, 1024),     # expand, two k steps
     (300, 7, 2, 256, 192),      # shrink with three 64-column blocks
-    (300, 7, 2, 96, 320),       # expand with a contraction above 64: the one-tile kernel's strided reads
+    (300, 7, 2, 96, 320),       # expand with a contraction above 64: 128 of k a piece
+    (300, 7, 2, 200, 320),      # ... two pieces
+    (700, 7, 2, 4096, 520),     # shrink with 440 workgroups of 128 columns
     (5000, 300, 20, 2048, 32),  # many segments, plan in two launches
-], ids=["shrink-r16", "expand-r16", "shrink-r64", "expand-r64", "shrink-wide", "expand-k96", "many-segments"])
+], ids=["shrink-r16", "expand-r16", "shrink-r64", "expand-r64", "shrink-wide", "expand-k96", "expand-k200", "shrink-128-columns",
+        "many-segments"])
 def test_row_major_forward_dyadic_bit_exact(K, oracle, gpu_device, shape, dt):
     T, S, NA, d_in, d_out = shape
     d = gpu_device
