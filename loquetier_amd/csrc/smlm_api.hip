@@ -527,8 +527,8 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
   ShrinkCfg c0{};
   size_t bits_off = 0;
   const int nw = shrink_waves(mt, nproj, d_in, d_out);
-  long wgs = 0;
-  for (int i = 0; i < nproj; ++i)
+  long wgs = 0;  // workgroups of 128 columns
+  for (int i = 0; mt > 1 && d_out > 64 && i < nproj; ++i)
     wgs += (long)ceil_div(T, kTileRows * mt) * shrink_cfg(T, d_in[i], d_out, nw, solo, mt).ksplit * ceil_div(d_out, 128);
   const bool wide = shrink_wide(mt, d_out, w_kn, wgs);
   for (int i = 0; i < nproj; ++i) {

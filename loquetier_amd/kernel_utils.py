@@ -113,7 +113,7 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
     `step` (mixed_lora.LayerStep or None): the backward's plan, the partitions'
     adapters, the weights' pointer tables and the layout of one buffer for all the
     gradients, prepared outside the layer loop; without it they are built here
-    (five small host-to-device copies and a plan launch per call)."""
+    (six small host-to-device copies, each of which the host waits for, and a plan launch per call)."""
     dev, dt = grad_output.device, grad_output.dtype
     T = grad_output.size(0)
     h_in = x_train.size(1)
