@@ -295,7 +295,7 @@ typedef struct smlm_dropout {
  *                  kernel_src/csrc/smlm_forward/smlm_forward_cutlass.cuh:31-46,76-79).  With
  *                  n_weights <= 1024 and either a batch of few rows (the single-tile
  *                  kernels: below 2048 rows at rank <= 16, 768 at rank <= 32, 512 at rank <= 48,
- *                  128 at rank <= 64, 640 at rank <= 96 (1024 with an h_in below 4096), 512 above),
+ *                  128 at rank <= 64, 512 above; 1024 at rank 65 to 96 with an h_in below 4096),
  *                  S <= 1024 and every h_in >= 2048, or a
  *                  larger batch with S <= 512 and T / 16 + S < 1024, this costs no
  *                  launch: the shrink's workgroups derive their own tiles from the two arrays

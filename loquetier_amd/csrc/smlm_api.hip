@@ -51,18 +51,17 @@ int launch(void (*kernel)(A), dim3 grid, dim3 block, hipStream_t st, const A& a)
 // projections, so that a launch of several gives the bits that launches of one give.
 // Ranks above 64: rank 128, 4096 -> 4096, prompts of 512 rows 22.9 / 20.2, of 640 rows 34.7 / 21.7, q/k/v/o at 512
 // rows 62.3 / 34.5, 1024 -> 4096 at 768 rows 23.6 / 18.8; the tile blocks lose where more than 512 segments take their
-// plan out of the launch and k is short (1024 -> 4096, 768 decoded rows 37.5 / 43.0) and where an odd split does (11008
-// -> 4096, 512 decoded rows 36.7 / 50.5).  Up to rank 96 the second block of 64 columns is at most half full, and the
+// plan out of the launch and k is short (1024 -> 4096, 768 decoded rows 37.5 / 43.0).
+// Up to rank 96 the second block of 64 columns is at most half full, and the
 // line also looks at the shortest k of the launch (h_in; projections of one input, as a group's, share it): rank 72,
-// 4096 -> 4096, 512 rows 17.0 / 18.3, 512 decoded rows 29.3 / 32.1, 640 rows 24.4 / 20.4; 2048 -> 2048, 768 rows
-// 16.3 / 17.5; 1024 -> 4096, 1000 rows 17.0 / 20.0.
+// 4096 -> 4096, 512 rows 17.0 / 18.3, q/k/v/o 45.5 / 30.4; 2048 -> 2048, 768 rows 16.3 / 17.5; 1024 -> 4096, 1000
+// rows 17.0 / 20.0.
 constexpr int kNoShrink = 1 << 30;  // k of an expand by itself
 inline int tiles_per_wave(int T, int r, int k) {
   int from;
   if (r <= 32) from = r <= 16 ? 2048 : 768;
   else if (r <= 64) from = r <= 48 ? 512 : 128;
-  else if (r <= 96) from = k >= 4096 ? 640 : 1024;
-  else from = 512;
+  else from = (r <= 96 && k < 4096) ? 1024 : 512;
   return T >= from ? kBlkTiles : 1;
 }
 // (The backward runs on tile blocks at every size and rank: they read the weights the other way round as they lie
@@ -114,7 +113,8 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
 // solo: the product is only ever launched by itself (the backward's dV and v products) and may take the
 // splits that suit a launch of one projection; the forward's projections keep one rule
 // whether they are launched alone or together, so that either way gives the same bits
-ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
+// plain: a product of smlm_gemm or smlm_gemm_planned
+ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt, bool plain = false) {
   ShrinkCfg c;
   c.MT = mt;
   c.NB = d_out <= 16 ? 1 : (d_out <= 32 ? 2 : 4);  // (run_shrink may turn 4 into 8: shrink_wide)
@@ -123,7 +123,11 @@ ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
   c.U = c.MT > 1 ? 4 : (c.NB == 4 ? 2 : 4);
   // k of a load batch of one wave, the unit the split is made in.  (Tile blocks: four steps, also for 128 columns a
   // workgroup, whose batches are two: slices of 256 of k instead of 512 double the partial sums, past
-  // smlm_gemm_static's scratch at 1024 rows and 128 columns.)
+  // smlm_gemm_static's scratch at 1024 rows and 128 columns.)  Above 64 columns the slices of a fused call come in
+  // multiples of 64 of k, so that 11008 falls into 16 instead of 15: an even number keeps batches of more than 256
+  // segments on the route that plans in the launch (896 rows in 298 segments at rank 256: 54.2 -> 42.6 us) and the
+  // same slices of the weights on an XCD (in three segments: 43.2 -> 37.5).  Plain products keep the fewer partial
+  // sums that smlm_gemm_static has room for.
   const int kq = c.MT > 1 ? 128 : 32 * c.U;
   c.NW = nw;
   const int units = ceil_div(T > 0 ? T : 1, kTileRows * c.MT);
@@ -146,7 +150,8 @@ ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
   // (the single-tile kernels' waves take a k range each: whole load batches a wave; a tile block's four
   // waves walk one slice together, which is cut to whole load batches, so its slices come out nearly equal:
   // k = 11008 in eight is seven slices of 1408 and one of 1152 instead of seven of 1536 and one of 256)
-  c.k_per_wave = round_up(ceil_div(d_in, c.NW * ks), c.MT > 1 ? kq / c.NW : kq);
+  const int step = c.MT == 1 ? kq : (d_out > 64 && !plain ? 64 : 128) / c.NW;
+  c.k_per_wave = round_up(ceil_div(d_in, c.NW * ks), step);
   c.ksplit = ceil_div(d_in, c.NW * c.k_per_wave);
   // An odd split (h_in = 14336 falls into seven slices of 2048) gives way to an even one of equal slices that
   // still fills the chip twice: 8192 rows, h_in = 14336, k in four instead of seven: rank 16 61.6 -> 53.1 us,
@@ -164,26 +169,28 @@ ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt) {
 }
 
 // Tile-block shrinks of more than 64 columns: 128 columns a workgroup, which then reads x once for them, instead of
-// 64 -- when that leaves workgroups enough (`wgs`, of 128 columns, over all projections of the launch).  The batches
-// are two k steps then (four would take 70 KB of LDS, two workgroups a CU: 27.5 us instead of 20.7 in the first line).
-// The choice does not touch the order of any sum.  64 / 128 columns, us (forward: the whole call; [k][n]: the product):
-//   forward, 2064 rows, two projections 4096 -> 4096 at rank 128 (528 workgroups): the shrink 25.5 / 20.7
-//   forward at rank 128, 4096 -> 4096: 512 rows (64) 20.2 / 23.0, 1024 rows (128) 23.0 / 25.7, 1500 rows (192)
-//     28.6 / 29.3, 2048 rows (256) 31.7 / 32.2, 3000 rows (282) 43.7 / 40.8; 11008 -> 4096: 512 rows (128) 25.5 / 27.8,
-//     640 rows (160) 30.8 / 29.2, 1024 rows (256) 34.4 / 31.5; q/k/v/o: 512 rows (256) 38.7 / 34.5
-//   weights [k][n], 4096 -> 128: 16 rows (8) 10.3 / 13.8, 1024 rows (128) 14.4 / 17.5, 4096 rows (256) 22.6 / 24.6;
-//     4096 -> 1024: 128 rows (128) 32.7 / 34.6, 512 rows (512) 41.2 / 39.4, 4096 rows (2048) 107.7 / 87.1
+// 64 -- when that leaves workgroups enough (`wgs`, of 128 columns, over all projections of the launch; a tile block per
+// 64 rows and half a one per adapter).  The batches are two k steps then (four would take 70 KB of LDS, two workgroups
+// a CU: 27.5 us instead of 20.7 in the first line).  The choice does not touch the order of any sum, so it may look at
+// the segmentation.  64 / 128 columns, us (forward: the whole call; [k][n]: the product), workgroups in parentheses:
+//   forward, 2064 rows, two projections 4096 -> 4096 at rank 128 (528): the shrink 25.5 / 20.7
+//   forward at rank 128, 4096 -> 4096: 512 rows (72) 20.2 / 23.0, 1024 rows (144) 23.0 / 25.7, 2048 rows (288)
+//     31.7 / 32.2, 3000 rows (306) 43.7 / 40.8; 11008 -> 4096: 512 rows (160) 25.5 / 27.8, 640 rows (192) 30.8 / 29.2,
+//     1024 rows (320) 34.4 / 31.5, 512 decoded rows over 32 adapters (384) 47.8 / 38.2; q/k/v/o: 512 rows (320)
+//     38.7 / 34.5
+//   weights [k][n], 4096 -> 128: 16 rows (16) 10.3 / 13.8, 1024 rows (144) 14.4 / 17.5, 4096 rows (264) 22.6 / 24.6;
+//     4096 -> 1024: 128 rows (256) 32.7 / 34.6, 512 rows (640) 41.2 / 39.4, 4096 rows (2112) 107.7 / 87.1
 inline bool shrink_wide(int mt, int d_out, bool w_kn, long wgs) {
-  return mt > 1 && d_out > 64 && (w_kn ? wgs > 256 : wgs >= 160);
+  return mt > 1 && d_out > 64 && (w_kn ? wgs > 300 : wgs >= 180);
 }
 
 // most k-split partials a shrink of this shape can leave behind, whichever wave count it runs with
-int fwd_ksplit_bound(int T, int d_in, int d_out) {
+int fwd_ksplit_bound(int T, int d_in, int d_out, bool plain = false) {
   int most = 1;
   for (int solo = 0; solo < 2; ++solo) {
-    const int a = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, 1).ksplit;
-    const int b = shrink_cfg(T, d_in, d_out, kDecodeWaves, solo != 0, 1).ksplit;
-    const int c = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles).ksplit;
+    const int a = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, 1, plain).ksplit;
+    const int b = shrink_cfg(T, d_in, d_out, kDecodeWaves, solo != 0, 1, plain).ksplit;
+    const int c = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain).ksplit;
     most = a > most ? a : most;
     most = b > most ? b : most;
     most = c > most ? c : most;
@@ -508,7 +515,7 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
                const float* seg_scale, int mt, hipStream_t st, bool fold = true, bool w_kn = false,
                const DropArgs* drop = nullptr, const int32_t* w_rank = nullptr, int packed = 0,
                const PlanSortArgs* build = nullptr, bool solo = false, const SideOut* side = nullptr,
-               bool* side_done = nullptr) {
+               bool* side_done = nullptr, bool plain = false) {
   if (drop && drop->seg_p && w_kn) return SMLM_ERR_ARG;
   if (side_done) *side_done = false;
   ShrinkArgs a{};
@@ -529,10 +536,12 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
   const int nw = shrink_waves(mt, nproj, d_in, d_out);
   long wgs = 0;  // workgroups of 128 columns
   for (int i = 0; mt > 1 && d_out > 64 && i < nproj; ++i)
-    wgs += (long)ceil_div(T, kTileRows * mt) * shrink_cfg(T, d_in[i], d_out, nw, solo, mt).ksplit * ceil_div(d_out, 128);
+    wgs += (long)(ceil_div(T, kTileRows * mt) + (groups > 0 && groups < S ? groups : S) / 2) *
+           shrink_cfg(T, d_in[i], d_out, nw, solo, mt, plain).ksplit *
+           ceil_div(d_out, 128);
   const bool wide = shrink_wide(mt, d_out, w_kn, wgs);
   for (int i = 0; i < nproj; ++i) {
-    ShrinkCfg c = shrink_cfg(T, d_in[i], d_out, nw, solo, mt);
+    ShrinkCfg c = shrink_cfg(T, d_in[i], d_out, nw, solo, mt, plain);
     if (wide) c.NB = 8, c.U = 2, c.zblocks = ceil_div(d_out, 128);
     if (i == 0) c0 = c;
     ShrinkProj& P = a.p[i];
@@ -728,7 +737,7 @@ SMLM_API int smlm_gemm_planned_workspace_size(int T, int d_in, int d_out, size_t
   if (T > (1 << 30)) return SMLM_ERR_LIMIT;
   size_t n = 256;
   if (d_in >= d_out) {
-    const int ks = fwd_ksplit_bound(T, d_in, d_out);
+    const int ks = fwd_ksplit_bound(T, d_in, d_out, true);
     if (ks > 1) n = align_up((size_t)ks * T * d_out * 4, 256);
   }
   *bytes = n;
@@ -780,9 +789,10 @@ SMLM_API int smlm_gemm_planned(void* y, const void* x, const void* const* w_ptrs
   float* partial = reinterpret_cast<float*>(workspace);
   if (w_row_major)  // the tile-block shrink stages [k][n] weights as they lie (as the backward's dV = dY B does)
     return run_shrink(dtype, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
-                      seg_scale, kBlkTiles, st, true, true);
+                      seg_scale, kBlkTiles, st, true, true, nullptr, nullptr, 0, nullptr, false, nullptr, nullptr, true);
   return run_shrink(dtype, pv, T, S, n_weights, 1, &x, &w_ptrs, &partial, &y, &d_in,
-                    d_out, &w_ld, beta, seg_scale, tiles_per_wave(T, d_out, d_in), st);
+                    d_out, &w_ld, beta, seg_scale, tiles_per_wave(T, d_out, d_in), st, true, false, nullptr, nullptr, 0,
+                    nullptr, false, nullptr, nullptr, true);
 }
 
 SMLM_API int smlm_gemm_workspace_size(int T, int S, int d_in, int d_out, size_t* bytes) {
@@ -821,7 +831,7 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
   // write the plan for the fold launch behind it (as the fused forward does with adapter ids).
   const int mt = tiles_per_wave(T, d_out, d_in);
   const int nw = shrink_waves(mt, 1, &d_in, d_out);
-  const int ks = shrink_cfg(T, d_in, d_out, nw, false, mt).ksplit;
+  const int ks = shrink_cfg(T, d_in, d_out, nw, false, mt, true).ksplit;
   const bool in_launch = d_in >= d_out && !w_row_major && self_planned_ok(T, S, S, pv.nt_max, mt) &&
                          (mt > 1 ? (S <= kFwdThreads || ks % 2 == 0)
                                  : (nw == kDecodeWaves && (S <= kSelfPlanThreads || ks % 2 == 0)));
@@ -830,7 +840,7 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
     const PlanSortArgs build{pv, seg_indptr, w_ptrs, SMLM_KEY_PTR2, S, next_pow2(S), w_ptrs};
     float* partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + plan_bytes);
     return run_shrink(dtype, pv, T, S, S, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
-                      seg_scale, mt, st, true, false, nullptr, nullptr, 0, &build);
+                      seg_scale, mt, st, true, false, nullptr, nullptr, 0, &build, false, nullptr, nullptr, true);
   }
   rc = plan_build_impl(pv, seg_indptr, w_ptrs, SMLM_KEY_PTR, S, st);
   if (rc) return rc;

@@ -17,16 +17,17 @@ SHAPES = [
     (1100, 9, 3, 2048, 1160, 128, None),
     (511, 4, 2, 2048, 72, 128, None),       # single tiles forward, the row below tile blocks
     (512, 4, 2, 2048, 72, 128, None),
-    (639, 5, 2, 4096, 72, 72, None),        # ... at ranks up to 96 and k of 4096
-    (640, 5, 2, 4096, 72, 96, None),
+    (511, 5, 2, 4096, 72, 72, None),        # ... at ranks up to 96 and k of 4096
+    (512, 5, 2, 4096, 72, 96, None),
+    (512, 5, 2, 5504, 5504, 128, None),     # k slices of 576, 64 columns a workgroup: a last batch of half its k
     (1023, 5, 2, 264, 88, 72, None),        # ... and at shorter k
     (1024, 5, 2, 264, 88, 96, None),
     (1040, 5, 2, 136, 88, 136, None),
     (1030, 6, 2, 328, 264, 256, None),
     (1200, 9, 3, 256, 520, 128, [8, 72, 128]),
-    (1100, 9, 3, 4096, 4096, 200, [200, 72, 136]),   # 288 workgroups of 128 columns: shrinks 128 columns wide, both ways
+    (1200, 9, 3, 4096, 4096, 200, [200, 72, 136]),   # workgroups enough for shrinks 128 columns wide, both ways
 ]
-IDS = ["3-rows", "rank72", "rank128", "511-rows", "512-rows", "639-rows", "640-rows", "1023-rows", "1024-rows", "rank136", "rank256", "packed", "wide-shrinks"]
+IDS = ["3-rows", "rank72", "rank128", "511-rows", "512-rows", "511-rows-rank72", "512-rows-rank96", "slices-of-576", "1023-rows", "1024-rows", "rank136", "rank256", "packed", "wide-shrinks"]
 
 
 def _inputs(case, dt, d, seed):
@@ -100,7 +101,8 @@ def test_backward_dyadic_bit_exact(K, oracle, gpu_device, case, drop, dt):
 @pytest.mark.parametrize("dt", ["fp16", "bf16"])
 @pytest.mark.parametrize("drop", [False, True], ids=["plain", "dropout"])
 @pytest.mark.parametrize("packed", [False, True], ids=["padded", "packed"])
-@pytest.mark.parametrize("k", [1024, 4096, 2560], ids=["64-columns", "128-columns", "odd-split-falls-back"])
+@pytest.mark.parametrize("k", [1024, 4096, 2560, 5504],
+                         ids=["64-columns", "128-columns", "odd-split-falls-back", "slices-of-576"])
 def test_plans_of_300_segments_built_in_the_shrinks(K, gpu_device, k, packed, drop, dt):
     """More segments than a four-wave workgroup has threads: the shrinks of both directions run two groups of waves a
     workgroup, 64 or 128 columns wide.  Everything they leave equals what plans built beforehand give, bit for bit."""

@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
     (300, 7, 2, 256, 192),      # shrink with three 64-column blocks
     (300, 7, 2, 96, 320),       # expand with a contraction above 64: 128 of k a piece
     (300, 7, 2, 200, 320),      # ... two pieces
-    (700, 7, 2, 4096, 520),     # shrink with 440 workgroups of 128 columns
+    (700, 7, 2, 4096, 520),     # shrink with workgroups enough for 128 columns each
     (5000, 300, 20, 2048, 32),  # many segments, plan in two launches
 ], ids=["shrink-r16", "expand-r16", "shrink-r64", "expand-r64", "shrink-wide", "expand-k96", "expand-k200", "shrink-128-columns",
         "many-segments"])
