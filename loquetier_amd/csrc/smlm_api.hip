@@ -353,32 +353,46 @@ int launch_shrink_self_planned(int dtype, const ShrinkCfg& c, int S, int groups,
                                  : launch_self_planned_dt<SMLM_DTYPE_BF16>(pairs, c, S, grid, st, sp);
 }
 
+template <int DT>
+int launch_side_fold(int ks, dim3 grid, hipStream_t st, const ReduceArgs& a) {
+  if (ks <= 4) return launch(side_fold_kernel<DT, 4>, grid, dim3(kSideThreads), st, a);
+  if (ks <= 8) return launch(side_fold_kernel<DT, 8>, grid, dim3(kSideThreads), st, a);
+  return launch(side_fold_kernel<DT, kMaxKsplit>, grid, dim3(kSideThreads), st, a);
+}
+template <int DT>
+int launch_reduce_rows(int ks, dim3 grid, hipStream_t st, const ReduceArgs& a) {
+  if (ks <= 4) return launch(reduce_rows_kernel<DT, 4>, grid, dim3(256), st, a);
+  if (ks <= 8) return launch(reduce_rows_kernel<DT, 8>, grid, dim3(256), st, a);
+  return launch(reduce_rows_kernel<DT, kMaxKsplit>, grid, dim3(256), st, a);
+}
+
 int launch_reduce(int dtype, int S, int groups, hipStream_t st, ReduceArgs& a, bool side = false) {
-  const int row_tiles = ceil_div(a.T, kTileRows);
+  const bool f16 = dtype == SMLM_DTYPE_F16;
+  int ks = 1;
+  for (int i = 0; i < a.nproj; ++i) ks = a.p[i].ksplit > ks ? a.p[i].ksplit : ks;
   if (side) {  // by tile slot: the by-products are stored in slot order
     const int units = tile_units_max(a.T, S, groups, 1);
-    const long items = (long)units * a.nproj;
+    const long items = (long)ceil_div(units, kBlkTiles) * ceil_div(a.d_out, 64) * a.nproj;
     a.units_max = items <= kDirectItems ? units : 0;
     const int zero_blocks = a.zero.n ? a.zero.first[a.zero.n] : 0;
     if (zero_blocks && !a.units_max) {  // (a launch that walks its items has no workgroups to spare)
       const int rc = launch(zero_spans_kernel, dim3((unsigned)zero_blocks), dim3(256), st, a.zero);
       if (rc) return rc;
     }
-    const dim3 grid = a.units_max ? dim3((unsigned)(items + zero_blocks)) : work_grid(items);
-    if (dtype == SMLM_DTYPE_F16) return launch(reduce_kernel<SMLM_DTYPE_F16, true>, grid, dim3(256), st, a);
-    return launch(reduce_kernel<SMLM_DTYPE_BF16, true>, grid, dim3(256), st, a);
+    const dim3 grid = a.units_max ? dim3((unsigned)(items + ceil_div(zero_blocks, kBlkTiles))) : work_grid(items);
+    return f16 ? launch_side_fold<SMLM_DTYPE_F16>(ks, grid, st, a) : launch_side_fold<SMLM_DTYPE_BF16>(ks, grid, st, a);
   }
-  if (!a.seg_scale && row_tiles <= kMaxGridY * 64) {  // no scale to look up: fold row by row
-    const dim3 grid((unsigned)row_tiles, (unsigned)a.nproj);
-    if (dtype == SMLM_DTYPE_F16) return launch(reduce_rows_kernel<SMLM_DTYPE_F16>, grid, dim3(256), st, a);
-    return launch(reduce_rows_kernel<SMLM_DTYPE_BF16>, grid, dim3(256), st, a);
+  const long fours = ((long)a.T * (a.d_out / 4) + 255) / 256;
+  if (!a.seg_scale && fours <= (1L << 23)) {  // no scale to look up: fold row by row
+    const dim3 grid((unsigned)fours, (unsigned)a.nproj);
+    return f16 ? launch_reduce_rows<SMLM_DTYPE_F16>(ks, grid, st, a) : launch_reduce_rows<SMLM_DTYPE_BF16>(ks, grid, st, a);
   }
   const int units = tile_units_max(a.T, S, groups, 1);
   const long items = (long)units * a.nproj;
   a.units_max = items <= kDirectItems ? units : 0;
   const dim3 grid = a.units_max ? dim3((unsigned)items) : work_grid(items);
-  if (dtype == SMLM_DTYPE_F16) return launch(reduce_kernel<SMLM_DTYPE_F16>, grid, dim3(256), st, a);
-  return launch(reduce_kernel<SMLM_DTYPE_BF16>, grid, dim3(256), st, a);
+  return f16 ? launch(reduce_kernel<SMLM_DTYPE_F16>, grid, dim3(256), st, a)
+             : launch(reduce_kernel<SMLM_DTYPE_BF16>, grid, dim3(256), st, a);
 }
 
 template <int DT, int NQ, bool DIRECT>

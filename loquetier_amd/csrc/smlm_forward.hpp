@@ -468,7 +468,7 @@ struct ZeroSpans {
   int first[kMaxProj + 1];
   int n;
 };
-__device__ __forceinline__ void zero_span_block(const ZeroSpans& z, int block) {
+__device__ __forceinline__ void zero_span_block(const ZeroSpans& z, int block, int thread) {
   int i = 0;
 #pragma unroll
   for (int j = 1; j < kMaxProj; ++j) i += (j < z.n && block >= z.first[j]) ? 1 : 0;
@@ -476,11 +476,11 @@ __device__ __forceinline__ void zero_span_block(const ZeroSpans& z, int block) {
   const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int e = 0; e < kZeroBlockBytes / (256 * 16); ++e) {
-    const long off = off0 + ((long)e * 256 + threadIdx.x) * 16;
+    const long off = off0 + ((long)e * 256 + thread) * 16;
     if (off < z.bytes[i]) stg16(reinterpret_cast<uint16_t*>(z.ptr[i] + off), zero);
   }
 }
-__global__ __launch_bounds__(256) void zero_spans_kernel(ZeroSpans z) { zero_span_block(z, (int)blockIdx.x); }
+__global__ __launch_bounds__(256) void zero_spans_kernel(ZeroSpans z) { zero_span_block(z, (int)blockIdx.x, threadIdx.x); }
 
 struct ReduceProj {
   const float* partial;  // [ksplit, T, d_out]
@@ -507,17 +507,11 @@ struct ReduceArgs {
 };
 
 // Folds the k-split partial sums of a shrink launch, in split order, into the
-// 16-bit result (the reference's "v in the I/O dtype"): work item -> (projection,
+// 16-bit result (the reference's "v in the I/O dtype"), scaled per segment: work item -> (projection,
 // tile), 16 threads per row.
-// SIDE: the fold of the backward's dV, which also leaves the by-products of write_side (further down)
-// behind -- the rounded sums and v2, scaled, by tile slot and transposed; slots without a row get zeros.
-template <int DT, bool SIDE = false>
+template <int DT>
 __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
   const int units = tile_units<1>(a.plan, a.units_max);
-  if (SIDE && a.units_max > 0 && (int)blockIdx.x >= units * a.nproj) {  // (uniform over the workgroup)
-    zero_span_block(a.zero, (int)blockIdx.x - units * a.nproj);
-    return;
-  }
   const int c = threadIdx.x >> 4, q = threadIdx.x & 15;
   const int last = a.units_max > 0 ? (int)blockIdx.x + 1 : units * a.nproj;
   for (int V = blockIdx.x; V < last; V += gridDim.x) {
@@ -527,8 +521,8 @@ __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
     if (!wid_ok(a.plan, uload(a.plan.tile_wid, tile))) continue;  // past the last tile (direct mode), or no such adapter
     const int slot = tile * kTileRows + c;
     const int row = a.plan.tile_row[slot];
-    if (!SIDE && row < 0) continue;
-    const float scale = (a.seg_scale && row >= 0) ? a.seg_scale[a.plan.tile_rseg[slot]] : 1.0f;
+    if (row < 0) continue;
+    const float scale = a.seg_scale ? a.seg_scale[a.plan.tile_rseg[slot]] : 1.0f;
     const float* zf = reinterpret_cast<const float*>(a.plan.hdr + kHdrZeros);
     for (int n = 4 * q; n < a.d_out; n += 64) {
       // all partials are requested before the first add waits for one; past ksplit the loads
@@ -536,53 +530,103 @@ __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
       f32x4 part[kMaxKsplit];
 #pragma unroll
       for (int z = 0; z < kMaxKsplit; ++z)
-        part[z] = ldg_f4((z < P.ksplit && row >= 0) ? P.partial + ((long)z * a.T + row) * a.d_out + n : zf);
-      u32x2 second = {0u, 0u};
-      if (SIDE && P.pt_b && row >= 0) second = *reinterpret_cast<const u32x2*>(P.v2 + (long)row * a.d_out + n);
+        part[z] = ldg_f4(z < P.ksplit ? P.partial + ((long)z * a.T + row) * a.d_out + n : zf);
       f32x4 sum = part[0];
 #pragma unroll
       for (int z = 1; z < kMaxKsplit; ++z) sum += part[z];
-      if (row >= 0) store4<DT>(P.out + (long)row * a.d_out + n, sum, scale, a.beta);
-      if (SIDE) {
-        const float ss = (a.side_scale && row >= 0) ? a.side_scale[a.plan.tile_rseg[slot]] : 1.0f;
-        // (from the rounded value, as a reader of `out` would scale it)
-        const u32x2 first = {pack2<DT>(scale * sum[0], scale * sum[1]), pack2<DT>(scale * sum[2], scale * sum[3])};
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          P.pt_a[(n + 2 * e) * a.side_pitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::lo(first[e]));
-          P.pt_a[(n + 2 * e + 1) * a.side_pitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::hi(first[e]));
-          if (P.pt_b) {
-            P.pt_b[(n + 2 * e) * a.side_pitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::lo(second[e]));
-            P.pt_b[(n + 2 * e + 1) * a.side_pitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::hi(second[e]));
-          }
-        }
-      }
+      store4<DT>(P.out + (long)row * a.d_out + n, sum, scale, a.beta);
     }
   }
 }
 
-// The same fold without a scale, walking the rows in order instead of through the plan's
-// tiles: grid (ceil(T / 16), projections), a workgroup folds 16 consecutive rows.  Nothing is
+// The same fold without a scale, four columns a thread over all rows in order instead of through the plan's
+// tiles: grid (T * d_out / 4 threads, projections).  Nothing is
 // looked up before the partials are requested; the rows that belong to a segment are the
 // range [hdr[5], hdr[5] + hdr[2]) (segments lie end to end) and only those are stored.
-template <int DT>
+// KS: upper bound of the launch's k splits.  Bound by its one round trip to memory: sixteen loads a thread whatever the
+// split, a row on sixteen lanes of which only d_out / 4 worked, 8600 rows, six projections at rank 64: 14.1 us, so 9.7;
+// 4224 rows, one projection at rank 16: 4.2 and 3.0.
+template <int DT, int KS>
 __global__ __launch_bounds__(256) void reduce_rows_kernel(ReduceArgs a) {
   const ReduceProj P = a.p[blockIdx.y];
   if (P.ksplit <= 1) return;
-  const int c = threadIdx.x >> 4, q = threadIdx.x & 15;
-  const int row = (int)blockIdx.x * kTileRows + c;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x, total = (long)a.T * (a.d_out / 4);
+  const int row = (int)(i / (a.d_out / 4));
   const int first = uload(a.plan.hdr, 5), count = uload(a.plan.hdr, 2);
-  const bool in_batch = row < a.T;
   const float* zf = reinterpret_cast<const float*>(a.plan.hdr + kHdrZeros);
-  for (int n = 4 * q; n < a.d_out; n += 64) {
-    f32x4 part[kMaxKsplit];
+  f32x4 part[KS];
 #pragma unroll
-    for (int z = 0; z < kMaxKsplit; ++z)
-      part[z] = ldg_f4((in_batch && z < P.ksplit) ? P.partial + ((long)z * a.T + row) * a.d_out + n : zf);
+  for (int z = 0; z < KS; ++z) part[z] = ldg_f4((i < total && z < P.ksplit) ? P.partial + (z * total + i) * 4 : zf);
+  f32x4 sum = part[0];
+#pragma unroll
+  for (int z = 1; z < KS; ++z) sum += part[z];
+  if (i < total && row >= first && row < first + count) store4<DT>(P.out + i * 4, sum, 1.0f, a.beta);
+}
+
+// The fold of the backward's dV, which also leaves the by-products of write_side (further down) behind: the rounded
+// sums and v2, scaled, by tile slot and transposed; slots without a row get zeros.  Work item -> (projection, 64
+// columns, four tiles), a thread per slot and four columns.  The transposed rows go through LDS, so that they are
+// written 128 bytes at a time: two bytes a lane straight from the registers, 268 partitions of 2080 rows, six
+// projections at ranks up to 64: 16.0 us, so 12.0; 2048 rows, two projections at rank 128: 11.3 and 7.5.  The
+// launch's workgroups past its items clear a.zero.
+constexpr int kSideThreads = kBlkTiles * 256;
+template <int DT, int KS>
+__global__ __launch_bounds__(kSideThreads) void side_fold_kernel(ReduceArgs a) {
+  constexpr int kSlots = kBlkTiles * kTileRows, kCols = 64;
+  constexpr int kTPitch = kSlots + 2;  // elements: columns 33 banks apart
+  __shared__ __attribute__((aligned(4))) uint16_t tr[2][kCols * kTPitch];
+  const int tiles = tile_units<1>(a.plan, a.units_max);
+  const int groups = (tiles + kBlkTiles - 1) / kBlkTiles, cols = (a.d_out + kCols - 1) / kCols;
+  const int items = groups * a.nproj * cols;
+  if (a.units_max > 0 && (int)blockIdx.x >= items) {  // (uniform over the workgroup)
+    const int block = ((int)blockIdx.x - items) * kBlkTiles + (int)(threadIdx.x >> 8);
+    if (block < a.zero.first[a.zero.n]) zero_span_block(a.zero, block, threadIdx.x & 255);
+    return;
+  }
+  const int slot = threadIdx.x >> 4, q = threadIdx.x & 15;
+  const float* zf = reinterpret_cast<const float*>(a.plan.hdr + kHdrZeros);
+  const int last = a.units_max > 0 ? (int)blockIdx.x + 1 : items;
+  for (int V = blockIdx.x; V < last; V += gridDim.x) {
+    const int pj = V / (groups * cols), in = V - pj * groups * cols;
+    const int n0 = in % cols * kCols, tile0 = in / cols * kBlkTiles;
+    const ReduceProj P = a.p[pj];
+    const int n = n0 + 4 * q;
+    // a tile past the last one or of no such adapter is left alone
+    auto tile_ok = [&](int t) {
+      return tile0 + t < tiles && wid_ok(a.plan, a.plan.tile_wid[tile0 + t < tiles ? tile0 + t : tile0]);
+    };
+    const int at = tile0 * kTileRows + (tile0 + (slot >> 4) < tiles ? slot : slot & 15);
+    int row = a.plan.tile_row[at];
+    const int seg = a.side_scale ? a.plan.tile_rseg[at] : -1;
+    if (!tile_ok(slot >> 4) || n >= a.d_out) row = -1;
+    f32x4 part[KS];
+#pragma unroll
+    for (int z = 0; z < KS; ++z)
+      part[z] = ldg_f4((z < P.ksplit && row >= 0) ? P.partial + ((long)z * a.T + row) * a.d_out + n : zf);
+    u32x2 second = {0u, 0u};
+    if (P.pt_b && row >= 0) second = *reinterpret_cast<const u32x2*>(P.v2 + (long)row * a.d_out + n);
+    const float ss = (row >= 0 && a.side_scale) ? a.side_scale[seg] : 1.0f;
     f32x4 sum = part[0];
 #pragma unroll
-    for (int z = 1; z < kMaxKsplit; ++z) sum += part[z];
-    if (in_batch && row >= first && row < first + count) store4<DT>(P.out + (long)row * a.d_out + n, sum, 1.0f, a.beta);
+    for (int z = 1; z < KS; ++z) sum += part[z];
+    if (row >= 0) store4<DT>(P.out + (long)row * a.d_out + n, sum, 1.0f, a.beta);
+    // (from the rounded value, as a reader of `out` would scale it)
+    const u32x2 one = {pack2<DT>(sum[0], sum[1]), pack2<DT>(sum[2], sum[3])};
+    __syncthreads();  // (the LDS of the previous item is read)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      tr[0][(4 * q + 2 * e) * kTPitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::lo(one[e]));
+      tr[0][(4 * q + 2 * e + 1) * kTPitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::hi(one[e]));
+      tr[1][(4 * q + 2 * e) * kTPitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::lo(second[e]));
+      tr[1][(4 * q + 2 * e + 1) * kTPitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::hi(second[e]));
+    }
+    __syncthreads();
+    const int which = threadIdx.x >> 9, m = (threadIdx.x >> 3) & 63, piece = threadIdx.x & 7;  // a piece: half a tile
+    uint16_t* pt = which ? P.pt_b : P.pt_a;
+    if (pt && n0 + m < a.d_out && tile_ok(piece >> 1)) {
+      const uint32_t* src = reinterpret_cast<const uint32_t*>(&tr[which][m * kTPitch + 8 * piece]);
+      stg16(pt + (long)(n0 + m) * a.side_pitch + (long)tile0 * kTileRows + 8 * piece, u32x4{src[0], src[1], src[2], src[3]});
+    }
   }
 }
 

@@ -136,3 +136,29 @@ def test_plans_of_300_segments_built_in_the_shrinks(K, gpu_device, k, packed, dr
 
     for a, b in zip(run(False), run(True)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1, 16, 63, 65, 200])
+@pytest.mark.parametrize("r", [8, 40, 64, 72, 136])
+def test_fold_of_dv_by_tile_slot(K, oracle, gpu_device, r, n):
+    """The fold of dV takes four tiles and 64 columns at a time and leaves s dV and s v transposed: pieces of both, rows
+    that end within a tile and within the four, an adapter without rows, scales; dyadic inputs, bit for bit."""
+    d, dt, NA, h = gpu_device, "bf16", 4, 1024
+    rng = np.random.default_rng(100 * r + n)
+    seg, ids = [0, n // 3, n // 3, n // 2, n], [0, 3, 1, 0]
+    A, B = [dyadic(rng, (r, h), 8, 64) for _ in range(NA)], [dyadic(rng, (h, r), 8, 8) for _ in range(NA)]
+    x, g = dyadic(rng, (n, h), 16, 8), dyadic(rng, (n, h), 16, 8)
+    Ad, Bd = [dev_t(a, dt, d) for a in A], [dev_t(b, dt, d) for b in B]
+    dA, dB = [torch.full_like(a, 9.0) for a in Ad], [torch.full_like(b, 9.0) for b in Bd]
+    dx = torch.empty(n, h, dtype=TDT[dt], device=d)
+    int32 = lambda v: torch.tensor(v, dtype=torch.int32, device=d)
+    _, v = oracle.add_lora_forward(x, [A[i] for i in ids], [B[i] for i in ids], seg, h, dt)
+    K.smlm_lora_backward(dx, ptrs(dA, d), ptrs(dB, d), dev_t(g, dt, d), dev_t(x, dt, d), dev_t(v, dt, d), ptrs(Ad, d),
+                         ptrs(Bd, d), K.SegmentPlan(int32(seg), int32(ids), n), r,
+                         torch.full((len(ids),), 2.0, device=d))
+    # a scale of two: every gradient is twice the unscaled one, bit for bit
+    gx, ga, gb = oracle.add_lora_backward(g, x, A, B, seg, ids, dt)
+    assert np.array_equal(to_np(dx), 2 * gx), "dX"
+    for a in range(NA):
+        assert np.array_equal(to_np(dA[a]), 2 * ga[a]), f"dA[{a}]"
+        assert np.array_equal(to_np(dB[a]), 2 * gb[a]), f"dB[{a}]"
