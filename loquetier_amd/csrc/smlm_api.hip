@@ -110,6 +110,49 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
   return all_long ? kDecodeWaves : kFwdWaves;
 }
 
+// Which of the two tile-block shrinks: shrink_block_kernel, whose waves read x and the weights for themselves, or
+// shrink_wide_kernel, whose workgroups stage the weights once for four waves.  Shrink and fold, us, wide / block, h_in =
+// 4096: one projection at rank 16, 2048 rows 13.0 / 11.6, 3000 rows 13.5 / 12.7; three at rank 32, 1000 rows 16.3 / 14.9,
+// 3000 rows 30 / 26.3; at rank 64 1500 rows 21 / 24.0, 2048 rows 23.5 / 25.8, 3000 rows 36 / 36, 7675 rows 68 / 60.
+// Above rank 64 x would be read once for every 64 columns.
+inline bool block_shrink(int mt, int T, int d_out) { return mt > 1 && (d_out <= 32 || (d_out <= 64 && T >= 3072)); }
+// ... of a launch: its weight rows must be within the block kernel's reach too (the slices are the same either way)
+inline bool block_shrink(int mt, const ShrinkArgs& a) {
+  bool near = block_shrink(mt, a.T, a.p[0].d_out);
+  for (int i = 0; i < a.items.nproj; ++i) near = near && a.p[i].ldw <= kBlockMaxLd;
+  return near;
+}
+
+// k slices of a tile-block shrink, in pieces of 256 of k (64 a wave): the split with the shortest time in steps of a
+// piece -- rounds of workgroups over the 256 CUs times (pieces of a slice + what starting one costs), an eighth more where
+// a CU has one workgroup only, the partial sums, and the fold, which costs as much as three pieces.  An uneven last
+// round is what costs most: 4096 rows, h_in = 11008 at rank 64, k in five 44.4 us, in four 30.4, in eight 33.6.
+// us with k in 1 / 2 / 4 / 8 / 16, one projection of h_in = 4096: 1024 rows at rank 64 - / - / - / 13.0 / 13.8; 2048
+// rows - / - / 15.2 / 14.7 / 18.1, at rank 128 - / 19.3 / 17.0 / 19.5 / 24.1; 4096 rows - / 20.0 / 17.3 / 19.1 / 24.6;
+// 8192 rows 27.1 / 29.3 / 27.0 / 30.9, at rank 16 20.2 / 25.3 / 22.1 / 21.5.  From about 7000 rows on slices of up to
+// 4608 fill the chip without being split, and a launch of several projections has no use for more workgroups
+// (8192 rows over 64 adapters, six projections at rank 64: 127 / 142 / 146 us).
+// Never more slices than `most`, which what callers' scratch holds was sized for.  `solo`: the backward's products,
+// whose fold leaves by-products behind and is wanted for that.
+int block_pieces(int T, int d_in, int d_out, int most, bool solo) {
+  const int P = ceil_div(d_in, 256), units = ceil_div(T > 0 ? T : 1, kTileRows * kBlkTiles) * ceil_div(d_out, 64);
+  if (most > kMaxKsplit) most = kMaxKsplit;
+  if (units >= 112 && !solo) {
+    const int ks = ceil_div(P, 18);
+    return ceil_div(P, ks < most ? ks : most);
+  }
+  int best = P;
+  float least = 0.0f;
+  for (int m = P; m >= 1; --m) {
+    const int ks = ceil_div(P, m);
+    const long wgs = (long)units * ks;
+    if (ks > most || (ks > 2 && wgs > 512) || (solo && ks == 1 && P > 1 && most > 1)) continue;
+    const float cost = (wgs + 255) / 256 * (m + 0.3f) * (wgs <= 256 ? 1.12f : 1.0f) + (0.1f + d_out / 160.0f) * ks + (ks > 1 ? 3.0f : 0.0f);
+    if (least == 0.0f || cost < least) least = cost, best = m;
+  }
+  return best;
+}
+
 // solo: the product is only ever launched by itself (the backward's dV and v products) and may take the
 // splits that suit a launch of one projection; the forward's projections keep one rule
 // whether they are launched alone or together, so that either way gives the same bits
@@ -147,6 +190,11 @@ ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt, bool
   if (max_split < 1) max_split = 1;
   if (max_split > kMaxKsplit) max_split = kMaxKsplit;
   const int ks = want < 1 ? 1 : (want > max_split ? max_split : want);
+  if (block_shrink(c.MT, T, d_out)) {
+    c.k_per_wave = 64 * block_pieces(T, d_in, d_out, ks, solo);
+    c.ksplit = ceil_div(d_in, c.NW * c.k_per_wave);
+    return c;
+  }
   // (the single-tile kernels' waves take a k range each: whole load batches a wave; a tile block's four
   // waves walk one slice together, which is cut to whole load batches, so its slices come out nearly equal:
   // k = 11008 in eight is seven slices of 1408 and one of 1152 instead of seven of 1536 and one of 256)
@@ -231,13 +279,35 @@ int launch_shrink_nb(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
 }
 
 template <int DT, bool DIRECT, bool WKN, bool DROP = false>
+int launch_shrink_wide(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
+  const dim3 block(kFwdThreads);  // U must match run_shrink
+  if (NB == 8) return launch(shrink_wide_kernel<DT, 8, 2, DIRECT, WKN, DROP>, grid, block, st, a);
+  return launch(shrink_wide_kernel<DT, 4, 4, DIRECT, WKN, DROP>, grid, block, st, a);
+}
+
+template <int DT, bool WKN, bool DROP = false>
 int launch_shrink_block(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
   const dim3 block(kFwdThreads);
-  if (NB == 1) return launch(shrink_block_kernel<DT, 1, 4, DIRECT, WKN, DROP>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_block_kernel<DT, 2, 4, DIRECT, WKN, DROP>, grid, block, st, a);
-  if (NB == 8) return launch(shrink_block_kernel<DT, 8, 2, DIRECT, WKN, DROP>, grid, block, st, a);
-  return launch(shrink_block_kernel<DT, 4, 4, DIRECT, WKN, DROP>, grid, block, st, a);
+  if (NB == 1) return launch(shrink_block_kernel<DT, 1, WKN, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_block_kernel<DT, 2, WKN, DROP>, grid, block, st, a);
+  return launch(shrink_block_kernel<DT, 4, WKN, DROP>, grid, block, st, a);
 }
+
+// Lists the chunk rows of a tile block are dealt out into, a workgroup (of four waves) each: what leaves the fewest
+// rounds of chunk rows a CU, within one generation of resident workgroups where that costs nothing, and the most
+// workgroups of those.  us, four / six / twelve lists, three projections of h_in = 4096 at rank 64, k in four: 4096 rows
+// 36.5 / 42.6 / 35.9, 8192 rows 59.4 / 64.4 / 61.7.
+int shrink_lists(int T, int S, int groups, int rows) {
+  const float units = ceil_div(T, kTileRows * kBlkTiles) + 0.5f * (groups > 0 && groups < S ? groups : S);
+  int best = rows;
+  float least = units * rows / 256 + 0.4f;
+  for (int lists = rows - 1; lists >= 1; --lists) {
+    const float cost = (float)((int)(1.05f * units * lists / 256) + 1) * ceil_div(rows, lists);
+    if (cost < least) least = cost, best = lists;
+  }
+  return best;
+}
+
 
 template <int DT, bool DIRECT>
 int launch_shrink_dt(int NB, int MT, int NW, dim3 grid, hipStream_t st,
@@ -246,13 +316,19 @@ int launch_shrink_dt(int NB, int MT, int NW, dim3 grid, hipStream_t st,
     if (MT == 1)
       return NW == kDecodeWaves ? launch_shrink_nb<DT, kDecodeWaves, DIRECT, true>(NB, grid, st, a)
                                 : launch_shrink_nb<DT, kFwdWaves, DIRECT, true>(NB, grid, st, a);
-    return launch_shrink_block<DT, DIRECT, false, true>(NB, grid, st, a);
+    return launch_shrink_wide<DT, DIRECT, false, true>(NB, grid, st, a);
   }
   if (MT == 1)
     return NW == kDecodeWaves ? launch_shrink_nb<DT, kDecodeWaves, DIRECT>(NB, grid, st, a)
                               : launch_shrink_nb<DT, kFwdWaves, DIRECT>(NB, grid, st, a);
-  return a.w_kn ? launch_shrink_block<DT, DIRECT, true>(NB, grid, st, a)
-                : launch_shrink_block<DT, DIRECT, false>(NB, grid, st, a);
+  return a.w_kn ? launch_shrink_wide<DT, DIRECT, true>(NB, grid, st, a)
+                : launch_shrink_wide<DT, DIRECT, false>(NB, grid, st, a);
+}
+
+template <int DT>
+int launch_shrink_block_dt(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
+  if (a.drop.seg_p) return launch_shrink_block<DT, false, true>(NB, grid, st, a);  // (weights [n][k])
+  return a.w_kn ? launch_shrink_block<DT, true>(NB, grid, st, a) : launch_shrink_block<DT, false>(NB, grid, st, a);
 }
 
 // all projections of one launch share NB / U / MT / NW (same rank, same T)
@@ -261,10 +337,18 @@ int launch_shrink(int dtype, const ShrinkCfg& c, int S, int groups, hipStream_t 
   const int MT = c.MT;
   a.items.interleave = 1;
   const int units = tile_units_max(a.T, S, groups, MT);
+  const bool f16 = dtype == SMLM_DTYPE_F16;
+  if (block_shrink(MT, a)) {
+    a.items.units_max = units;
+    const int y = units < kMaxGridY ? units : kMaxGridY;
+    const dim3 grid((unsigned)shrink_lists(a.T, S, groups, a.items.row_start[a.items.nproj]), (unsigned)y,
+                    (unsigned)ceil_div(units, y));
+    return f16 ? launch_shrink_block_dt<SMLM_DTYPE_F16>(c.NB, grid, st, a)
+               : launch_shrink_block_dt<SMLM_DTYPE_BF16>(c.NB, grid, st, a);
+  }
   const long items = (long)units * a.items.row_start[a.items.nproj];
   a.items.units_max = (items <= kDirectItems && units <= kMaxGridY) ? units : 0;
   const dim3 grid = item_grid(a.items, items);
-  const bool f16 = dtype == SMLM_DTYPE_F16;
   if (a.items.units_max)
     return f16 ? launch_shrink_dt<SMLM_DTYPE_F16, true>(c.NB, MT, c.NW, grid, st, a)
                : launch_shrink_dt<SMLM_DTYPE_BF16, true>(c.NB, MT, c.NW, grid, st, a);
@@ -283,16 +367,18 @@ int launch_self_planned_nb(int NB, dim3 grid, hipStream_t st, const SelfPlanArgs
 template <int DT, bool WKN, int THREADS, bool PAIRS, bool DROP = false>
 int launch_self_planned_block_nb(int NB, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
   const dim3 block(THREADS);  // U must match shrink_cfg
-  if (NB == 1) return launch(shrink_block_self_planned_kernel<DT, 1, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_block_self_planned_kernel<DT, 2, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
-  if (NB == 8) return launch(shrink_block_self_planned_kernel<DT, 8, 2, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
-  return launch(shrink_block_self_planned_kernel<DT, 4, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (!block_shrink(kBlkTiles, a.sh))
+    return NB == 8 ? launch(shrink_wide_self_planned_kernel<DT, 8, 2, WKN, THREADS, PAIRS, DROP>, grid, block, st, a)
+                   : launch(shrink_wide_self_planned_kernel<DT, 4, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 1) return launch(shrink_block_self_planned_kernel<DT, 1, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_block_self_planned_kernel<DT, 2, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  return launch(shrink_block_self_planned_kernel<DT, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
 }
 template <int DT, bool WKN, bool PAIRS, bool DROP = false>
 int launch_self_planned_block(int NB, int S, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
   if (S <= kFwdThreads) return launch_self_planned_block_nb<DT, WKN, kFwdThreads, PAIRS, DROP>(NB, grid, st, a);
-  // more segments than the four-wave workgroup has threads: two such groups a workgroup, each
-  // taking one of two neighbouring k slices (the caller has checked that the splits are even)
+  // more segments than the four-wave workgroup has threads: two such groups a workgroup, each taking a list of chunk
+  // rows or (ranks above 64) one of two neighbouring k slices (the caller has checked that the splits are even)
   grid.x = (grid.x + 1) / 2;
   return launch_self_planned_block_nb<DT, WKN, 2 * kFwdThreads, PAIRS, DROP>(NB, grid, st, a);
 }
@@ -349,6 +435,11 @@ int launch_shrink_self_planned(int dtype, const ShrinkCfg& c, int S, int groups,
   for (int i = 0; i < a.items.nproj; ++i)
     if (a.items.row_start[i + 1] - a.items.row_start[i] > rows) rows = a.items.row_start[i + 1] - a.items.row_start[i];
   dim3 grid((unsigned)rows, (unsigned)sp.units + 1u, (unsigned)a.items.nproj);
+  if (block_shrink(c.MT, a)) {
+    const int lists = shrink_lists(a.T, S, groups, a.items.row_start[a.items.nproj]);
+    sp.builder_rows = ceil_div(kSelfPlanBuilders, S <= kFwdThreads ? lists : ceil_div(lists, 2));
+    grid = dim3((unsigned)lists, (unsigned)(sp.units + sp.builder_rows));
+  }
   return dtype == SMLM_DTYPE_F16 ? launch_self_planned_dt<SMLM_DTYPE_F16>(pairs, c, S, grid, st, sp)
                                  : launch_self_planned_dt<SMLM_DTYPE_BF16>(pairs, c, S, grid, st, sp);
 }
@@ -575,7 +666,7 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
     // 59.6 us; 6144 rows, h_in = 4096, in three: 27.2 -> 25.0; launches of several projections and those that
     // build their plan keep their grid)
     int rows = c.ksplit * c.zblocks;
-    if (nproj == 1 && !build && rows > 1 && (rows & 1)) rows += 1;
+    if (nproj == 1 && !build && !block_shrink(mt, T, d_out) && rows > 1 && (rows & 1)) rows += 1;
     a.items.row_start[i + 1] = a.items.row_start[i] + rows;
     ra.p[i] = ReduceProj{partial[i], P.out, c.ksplit, side ? side->pt_a[i] : nullptr, side ? side->pt_b[i] : nullptr,
                          side ? side->v2[i] : nullptr};
@@ -847,7 +938,7 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
   const int nw = shrink_waves(mt, 1, &d_in, d_out);
   const int ks = shrink_cfg(T, d_in, d_out, nw, false, mt, true).ksplit;
   const bool in_launch = d_in >= d_out && !w_row_major && self_planned_ok(T, S, S, pv.nt_max, mt) &&
-                         (mt > 1 ? (S <= kFwdThreads || ks % 2 == 0)
+                         (mt > 1 ? (S <= kFwdThreads || block_shrink(mt, T, d_out) || ks % 2 == 0)
                                  : (nw == kDecodeWaves && (S <= kSelfPlanThreads || ks % 2 == 0)));
   if (in_launch) {
     if (!aligned16(y) || !aligned16(x)) return SMLM_ERR_ALIGN;
@@ -1005,7 +1096,7 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
   // (both routes pair k slices up in one workgroup beyond 512 / 256 segments)
   const bool self_planned = build_s && (!drop.seg_p || build_kind == SMLM_KEY_I32) &&
                             self_planned_ok(T, S, n_weights, pv.nt_max, mt) &&
-                            (mt > 1 ? (S <= kFwdThreads || even_splits)
+                            (mt > 1 ? (S <= kFwdThreads || block_shrink(mt, T, r) || even_splits)
                                                    : (expand_folds && (S <= kSelfPlanThreads || even_splits)));
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, build_kind, S, st, build_k2))) return rc;
   if (stages & SMLM_STAGE_SHRINK) {
@@ -1155,7 +1246,7 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   bool even_dv = true;  // (k slices in pairs beyond 256 partitions)
   for (int i = 0; i < n_proj; ++i) even_dv = even_dv && shrink_cfg(n_rows, h_out[i], r, kFwdWaves, true, mt).ksplit % 2 == 0;
   const bool self_planned = build_s && have_v && (!drop.seg_p || drop.bits) &&
-                            self_planned_ok(n_rows, P, NA, pv.nt_max, mt) && (P <= kFwdThreads || even_dv);
+                            self_planned_ok(n_rows, P, NA, pv.nt_max, mt) && (P <= kFwdThreads || block_shrink(mt, n_rows, r) || even_dv);
   const bool products = (stages & SMLM_BWD_PRODUCTS) != 0;
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, SMLM_KEY_I32, P, st))) return rc;
 

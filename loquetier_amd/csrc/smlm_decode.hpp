@@ -17,8 +17,8 @@
 // rows.  The plan orders groups by ascending id and a group's segments by index, which is
 // what the two scans walk, so unit u here is unit u of the plan.
 //
-// The products themselves repeat shrink_kernel / shrink_block_kernel step for step (same MFMA
-// sequence over k, same cross-wave sum): a call that builds its plan here and a call over the
+// The products themselves repeat shrink_kernel / shrink_wide_kernel step for step, or are the same code as
+// shrink_block_kernel's (same MFMA sequence over k, same cross-wave sum): a call that builds its plan here and a call over the
 // finished plan give the same bits, which the tests hold them to.  What differs is the order of
 // the loads -- the weights are requested as soon as the adapter is known, before the rows are.
 #pragma once
@@ -38,7 +38,8 @@ struct SelfPlanArgs {
   ShrinkArgs sh;        // sh.plan is not read (the plan does not exist yet), except w_rank
   PlanSortArgs plan;    // what the extra workgroups build; key_kind = SMLM_KEY_I32
   int n_weights;
-  int units;            // unit bound = grid.y - 1; workgroups with blockIdx.y == units: the plan builders
+  int units;            // unit bound; single tiles, wide tile blocks: workgroups with blockIdx.y == units are the plan builders
+  int builder_rows;     // tile blocks up to rank 64: the plan builders are the first rows of the grid (blockIdx.y < builder_rows)
 };
 
 // sixteen zero bytes for predicated-off loads (the other kernels read the plan header's)
@@ -366,36 +367,36 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   }
 }
 
-// ---- larger batches: the tile-block shrink_block_kernel ------------------------
+// ---- larger batches at ranks above 64: shrink_wide_kernel ----------------------------
 // WKN: the weights are stored [k][n], as B is for the backward's dV = dY B.
-// THREADS = 256: a workgroup is the four waves of shrink_block_kernel and takes one k slice of its
+// THREADS = 256: a workgroup is the four waves of shrink_wide_kernel and takes one k slice of its
 // tile block.  THREADS = 512 (more than 256 segments; finder and plan builders hold a segment per
 // thread): two such groups of four waves, each with its own staging buffers, which take two
 // neighbouring k slices -- the same sums as two workgroups of the 256-thread kind.  Both groups
 // walk a whole slice's worth of batches (past the end of k they multiply zeros) so that they meet
 // at the same barriers.
 template <int NB, int U, bool WKN, int GROUPS>
-struct SelfPlanBlockStage {
+struct SelfPlanWideStage {
   static constexpr int kPitch = WKN ? 16 * NB + 8 : 32 * U + 8;
   uint16_t wlds[GROUPS][2][(WKN ? 32 * U : 16 * NB) * kPitch];
 };
 template <int NB, int U, bool WKN, int THREADS, bool PAIRS>
-union SelfPlanBlockLds {
+union SelfPlanWideLds {
   PlanSmallLdsT<THREADS> plan;                                  // the plan-building workgroups
   FindLds<THREADS, PAIRS> find;                                 // the others: first while they find their tile block ...
-  SelfPlanBlockStage<NB, U, WKN, THREADS / kFwdThreads> stage;  // ... then the staged weight batches
+  SelfPlanWideStage<NB, U, WKN, THREADS / kFwdThreads> stage;  // ... then the staged weight batches
 };
 
 template <int DT, int NB, int U, bool WKN, int THREADS, bool PAIRS = false, bool DROP = false>
-__global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(SelfPlanArgs a) {
+__global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfPlanArgs a) {
   static_assert(THREADS == kFwdThreads || THREADS == 2 * kFwdThreads, "one or two groups of four waves");
   constexpr int GROUPS = THREADS / kFwdThreads;
   constexpr int KB = 32 * U;                 // k per batch
   constexpr int kRowsW = 16 * NB;            // weight rows (output columns) per workgroup
-  constexpr int kPitch = SelfPlanBlockStage<NB, U, WKN, GROUPS>::kPitch;
+  constexpr int kPitch = SelfPlanWideStage<NB, U, WKN, GROUPS>::kPitch;
   constexpr int kPieces = kRowsW * (KB / 8); // 16-byte pieces of one staged batch
   constexpr int kPer = (kPieces + kFwdThreads - 1) / kFwdThreads;
-  __shared__ __attribute__((aligned(16))) SelfPlanBlockLds<NB, U, WKN, THREADS, PAIRS> sm;
+  __shared__ __attribute__((aligned(16))) SelfPlanWideLds<NB, U, WKN, THREADS, PAIRS> sm;
   if ((int)blockIdx.y == a.units) {  // the extra row of the grid: up to kSelfPlanBuilders workgroups build the plan
     const int part = (int)(blockIdx.z * gridDim.x + blockIdx.x), all = (int)(gridDim.x * gridDim.z);
     if (part < kSelfPlanBuilders) plan_small_body(a.plan, sm.plan, part, all < kSelfPlanBuilders ? all : kSelfPlanBuilders);
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(Self
     }
   };
   auto weight_frag = [&](int buf, int u, int nb) -> u32x4 {
-    if (WKN) {  // as in shrink_block_kernel: four consecutive k rows of one column per transposing read
+    if (WKN) {  // as in shrink_wide_kernel: four consecutive k rows of one column per transposing read
       const uint16_t* base = &sm.stage.wlds[grp][buf][(32 * u + 8 * g + (c >> 2)) * kPitch + 16 * nb + 4 * (c & 3)];
       const u32x2 q0 = lds_read_tr16(base), q1 = lds_read_tr16(base + 4 * kPitch);
       return u32x4{q0[0], q0[1], q1[0], q1[1]};
@@ -487,7 +488,7 @@ __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(Self
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // ---- the product, as shrink_block_kernel does it
+  // ---- the product, as shrink_wide_kernel does it
   u32x4 xf[U];
   load_x(kbeg, xf);
   __syncthreads();  // every wave holds its rows: the finder's LDS turns into the weight staging area
@@ -530,6 +531,88 @@ __global__ __launch_bounds__(THREADS) void shrink_block_self_planned_kernel(Self
   }
   if (!PAIRS || tb + a.units >= un.total) return;  // uniform over the workgroup: no tile block is left for it
   __syncthreads();                       // the staged weights are read: the finder takes its LDS back
+  }
+}
+
+// ---- larger batches: shrink_block_kernel -------------------------------------------
+// WKN: the weights are stored [k][n], as B is for the backward's dV = dY B.
+// THREADS = 256: a workgroup is the four waves of shrink_block_kernel and takes one k slice of its
+// tile block.  THREADS = 512 (more than 256 segments; finder and plan builders hold a segment per
+// thread): two such groups of four waves, each with its own LDS area, which take two
+// neighbouring k slices -- the same sums as two workgroups of the 256-thread kind.
+template <int THREADS, bool PAIRS, int BYTES>
+union SelfPlanBlockLds {
+  PlanSmallLdsT<THREADS> plan;        // the plan-building workgroups
+  FindLds<THREADS, PAIRS> find;       // the others: first while they find their tile block ...
+  char area[THREADS / kFwdThreads][BYTES];  // ... then the product's
+};
+
+template <int DT, int NB, bool WKN, int THREADS, bool PAIRS = false, bool DROP = false>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB, DROP))))
+void shrink_block_self_planned_kernel(SelfPlanArgs a) {
+  static_assert(THREADS == kFwdThreads || THREADS == 2 * kFwdThreads, "one or two groups of four waves");
+  typedef BlockProduct<DT, NB, WKN, DROP> Product;
+  constexpr int GROUPS = THREADS / kFwdThreads;
+  __shared__ __attribute__((aligned(16))) SelfPlanBlockLds<THREADS, PAIRS, Product::kLdsBytes> sm;
+  if ((int)blockIdx.y < a.builder_rows) {  // up to kSelfPlanBuilders workgroups build the plan
+    const int part = (int)(blockIdx.y * gridDim.x + blockIdx.x), all = a.builder_rows * (int)gridDim.x;
+    if (part < kSelfPlanBuilders) plan_small_body(a.plan, sm.plan, part, all < kSelfPlanBuilders ? all : kSelfPlanBuilders);
+    return;
+  }
+  // grid x: the lists of chunk rows (as shrink_block_kernel's), a list a group
+  const int rows = a.sh.items.row_start[a.sh.items.nproj], lists = (int)gridDim.x * GROUPS;
+  const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kFwdThreads) : 0;
+  const int tl = threadIdx.x % kFwdThreads;
+  const int list = (int)blockIdx.x * GROUPS + grp;
+  const int wave = tl >> 6, c = threadIdx.x & 15;
+  const int turns = (rows - (int)blockIdx.x * GROUPS + lists - 1) / lists;  // of the workgroup's first group
+  if (turns <= 0) return;
+  int pj = 0;  // projection of the workgroup's first chunk row
+#pragma unroll
+  for (int i = 1; i < kMaxProj; ++i)
+    pj += (i < a.sh.items.nproj && (int)blockIdx.x * GROUPS >= a.sh.items.row_start[i]) ? 1 : 0;
+
+  // (PAIRS: a row of workgroups for every tile block the batch usually has; the others go round again, as in
+  // shrink_self_planned_kernel)
+  for (int tb = (int)blockIdx.y - a.builder_rows;; tb += a.units) {
+  FindSeg seg;
+  const FoundUnit un = find_adapter<THREADS, kBlkTiles, PAIRS>(sm.find, a.plan, a.sh.p[pj].w_ptrs, a.sh.plan.w_rank,
+                                                               a.n_weights, tb, &seg);
+  if (un.wid < 0) return;  // past the last tile block; uniform over the workgroup
+  const int wid = __builtin_amdgcn_readfirstlane(un.wid);
+  const uint64_t wp = sm.find.wtab[wid];  // (the same in every lane)
+  const uint16_t* W = reinterpret_cast<const uint16_t*>(
+      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)wp) |
+      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(wp >> 32)) << 32);
+  int nlim = a.sh.p[0].d_out;  // weight rows at or past it are zero padding
+  if (a.sh.plan.w_rank) {
+    const int r8 = (__builtin_amdgcn_readfirstlane(sm.find.rtab[wid]) + 7) & ~7;
+    nlim = r8 < nlim ? r8 : nlim;
+  }
+  // the adapter is known: its first weights are requested while the rows are still being found
+  Product pr(a.sh, tl, wid, nlim, __builtin_amdgcn_readfirstlane(un.tiles), list, lists);
+  typename Product::Stage first;
+  if (!pr.exists(list)) pr.r = (int)blockIdx.x * GROUPS;  // (a second group without a row: multiplies, stores nothing)
+  pr.open_w(GROUPS > 1 && pr.item(pr.r).pj != pj ? nullptr : W);
+  pr.load_w(first);
+
+  find_rows<THREADS, kBlkTiles, PAIRS>(sm.find, seg, un);
+  pr.set_rows([&](int i) { return sm.find.rows[i]; });  // -1: empty
+  if (DROP) {
+    const DropArgs dp = drop_proj(a.sh.drop, 0);  // (the rows' probabilities are the same for every projection)
+#pragma unroll
+    for (int t = 0; t < kBlkTiles; ++t)
+      pr.dr[DROP ? t : 0] = drop_row_of(dp, pr.frow[DROP ? t : 0], sm.find.rseg[t * kTileRows + c]);
+  }
+  if (!pr.exists(list)) pr.rw = -1;
+  if (a.sh.seg_scale && pr.rw >= 0) pr.scale = a.sh.seg_scale[sm.find.rseg[wave * kTileRows + c]];
+  pr.fill_rows();
+  pr.open_x();
+  __syncthreads();  // every wave holds its rows: the finder's LDS turns into the product's area
+
+  pr.run(first, sm.area[grp], turns);
+  if (!PAIRS || tb + a.units >= un.total) return;  // uniform over the workgroup: no tile block is left for it
+  __syncthreads();                       // the sums are read: the finder takes its LDS back
   }
 }
 

@@ -317,7 +317,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
   }
 }
 
-// Shrink for tile blocks (larger batches, and the backward).  Work item -> (projection, k
+// Shrink for tile blocks (larger batches, and the backward) at ranks above 64.  Work item -> (projection, k
 // slice, column block of 16 * NB, tile block) as above, but here wave w owns tile w of the block
 // and all four waves walk the whole k slice together: each 32*U-wide batch of the weight
 // rows is staged once in LDS (two buffers in turn, one barrier a batch) and shared by the
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
 // it lies in memory and the MFMA operand, which wants eight consecutive k of one column,
 // is read out of LDS with the transposing read.
 template <int DT, int NB, int U, bool DIRECT, bool WKN, bool DROP = false>
-__global__ __launch_bounds__(kFwdThreads) void shrink_block_kernel(ShrinkArgs a) {
+__global__ __launch_bounds__(kFwdThreads) void shrink_wide_kernel(ShrinkArgs a) {
   constexpr int KB = 32 * U;                 // k per batch
   constexpr int kRowsW = 16 * NB;            // weight rows (output columns) per workgroup
   constexpr int kPitch = WKN ? kRowsW + 8 : KB + 8;  // LDS row pitch in elements
@@ -455,6 +455,367 @@ __global__ __launch_bounds__(kFwdThreads) void shrink_block_kernel(ShrinkArgs a)
       }
     }
   }
+}
+
+// ---- the products of a tile block: x [64 rows, k slice] W^T, for one or more (projection, k slice) ----
+// Each of the four waves multiplies all four tiles of the block (64 rows) with 16 * NB weight columns over its own part
+// of the k slice -- pieces of 64 of k, the four waves' pieces side by side, so that the workgroup reads 512 consecutive
+// bytes of every row at a time -- and the waves' sums are added through LDS, in wave order, at the end of the slice.  No
+// wave waits for another before that: two pieces are held in registers in turn, of which one or two are on their way at
+// any time, the first of the next slice among them while a slice is finished.
+//
+// x and the weights are requested in full lines, eight lanes to 128 bytes of a row, and change layout through an LDS area
+// of the wave's own.  Requested as the MFMA wants them, sixteen rows to the sixteen neighbouring lanes, a load occupies
+// the CU's address unit for 65 cycles instead of 18 (measured with data out of L2), which alone holds x and the weights
+// together to 9.4 TB/s.
+//
+// Bound by HBM and by what surrounds it: 7675 rows, three projections 4096 -> 64: 59.4 us with the weights staged for
+// four waves at a barrier a batch, 50 so (189 MB of x; 245 MB fetched from beyond the L2s); whole pass of 7675 rows at
+// rank 64, 4096 -> 14336 twice and back, 281 -> 259 us; 8600 rows over 64 adapters, six projections, 826 -> 809 us.
+//
+// WKN: the weight matrices are stored [k][n] (k rows of d_out contiguous columns, as B
+// [h_out, r] is for the backward's dV = dY B) instead of [n][k]: a piece lies in LDS as it does in memory and the MFMA
+// operand, which wants eight consecutive k of one column, is read out of it with the transposing read.
+//
+// Slots without a row multiply the block's first row and columns at or past the adapter's rank another column's
+// weights: MFMA columns and rows do not mix, the former are not stored and the latter are stored as zeros.
+__device__ __attribute__((aligned(16))) uint32_t product_zeros[4];  // what loads past the end of a slice read
+
+constexpr int kBlockMaxLd = 1 << 25;  // longest weight row, in elements: a lane's offset in the weights has 32 bits
+
+// waves a SIMD the registers are held to
+constexpr int block_product_waves(int NB, bool DROP) { return NB >= 4 || (DROP && NB >= 2) ? 2 : 3; }
+
+template <int DT, int NB, bool WKN, bool DROP>
+struct BlockProduct {
+  static constexpr int KB = 64, U = KB / 32;      // k of a wave's piece, its 32-wide steps
+  static constexpr int kPitch = 16 * NB + 8;      // WKN: LDS row pitch of the weights in elements
+  static constexpr int kTileBytes = kTileRows * KB * 2;             // 16 rows of x (or of the weights) on their way
+  static constexpr int kWBytes = WKN ? KB * kPitch * 2 : NB * kTileBytes;
+  static constexpr int kStageBytes = kWBytes + 2 * kTileBytes;      // of a wave
+  static constexpr int kRedBytes = kFwdWaves * kBlkTiles * NB * kWaveSize * 16;
+  static constexpr int kLdsBytes = kFwdWaves * kStageBytes > kRedBytes ? kFwdWaves * kStageBytes : kRedBytes;
+
+  struct Stage {
+    u32x4 x[kBlkTiles][2], w[2 * NB];  // as they are loaded: eight rows of eight 16-byte pieces an element
+    int k0;
+  };
+  struct Item {  // (all uniform over the four waves)
+    int pj, kz, zb, kbeg, kend, n;  // n: pieces a wave takes
+  };
+
+  const ShrinkArgs& a;
+  const int lane, wave, c, g;
+  const int wid, nlim;       // the block's adapter; weight rows at or past nlim are zero padding
+  const int tiles;           // tiles of the block
+  const int nlists;          // the chunk rows r, r + nlists ... are this group's
+  int lrow[kBlkTiles][2];    // the rows this lane loads: 8 i + lane / 8 of tile t (the block's first row: none)
+  int frow[DROP ? kBlkTiles : 1];  // DROP: the rows it multiplies, lane % 16 of tile t (-1: none)
+  int rw;                    // its row of tile `wave`, which it stores
+  float scale;               //   ... and what that is scaled with when no partial sums are stored
+  DropRow dr[DROP ? kBlkTiles : 1];
+  f32x4 acc[kBlkTiles][NB];
+  // what is loaded next
+  int r, s;
+  Item li;
+  const uint16_t *wbase, *xbase;
+  int d_in, ldw, ncols;      // ncols: columns of the block that have weights (a multiple of 8, may be 0 or less)
+  uint32_t woff;             // the lane's byte offset in the weights (up to 31 rows: ldw <= kBlockMaxLd)
+
+  __device__ __forceinline__ BlockProduct(const ShrinkArgs& args, int thread, int wid_, int nlim_, int tiles_, int list,
+                                          int lists)
+      : a(args), lane(thread & 63), wave(__builtin_amdgcn_readfirstlane(thread >> 6)), c(thread & 15),
+        g((thread & 63) >> 4), wid(wid_), nlim(nlim_), tiles(tiles_), nlists(lists), rw(-1), scale(1.0f), r(list), s(0) {
+#pragma unroll
+    for (int t = 0; t < kBlkTiles; ++t)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[t][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // the rows of the block, row_of(slot): row of slot 16 t + i of the block, -1 where there is none (not slot 0)
+  template <typename F>
+  __device__ __forceinline__ void set_rows(const F& row_of) {
+#pragma unroll
+    for (int t = 0; t < kBlkTiles; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) lrow[t][i] = row_of(kTileRows * t + 8 * i + (lane >> 3));
+    rw = row_of(kTileRows * wave + c);
+    if (DROP) {
+#pragma unroll
+      for (int t = 0; t < kBlkTiles; ++t) frow[DROP ? t : 0] = row_of(kTileRows * t + c);
+    }
+  }
+
+  __device__ __forceinline__ bool exists(int row_) const { return row_ < a.items.row_start[a.items.nproj]; }
+  __device__ __forceinline__ Item item(int row_) const {
+    Item it;
+    it.pj = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxProj; ++i) it.pj += (i < a.items.nproj && row_ >= a.items.row_start[i]) ? 1 : 0;
+    const int yy = row_ - a.items.row_start[it.pj];
+    const ShrinkProj& P = a.p[it.pj];
+    it.kz = yy / P.zblocks, it.zb = yy % P.zblocks;  // (the column blocks of a slice side by side: they read the same x)
+    it.kbeg = it.kz * kFwdWaves * P.k_per_wave;
+    it.kend = min(it.kbeg + kFwdWaves * P.k_per_wave, P.d_in);
+    it.n = (it.kend - it.kbeg + kFwdWaves * KB - 1) / (kFwdWaves * KB);
+    return it;
+  }
+  // the weights of chunk row r; `W`: their address where the caller already knows it
+  __device__ __forceinline__ void open_w(const uint16_t* W = nullptr) {
+    li = item(r);
+    const ShrinkProj& P = a.p[li.pj];
+    if (!W) W = uload_ptr(P.w_ptrs, wid);
+    const int n0 = li.zb * 16 * NB;
+    ldw = WKN ? rank_ld(a.plan, P.ldw, nlim) : P.ldw;  // [k][n] weights (B) have the rank contiguous
+    ncols = nlim - n0;
+    if (WKN) {
+      wbase = W + n0;
+      const int n8 = (lane % (2 * NB)) * 8;
+      woff = ((uint32_t)(lane / (2 * NB)) * (uint32_t)ldw + (uint32_t)(n8 < ncols ? n8 : 0)) * 2u;
+    } else {
+      wbase = W + (long)n0 * ldw;
+      woff = ((uint32_t)(lane >> 3) * (uint32_t)ldw + 8u * (lane & 7)) * 2u;
+    }
+    s = 0;
+  }
+  __device__ __forceinline__ void open_x() {
+    const ShrinkProj& P = a.p[li.pj];
+    d_in = P.d_in;
+    xbase = P.x + 8 * (lane & 7);
+  }
+  // slots without a row load the block's first row
+  __device__ __forceinline__ void fill_rows() {
+    const int any = max(__builtin_amdgcn_readfirstlane(lrow[0][0]), 0);
+#pragma unroll
+    for (int t = 0; t < kBlkTiles; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) lrow[t][i] = lrow[t][i] >= 0 ? lrow[t][i] : any;
+  }
+  __device__ __forceinline__ int piece_k() const {
+    int k0 = li.kbeg + (wave + kFwdWaves * s) * KB;
+    // (opaque: the compiler otherwise keeps an induction register pair for every address)
+    asm volatile("" : "+s"(k0));
+    return k0;
+  }
+  // a piece past the end of its slice (every wave takes as many) or the list reads zeros, as does its part past the end
+  __device__ __forceinline__ void load_w(Stage& st) {
+    const int k0 = st.k0 = piece_k();
+    const uint16_t* zeros = reinterpret_cast<const uint16_t*>(product_zeros);
+    const int kend = ncols > 0 ? li.kend : 0;  // (a block of which no column has weights)
+#pragma unroll
+    for (int j = 0; j < 2 * NB; ++j) {
+      if (WKN) {
+        const int kj = k0 + (32 / NB) * j;
+        const uint16_t* p = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(wbase + (long)kj * ldw) + woff);
+        st.w[j] = ldg16_or(p, kj + lane / (2 * NB) < kend, zeros);
+      } else {
+        const uint16_t* p = reinterpret_cast<const uint16_t*>(
+            reinterpret_cast<const char*>(wbase + (long)(8 * j < ncols ? 8 * j : 0) * ldw + k0) + woff);
+        st.w[j] = ldg16_or(p, k0 + 8 * (lane & 7) < kend, zeros);
+      }
+    }
+  }
+  __device__ __forceinline__ void load_x(Stage& st) {
+    const uint16_t* zeros = reinterpret_cast<const uint16_t*>(product_zeros);
+    const bool in = st.k0 + 8 * (lane & 7) < li.kend;
+    const uint16_t* base = in ? xbase + st.k0 : zeros;
+    const uint32_t pitch = in ? (uint32_t)d_in * 2u : 0u;
+#pragma unroll
+    for (int t = 0; t < kBlkTiles; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        st.x[t][i] = ldg16(reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(base) +
+                                                             (uint64_t)(uint32_t)lrow[t][i] * pitch));
+    ++s;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void load(Stage& st) {
+    if (s >= li.n) {  // (no vector memory access in here: the compiler would wait for the loads in flight)
+      r += nlists;
+      if (exists(r)) {
+        open_w();
+        open_x();
+      } else {
+        li.kend = 0;  // zeros from here on
+      }
+    }
+    load_w(st);
+    load_x(st);
+  }
+  // Through the wave's LDS area from rows of full lines, as they are loaded, to MFMA operands.  Piece p of row i lies in
+  // place p ^ (i / 2) of its row: both ways every instruction touches each bank once.
+  __device__ __forceinline__ void put(char* lds, int i, u32x4 v) const {
+    const int row = 8 * i + (lane >> 3);
+    *reinterpret_cast<u32x4*>(lds + row * (KB * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4)) = v;
+  }
+  __device__ __forceinline__ u32x4 get(const char* lds, int u) const {
+    return *reinterpret_cast<const u32x4*>(lds + c * (KB * 2) + (((4 * u + g) ^ ((c >> 1) & 7)) << 4));
+  }
+  // a wave's own LDS accesses are served in order; the compiler must keep them in order too
+  static __device__ __forceinline__ void lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  __device__ __forceinline__ void multiply(const Stage& st, char* lds, const DropArgs& dp, const Item& it) {
+    uint16_t* wl = reinterpret_cast<uint16_t*>(lds);
+#pragma unroll
+    for (int j = 0; j < 2 * NB; ++j) {
+      if (WKN) *reinterpret_cast<u32x4*>(&wl[((32 / NB) * j + lane / (2 * NB)) * kPitch + (lane % (2 * NB)) * 8]) = st.w[j];
+      else put(lds + (j >> 1) * kTileBytes, j & 1, st.w[j]);
+    }
+    u32x4 wf[NB][U];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (h == 1 && tiles <= 2) break;  // (uniform over the four waves)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) put(lds + kWBytes + (e >> 1) * kTileBytes, e & 1, st.x[2 * h + (e >> 1)][e & 1]);
+      lds_order();
+      if (h == 0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            if (WKN) {
+              // lane c names k row 32u + 8g (+4) + c/4 and columns 16nb + 4(c%4) .. +3; it receives
+              // column 16nb + c of four consecutive k rows per read
+              const uint16_t* base = &wl[(32 * u + 8 * g + (c >> 2)) * kPitch + 16 * nb + 4 * (c & 3)];
+              const u32x2 q0 = lds_read_tr16(base), q1 = lds_read_tr16(base + 4 * kPitch);
+              wf[nb][u] = u32x4{q0[0], q0[1], q1[0], q1[1]};
+            } else {
+              wf[nb][u] = get(lds + nb * kTileBytes, u);
+            }
+          }
+      }
+      u32x4 xf[2][U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          xf[e][u] = get(lds + kWBytes + e * kTileBytes, u);
+          if (DROP) {
+            const ShrinkProj& P = a.p[it.pj];
+            const int t = 2 * h + e, kk = st.k0 + 32 * u + 8 * g;
+            xf[e][u] = drop8<DT>(xf[e][u], dp, dr[DROP ? t : 0], frow[DROP ? t : 0], kk >> 3, P.drop_bits, P.d_in >> 3,
+                                 it.zb == 0 && kk < it.kend);
+          }
+        }
+      lds_order();
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) acc[2 * h + e][nb] = Num<DT>::mfma(wf[nb][u], xf[e][u], acc[2 * h + e][nb]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // Sum over the waves and store: wave w the rows of tile w.  Every thread of the four waves calls it.
+  __device__ __forceinline__ void finish(char* smem, const Item& it, bool real) {
+    f32x4(*red)[kBlkTiles][NB][kWaveSize] = reinterpret_cast<f32x4(*)[kBlkTiles][NB][kWaveSize]>(smem);
+    const ShrinkProj& P = a.p[it.pj];
+    const bool as_partial = P.ksplit > 1 || P.to_partial;
+    const int n0 = it.zb * 16 * NB;
+    __syncthreads();  // every wave is done with the area
+#pragma unroll
+    for (int t = 0; t < kBlkTiles; ++t)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        red[wave][t][nb][lane] = acc[t][nb];
+        acc[t][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    __syncthreads();
+    if (rw >= 0 && real) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        f32x4 part[kFwdWaves];
+#pragma unroll
+        for (int w = 0; w < kFwdWaves; ++w) part[w] = red[w][wave][nb][lane];
+        f32x4 sum = part[0];
+#pragma unroll
+        for (int w = 1; w < kFwdWaves; ++w) sum += part[w];
+        const int n = n0 + 16 * nb + 4 * g;  // lane holds columns n .. n+3 of its token
+        if (n >= P.d_out) continue;
+        if (n >= nlim) sum = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (as_partial)
+          *(SMLM_GLOBAL f32x4*)(P.partial + ((long)it.kz * a.T + rw) * P.d_out + n) = sum;
+        else
+          store4<DT>(P.out + (long)rw * P.d_out + n, sum, scale, a.beta);
+      }
+    }
+    __syncthreads();  // the sums are read: the area takes rows again
+  }
+  // The products of the group's chunk rows, the weights of the first piece (`sa`) already requested.  `turns`: how many,
+  // turns past the group's last row among them (every group of a workgroup takes as many: there are barriers inside).
+  __device__ __forceinline__ void run(Stage& sa, char* smem, int turns) {
+    char* lds = smem + wave * kStageBytes;
+    int mr = r, ms = 0;  // what is multiplied: chunk row, piece
+    Item mi = li;
+    DropArgs dp{};
+    if (DROP) dp = drop_proj(a.drop, mi.pj);
+    auto next = [&] {
+      if (++ms < mi.n) return;
+      finish(smem, mi, exists(mr));
+      mr += nlists;
+      --turns;
+      ms = 0;
+      if (exists(mr)) {
+        mi = item(mr);
+        if (DROP) dp = drop_proj(a.drop, mi.pj);
+      } else {
+        mi.n = 1;
+      }
+    };
+    Stage sb;
+    load_x(sa);
+    // (all loads are unconditional: where branches join the compiler waits for every load in flight)
+#pragma unroll 1
+    while (true) {
+      load(sb);
+      multiply(sa, lds, dp, mi);
+      next();
+      if (turns <= 0) break;
+      load(sa);
+      multiply(sb, lds, dp, mi);
+      next();
+      if (turns <= 0) break;
+    }
+  }
+};
+
+// Shrink for tile blocks (larger batches, and the backward).  Grid (lists, tile blocks): a workgroup takes the chunk rows
+// (projection, k slice, column block of 16 * NB) blockIdx.x, blockIdx.x + gridDim.x ... of its tile block.
+template <int DT, int NB, bool WKN, bool DROP = false>
+__global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB, DROP))))
+void shrink_block_kernel(ShrinkArgs a) {
+  typedef BlockProduct<DT, NB, WKN, DROP> Product;
+  __shared__ __attribute__((aligned(16))) char smem[Product::kLdsBytes];
+  const int tb = (int)(blockIdx.y + blockIdx.z * gridDim.y);
+  if (tb >= a.items.units_max) return;
+  int t0, cnt, wid;
+  pick_tiles<kBlkTiles>(a.plan, tb, &t0, &cnt, &wid);
+  if (cnt == 0) return;  // uniform over the workgroup
+  const int c = threadIdx.x & 15, wave = threadIdx.x >> 6;
+  const int nlim = rank_limit(a.plan, wid, a.p[0].d_out);
+  Product pr(a, threadIdx.x, wid, nlim, cnt, blockIdx.x, gridDim.x);
+  pr.set_rows([&](int i) {
+    const int row = a.plan.tile_row[(i < cnt * kTileRows ? t0 * kTileRows : t0 * kTileRows - i) + i];
+    return i < cnt * kTileRows ? row : -1;
+  });
+  const int slot = (t0 + wave) * kTileRows + c;
+  typename Product::Stage first;
+  pr.open_w();
+  pr.load_w(first);
+  if (a.seg_scale && pr.rw >= 0) pr.scale = a.seg_scale[a.plan.tile_rseg[slot]];
+  if (DROP) {
+    const DropArgs dp = drop_proj(a.drop, 0);  // (the rows' probabilities are the same for every projection)
+#pragma unroll
+    for (int t = 0; t < kBlkTiles; ++t)
+      pr.dr[DROP ? t : 0] = drop_row(dp, pr.frow[DROP ? t : 0], a.plan.tile_rseg, (t0 + t) * kTileRows + c);
+  }
+  pr.fill_rows();
+  pr.open_x();
+  const int rows = a.items.row_start[a.items.nproj];
+  pr.run(first, smem, (rows - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
 }
 
 constexpr int kMaxKsplit = 16;  // upper bound of the k split over workgroups
