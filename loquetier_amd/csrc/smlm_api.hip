@@ -610,7 +610,6 @@ struct SideOut {
   uint16_t* pt_b[kMaxProj];
   const uint16_t* v2[kMaxProj];
   const float* scale;
-  long pitch;
   ZeroSpans zero;  // memory the fold's launch is to clear as well (n = 0: none)
 };
 
@@ -690,7 +689,6 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
   const bool with_side = side && all_reduce;
   if (with_side) {
     ra.side_scale = side->scale;
-    ra.side_pitch = side->pitch;
     ra.zero = side->zero;
   }
   if (side_done) *side_done = with_side;
@@ -719,7 +717,6 @@ struct BwdProjLayout {
 struct BwdLayout {
   BwdProjLayout p[kMaxProj];
   size_t total;
-  long pitch;
 };
 
 // the projections' areas lie end to end, each laid out as a backward of that projection alone
@@ -731,7 +728,7 @@ BwdLayout bwd_layout(int n_proj, int n_rows, int P, int NA, const int* h_in, con
     off = align_up(off + bytes, 256);
     return o;
   };
-  L.pitch = (long)plan_nt_max(n_rows, P) * kTileRows;
+  const size_t slots = (size_t)plan_nt_max(n_rows, P) * kTileRows;
   for (int i = 0; i < n_proj; ++i) {
     BwdProjLayout& Q = L.p[i];
     const int ks_dv = fwd_ksplit_bound(n_rows, h_out[i], r), ks_v = fwd_ksplit_bound(n_rows, h_in[i], r);
@@ -739,8 +736,8 @@ BwdLayout bwd_layout(int n_proj, int n_rows, int P, int NA, const int* h_in, con
     Q.partial = take((size_t)ks * n_rows * r * 4);
     Q.dv16 = take((size_t)n_rows * r * 2);
     Q.v16 = take((size_t)n_rows * r * 2);
-    Q.pt_a = take((size_t)r * L.pitch * 2);
-    Q.pt_b = take((size_t)r * L.pitch * 2);
+    Q.pt_a = take(r * slots * 2);
+    Q.pt_b = take(r * slots * 2);
     Q.bits = take((size_t)n_rows * (h_in[i] / 8));  // keep bits of x's dropout mask when the caller has none
   }
   L.total = off;
@@ -1320,7 +1317,6 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
     side.v2[i] = reinterpret_cast<const uint16_t*>(vv[i]);
   }
   side.scale = part_scale;
-  side.pitch = L.pitch;
   // rows of dX past the backward's own (opts->dx_rows): cleared by the fold's launch when it runs in direct mode,
   // else by a launch of their own
   ZeroSpans tail{};
@@ -1421,7 +1417,6 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
     Q.drop_pitch = h_in[i] / 8;
     units += Q.units_a + ceil_div(ceil_div(Q.h_out, kWgCols), walk);
   }
-  wa.pitch = L.pitch;
   wa.r = r;
   wa.n_parts = P;
   wa.grp_seg = pv.grp_seg;

@@ -15,8 +15,8 @@ constexpr int kWgMaxProj = 8;  // projections one weight-gradient launch can ser
 struct WgradProj {
   const uint16_t* q_a;   // x  [n_rows, h_in]   -> dA
   const uint16_t* q_b;   // dY [n_rows, h_out]  -> dB
-  const uint16_t* pt_a;  // scale*dV by slot, transposed [r, pitch]
-  const uint16_t* pt_b;  // scale*v  by slot, transposed [r, pitch]
+  const uint16_t* pt_a;  // scale*dV by tile slot, transposed (side_piece)
+  const uint16_t* pt_b;  // scale*v, likewise
   void* const* da_ptrs;  // [NA] -> [r, h_in]
   void* const* db_ptrs;  // [NA] -> [h_out, r]
   int h_in, h_out, chunks_a;  // chunks_a = ceil(h_in/64) 64-column chunks of dA (dB: ceil(h_out/64))
@@ -36,7 +36,6 @@ struct WgradArgs {
   int units;               // units of all projections
   int zcount;              // workgroups along the rank, see wgrad_kernel
   int walk;                // chunks a one-wave workgroup takes in turn (NW = 1 kernels; else 1)
-  long pitch;
   int r;
   int n_parts;             // partitions the plan was laid out for (>= 1): its group tables hold n_parts + 1 entries
   const int32_t* w_rank;   // optional [NA]: true rank of each adapter (rows of dV / v past it are zero padding)
@@ -75,6 +74,11 @@ __device__ __forceinline__ int wg_lds_row(int s) {
 // token-innermost with the transposing LDS read; no workgroup barrier is needed
 // inside the loop, and the rows of the next step are already on their way from
 // memory while the current step is multiplied.
+// Bound by the loads a CU's address unit can take besides HBM: the token-side operand comes in lines (side_piece) and
+// the row numbers of a step in one load, dealt out by lane exchange.  With the operand in rows of slots, sixteen rows a
+// load, and eight loads of row numbers a step, us: 2080 rows in 268 partitions over 64 adapters of ranks up to 64, six
+// projections 156 (and 44 bytes of spills), so 138; 2048 rows over two adapters, two projections at rank 128 32.3 and
+// 26.5; 2754 rows with dropout at rank 32, two projections 26.0 and 24.6; 4096 rows at rank 16, one 15.2 and 14.2.
 //
 // DROP (dA only): the forward multiplied the dropped x, so dA = dV^T dropout(x).  The keep
 // bits (one byte per eight columns, the projection's drop_bits) travel with the rows and are applied while the
@@ -143,28 +147,26 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   const int tr_row = wg_lds_row(8 * g + (c >> 2));  // + 4h -> LDS row + 8h; + 32 per k step
   const int tr_col = 4 * (c & 3);
 
-  auto load_rows = [&](int step, int32_t (&row)[8]) {
-    const int tile0 = t_beg + kStepTiles * step;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int s = wg_lds_row(8 * u + rlow);  // the swap is its own inverse
-      const int tile = tile0 + (s >> 4);
-      row[u] = (step < n_steps && tile < t_end) ? a.tile_row[tile * kTileRows + (s & 15)] : -1;
-    }
+  // row numbers: slot `lane` of the step in every lane, dealt out when the rows are requested
+  auto load_rows = [&](int step) -> int32_t {
+    const int tile = t_beg + kStepTiles * step + (lane >> 4);
+    return (step < n_steps && tile < t_end) ? a.tile_row[tile * kTileRows + c] : -1;
   };
+  const int slot0 = wg_lds_row(rlow);
   const uint8_t* zero_bytes = reinterpret_cast<const uint8_t*>(zeros);
-  auto load_data = [&](const int32_t (&row)[8], int n0, u32x4 (&val)[8], uint32_t (&keep)[DROP ? 8 : 1]) {
+  auto load_data = [&](int32_t rows, int n0, u32x4 (&val)[8], uint32_t (&keep)[DROP ? 8 : 1]) {
     const bool col_ok = n0 + lcol < h;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const bool ok = row[u] >= 0 && col_ok;
+      const int32_t row = __shfl(rows, slot0 + wg_lds_row(8 * u));  // (wg_lds_row is its own inverse)
+      const bool ok = row >= 0 && col_ok;
       // x and dY are read here for the last time in the backward: non-temporal, unless the workgroup next door
       // reads the same lines for other ranks
-      const uint16_t* q = Q + (long)row[u] * h + n0 + lcol;
+      const uint16_t* q = Q + (long)row * h + n0 + lcol;
       val[u] = ZSPLIT ? ldg16_or(q, ok, zeros) : ldg16_or_nt(q, ok, zeros);
       if (DROP) {  // rows at or past drop.rows keep everything: their byte is never applied
-        const bool dropped = ok && row[u] < a.drop.rows;
-        keep[u] = *(const SMLM_GLOBAL uint8_t*)(dropped ? P.drop_bits + (long)row[u] * P.drop_pitch + ((n0 + lcol) >> 3)
+        const bool dropped = ok && row < a.drop.rows;
+        keep[u] = *(const SMLM_GLOBAL uint8_t*)(dropped ? P.drop_bits + (long)row * P.drop_pitch + ((n0 + lcol) >> 3)
                                                         : zero_bytes) | (dropped ? 0u : 0x100u);
       }
     }
@@ -178,7 +180,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
         const int j = j0 + 16 * jb + c;
         const int tile = tile0 + 2 * ks + (g >> 1);
         const bool ok = step < n_steps && tile < t_end && j < rlim;
-        pf[jb][ks] = ldg16_or(PT + (long)j * a.pitch + (long)tile0 * kTileRows + 32 * ks + 8 * g, ok, zeros);
+        pf[jb][ks] = ldg16_or(PT + side_piece(a.r, tile, j, g & 1), ok, zeros);
       }
   };
 
@@ -190,13 +192,12 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   }
 
   // the first step of the first chunk
-  int32_t row_first[8], row_next[8];  // the rows of the wave's first step (every chunk starts with them), of the step ahead
+  const int32_t row_first = load_rows(wave);  // the rows of the wave's first step: every chunk starts with them
   uint32_t keep[DROP ? 8 : 1];  // bit 8 set: the row is not dropped
   u32x4 val[8], pf[NBJ][2];
-  load_rows(wave, row_first);
   load_data(row_first, chunk_first * kWgCols, val, keep);
   load_p(wave, pf);
-  load_rows(wave + kWgWaves, row_next);
+  int32_t row_next = load_rows(wave + kWgWaves);
 
   f32x4(*red)[4][kWaveSize] = reinterpret_cast<f32x4(*)[4][kWaveSize]>(smem);
   // Store staging.  The MFMA leaves 32-byte pieces per output row; the totals go through LDS once
@@ -236,7 +237,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
       uint32_t keep_next[DROP ? 8 : 1];
       if (wrap) load_data(row_first, n0 + kWgCols, val_next, keep_next);
       else load_data(row_next, n0, val_next, keep_next);
-      load_rows(wrap ? wave + kWgWaves : step + 2 * kWgWaves, row_next);
+      row_next = load_rows(wrap ? wave + kWgWaves : step + 2 * kWgWaves);
 
       if (DROP && drop_on) {  // uniform over the workgroup
 #pragma unroll
@@ -363,8 +364,8 @@ constexpr int wgrad_nbj_a(int nbj, int nw, bool drop) { return (drop && nw == 1 
 // 32 in the one-wave kernel under dropout, whose dA workgroups take 32 each).  They are
 // numbered eight apart, so that they run at about the same time on one XCD (workgroup number modulo eight) and the
 // rows of x and dY, which all of them read, come out of its L2 for the second (2048 rows, two projections
-// 4096 -> 4096 at rank 128: 40.2 us with the ranks along the grid's z axis, 37.4 eight apart, 32.9 with loads that
-// are not marked non-temporal as well).
+// 4096 -> 4096 at rank 128, before the operand came in lines: 40.2 us with the ranks along the grid's z axis, 37.4 eight
+// apart, 32.9 with loads that are not marked non-temporal as well).
 template <int DT, int NBJ, int NW, bool DROP, bool ZSPLIT>
 // (two waves a SIMD at every rank: the one-wave kernels hide their latencies through occupancy)
 __global__ __launch_bounds__(NW * kWaveSize) __attribute__((amdgpu_waves_per_eu(2))) void wgrad_kernel(WgradArgs a) {

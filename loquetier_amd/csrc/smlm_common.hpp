@@ -137,6 +137,14 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* lds_addr) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_vec*)lds_addr));
 }
 
+// s*dV and s*v as the weight gradients read them, by tile slot with the token index innermost: [tile][rank / 8][half of
+// the tile][rank % 8][8 slots].  The first element of rank j's eight slots: a piece of 16 bytes, eight ranks' pieces a
+// line.  (With a row of slots per rank sixteen neighbouring lanes, which hold the operand of sixteen ranks, read sixteen
+// lines, and such a load occupies a CU's address unit for 65 cycles instead of 18.)
+__device__ __forceinline__ long side_piece(int r, int tile, int j, int half) {
+  return (long)tile * (r * kTileRows) + (j >> 3) * (8 * kTileRows) + half * 64 + (j & 7) * 8;
+}
+
 // Reads of plan tables and pointer tables at a wave-uniform index.  These are
 // written by an earlier kernel and never by the kernel that reads them, so they
 // may go through the scalar (constant) path: the loads then cost no vector

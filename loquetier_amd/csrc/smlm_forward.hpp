@@ -847,7 +847,7 @@ struct ReduceProj {
   const float* partial;  // [ksplit, T, d_out]
   uint16_t* out;         // [T, d_out]
   int ksplit;            // 1: nothing to fold for this projection
-  // SIDE folds (the backward's dV): side_scale * out by tile slot, transposed ([d_out][side_pitch]), and the
+  // SIDE folds (the backward's dV): side_scale * out by tile slot, transposed (side_piece), and the
   // same treatment of v2 (a second [T, d_out] matrix) -- what the weight-gradient kernel reads
   uint16_t* pt_a;
   uint16_t* pt_b;
@@ -862,7 +862,6 @@ struct ReduceArgs {
   int T, d_out, nproj;
   int units_max;  // > 0: direct mode, one (projection, tile) per workgroup over this tile bound
   const float* side_scale;  // SIDE folds: per segment, or null for 1
-  long side_pitch;          // SIDE folds: slots per row of pt_a / pt_b
   ZeroSpans zero;           // SIDE folds, direct mode: memory the launch's last workgroups clear (the rows of dX
                             //   past the backward's own)
 };
@@ -982,11 +981,12 @@ __global__ __launch_bounds__(kSideThreads) void side_fold_kernel(ReduceArgs a) {
       tr[1][(4 * q + 2 * e + 1) * kTPitch + slot] = (uint16_t)Num<DT>::bits(ss * Num<DT>::hi(second[e]));
     }
     __syncthreads();
-    const int which = threadIdx.x >> 9, m = (threadIdx.x >> 3) & 63, piece = threadIdx.x & 7;  // a piece: half a tile
+    // piece: half a tile; eight neighbouring threads write a line
+    const int which = threadIdx.x >> 9, m = (threadIdx.x >> 3 & 56) | (threadIdx.x & 7), piece = threadIdx.x >> 3 & 7;
     uint16_t* pt = which ? P.pt_b : P.pt_a;
     if (pt && n0 + m < a.d_out && tile_ok(piece >> 1)) {
       const uint32_t* src = reinterpret_cast<const uint32_t*>(&tr[which][m * kTPitch + 8 * piece]);
-      stg16(pt + (long)(n0 + m) * a.side_pitch + (long)tile0 * kTileRows + 8 * piece, u32x4{src[0], src[1], src[2], src[3]});
+      stg16(pt + side_piece(a.d_out, tile0 + (piece >> 1), n0 + m, piece & 1), u32x4{src[0], src[1], src[2], src[3]});
     }
   }
 }
@@ -1000,7 +1000,7 @@ struct ExpandProj {
   const float* vpart;         // VFOLD wave kernels: v arrives as vsplit (1..4) fp32 k-split partials
   int vsplit;                 //   [vsplit, T, d_in], summed here in split order and rounded
   int d_in, d_out, ldw;
-  uint16_t* pt_a;             // block kernels, optional [d_in, nt_max*16]: scale*v by tile slot, transposed
+  uint16_t* pt_a;             // block kernels, optional: scale*v by tile slot, transposed (side_piece)
   uint16_t* pt_b;             // optional: same treatment of v2 (a second [T, d_in] matrix)
   const uint16_t* v2;
   const uint8_t* drop_bits;   // DROP kernels: keep bits of this projection's mask, [rows, drop_pitch]
@@ -1021,22 +1021,22 @@ struct ExpandArgs {
                              //   (probabilities and row count; the keep bits are each projection's own)
 };
 
-// by-products one wave per tile writes: scale*v / scale*v2 by tile slot, transposed ([k][slot]),
+// by-products one wave per tile writes: scale*v / scale*v2 by tile slot, transposed (side_piece),
 // which the weight-gradient kernel reads with the token index innermost
 template <int DT>
 __device__ __forceinline__ void write_side(const ExpandArgs& a, const ExpandProj& P, int slot, int row,
                                            int kk, u32x4 vf, float scale) {
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  const long pitch = (long)a.nt_max * kTileRows;
+  const long at = side_piece(P.d_in, slot / kTileRows, kk, slot >> 3 & 1) + (slot & 7);
   u32x4 v2f = zero;
   if (P.pt_b && row >= 0) v2f = ldg16(P.v2 + (long)row * P.d_in + kk);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    P.pt_a[(kk + 2 * e) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(vf[e]));
-    P.pt_a[(kk + 2 * e + 1) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(vf[e]));
+    P.pt_a[at + 16 * e] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(vf[e]));
+    P.pt_a[at + 16 * e + 8] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(vf[e]));
     if (P.pt_b) {
-      P.pt_b[(kk + 2 * e) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(v2f[e]));
-      P.pt_b[(kk + 2 * e + 1) * pitch + slot] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(v2f[e]));
+      P.pt_b[at + 16 * e] = (uint16_t)Num<DT>::bits(scale * Num<DT>::lo(v2f[e]));
+      P.pt_b[at + 16 * e + 8] = (uint16_t)Num<DT>::bits(scale * Num<DT>::hi(v2f[e]));
     }
   }
 }
