@@ -744,6 +744,33 @@ BwdLayout bwd_layout(int n_proj, int n_rows, int P, int NA, const int* h_in, con
   return L;
 }
 
+template <int DT>
+int launch_expand_found_dt(int nq, int KS, dim3 grid, hipStream_t st, const FoundExpandArgs& a) {
+  const dim3 block(kFwdThreads);
+  if (nq == 4) {
+    if (KS == 1) return launch(expand_found_kernel<DT, 4, 1>, grid, block, st, a);
+    if (KS == 2) return launch(expand_found_kernel<DT, 4, 2>, grid, block, st, a);
+    return launch(expand_found_kernel<DT, 4, 0>, grid, block, st, a);
+  }
+  if (KS == 1) return launch(expand_found_kernel<DT, 2, 1>, grid, block, st, a);
+  if (KS == 2) return launch(expand_found_kernel<DT, 2, 2>, grid, block, st, a);
+  return launch(expand_found_kernel<DT, 2, 0>, grid, block, st, a);
+}
+// An expand of smlm_gemm on single tiles: about five workgroups a CU, each with its share of a tile's column chunks;
+// lists in multiples of eight, so that a chunk's weights stay on an XCD (workgroups go to the XCDs in turn).
+int launch_expand_found(int dtype, int T, int S, hipStream_t st, FoundExpandArgs& a) {
+  const int nq = expand_nq(T, a.p.d_out);
+  const int KS = a.p.d_in <= 32 ? 1 : (a.p.d_in <= 64 ? 2 : 0);
+  a.chunks = ceil_div(a.p.d_out, kFwdWaves * 32 * nq);
+  const int most = tile_units_max(T, S, S, 1), usual = T / kTileRows + 1 + 32;  // (as launch_shrink_self_planned)
+  a.units = most < usual ? most : usual;
+  int lists = ceil_div(a.chunks, ceil_div(a.units * a.chunks, 1280));
+  if (lists > kWgXcd / 2) lists = round_up(lists, kWgXcd);
+  const dim3 grid((unsigned)lists, (unsigned)a.units);
+  return dtype == SMLM_DTYPE_F16 ? launch_expand_found_dt<SMLM_DTYPE_F16>(nq, KS, grid, st, a)
+                                 : launch_expand_found_dt<SMLM_DTYPE_BF16>(nq, KS, grid, st, a);
+}
+
 // Scratch of smlm_gemm_static: part of the code object, so every device the library is loaded
 // on has its own copy at its own address.  In host code the name is only a handle for
 // hipGetSymbolAddress; kernels and copies get the looked-up device address.
@@ -943,6 +970,19 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
     float* partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + plan_bytes);
     return run_shrink(dtype, pv, T, S, S, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
                       seg_scale, mt, st, true, false, nullptr, nullptr, 0, &build, false, nullptr, nullptr, true);
+  }
+  // An expanding product on single tiles finds them itself (expand_found_kernel): up to a segment a thread.  Larger
+  // batches, on tile blocks, keep the plan's launch: it is the smaller part of theirs.
+  if (d_in < d_out && !w_row_major && S <= kFoundSegs && tiles_per_wave(T, d_in, kNoShrink) == 1) {
+    FoundExpandArgs a{};
+    a.plan = PlanSortArgs{pv, seg_indptr, w_ptrs, SMLM_KEY_PTR2, S, next_pow2(S), w_ptrs};
+    a.seg_scale = seg_scale;
+    a.beta = beta;
+    a.p.y = reinterpret_cast<uint16_t*>(y);
+    a.p.v = reinterpret_cast<const uint16_t*>(x);
+    a.p.w_ptrs = w_ptrs;
+    a.p.d_in = d_in; a.p.d_out = d_out; a.p.ldw = w_ld;
+    return launch_expand_found(dtype, T, S, st, a);
   }
   rc = plan_build_impl(pv, seg_indptr, w_ptrs, SMLM_KEY_PTR, S, st);
   if (rc) return rc;

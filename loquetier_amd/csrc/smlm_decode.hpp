@@ -58,12 +58,12 @@ struct FindPairs {
 };
 template <>
 struct FindPairs<0> {};
-template <int THREADS, bool PAIRS>
+template <int THREADS, bool PAIRS, int N = kSelfPlanWeights>
 struct FindLds {
-  int32_t hist[kSelfPlanWeights];   // rows per adapter
-  uint64_t wtab[kSelfPlanWeights];  // this projection's weight table
-  int32_t rtab[kSelfPlanWeights];   // true ranks, when given
-  FindPairs<PAIRS ? kSelfPlanWeights : 0> pr;
+  int32_t hist[N];   // rows per adapter
+  uint64_t wtab[N];  // this projection's weight table
+  int32_t rtab[N];   // true ranks, when given
+  FindPairs<PAIRS ? N : 0> pr;
   uint32_t tot_a[THREADS / kWaveSize], tot_b[THREADS / kWaveSize];  // wave totals of the two scans
   int32_t rows[kBlkTiles * kTileRows], rseg[kBlkTiles * kTileRows];
   int32_t sel[3];                   // adapter of the unit (-1: no such unit), unit's index within the adapter, units in all
@@ -97,11 +97,11 @@ __device__ __forceinline__ uint32_t block_scan_excl_1(uint32_t v, uint32_t* tot,
 // Which adapter owns unit `unit` (a unit = UT consecutive tiles of one adapter; adapters in
 // ascending order, as the plan's groups are).  Everything global is requested at once; the
 // first barrier (LDS cleared) passes while those loads are on their way.  THREADS >= S.
-template <int THREADS, int UT, bool PAIRS>
-__device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS>& F, const PlanSortArgs& pa,
+template <int THREADS, int UT, bool PAIRS, int N>
+__device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS, N>& F, const PlanSortArgs& pa,
                                                   const void* const* w_ptrs, const int32_t* w_rank, int NA,
                                                   int unit, FindSeg* seg) {
-  constexpr int kEnt = kSelfPlanWeights / THREADS;  // table entries a thread holds: kEnt * tid ...
+  constexpr int kEnt = N / THREADS;  // table entries a thread holds: kEnt * tid ...
   const int tid = threadIdx.x, lane = tid & 63;
   int key = -1, s0 = 0, len = 0;
   uint64_t pair_a = 0, pair_b = 0;
@@ -134,7 +134,7 @@ __device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS>& F, co
     // groups by pairs of addresses: the id of a segment is the first segment with its pair, as the plan
     // builders number them (first_equal_pair; its barriers also cover the clearing above)
     if (tid < pa.S) F.pr.ka[tid] = pair_a, F.pr.kb[tid] = pair_b;
-    first_equal_pair<kSelfPlanWeights>(F.pr.ka, F.pr.kb, F.pr.first, F.pr.slot[0], F.pr.slot[1], pa.S);
+    first_equal_pair<N>(F.pr.ka, F.pr.kb, F.pr.first, F.pr.slot[0], F.pr.slot[1], pa.S);
     if (tid < pa.S) key = F.pr.first[tid];
   } else {
     __syncthreads();
@@ -197,8 +197,8 @@ __device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS>& F, co
 
 // The rows of the unit, into F.rows / F.rseg (slot 16 w + c = row c of the unit's tile w; -1 =
 // empty): the adapter's rows in segment order, of which the unit holds 16 UT sub ... + 16 UT - 1.
-template <int THREADS, int UT, bool PAIRS>
-__device__ __forceinline__ void find_rows(FindLds<THREADS, PAIRS>& F, const FindSeg& seg, const FoundUnit& u) {
+template <int THREADS, int UT, bool PAIRS, int N>
+__device__ __forceinline__ void find_rows(FindLds<THREADS, PAIRS, N>& F, const FindSeg& seg, const FoundUnit& u) {
   const int q_lo = u.sub * UT * kTileRows;
   const uint32_t mine = (seg.counted && seg.key == u.wid) ? (uint32_t)seg.len : 0u;
   uint32_t hi_u;
@@ -364,6 +364,113 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   }
   if (!PAIRS || tile + a.units >= un.total) return;  // uniform over the workgroup: no tile is left for it
   __syncthreads();                         // the sums are read: the finder takes its LDS back
+  }
+}
+
+// ---- expand by itself (smlm_gemm), single tiles: expand_wave_kernel without a plan --------------------
+// One weight address per segment, as many table entries as segments.  A product that expands is the last of its call:
+// nobody reads its plan, which took a launch of its own (5.4 us of a single workgroup and the gap behind it).  Every
+// workgroup finds its tile, asks for its first weights while it finds the rows, and walks the column chunks
+// blockIdx.x, blockIdx.x + gridDim.x ... of it with the next chunk's weights on their way.  A tile's rows get the bits
+// they get from expand_wave_kernel: MFMA columns do not mix.
+// Bound by the finding (about 3 us before a workgroup's first row is known) and the stores behind it: 1856 rows in 24
+// segments, 16 -> 11008, us: plan 5.4, gap 1.5 and expand 11.9 with a plan; 15.3 so, with eight lists of three chunks a
+// tile, 20.7 with sixteen, 22.3 with a workgroup a chunk.  Both products of that batch 29.3 -> 26.6; 40 segments of 8
+// rows, 128 -> 4096, 29.8 -> 23.8, and what is smaller is host time (26.7 -> 23.7).
+constexpr int kFoundSegs = kFwdThreads;  // most segments: one a thread
+
+struct FoundExpandArgs {
+  ExpandProj p;        // y, v, w_ptrs (one per segment), d_in, d_out, ldw
+  PlanSortArgs plan;   // s, key = key2 = w_ptrs, S
+  const float* seg_scale;
+  float beta;
+  int units;           // rows of workgroups (tiles beyond them: further rounds)
+  int chunks;          // column chunks of kFwdWaves * 32 * NQ
+};
+
+template <int DT, int NQ, int KS>
+__global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandArgs a) {
+  __shared__ FindLds<kFwdThreads, true, kFoundSegs> F;
+  __shared__ __attribute__((aligned(16))) float olds[kFwdWaves][kTileRows * kOPitch];
+  if ((int)blockIdx.x >= a.chunks) return;  // (lists rounded up)
+  const ExpandProj& P = a.p;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int c = lane & 15, g = lane >> 4;
+  const int mrow = 8 * (c >> 2) + (c & 3);  // column offset of MFMA row c inside a (q,p) block
+  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
+  constexpr int KSU = KS > 0 ? KS : 1;
+
+  for (int tile = blockIdx.y;; tile += a.units) {
+    FindSeg seg;
+    const FoundUnit un = find_adapter<kFwdThreads, 1, true>(F, a.plan, P.w_ptrs, nullptr, a.plan.S, tile, &seg);
+    if (un.wid < 0) return;  // past the last tile; uniform over the workgroup
+    const uint16_t* W = reinterpret_cast<const uint16_t*>(F.wtab[un.wid]);
+    u32x4 wf[KSU][NQ][2];
+    auto load_w = [&](int yy, int ks, u32x4 (&w)[NQ][2]) {
+      const int ncol0 = (yy * kFwdWaves + wave) * 32 * NQ, kk = 32 * ks + 8 * g;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const int n = ncol0 + 32 * q + 4 * p + mrow;
+          w[q][p] = ldg16_or(W + (long)n * P.ldw + kk, kk < P.d_in && n < P.d_out, zeros);
+        }
+    };
+    if (KS > 0) {
+#pragma unroll
+      for (int ks = 0; ks < KSU; ++ks) load_w(blockIdx.x, ks, wf[ks]);
+    }
+
+    find_rows<kFwdThreads, 1, true>(F, seg, un);
+    const int row = F.rows[c];
+    LineLane L;
+    L.orow = lane >> 3;
+    L.ocol = (lane & 7) * 8;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      L.srow[j] = F.rows[L.orow + 8 * j];
+      L.scale[j] = (a.seg_scale && L.srow[j] >= 0) ? a.seg_scale[F.rseg[L.orow + 8 * j]] : 1.0f;
+    }
+    auto load_v = [&](int ks) {
+      const int kk = 32 * ks + 8 * g;
+      return ldg16_or(P.v + (long)row * P.d_in + kk, kk < P.d_in && row >= 0, zeros);
+    };
+    u32x4 vf[KSU];
+    if (KS > 0) {
+#pragma unroll
+      for (int ks = 0; ks < KSU; ++ks) vf[ks] = load_v(ks);
+    }
+
+#pragma unroll 1
+    for (int yy = blockIdx.x; yy < a.chunks; yy += gridDim.x) {
+      const int ncol0 = (yy * kFwdWaves + wave) * 32 * NQ;
+      if (ncol0 >= P.d_out) break;  // (no barrier in this loop)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        L.yrow[j] = P.y + (long)(L.srow[j] < 0 ? 0 : L.srow[j]) * P.d_out + ncol0 + L.ocol;
+      u32x4 yold[NQ / 2][2];
+      load_y_lines<NQ>(yold, L, ncol0, P.d_out, a.beta != 0.0f, zeros);
+      f32x4 acc[NQ][2];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) acc[q][0] = acc[q][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int nks = KS > 0 ? KS : (P.d_in + 31) / 32;
+#pragma unroll KSU
+      for (int ks = 0; ks < nks; ++ks) {
+        if (KS == 0) load_w(yy, ks, wf[0]), vf[0] = load_v(ks);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+            acc[q][p] = Num<DT>::mfma(wf[KS > 0 ? ks : 0][q][p], vf[KS > 0 ? ks : 0], acc[q][p]);
+      }
+      if (KS > 0 && yy + (int)gridDim.x < a.chunks) {
+#pragma unroll
+        for (int ks = 0; ks < KSU; ++ks) load_w(yy + gridDim.x, ks, wf[ks]);
+      }
+      store_y_lines<DT, NQ>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
+    }
+    if (tile + a.units >= un.total) return;  // uniform over the workgroup: no tile is left for it
+    __syncthreads();                         // every wave has read its rows: the finder takes its LDS back
   }
 }
 
