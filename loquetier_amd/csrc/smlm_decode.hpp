@@ -228,31 +228,25 @@ __device__ __forceinline__ void find_rows(FindLds<THREADS, PAIRS, N>& F, const F
 // THREADS = 1024 (more than 512 segments; the finder and the plan builders hold a segment per
 // thread): two such groups of eight waves, which take two neighbouring k slices of the tile and sum
 // each for itself -- the same sums as two workgroups of the 512-thread kind.
-// The sums' staging area lies behind the finder's LDS where both fit under the plan builders'
-// and over it otherwise.
-template <int NB, int THREADS, bool PAIRS>
-struct SelfPlanWork {
-  static constexpr int kWaves = THREADS / kWaveSize;
-  static constexpr bool kOverlay = sizeof(FindLds<THREADS, PAIRS>) + sizeof(f32x4) * kWaves * NB * kWaveSize >
-                                   sizeof(PlanSmallLdsT<THREADS>);
-  FindLds<THREADS, PAIRS> find;
-  f32x4 red[kOverlay ? 1 : kWaves][NB][kWaveSize];
-};
-template <int NB, int THREADS, bool PAIRS>
+// The finder's LDS turns into the product's once every wave holds its rows.
+template <int NB, int U, int THREADS, bool PAIRS>
 union SelfPlanLds {
-  PlanSmallLdsT<THREADS> plan;                      // the plan-building workgroups
-  SelfPlanWork<NB, THREADS, PAIRS> work;            // the others: finding their tile, then the cross-wave sums
-  f32x4 red[THREADS / kWaveSize][NB][kWaveSize];    // ... which reuse the finder's memory when the two do not fit side by side
+  PlanSmallLdsT<THREADS> plan;   // the plan-building workgroups
+  FindLds<THREADS, PAIRS> find;  // the others: finding their tile ...
+  union {
+    char turn[LineTurn<U>::kBytes];  // ... then, a part for each wave, x and the weights on their way to the MFMA
+    f32x4 sum[NB][kWaveSize];        // and its sums
+  } wave[THREADS / kWaveSize];
 };
 
 // DROP (plans keyed by ids): dropout of the training rows of x, as shrink_kernel applies it.
 template <int DT, int NB, int U, int THREADS, bool PAIRS = false, bool DROP = false>
 __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanArgs a) {
   static_assert(THREADS == kSelfPlanThreads || THREADS == 2 * kSelfPlanThreads, "one or two groups of eight waves");
-  __shared__ SelfPlanLds<NB, THREADS, PAIRS> sm;
+  typedef LineTurn<U> Turn;
+  __shared__ __attribute__((aligned(16))) SelfPlanLds<NB, U, THREADS, PAIRS> sm;
   constexpr int NW = kSelfPlanThreads / kWaveSize;  // waves that sum one k slice
   constexpr int HALVES = THREADS / kSelfPlanThreads;
-  constexpr bool kOverlay = SelfPlanWork<NB, THREADS, PAIRS>::kOverlay;
   const int tid = threadIdx.x;
   if ((int)blockIdx.y == a.units) {  // the extra row of the grid: up to kSelfPlanBuilders workgroups build the plan
     const int part = (int)(blockIdx.z * gridDim.x + blockIdx.x), all = (int)(gridDim.x * gridDim.z);
@@ -264,7 +258,7 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   const int pj = blockIdx.z;
   if ((int)blockIdx.x * HALVES >= a.sh.items.row_start[pj + 1] - a.sh.items.row_start[pj]) return;
   const ShrinkProj P = a.sh.p[pj];
-  FindLds<THREADS, PAIRS>& F = sm.work.find;
+  FindLds<THREADS, PAIRS>& F = sm.find;
   const int wave_all = tid >> 6, lane = tid & 63;
   const int wave = wave_all % NW;           // wave within its group of eight
   const int yy = (int)blockIdx.x * HALVES + wave_all / NW;
@@ -293,22 +287,24 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   }
   // the adapter is known: its weights are requested while the rows are still being found
   auto load_w = [&](int k, u32x4 (&wf)[NB][U]) {
+    const int kk = k + 8 * Turn::piece(lane);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int kk = k + 32 * u + 8 * g;
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int n = n0 + 16 * nb + c;
-        wf[nb][u] = ldg16_or(W + (long)n * P.ldw + kk, kk < kend && n < nlim, zeros);
+      for (int i = 0; i < U; ++i) {
+        const int n = n0 + 16 * nb + Turn::row(lane, i);
+        wf[nb][i] = ldg16_or(W + (long)n * P.ldw + kk, kk < kend && n < nlim, zeros);
       }
-    }
   };
   u32x4 wf[NB][U];
   load_w(kbeg, wf);
 
   find_rows<THREADS, 1, PAIRS>(F, seg, un);
   const int row = F.rows[c], rseg = F.rseg[c];
-  if (kOverlay) __syncthreads();  // every wave holds its tile: the finder's LDS turns into the sum's staging area
+  int lrow[U];  // the rows this lane requests
+#pragma unroll
+  for (int i = 0; i < U; ++i) lrow[i] = F.rows[Turn::row(lane, i)];
+  __syncthreads();  // every wave holds its rows: the finder's LDS turns into the product's
   DropRow dr{};
   DropArgs dp{};
   if (DROP) dp = drop_proj(a.sh.drop, pj), dr = drop_row_of(dp, row, rseg);
@@ -320,12 +316,14 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
 #pragma unroll 1
   for (int k = kbeg; k < kend; k += 32 * U) {
     u32x4 xf[U];
+    const int kl = k + 8 * Turn::piece(lane);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int kk = k + 32 * u + 8 * g;
-      xf[u] = ldg16_or(P.x + (long)row * P.d_in + kk, kk < kend && row >= 0, zeros);
-    }
+    for (int i = 0; i < U; ++i)
+      xf[i] = ldg16_or(P.x + (long)lrow[i] * P.d_in + kl, kl < kend && lrow[i] >= 0, zeros);
     if (k != kbeg) load_w(k, wf);  // uniform over the wave (k is usually one batch)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) Turn::turn(sm.wave[wave_all].turn, lane, wf[nb]);
+    Turn::turn(sm.wave[wave_all].turn, lane, xf);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kk = k + 32 * u + 8 * g;
@@ -335,11 +333,10 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
     }
   }
 
-  // decided at compile time; every group of eight waves has its own part of the area
-  f32x4 (*red)[NB][kWaveSize] = (kOverlay ? sm.red : sm.work.red) + (wave_all - wave);
+  auto* const sums = sm.wave + (wave_all - wave);  // of the group of eight waves
   // cross-wave sum in wave order; the group's first wave writes the tile
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) red[wave][nb][lane] = acc[nb];
+  for (int nb = 0; nb < NB; ++nb) sums[wave].sum[nb][lane] = acc[nb];
   __syncthreads();
   if (wave == 0 && row >= 0) {
     const bool as_partial = P.ksplit > 1 || P.to_partial;
@@ -349,7 +346,7 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
     for (int nb = 0; nb < NB; ++nb) {
       f32x4 part[NW];
 #pragma unroll
-      for (int w = 0; w < NW; ++w) part[w] = red[w][nb][lane];
+      for (int w = 0; w < NW; ++w) part[w] = sums[w].sum[nb][lane];
       __builtin_amdgcn_sched_barrier(0);
       f32x4 sum = part[0];
 #pragma unroll

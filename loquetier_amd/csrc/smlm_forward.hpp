@@ -210,6 +210,36 @@ struct ShrinkArgs {
   DropArgs drop;              // DROP kernels: dropout of the training rows of x
 };
 
+// Sixteen rows of 32 * U of k on their way from memory to the MFMA.  They are requested along the rows, load i of a lane
+// piece `piece` of row `row(i)`, and change layout in an LDS area of the wave's own: afterwards register u of lane (c, g)
+// holds row c, k 32 u + 8 g .. + 7.  Requested in that layout, sixteen rows to sixteen neighbouring lanes, a load occupies
+// the CU's address unit for 65 cycles instead of 18.
+template <int U>
+struct LineTurn {
+  static constexpr int kRow = 4 * U;  // 16-byte pieces of a row
+  static constexpr int kBytes = kTileRows * kRow * 16;
+  static_assert(U == 2 || U == 4, "rows of one or two lines");
+  static __device__ __forceinline__ int row(int lane, int i) { return (lane + kWaveSize * i) / kRow; }
+  static __device__ __forceinline__ int piece(int lane) { return lane % kRow; }
+  // (pieces change places within their row so that reads and writes touch each bank once)
+  static __device__ __forceinline__ int at(int r, int p) { return r * kRow + (p ^ (U == 4 ? r : (r >> 1) & 7)); }
+  static __device__ __forceinline__ void turn(char* lds, int lane, u32x4 (&v)[U]) {
+    u32x4* a = reinterpret_cast<u32x4*>(lds);
+#pragma unroll
+    for (int i = 0; i < U; ++i) a[at(row(lane, i), piece(lane))] = v[i];
+    order();
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = a[at(lane & 15, 4 * u + (lane >> 4))];
+    order();
+  }
+  // a wave's own LDS accesses are served in order; the compiler must keep them in order too
+  static __device__ __forceinline__ void order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+};
+
 // Shrink for single tiles (batches of few rows).  Work item -> (projection, k
 // slice, 64-column block, tile).  The NW waves of a workgroup take consecutive k
 // ranges; their accumulators are summed through LDS in wave order and written
@@ -217,7 +247,11 @@ struct ShrinkArgs {
 // or as the final 16-bit value.  NW = 8 is for decode batches: few tiles, long k.
 template <int DT, int NB, int U, int NW, bool DIRECT, bool DROP = false>
 __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
-  __shared__ f32x4 red[NW][NB][kWaveSize];
+  typedef LineTurn<U> Turn;
+  // a wave's part: x and the weights on their way to the MFMA, then its sums
+  constexpr int kSums = NB * kWaveSize;
+  __shared__ __attribute__((aligned(16))) char area[NW][Turn::kBytes > kSums * 16 ? Turn::kBytes : kSums * 16];
+  auto red = [&](int w, int nb) -> f32x4& { return reinterpret_cast<f32x4*>(area[w])[nb * kWaveSize + (threadIdx.x & 63)]; };
   const int units = DIRECT ? 0 : tile_units<1>(a.plan, 0);
   const WorkRange wr = item_range<DIRECT>(a.items, units);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -234,6 +268,9 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
     const int n0 = zb * 64;
     const int slot = tile * kTileRows + c;
     const int row = a.plan.tile_row[slot];
+    int lrow[U];  // the rows this lane requests
+#pragma unroll
+    for (int i = 0; i < U; ++i) lrow[i] = a.plan.tile_row[tile * kTileRows + Turn::row(lane, i)];
     const uint16_t* W = uload_ptr(P.w_ptrs, wid);
     const int nlim = rank_limit(a.plan, wid, P.d_out);  // weight rows at or past it are zero padding
     DropRow dr{};
@@ -249,19 +286,23 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
     for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     auto load_batch = [&](int k, u32x4 (&xf)[U], u32x4 (&wf)[NB][U]) {
+      const int kk = k + 8 * Turn::piece(lane);
+      const bool kin = kk < kend;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int kk = k + 32 * u + 8 * g;
-        const bool kin = kk < kend;
-        xf[u] = ldg16_or(P.x + (long)row * P.d_in + kk, kin && row >= 0, zeros);
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const int n = n0 + 16 * nb + c;
-          wf[nb][u] = load_w8(W, n, kk, P.ldw, kin && n < nlim, zeros);
+        for (int i = 0; i < U; ++i) {
+          const int n = n0 + 16 * nb + Turn::row(lane, i);
+          wf[nb][i] = load_w8(W, n, kk, P.ldw, kin && n < nlim, zeros);
         }
-      }
+#pragma unroll
+      for (int i = 0; i < U; ++i)
+        xf[i] = ldg16_or(P.x + (long)lrow[i] * P.d_in + kk, kin && lrow[i] >= 0, zeros);
     };
-    auto multiply = [&](int k, const u32x4 (&xf)[U], const u32x4 (&wf)[NB][U]) {
+    auto multiply = [&](int k, u32x4 (&xf)[U], u32x4 (&wf)[NB][U]) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) Turn::turn(area[wave], lane, wf[nb]);
+      Turn::turn(area[wave], lane, xf);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int kk = k + 32 * u + 8 * g;
@@ -287,7 +328,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
 
     // cross-wave sum in wave order; wave 0 writes the tile
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) red[wave][nb][lane] = acc[nb];
+    for (int nb = 0; nb < NB; ++nb) red(wave, nb) = acc[nb];
     __syncthreads();
     if (wave == 0 && row >= 0) {
       float scale = 1.0f;
@@ -300,7 +341,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
         // in its k loop)
         f32x4 part[NW];
 #pragma unroll
-        for (int w = 0; w < NW; ++w) part[w] = red[w][nb][lane];
+        for (int w = 0; w < NW; ++w) part[w] = red(w, nb);
         __builtin_amdgcn_sched_barrier(0);
         f32x4 sum = part[0];
 #pragma unroll
