@@ -247,6 +247,9 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   __shared__ __attribute__((aligned(16))) SelfPlanLds<NB, U, THREADS, PAIRS> sm;
   constexpr int NW = kSelfPlanThreads / kWaveSize;  // waves that sum one k slice
   constexpr int HALVES = THREADS / kSelfPlanThreads;
+  // x and the weights along the rows (LineTurn), but for sixteen waves a workgroup, two of which fill a CU: q/k/v/o of
+  // 900 decoded rows at rank 16 32.4 us in the MFMA's layout, 35.2 along the rows
+  constexpr bool kLines = HALVES == 1;
   const int tid = threadIdx.x;
   if ((int)blockIdx.y == a.units) {  // the extra row of the grid: up to kSelfPlanBuilders workgroups build the plan
     const int part = (int)(blockIdx.z * gridDim.x + blockIdx.x), all = (int)(gridDim.x * gridDim.z);
@@ -286,13 +289,14 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
     nlim = r8 < nlim ? r8 : nlim;
   }
   // the adapter is known: its weights are requested while the rows are still being found
+  auto load_row = [&](int i) { return kLines ? Turn::row(lane, i) : c; };  // what load i of a lane brings
+  auto load_k = [&](int i) { return kLines ? 8 * Turn::piece(lane) : 32 * i + 8 * g; };
   auto load_w = [&](int k, u32x4 (&wf)[NB][U]) {
-    const int kk = k + 8 * Turn::piece(lane);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < U; ++i) {
-        const int n = n0 + 16 * nb + Turn::row(lane, i);
+        const int kk = k + load_k(i), n = n0 + 16 * nb + load_row(i);
         wf[nb][i] = ldg16_or(W + (long)n * P.ldw + kk, kk < kend && n < nlim, zeros);
       }
   };
@@ -303,7 +307,7 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   const int row = F.rows[c], rseg = F.rseg[c];
   int lrow[U];  // the rows this lane requests
 #pragma unroll
-  for (int i = 0; i < U; ++i) lrow[i] = F.rows[Turn::row(lane, i)];
+  for (int i = 0; i < U; ++i) lrow[i] = F.rows[load_row(i)];
   __syncthreads();  // every wave holds its rows: the finder's LDS turns into the product's
   DropRow dr{};
   DropArgs dp{};
@@ -316,14 +320,17 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
 #pragma unroll 1
   for (int k = kbeg; k < kend; k += 32 * U) {
     u32x4 xf[U];
-    const int kl = k + 8 * Turn::piece(lane);
 #pragma unroll
-    for (int i = 0; i < U; ++i)
-      xf[i] = ldg16_or(P.x + (long)lrow[i] * P.d_in + kl, kl < kend && lrow[i] >= 0, zeros);
+    for (int i = 0; i < U; ++i) {
+      const int kk = k + load_k(i);
+      xf[i] = ldg16_or(P.x + (long)lrow[i] * P.d_in + kk, kk < kend && lrow[i] >= 0, zeros);
+    }
     if (k != kbeg) load_w(k, wf);  // uniform over the wave (k is usually one batch)
+    if (kLines) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) Turn::turn(sm.wave[wave_all].turn, lane, wf[nb]);
-    Turn::turn(sm.wave[wave_all].turn, lane, xf);
+      for (int nb = 0; nb < NB; ++nb) Turn::turn(sm.wave[wave_all].turn, lane, wf[nb]);
+      Turn::turn(sm.wave[wave_all].turn, lane, xf);
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kk = k + 32 * u + 8 * g;
