@@ -115,10 +115,16 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
 // 4096: one projection at rank 16, 2048 rows 13.0 / 11.6, 3000 rows 13.5 / 12.7; three at rank 32, 1000 rows 16.3 / 14.9,
 // 3000 rows 30 / 26.3; at rank 64 1500 rows 21 / 24.0, 2048 rows 23.5 / 25.8, 3000 rows 36 / 36, 7675 rows 68 / 60.
 // Above rank 64 x would be read once for every 64 columns.
-inline bool block_shrink(int mt, int T, int d_out) { return mt > 1 && (d_out <= 32 || (d_out <= 64 && T >= 3072)); }
+// Below 1024 rows adapters have few rows each, and the block kernel reads 64 rows for however few: 867 rows over 48
+// adapters, three projections at rank 32, forward 15.6 / 19.4, backward (567 rows) 14.0 / 18.0.  Under dropout the
+// generator keeps the vector units busy and the wide kernel's waves, more of them on a CU, share it better: 2436 rows, two
+// projections at rank 16 21.7 / 28.3.
+inline bool block_shrink(int mt, int T, int d_out, bool drop = false) {
+  return mt > 1 && !drop && T >= (d_out <= 32 ? 1024 : 3072) && d_out <= 64;
+}
 // ... of a launch: its weight rows must be within the block kernel's reach too (the slices are the same either way)
 inline bool block_shrink(int mt, const ShrinkArgs& a) {
-  bool near = block_shrink(mt, a.T, a.p[0].d_out);
+  bool near = block_shrink(mt, a.T, a.p[0].d_out, a.drop.seg_p != nullptr);
   for (int i = 0; i < a.items.nproj; ++i) near = near && a.p[i].ldw <= kBlockMaxLd;
   return near;
 }
@@ -156,8 +162,8 @@ int block_pieces(int T, int d_in, int d_out, int most, bool solo) {
 // solo: the product is only ever launched by itself (the backward's dV and v products) and may take the
 // splits that suit a launch of one projection; the forward's projections keep one rule
 // whether they are launched alone or together, so that either way gives the same bits
-// plain: a product of smlm_gemm or smlm_gemm_planned
-ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt, bool plain = false) {
+// plain: a product of smlm_gemm or smlm_gemm_planned; drop: of x under dropout
+ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt, bool plain = false, bool drop = false) {
   ShrinkCfg c;
   c.MT = mt;
   c.NB = d_out <= 16 ? 1 : (d_out <= 32 ? 2 : 4);  // (run_shrink may turn 4 into 8: shrink_wide)
@@ -190,7 +196,7 @@ ShrinkCfg shrink_cfg(int T, int d_in, int d_out, int nw, bool solo, int mt, bool
   if (max_split < 1) max_split = 1;
   if (max_split > kMaxKsplit) max_split = kMaxKsplit;
   const int ks = want < 1 ? 1 : (want > max_split ? max_split : want);
-  if (block_shrink(c.MT, T, d_out)) {
+  if (block_shrink(c.MT, T, d_out, drop)) {
     c.k_per_wave = 64 * block_pieces(T, d_in, d_out, ks, solo);
     c.ksplit = ceil_div(d_in, c.NW * c.k_per_wave);
     return c;
@@ -239,9 +245,11 @@ int fwd_ksplit_bound(int T, int d_in, int d_out, bool plain = false) {
     const int a = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, 1, plain).ksplit;
     const int b = shrink_cfg(T, d_in, d_out, kDecodeWaves, solo != 0, 1, plain).ksplit;
     const int c = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain).ksplit;
+    const int d = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain, !plain).ksplit;
     most = a > most ? a : most;
     most = b > most ? b : most;
     most = c > most ? c : most;
+    most = d > most ? d : most;
   }
   return most;
 }
@@ -281,6 +289,8 @@ int launch_shrink_nb(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
 template <int DT, bool DIRECT, bool WKN, bool DROP = false>
 int launch_shrink_wide(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
   const dim3 block(kFwdThreads);  // U must match run_shrink
+  if (NB == 1) return launch(shrink_wide_kernel<DT, 1, 4, DIRECT, WKN, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_wide_kernel<DT, 2, 4, DIRECT, WKN, DROP>, grid, block, st, a);
   if (NB == 8) return launch(shrink_wide_kernel<DT, 8, 2, DIRECT, WKN, DROP>, grid, block, st, a);
   return launch(shrink_wide_kernel<DT, 4, 4, DIRECT, WKN, DROP>, grid, block, st, a);
 }
@@ -367,12 +377,17 @@ int launch_self_planned_nb(int NB, dim3 grid, hipStream_t st, const SelfPlanArgs
 template <int DT, bool WKN, int THREADS, bool PAIRS, bool DROP = false>
 int launch_self_planned_block_nb(int NB, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
   const dim3 block(THREADS);  // U must match shrink_cfg
-  if (!block_shrink(kBlkTiles, a.sh))
-    return NB == 8 ? launch(shrink_wide_self_planned_kernel<DT, 8, 2, WKN, THREADS, PAIRS, DROP>, grid, block, st, a)
-                   : launch(shrink_wide_self_planned_kernel<DT, 4, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
-  if (NB == 1) return launch(shrink_block_self_planned_kernel<DT, 1, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_block_self_planned_kernel<DT, 2, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
-  return launch(shrink_block_self_planned_kernel<DT, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if constexpr (!DROP) {
+    if (block_shrink(kBlkTiles, a.sh)) {
+      if (NB == 1) return launch(shrink_block_self_planned_kernel<DT, 1, WKN, THREADS, PAIRS>, grid, block, st, a);
+      if (NB == 2) return launch(shrink_block_self_planned_kernel<DT, 2, WKN, THREADS, PAIRS>, grid, block, st, a);
+      return launch(shrink_block_self_planned_kernel<DT, 4, WKN, THREADS, PAIRS>, grid, block, st, a);
+    }
+  }
+  if (NB == 1) return launch(shrink_wide_self_planned_kernel<DT, 1, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_wide_self_planned_kernel<DT, 2, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 8) return launch(shrink_wide_self_planned_kernel<DT, 8, 2, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
+  return launch(shrink_wide_self_planned_kernel<DT, 4, 4, WKN, THREADS, PAIRS, DROP>, grid, block, st, a);
 }
 template <int DT, bool WKN, bool PAIRS, bool DROP = false>
 int launch_self_planned_block(int NB, int S, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
@@ -638,14 +653,15 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
   ShrinkCfg c0{};
   size_t bits_off = 0;
   const int nw = shrink_waves(mt, nproj, d_in, d_out);
+  const bool dropped = drop && drop->seg_p;
   long wgs = 0;  // workgroups of 128 columns
   for (int i = 0; mt > 1 && d_out > 64 && i < nproj; ++i)
     wgs += (long)(ceil_div(T, kTileRows * mt) + (groups > 0 && groups < S ? groups : S) / 2) *
-           shrink_cfg(T, d_in[i], d_out, nw, solo, mt, plain).ksplit *
+           shrink_cfg(T, d_in[i], d_out, nw, solo, mt, plain, dropped).ksplit *
            ceil_div(d_out, 128);
   const bool wide = shrink_wide(mt, d_out, w_kn, wgs);
   for (int i = 0; i < nproj; ++i) {
-    ShrinkCfg c = shrink_cfg(T, d_in[i], d_out, nw, solo, mt, plain);
+    ShrinkCfg c = shrink_cfg(T, d_in[i], d_out, nw, solo, mt, plain, dropped);
     if (wide) c.NB = 8, c.U = 2, c.zblocks = ceil_div(d_out, 128);
     if (i == 0) c0 = c;
     ShrinkProj& P = a.p[i];
@@ -665,7 +681,7 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
     // 59.6 us; 6144 rows, h_in = 4096, in three: 27.2 -> 25.0; launches of several projections and those that
     // build their plan keep their grid)
     int rows = c.ksplit * c.zblocks;
-    if (nproj == 1 && !build && !block_shrink(mt, T, d_out) && rows > 1 && (rows & 1)) rows += 1;
+    if (nproj == 1 && !build && !block_shrink(mt, T, d_out, dropped) && rows > 1 && (rows & 1)) rows += 1;
     a.items.row_start[i + 1] = a.items.row_start[i] + rows;
     ra.p[i] = ReduceProj{partial[i], P.out, c.ksplit, side ? side->pt_a[i] : nullptr, side ? side->pt_b[i] : nullptr,
                          side ? side->v2[i] : nullptr};
@@ -1115,7 +1131,7 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
   {
     char* w = reinterpret_cast<char*>(workspace);
     for (int i = 0; i < n_proj; ++i) {
-      vsplit[i] = shrink_cfg(T, h_in[i], r, nw, false, mt).ksplit;
+      vsplit[i] = shrink_cfg(T, h_in[i], r, nw, false, mt, false, drop.seg_p != nullptr).ksplit;
       expand_folds = expand_folds && vsplit[i] <= kMaxExpandFold;
       partial[i] = reinterpret_cast<float*>(w);
       w += align_up((size_t)fwd_ksplit_bound(T, h_in[i], r) * T * r * 4, 256);
@@ -1133,7 +1149,7 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
   // (both routes pair k slices up in one workgroup beyond 512 / 256 segments)
   const bool self_planned = build_s && (!drop.seg_p || build_kind == SMLM_KEY_I32) &&
                             self_planned_ok(T, S, n_weights, pv.nt_max, mt) &&
-                            (mt > 1 ? (S <= kFwdThreads || block_shrink(mt, T, r) || even_splits)
+                            (mt > 1 ? (S <= kFwdThreads || block_shrink(mt, T, r, drop.seg_p != nullptr) || even_splits)
                                                    : (expand_folds && (S <= kSelfPlanThreads || even_splits)));
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, build_kind, S, st, build_k2))) return rc;
   if (stages & SMLM_STAGE_SHRINK) {
