@@ -295,12 +295,12 @@ int launch_shrink_wide(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
   return launch(shrink_wide_kernel<DT, 4, 4, DIRECT, WKN, DROP>, grid, block, st, a);
 }
 
-template <int DT, bool WKN, bool DROP = false>
+template <int DT, bool WKN>
 int launch_shrink_block(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
   const dim3 block(kFwdThreads);
-  if (NB == 1) return launch(shrink_block_kernel<DT, 1, WKN, DROP>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_block_kernel<DT, 2, WKN, DROP>, grid, block, st, a);
-  return launch(shrink_block_kernel<DT, 4, WKN, DROP>, grid, block, st, a);
+  if (NB == 1) return launch(shrink_block_kernel<DT, 1, WKN>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_block_kernel<DT, 2, WKN>, grid, block, st, a);
+  return launch(shrink_block_kernel<DT, 4, WKN>, grid, block, st, a);
 }
 
 // Lists the chunk rows of a tile block are dealt out into, a workgroup (of four waves) each: what leaves the fewest
@@ -337,7 +337,6 @@ int launch_shrink_dt(int NB, int MT, int NW, dim3 grid, hipStream_t st,
 
 template <int DT>
 int launch_shrink_block_dt(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) {
-  if (a.drop.seg_p) return launch_shrink_block<DT, false, true>(NB, grid, st, a);  // (weights [n][k])
   return a.w_kn ? launch_shrink_block<DT, true>(NB, grid, st, a) : launch_shrink_block<DT, false>(NB, grid, st, a);
 }
 

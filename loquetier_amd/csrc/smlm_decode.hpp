@@ -658,11 +658,11 @@ union SelfPlanBlockLds {
   char area[THREADS / kFwdThreads][BYTES];  // ... then the product's
 };
 
-template <int DT, int NB, bool WKN, int THREADS, bool PAIRS = false, bool DROP = false>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB, DROP))))
+template <int DT, int NB, bool WKN, int THREADS, bool PAIRS = false>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB))))
 void shrink_block_self_planned_kernel(SelfPlanArgs a) {
   static_assert(THREADS == kFwdThreads || THREADS == 2 * kFwdThreads, "one or two groups of four waves");
-  typedef BlockProduct<DT, NB, WKN, DROP> Product;
+  typedef BlockProduct<DT, NB, WKN> Product;
   constexpr int GROUPS = THREADS / kFwdThreads;
   __shared__ __attribute__((aligned(16))) SelfPlanBlockLds<THREADS, PAIRS, Product::kLdsBytes> sm;
   if ((int)blockIdx.y < a.builder_rows) {  // up to kSelfPlanBuilders workgroups build the plan
@@ -709,12 +709,6 @@ void shrink_block_self_planned_kernel(SelfPlanArgs a) {
 
   find_rows<THREADS, kBlkTiles, PAIRS>(sm.find, seg, un);
   pr.set_rows([&](int i) { return sm.find.rows[i]; });  // -1: empty
-  if (DROP) {
-    const DropArgs dp = drop_proj(a.sh.drop, 0);  // (the rows' probabilities are the same for every projection)
-#pragma unroll
-    for (int t = 0; t < kBlkTiles; ++t)
-      pr.dr[DROP ? t : 0] = drop_row_of(dp, pr.frow[DROP ? t : 0], sm.find.rseg[t * kTileRows + c]);
-  }
   if (!pr.exists(list)) pr.rw = -1;
   if (a.sh.seg_scale && pr.rw >= 0) pr.scale = a.sh.seg_scale[sm.find.rseg[wave * kTileRows + c]];
   pr.fill_rows();

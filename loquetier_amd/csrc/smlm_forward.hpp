@@ -525,9 +525,9 @@ __device__ __attribute__((aligned(16))) uint32_t product_zeros[4];  // what load
 constexpr int kBlockMaxLd = 1 << 25;  // longest weight row, in elements: a lane's offset in the weights has 32 bits
 
 // waves a SIMD the registers are held to
-constexpr int block_product_waves(int NB, bool DROP) { return NB >= 4 || (DROP && NB >= 2) ? 2 : 3; }
+constexpr int block_product_waves(int NB) { return NB >= 4 ? 2 : 3; }
 
-template <int DT, int NB, bool WKN, bool DROP>
+template <int DT, int NB, bool WKN>
 struct BlockProduct {
   static constexpr int KB = 64, U = KB / 32;      // k of a wave's piece, its 32-wide steps
   static constexpr int kPitch = 16 * NB + 8;      // WKN: LDS row pitch of the weights in elements
@@ -551,10 +551,8 @@ struct BlockProduct {
   const int tiles;           // tiles of the block
   const int nlists;          // the chunk rows r, r + nlists ... are this group's
   int lrow[kBlkTiles][2];    // the rows this lane loads: 8 i + lane / 8 of tile t (the block's first row: none)
-  int frow[DROP ? kBlkTiles : 1];  // DROP: the rows it multiplies, lane % 16 of tile t (-1: none)
   int rw;                    // its row of tile `wave`, which it stores
   float scale;               //   ... and what that is scaled with when no partial sums are stored
-  DropRow dr[DROP ? kBlkTiles : 1];
   f32x4 acc[kBlkTiles][NB];
   // what is loaded next
   int r, s;
@@ -580,10 +578,6 @@ struct BlockProduct {
 #pragma unroll
       for (int i = 0; i < 2; ++i) lrow[t][i] = row_of(kTileRows * t + 8 * i + (lane >> 3));
     rw = row_of(kTileRows * wave + c);
-    if (DROP) {
-#pragma unroll
-      for (int t = 0; t < kBlkTiles; ++t) frow[DROP ? t : 0] = row_of(kTileRows * t + c);
-    }
   }
 
   __device__ __forceinline__ bool exists(int row_) const { return row_ < a.items.row_start[a.items.nproj]; }
@@ -697,7 +691,7 @@ struct BlockProduct {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  __device__ __forceinline__ void multiply(const Stage& st, char* lds, const DropArgs& dp, const Item& it) {
+  __device__ __forceinline__ void multiply(const Stage& st, char* lds) {
     uint16_t* wl = reinterpret_cast<uint16_t*>(lds);
 #pragma unroll
     for (int j = 0; j < 2 * NB; ++j) {
@@ -731,15 +725,7 @@ struct BlockProduct {
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          xf[e][u] = get(lds + kWBytes + e * kTileBytes, u);
-          if (DROP) {
-            const ShrinkProj& P = a.p[it.pj];
-            const int t = 2 * h + e, kk = st.k0 + 32 * u + 8 * g;
-            xf[e][u] = drop8<DT>(xf[e][u], dp, dr[DROP ? t : 0], frow[DROP ? t : 0], kk >> 3, P.drop_bits, P.d_in >> 3,
-                                 it.zb == 0 && kk < it.kend);
-          }
-        }
+        for (int e = 0; e < 2; ++e) xf[e][u] = get(lds + kWBytes + e * kTileBytes, u);
       lds_order();
 #pragma unroll
       for (int u = 0; u < U; ++u)
@@ -791,20 +777,14 @@ struct BlockProduct {
     char* lds = smem + wave * kStageBytes;
     int mr = r, ms = 0;  // what is multiplied: chunk row, piece
     Item mi = li;
-    DropArgs dp{};
-    if (DROP) dp = drop_proj(a.drop, mi.pj);
     auto next = [&] {
       if (++ms < mi.n) return;
       finish(smem, mi, exists(mr));
       mr += nlists;
       --turns;
       ms = 0;
-      if (exists(mr)) {
-        mi = item(mr);
-        if (DROP) dp = drop_proj(a.drop, mi.pj);
-      } else {
-        mi.n = 1;
-      }
+      if (exists(mr)) mi = item(mr);
+      else mi.n = 1;
     };
     Stage sb;
     load_x(sa);
@@ -812,11 +792,11 @@ struct BlockProduct {
 #pragma unroll 1
     while (true) {
       load(sb);
-      multiply(sa, lds, dp, mi);
+      multiply(sa, lds);
       next();
       if (turns <= 0) break;
       load(sa);
-      multiply(sb, lds, dp, mi);
+      multiply(sb, lds);
       next();
       if (turns <= 0) break;
     }
@@ -825,10 +805,10 @@ struct BlockProduct {
 
 // Shrink for tile blocks (larger batches, and the backward).  Grid (lists, tile blocks): a workgroup takes the chunk rows
 // (projection, k slice, column block of 16 * NB) blockIdx.x, blockIdx.x + gridDim.x ... of its tile block.
-template <int DT, int NB, bool WKN, bool DROP = false>
-__global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB, DROP))))
+template <int DT, int NB, bool WKN>
+__global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB))))
 void shrink_block_kernel(ShrinkArgs a) {
-  typedef BlockProduct<DT, NB, WKN, DROP> Product;
+  typedef BlockProduct<DT, NB, WKN> Product;
   __shared__ __attribute__((aligned(16))) char smem[Product::kLdsBytes];
   const int tb = (int)(blockIdx.y + blockIdx.z * gridDim.y);
   if (tb >= a.items.units_max) return;
@@ -847,12 +827,6 @@ void shrink_block_kernel(ShrinkArgs a) {
   pr.open_w();
   pr.load_w(first);
   if (a.seg_scale && pr.rw >= 0) pr.scale = a.seg_scale[a.plan.tile_rseg[slot]];
-  if (DROP) {
-    const DropArgs dp = drop_proj(a.drop, 0);  // (the rows' probabilities are the same for every projection)
-#pragma unroll
-    for (int t = 0; t < kBlkTiles; ++t)
-      pr.dr[DROP ? t : 0] = drop_row(dp, pr.frow[DROP ? t : 0], a.plan.tile_rseg, (t0 + t) * kTileRows + c);
-  }
   pr.fill_rows();
   pr.open_x();
   const int rows = a.items.row_start[a.items.nproj];
