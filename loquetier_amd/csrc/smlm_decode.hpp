@@ -50,20 +50,20 @@ __device__ __attribute__((aligned(16))) uint32_t self_plan_zeros[4];
 // own because what they add costs the others dearly: the arrays below triple the finder's LDS, and their
 // workgroups may take several units in turn (see shrink_self_planned_kernel), a loop around the whole body
 // that takes the tile-block kernel from 68 to 128 registers a lane.
-template <int N>
+template <int N, int SLOTS>
 struct FindPairs {
   uint64_t ka[N], kb[N];  // the segments' pairs of addresses
   int32_t first[N];       // the first segment with the same pair: the segment's id
-  int32_t slot[2][N];     // (scratch of first_equal_pair)
+  int32_t slot[2][SLOTS]; // (scratch of first_equal_pair)
 };
-template <>
-struct FindPairs<0> {};
-template <int THREADS, bool PAIRS, int N = kSelfPlanWeights>
+template <int SLOTS>
+struct FindPairs<0, SLOTS> {};
+template <int THREADS, bool PAIRS, int N = kSelfPlanWeights, int SLOTS = N>
 struct FindLds {
   int32_t hist[N];   // rows per adapter
   uint64_t wtab[N];  // this projection's weight table
   int32_t rtab[N];   // true ranks, when given
-  FindPairs<PAIRS ? N : 0> pr;
+  FindPairs<PAIRS ? N : 0, SLOTS> pr;
   uint32_t tot_a[THREADS / kWaveSize], tot_b[THREADS / kWaveSize];  // wave totals of the two scans
   int32_t rows[kBlkTiles * kTileRows], rseg[kBlkTiles * kTileRows];
   int32_t sel[3];                   // adapter of the unit (-1: no such unit), unit's index within the adapter, units in all
@@ -94,15 +94,13 @@ __device__ __forceinline__ uint32_t block_scan_excl_1(uint32_t v, uint32_t* tot,
   return before + in_wave - v;
 }
 
-// Which adapter owns unit `unit` (a unit = UT consecutive tiles of one adapter; adapters in
-// ascending order, as the plan's groups are).  Everything global is requested at once; the
-// first barrier (LDS cleared) passes while those loads are on their way.  THREADS >= S.
-template <int THREADS, int UT, bool PAIRS, int N>
-__device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS, N>& F, const PlanSortArgs& pa,
-                                                  const void* const* w_ptrs, const int32_t* w_rank, int NA,
-                                                  int unit, FindSeg* seg) {
+// The rows of every adapter and the tables, into F; returns the thread's segment.  Everything global is requested at
+// once; the first barrier (LDS cleared) passes while those loads are on their way.  THREADS >= S.
+template <int THREADS, int UT, bool PAIRS, int N, int SLOTS>
+__device__ __forceinline__ FindSeg find_tables(FindLds<THREADS, PAIRS, N, SLOTS>& F, const PlanSortArgs& pa,
+                                               const void* const* w_ptrs, const int32_t* w_rank, int NA) {
   constexpr int kEnt = N / THREADS;  // table entries a thread holds: kEnt * tid ...
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   int key = -1, s0 = 0, len = 0;
   uint64_t pair_a = 0, pair_b = 0;
   if (tid < pa.S) {
@@ -134,7 +132,7 @@ __device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS, N>& F,
     // groups by pairs of addresses: the id of a segment is the first segment with its pair, as the plan
     // builders number them (first_equal_pair; its barriers also cover the clearing above)
     if (tid < pa.S) F.pr.ka[tid] = pair_a, F.pr.kb[tid] = pair_b;
-    first_equal_pair<N>(F.pr.ka, F.pr.kb, F.pr.first, F.pr.slot[0], F.pr.slot[1], pa.S);
+    first_equal_pair<SLOTS>(F.pr.ka, F.pr.kb, F.pr.first, F.pr.slot[0], F.pr.slot[1], pa.S);
     if (tid < pa.S) key = F.pr.first[tid];
   } else {
     __syncthreads();
@@ -144,8 +142,15 @@ __device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS, N>& F,
 #pragma unroll
   for (int e = 0; e < kEnt; ++e) F.wtab[kEnt * tid + e] = wp[e], F.rtab[kEnt * tid + e] = wr[e];
   __syncthreads();
-  *seg = FindSeg{key, s0, len, counted};
+  return FindSeg{key, s0, len, counted};
+}
 
+// Which adapter owns unit `unit` (a unit = UT consecutive tiles of one adapter; adapters in
+// ascending order, as the plan's groups are).
+template <int THREADS, int UT, bool PAIRS, int N, int SLOTS>
+__device__ __forceinline__ FoundUnit find_unit(FindLds<THREADS, PAIRS, N, SLOTS>& F, int NA, int unit) {
+  constexpr int kEnt = N / THREADS;
+  const int tid = threadIdx.x, lane = tid & 63;
   auto units_of = [&](int a) -> uint32_t {
     return a < NA ? (uint32_t)((F.hist[a] + UT * kTileRows - 1) / (UT * kTileRows)) : 0u;
   };
@@ -195,10 +200,18 @@ __device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS, N>& F,
   return u;
 }
 
+template <int THREADS, int UT, bool PAIRS, int N, int SLOTS>
+__device__ __forceinline__ FoundUnit find_adapter(FindLds<THREADS, PAIRS, N, SLOTS>& F, const PlanSortArgs& pa,
+                                                  const void* const* w_ptrs, const int32_t* w_rank, int NA,
+                                                  int unit, FindSeg* seg) {
+  *seg = find_tables<THREADS, UT>(F, pa, w_ptrs, w_rank, NA);
+  return find_unit<THREADS, UT>(F, NA, unit);
+}
+
 // The rows of the unit, into F.rows / F.rseg (slot 16 w + c = row c of the unit's tile w; -1 =
 // empty): the adapter's rows in segment order, of which the unit holds 16 UT sub ... + 16 UT - 1.
-template <int THREADS, int UT, bool PAIRS, int N>
-__device__ __forceinline__ void find_rows(FindLds<THREADS, PAIRS, N>& F, const FindSeg& seg, const FoundUnit& u) {
+template <int THREADS, int UT, bool PAIRS, int N, int SLOTS>
+__device__ __forceinline__ void find_rows(FindLds<THREADS, PAIRS, N, SLOTS>& F, const FindSeg& seg, const FoundUnit& u) {
   const int q_lo = u.sub * UT * kTileRows;
   const uint32_t mine = (seg.counted && seg.key == u.wid) ? (uint32_t)seg.len : 0u;
   uint32_t hi_u;
@@ -279,7 +292,7 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   for (int tile = blockIdx.y;; tile += a.units) {
   FindSeg seg;
   const FoundUnit un =
-      find_adapter<THREADS, 1, PAIRS>(F, a.plan, P.w_ptrs, a.sh.plan.w_rank, a.n_weights, tile, &seg);
+      find_adapter<THREADS, 1>(F, a.plan, P.w_ptrs, a.sh.plan.w_rank, a.n_weights, tile, &seg);
   const int wid = un.wid;
   if (wid < 0) return;  // past the last tile; uniform over the workgroup
   const uint16_t* W = reinterpret_cast<const uint16_t*>(F.wtab[wid]);
@@ -303,7 +316,7 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   u32x4 wf[NB][U];
   load_w(kbeg, wf);
 
-  find_rows<THREADS, 1, PAIRS>(F, seg, un);
+  find_rows<THREADS, 1>(F, seg, un);
   const int row = F.rows[c], rseg = F.rseg[c];
   int lrow[U];  // the rows this lane requests
 #pragma unroll
@@ -376,12 +389,16 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
 // nobody reads its plan, which took a launch of its own (5.4 us of a single workgroup and the gap behind it).  Every
 // workgroup finds its tile, asks for its first weights while it finds the rows, and walks the column chunks
 // blockIdx.x, blockIdx.x + gridDim.x ... of it with the next chunk's weights on their way.  A tile's rows get the bits
-// they get from expand_wave_kernel: MFMA columns do not mix.
-// Bound by the finding (about 3 us before a workgroup's first row is known) and the stores behind it: 1856 rows in 24
+// they get from expand_wave_kernel: MFMA columns do not mix.  The addresses are numbered and the rows counted once; a
+// further tile costs a walk over the counts and the scan for its rows (256 one-row segments on 256 addresses, 4096 wide:
+// 127.8 us a pass of both products with all of it done again for every tile and a hash slot a segment, 58.8 so, 63.0
+// with a plan).
+// Bound by the finding (about 3 us before a workgroup's first row is known) and the stores behind it: 1826 rows in 24
 // segments, 16 -> 11008, us: plan 5.4, gap 1.5 and expand 11.9 with a plan; 15.3 so, with eight lists of three chunks a
 // tile, 20.7 with sixteen, 22.3 with a workgroup a chunk.  Both products of that batch 29.3 -> 26.6; 40 segments of 8
 // rows, 128 -> 4096, 29.8 -> 23.8, and what is smaller is host time (26.7 -> 23.7).
-constexpr int kFoundSegs = kFwdThreads;  // most segments: one a thread
+constexpr int kFoundSegs = kFwdThreads;      // most segments: one a thread
+constexpr int kFoundSlots = 4 * kFoundSegs;  // hash slots of their addresses, so that few of them collide
 
 struct FoundExpandArgs {
   ExpandProj p;        // y, v, w_ptrs (one per segment), d_in, d_out, ldw
@@ -394,7 +411,7 @@ struct FoundExpandArgs {
 
 template <int DT, int NQ, int KS>
 __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandArgs a) {
-  __shared__ FindLds<kFwdThreads, true, kFoundSegs> F;
+  __shared__ FindLds<kFwdThreads, true, kFoundSegs, kFoundSlots> F;
   __shared__ __attribute__((aligned(16))) float olds[kFwdWaves][kTileRows * kOPitch];
   if ((int)blockIdx.x >= a.chunks) return;  // (lists rounded up)
   const ExpandProj& P = a.p;
@@ -404,9 +421,9 @@ __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandAr
   const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
   constexpr int KSU = KS > 0 ? KS : 1;
 
+  const FindSeg seg = find_tables<kFwdThreads, 1>(F, a.plan, P.w_ptrs, nullptr, a.plan.S);
   for (int tile = blockIdx.y;; tile += a.units) {
-    FindSeg seg;
-    const FoundUnit un = find_adapter<kFwdThreads, 1, true>(F, a.plan, P.w_ptrs, nullptr, a.plan.S, tile, &seg);
+    const FoundUnit un = find_unit<kFwdThreads, 1>(F, a.plan.S, tile);
     if (un.wid < 0) return;  // past the last tile; uniform over the workgroup
     const uint16_t* W = reinterpret_cast<const uint16_t*>(F.wtab[un.wid]);
     u32x4 wf[KSU][NQ][2];
@@ -425,7 +442,7 @@ __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandAr
       for (int ks = 0; ks < KSU; ++ks) load_w(blockIdx.x, ks, wf[ks]);
     }
 
-    find_rows<kFwdThreads, 1, true>(F, seg, un);
+    find_rows<kFwdThreads, 1>(F, seg, un);
     const int row = F.rows[c];
     LineLane L;
     L.orow = lane >> 3;
@@ -474,7 +491,8 @@ __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandAr
       store_y_lines<DT, NQ>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
     }
     if (tile + a.units >= un.total) return;  // uniform over the workgroup: no tile is left for it
-    __syncthreads();                         // every wave has read its rows: the finder takes its LDS back
+    __syncthreads();                         // every wave has read its rows
+    if (threadIdx.x < kTileRows) F.rows[threadIdx.x] = -1, F.rseg[threadIdx.x] = -1;  // (find_rows starts with a barrier)
   }
 }
 
@@ -534,7 +552,7 @@ __global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfP
   for (int tb = blockIdx.y;; tb += a.units) {
   FindSeg seg;
   const FoundUnit un =
-      find_adapter<THREADS, kBlkTiles, PAIRS>(sm.find, a.plan, P.w_ptrs, a.sh.plan.w_rank, a.n_weights, tb, &seg);
+      find_adapter<THREADS, kBlkTiles>(sm.find, a.plan, P.w_ptrs, a.sh.plan.w_rank, a.n_weights, tb, &seg);
   if (un.wid < 0) return;  // past the last tile block; uniform over the workgroup
   const uint16_t* W = reinterpret_cast<const uint16_t*>(sm.find.wtab[un.wid]);
   int nlim = P.d_out;  // weight rows at or past it are zero padding
@@ -579,7 +597,7 @@ __global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfP
   u32x4 wst[kPer];
   load_w(kbeg, wst);
 
-  find_rows<THREADS, kBlkTiles, PAIRS>(sm.find, seg, un);
+  find_rows<THREADS, kBlkTiles>(sm.find, seg, un);
   const bool active = wave < un.tiles;
   const int row = active ? sm.find.rows[wave * kTileRows + c] : -1;
   const int rseg = active ? sm.find.rseg[wave * kTileRows + c] : -1;
@@ -687,7 +705,7 @@ void shrink_block_self_planned_kernel(SelfPlanArgs a) {
   // shrink_self_planned_kernel)
   for (int tb = (int)blockIdx.y - a.builder_rows;; tb += a.units) {
   FindSeg seg;
-  const FoundUnit un = find_adapter<THREADS, kBlkTiles, PAIRS>(sm.find, a.plan, a.sh.p[pj].w_ptrs, a.sh.plan.w_rank,
+  const FoundUnit un = find_adapter<THREADS, kBlkTiles>(sm.find, a.plan, a.sh.p[pj].w_ptrs, a.sh.plan.w_rank,
                                                                a.n_weights, tb, &seg);
   if (un.wid < 0) return;  // past the last tile block; uniform over the workgroup
   const int wid = __builtin_amdgcn_readfirstlane(un.wid);
@@ -707,7 +725,7 @@ void shrink_block_self_planned_kernel(SelfPlanArgs a) {
   pr.open_w(GROUPS > 1 && pr.item(pr.r).pj != pj ? nullptr : W);
   pr.load_w(first);
 
-  find_rows<THREADS, kBlkTiles, PAIRS>(sm.find, seg, un);
+  find_rows<THREADS, kBlkTiles>(sm.find, seg, un);
   pr.set_rows([&](int i) { return sm.find.rows[i]; });  // -1: empty
   if (!pr.exists(list)) pr.rw = -1;
   if (a.sh.seg_scale && pr.rw >= 0) pr.scale = a.sh.seg_scale[sm.find.rseg[wave * kTileRows + c]];

@@ -21,6 +21,9 @@ CASES = {
     "rounds": ([1] * 256, 256, 16, 1032, 0),        # a tile a segment: more than the launch has rows of workgroups
     "planned-257": ([2] * 257, 9, 16, 1032, 0),     # one segment too many: the plan's launch
     "equal-width": ([5, 6], 2, 8, 24, 0),
+    "128-wide": ([1] * 128, 40, 16, 12296, 0),
+    "planned-129-wide": ([1] * 129, 40, 16, 12296, 0),  # too many column chunks for so many segments: the plan's launch
+    "planned-256-13-chunks": ([1] * 256, 40, 16, 6152, 0),
 }
 
 
@@ -52,3 +55,42 @@ def test_equals_the_planned_product(K, gpu_device, name, dt):
         assert torch.equal(got, want)
         outside = list(range(first)) + list(range(int(seg[-1]), T))
         assert torch.equal(got[outside], y0[outside])
+
+
+def test_many_addresses_take_no_longer_than_the_planned_product(K, gpu_device):
+    """256 one-row segments on as many addresses: more tiles than the launch has rows of workgroups, and as many addresses
+    as can be to tell apart.  The planned product does the same work plus the plan's launch, so its time is the bound;
+    half as much again for what two timings differ by (140 us against 20 with the search done again for every tile)."""
+    from loquetier_amd import _lib as lib
+    d, S, d_in, d_out, n = gpu_device, 256, 16, 6144, 20
+    x, W = torch.randn(S, d_in, device=d).half(), torch.randn(S, d_out, d_in, device=d).half()
+    seg, table = torch.arange(S + 1, dtype=torch.int32, device=d), ptrs(list(W), d)
+    y = torch.empty(S, d_out, dtype=torch.float16, device=d)
+    need = lib.size_query("smlm_gemm_workspace_size", S, S, d_in, d_out)
+    ws = torch.empty(need, dtype=torch.uint8, device=d)
+    code, stream, lib_ = lib.SMLM_DTYPE_F16, torch.cuda.current_stream(d).cuda_stream, lib.load()
+    plan = torch.empty(K.SegmentPlan.nbytes(S, S), dtype=torch.uint8, device=d)
+
+    def found():
+        return lib_.smlm_gemm(y.data_ptr(), x.data_ptr(), table.data_ptr(), seg.data_ptr(), ws.data_ptr(), need, S, S, d_in,
+                              d_out, d_in, 0, code, 0.0, None, stream)
+
+    def planned():
+        return lib_.smlm_plan_build(plan.data_ptr(), plan.numel(), seg.data_ptr(), table.data_ptr(), lib.SMLM_KEY_PTR, S, S,
+                                    stream) or \
+            lib_.smlm_gemm_planned(y.data_ptr(), x.data_ptr(), table.data_ptr(), S, plan.data_ptr(), ws.data_ptr(), need, S,
+                                   S, d_in, d_out, d_in, 0, code, 0.0, None, stream)
+
+    def time(call):
+        best = []
+        for _ in range(7):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(n):
+                assert call() == 0
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_time(b))
+        return sorted(best)[1]
+    time(found), time(planned)
+    assert time(found) <= 1.5 * time(planned)
