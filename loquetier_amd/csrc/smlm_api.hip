@@ -122,11 +122,18 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
 inline bool block_shrink(int mt, int T, int d_out, bool drop = false) {
   return mt > 1 && !drop && T >= (d_out <= 32 ? 1024 : 3072) && d_out <= 64;
 }
-// ... of a launch: its weight rows must be within the block kernel's reach too (the slices are the same either way)
-inline bool block_shrink(int mt, const ShrinkArgs& a) {
-  bool near = block_shrink(mt, a.T, a.p[0].d_out, a.drop.seg_p != nullptr);
-  for (int i = 0; i < a.items.nproj; ++i) near = near && a.p[i].ldw <= kBlockMaxLd;
+// ... of a launch: its weight rows must be within the block kernel's reach too (the slices are the same either way).
+// Whoever decides on the plan's route asks this, as the launch does: the wide kernel needs the splits even where two
+// groups of waves share a workgroup, and would store a slice past the last one.
+inline bool block_shrink(int mt, int T, int d_out, bool drop, int nproj, const int* ldw) {
+  bool near = block_shrink(mt, T, d_out, drop);
+  for (int i = 0; i < nproj; ++i) near = near && ldw[i] <= kBlockMaxLd;
   return near;
+}
+inline bool block_shrink(int mt, const ShrinkArgs& a) {
+  int ldw[kMaxProj];
+  for (int i = 0; i < a.items.nproj; ++i) ldw[i] = a.p[i].ldw;
+  return block_shrink(mt, a.T, a.p[0].d_out, a.drop.seg_p != nullptr, a.items.nproj, ldw);
 }
 
 // k slices of a tile-block shrink, in pieces of 256 of k (64 a wave): the split with the shortest time in steps of a
@@ -991,7 +998,7 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
   const int nw = shrink_waves(mt, 1, &d_in, d_out);
   const int ks = shrink_cfg(T, d_in, d_out, nw, false, mt, true).ksplit;
   const bool in_launch = d_in >= d_out && !w_row_major && self_planned_ok(T, S, S, pv.nt_max, mt) &&
-                         (mt > 1 ? (S <= kFwdThreads || block_shrink(mt, T, d_out) || ks % 2 == 0)
+                         (mt > 1 ? (S <= kFwdThreads || block_shrink(mt, T, d_out, false, 1, &w_ld) || ks % 2 == 0)
                                  : (nw == kDecodeWaves && (S <= kSelfPlanThreads || ks % 2 == 0)));
   if (in_launch) {
     if (!aligned16(y) || !aligned16(x)) return SMLM_ERR_ALIGN;
@@ -1162,8 +1169,9 @@ SMLM_API int smlm_lora_fwd_multi_ex(int n_proj, void* const* y, const void* cons
   // (both routes pair k slices up in one workgroup beyond 512 / 256 segments)
   const bool self_planned = build_s && (!drop.seg_p || build_kind == SMLM_KEY_I32) &&
                             self_planned_ok(T, S, n_weights, pv.nt_max, mt) &&
-                            (mt > 1 ? (S <= kFwdThreads || block_shrink(mt, T, r, drop.seg_p != nullptr) || even_splits)
-                                                   : (expand_folds && (S <= kSelfPlanThreads || even_splits)));
+                            (mt > 1 ? (S <= kFwdThreads ||
+                                       block_shrink(mt, T, r, drop.seg_p != nullptr, n_proj, h_in) || even_splits)
+                                    : (expand_folds && (S <= kSelfPlanThreads || even_splits)));
   if (build_s && !self_planned && (rc = plan_build_impl(pv, build_s, build_k, build_kind, S, st, build_k2))) return rc;
   if (stages & SMLM_STAGE_SHRINK) {
     rc = run_shrink(dtype, pv, T, S, n_weights, n_proj, x, a_ptrs, partial, v16, h_in, r, h_in,

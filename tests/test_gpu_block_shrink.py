@@ -94,3 +94,25 @@ def test_inf_and_nan_stay_in_their_rows_and_columns(K, gpu_device, r):
     mid[70:3000] = True
     assert v[ok & ~mid].isfinite().all() and not v[~ok].isfinite().any()
     assert v[mid][:, 3].isnan().all() and v[mid][:, [0, 1, 2, 4, 5, 6, 7]].isfinite().all() and not v[mid][:, 8:].any()
+
+
+@pytest.mark.parametrize("S", [200, 300])
+def test_weight_rows_out_of_the_block_kernels_reach(K, gpu_device, S):
+    """Rows of 2 ** 25 elements and more go to the wide kernel: beyond 256 segments, with k in three, its two groups of
+    waves a workgroup may not pair the slices up.  Whole numbers, so any order of the sums gives the same bits."""
+    from loquetier_amd import _lib as lib
+    d, T, d_in, d_out, ld = gpu_device, 2100, 1536, 16, 2 ** 25 + 8
+    g = torch.Generator().manual_seed(1)
+    whole = lambda *s: torch.randint(-3, 4, s, generator=g).half().to(d)
+    seg = (torch.arange(S + 1) * T // S).to(torch.int32).to(d)
+    x, w = whole(T, d_in), whole(d_out, d_in)
+    far = torch.empty((d_out - 1) * ld + d_in, dtype=torch.float16, device=d)
+    far.as_strided((d_out, d_in), (ld, 1)).copy_(w)
+    need = lib.size_query("smlm_gemm_workspace_size", T, S, d_in, d_out)
+    ws = torch.full((need + T * d_out * 4,), 0xA5, dtype=torch.uint8, device=d)
+    y, table = torch.empty(T, d_out, dtype=torch.float16, device=d), ptrs([far] * S, d)
+    rc = lib.load().smlm_gemm(y.data_ptr(), x.data_ptr(), table.data_ptr(), seg.data_ptr(), ws.data_ptr(), need,
+                              T, S, d_in, d_out, ld, 0, lib.SMLM_DTYPE_F16, 0.0, None,
+                              torch.cuda.current_stream(d).cuda_stream)
+    assert rc == 0, lib.strerror(rc)
+    assert torch.equal(y, (x.double() @ w.double().T).half()) and bool((ws[need:] == 0xA5).all())
