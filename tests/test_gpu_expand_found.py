@@ -1,6 +1,7 @@
 """Expanding products of smlm_gemm whose workgroups find their tiles without a plan: bit for bit what the same product
 over a finished plan gives, at the edges of its range -- segments up to a thread each, empty and repeated ones, more tiles
 than rows of workgroups, k and columns short of a step and of a chunk, beta and scale, rows no segment covers."""
+import numpy as np
 import pytest
 import torch
 
@@ -55,6 +56,40 @@ def test_equals_the_planned_product(K, gpu_device, name, dt):
         assert torch.equal(got, want)
         outside = list(range(first)) + list(range(int(seg[-1]), T))
         assert torch.equal(got[outside], y0[outside])
+
+
+def _colliding(base, n, slots, per):
+    """Addresses in `n` sixteenths of bytes from `base` of which `per` share both hash slots of first_equal_pair."""
+    at = (np.uint64(base >> 4) + np.arange(n, dtype=np.uint64))
+    with np.errstate(over="ignore"):
+        h = (at * np.uint64(0x9E3779B97F4A7C15)) ^ (at * np.uint64(0xC2B2AE3D27D4EB4F))
+    both = (h >> np.uint64(40)) % np.uint64(slots) * np.uint64(slots) + (h >> np.uint64(24)) % np.uint64(slots)
+    order = np.argsort(both, kind="stable")
+    run = np.flatnonzero(both[order[:-per + 1]] == both[order[per - 1:]])
+    first = run[np.concatenate([[True], np.diff(run) >= per])]
+    return [int(at[order[i + j]]) << 4 for i in first[:250 // per] for j in range(per)]
+
+
+def test_addresses_that_collide_twice(K, gpu_device):
+    """Segments whose address loses its slot in both rounds of the numbering: three of every four here, each address
+    twice.  The product equals the one over a plan, which sorts the addresses."""
+    from loquetier_amd import _lib as lib
+    d, d_in, d_out = gpu_device, 16, 64
+    g = torch.Generator().manual_seed(3)
+    pool = torch.randn(1 << 25, generator=g).half().to(d)  # the weights overlap in it
+    some = _colliding(pool.data_ptr(), pool.numel() // 8 - d_in * d_out, 1024, 4)[:128]
+    assert len(some) == 128
+    table = torch.tensor(some + some[::-1], dtype=torch.int64, device=d)
+    S = 256
+    seg = torch.arange(S + 1, dtype=torch.int32, device=d)
+    x, want, got = torch.randn(S, d_in, generator=g).half().to(d), *torch.zeros(2, S, d_out, dtype=torch.float16, device=d)
+    K.smlm_gemm_planned(want, x, table, K.SegmentPlan(seg, None, S))
+    need = lib.size_query("smlm_gemm_workspace_size", S, S, d_in, d_out)
+    ws = torch.empty(need, dtype=torch.uint8, device=d)
+    rc = lib.load().smlm_gemm(got.data_ptr(), x.data_ptr(), table.data_ptr(), seg.data_ptr(), ws.data_ptr(), need, S, S, d_in,
+                              d_out, d_in, 0, lib.SMLM_DTYPE_F16, 0.0, None, torch.cuda.current_stream(d).cuda_stream)
+    assert rc == 0, lib.strerror(rc)
+    assert torch.equal(got, want)
 
 
 def test_many_addresses_take_no_longer_than_the_planned_product(K, gpu_device):
