@@ -778,31 +778,13 @@ int launch_expand_found_dt(int nq, int KS, dim3 grid, hipStream_t st, const Foun
   if (KS == 2) return launch(expand_found_kernel<DT, 2, 2>, grid, block, st, a);
   return launch(expand_found_kernel<DT, 2, 0>, grid, block, st, a);
 }
-inline int found_chunks(int T, int d_out) { return ceil_div(d_out, kFwdWaves * 32 * expand_nq(T, d_out)); }
-// Whether an expand of smlm_gemm on single tiles finds its tiles itself (expand_found_kernel) or takes the plan's launch.
-// It holds weights of a chunk or two in flight a workgroup, and where every segment has an address of its own and their
-// weights come out of HBM the planned kernel's single-chunk workgroups fetch them faster.  Both products of smlm_gemm
-// with one-row segments on as many addresses, rank 16, us, planned / found: 64 segments 11008 wide 25.0 / 22.7; 128
-// segments 4096 wide 32.7 / 27.5, 11008 35.7 / 34.1, 14336 37.8 / 37.7; 192 segments 8192 wide 42.1 / 36.6 (7 rows each,
-// 11008: 44.2 / 46.4); 256 segments 4096 wide 63.0 / 58.8, 6144 48.5 / 45.5, 8192 53.7 / 84.5, 11008 58.9 / 79.1.
-inline bool expand_found(int T, int S, int d_out) {
-  return S <= kFoundSegs && (S <= 128 || (long)S * found_chunks(T, d_out) <= 3072);
-}
-// About five workgroups a CU, each with its share of a tile's column chunks; lists in multiples of eight, so that a
-// chunk's weights stay on an XCD (workgroups go to the XCDs in turn).  Rows of workgroups: as launch_shrink_self_planned
-// counts them, but at least 160 where there can be as many tiles (256 segments on 256 addresses, 11008 wide: 82.8 us in
-// the six rounds of 49 rows, 73.6 in two; 32 addresses 23.8 and 24.2).
 int launch_expand_found(int dtype, int T, int S, hipStream_t st, FoundExpandArgs& a) {
   const int nq = expand_nq(T, a.p.d_out);
   const int KS = a.p.d_in <= 32 ? 1 : (a.p.d_in <= 64 ? 2 : 0);
-  a.chunks = found_chunks(T, a.p.d_out);
-  const int most = tile_units_max(T, S, S, 1);
-  int usual = T / kTileRows + 1 + 32;
-  if (usual < 160) usual = 160;
-  a.units = most < usual ? most : usual;
-  int lists = ceil_div(a.chunks, ceil_div(a.units * a.chunks, 1280));
-  if (lists > kWgXcd / 2) lists = round_up(lists, kWgXcd);
-  const dim3 grid((unsigned)lists, (unsigned)a.units);
+  a.chunks = ceil_div(a.p.d_out, kFwdWaves * 32 * nq);
+  const long items = (long)tile_units_max(T, S, S, 1) * a.chunks, wgs = 256 * found_wgs(nq, KS);
+  a.lists = items <= wgs ? a.chunks : 0;  // (a workgroup for every chunk there can be)
+  const dim3 grid((unsigned)(items < wgs ? items : wgs));
   return dtype == SMLM_DTYPE_F16 ? launch_expand_found_dt<SMLM_DTYPE_F16>(nq, KS, grid, st, a)
                                  : launch_expand_found_dt<SMLM_DTYPE_BF16>(nq, KS, grid, st, a);
 }
@@ -1007,9 +989,9 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
     return run_shrink(dtype, pv, T, S, S, 1, &x, &w_ptrs, &partial, &y, &d_in, d_out, &w_ld, beta,
                       seg_scale, mt, st, true, false, nullptr, nullptr, 0, &build, false, nullptr, nullptr, true);
   }
-  // An expanding product on single tiles may find them itself.  Larger batches, on tile blocks, keep the plan's launch:
-  // it is the smaller part of theirs.
-  if (d_in < d_out && !w_row_major && expand_found(T, S, d_out) && tiles_per_wave(T, d_in, kNoShrink) == 1) {
+  // An expanding product on single tiles finds them itself, up to a segment a thread.  Larger batches, on tile blocks,
+  // keep the plan's launch: it is the smaller part of theirs.
+  if (d_in < d_out && !w_row_major && S <= kFoundSegs && tiles_per_wave(T, d_in, kNoShrink) == 1) {
     FoundExpandArgs a{};
     a.plan = PlanSortArgs{pv, seg_indptr, w_ptrs, SMLM_KEY_PTR2, S, next_pow2(S), w_ptrs};
     a.seg_scale = seg_scale;

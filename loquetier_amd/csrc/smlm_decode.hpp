@@ -386,17 +386,15 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
 
 // ---- expand by itself (smlm_gemm), single tiles: expand_wave_kernel without a plan --------------------
 // One weight address per segment, as many table entries as segments.  A product that expands is the last of its call:
-// nobody reads its plan, which took a launch of its own (5.4 us of a single workgroup and the gap behind it).  Every
-// workgroup finds its tile, asks for its first weights while it finds the rows, and walks the column chunks
-// blockIdx.x, blockIdx.x + gridDim.x ... of it with the next chunk's weights on their way.  A tile's rows get the bits
-// they get from expand_wave_kernel: MFMA columns do not mix.  The addresses are numbered and the rows counted once; a
-// further tile costs a walk over the counts and the scan for its rows (256 one-row segments on 256 addresses, 4096 wide:
-// 127.8 us a pass of both products with all of it done again for every tile and a hash slot a segment, 58.8 so, 63.0
-// with a plan).
-// Bound by the finding (about 3 us before a workgroup's first row is known) and the stores behind it: 1826 rows in 24
-// segments, 16 -> 11008, us: plan 5.4, gap 1.5 and expand 11.9 with a plan; 15.3 so, with eight lists of three chunks a
-// tile, 20.7 with sixteen, 22.3 with a workgroup a chunk.  Both products of that batch 29.3 -> 26.6; 40 segments of 8
-// rows, 128 -> 4096, 29.8 -> 23.8, and what is smaller is host time (26.7 -> 23.7).
+// nobody reads its plan, which took a launch of its own (5.4 us of a single workgroup and the gap behind it).  As many
+// workgroups as the chip holds number the addresses and count the rows once each, and deal out items (tile, list of column
+// chunks) by what they found: the host knows only how many tiles there can be.  The weights of an item's first chunk are
+// requested before its rows are found, the next chunk's while one is multiplied.  A tile's rows get the bits
+// they get from expand_wave_kernel: MFMA columns do not mix.
+// Bound by the finding (about 3 us before a workgroup's first row is known), then by the weights and the stores.  us, a
+// plan and its expand / lists and rows of workgroups fixed by the host / so: 1826 rows in 24 segments, 16 -> 4096 12.5 /
+// 10.4 / 8.2, 16 -> 11008 16.8 / 15.8 / 12.9; 64 one-row segments on as many addresses, 16 -> 11008 11.7 / 13.2 / 7.9; 256
+// on 256 addresses 25.9 / 216 / 19.7, on 32 13.1 / 10.6 / 7.0; one row, 16 -> 4096 8.0 / 4.8 / 4.9.
 constexpr int kFoundSegs = kFwdThreads;      // most segments: one a thread
 constexpr int kFoundSlots = 4 * kFoundSegs;  // hash slots of their addresses, so that few of them collide
 
@@ -405,15 +403,30 @@ struct FoundExpandArgs {
   PlanSortArgs plan;   // s, key = key2 = w_ptrs, S
   const float* seg_scale;
   float beta;
-  int units;           // rows of workgroups (tiles beyond them: further rounds)
   int chunks;          // column chunks of kFwdWaves * 32 * NQ
+  int lists;           // lists of chunks a tile, or 0: as found_lists says
 };
 
+// workgroups a CU (what the registers of the kernel below leave room for)
+constexpr int found_wgs(int nq, int KS) { return nq == 2 || KS == 1 ? 3 : 2; }
+
+// Lists the chunks of every tile are dealt out into: with `wgs` workgroups that take an item (tile, list) each in turn,
+// the fewest turns times what one takes -- a change of tile, as much as kFoundSwitch chunks, and its chunks.  Every lane
+// prices one number of lists; all workgroups come to the same one.
+constexpr float kFoundSwitch = 2.0f;
+__device__ __forceinline__ int found_lists(int tiles, int chunks, int wgs) {
+  const int lists = (int)(threadIdx.x & 63) + 1;
+  const float each = ceilf((float)chunks * __builtin_amdgcn_rcpf((float)lists) - 1e-3f);
+  const float turns = ceilf((float)(tiles * lists) * __builtin_amdgcn_rcpf((float)wgs) - 1e-3f);
+  const uint32_t price = lists <= chunks ? (uint32_t)(turns * (kFoundSwitch + each)) * kWaveSize + lists - 1 : ~0u;
+  return (int)(wave_min_u32(price) % kWaveSize) + 1;
+}
+
 template <int DT, int NQ, int KS>
-__global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandArgs a) {
+__global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(found_wgs(NQ, KS))))
+void expand_found_kernel(FoundExpandArgs a) {
   __shared__ FindLds<kFwdThreads, true, kFoundSegs, kFoundSlots> F;
   __shared__ __attribute__((aligned(16))) float olds[kFwdWaves][kTileRows * kOPitch];
-  if ((int)blockIdx.x >= a.chunks) return;  // (lists rounded up)
   const ExpandProj& P = a.p;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
@@ -422,9 +435,34 @@ __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandAr
   constexpr int KSU = KS > 0 ? KS : 1;
 
   const FindSeg seg = find_tables<kFwdThreads, 1>(F, a.plan, P.w_ptrs, nullptr, a.plan.S);
-  for (int tile = blockIdx.y;; tile += a.units) {
-    const FoundUnit un = find_unit<kFwdThreads, 1>(F, a.plan.S, tile);
-    if (un.wid < 0) return;  // past the last tile; uniform over the workgroup
+  // tiles of the addresses, 64 a step, and where they end
+  uint32_t own[kFoundSegs / kWaveSize], end[kFoundSegs / kWaveSize], tiles = 0;
+#pragma unroll
+  for (int i = 0; i < kFoundSegs / kWaveSize; ++i)
+    own[i] = (uint32_t)(F.hist[kWaveSize * i + lane] + kTileRows - 1) / kTileRows;  // (entries past S are zero)
+#pragma unroll
+  for (int i = 0; i < kFoundSegs / kWaveSize; ++i) {
+    if (kWaveSize * i >= a.plan.S) break;
+    end[i] = tiles + wave_scan_incl_u32(own[i]);
+    tiles = (uint32_t)__builtin_amdgcn_readlane((int)end[i], kWaveSize - 1);
+  }
+  const int lists = a.lists ? a.lists : found_lists((int)tiles, a.chunks, gridDim.x);
+  const float per = __builtin_amdgcn_rcpf((float)lists);
+  for (int item = blockIdx.x;; item += gridDim.x) {
+    const uint32_t tile = __builtin_amdgcn_readfirstlane((int)(((float)item + 0.5f) * per));
+    if (tile >= tiles) return;  // uniform over the workgroup
+    const int list = item - (int)tile * lists;  // its chunks: list, list + lists ...
+    FoundUnit un{-1, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < kFoundSegs / kWaveSize; ++i) {
+      if (kWaveSize * i >= a.plan.S) break;
+      const uint64_t hit = __ballot(tile < end[i] && tile >= end[i] - own[i]);
+      if (hit) {  // uniform over the wave; one lane
+        const int l = __builtin_ctzll(hit);
+        un.wid = kWaveSize * i + l;
+        un.sub = (int)(tile - (uint32_t)__builtin_amdgcn_readlane((int)(end[i] - own[i]), l));
+      }
+    }
     const uint16_t* W = reinterpret_cast<const uint16_t*>(F.wtab[un.wid]);
     u32x4 wf[KSU][NQ][2];
     auto load_w = [&](int yy, int ks, u32x4 (&w)[NQ][2]) {
@@ -439,7 +477,7 @@ __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandAr
     };
     if (KS > 0) {
 #pragma unroll
-      for (int ks = 0; ks < KSU; ++ks) load_w(blockIdx.x, ks, wf[ks]);
+      for (int ks = 0; ks < KSU; ++ks) load_w(list, ks, wf[ks]);
     }
 
     find_rows<kFwdThreads, 1>(F, seg, un);
@@ -463,7 +501,7 @@ __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandAr
     }
 
 #pragma unroll 1
-    for (int yy = blockIdx.x; yy < a.chunks; yy += gridDim.x) {
+    for (int yy = list; yy < a.chunks; yy += lists) {
       const int ncol0 = (yy * kFwdWaves + wave) * 32 * NQ;
       if (ncol0 >= P.d_out) break;  // (no barrier in this loop)
 #pragma unroll
@@ -484,14 +522,13 @@ __global__ __launch_bounds__(kFwdThreads) void expand_found_kernel(FoundExpandAr
           for (int p = 0; p < 2; ++p)
             acc[q][p] = Num<DT>::mfma(wf[KS > 0 ? ks : 0][q][p], vf[KS > 0 ? ks : 0], acc[q][p]);
       }
-      if (KS > 0 && yy + (int)gridDim.x < a.chunks) {
+      if (KS > 0 && yy + lists < a.chunks) {
 #pragma unroll
-        for (int ks = 0; ks < KSU; ++ks) load_w(yy + gridDim.x, ks, wf[ks]);
+        for (int ks = 0; ks < KSU; ++ks) load_w(yy + lists, ks, wf[ks]);
       }
       store_y_lines<DT, NQ>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
     }
-    if (tile + a.units >= un.total) return;  // uniform over the workgroup: no tile is left for it
-    __syncthreads();                         // every wave has read its rows
+    __syncthreads();  // every wave has read its rows
     if (threadIdx.x < kTileRows) F.rows[threadIdx.x] = -1, F.rseg[threadIdx.x] = -1;  // (find_rows starts with a barrier)
   }
 }

@@ -90,6 +90,17 @@ __device__ __forceinline__ void first_equal_pair(A64& ka, A64& kb, A32& first, T
   __syncthreads();
 }
 
+// The smallest value of the wave, in every lane: minima in the steps of the scan below, of which lane 63 has the last.
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x111, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x112, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x114, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x118, 0xf, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x142, 0xa, 0xf, false));
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x143, 0xc, 0xf, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, kWaveSize - 1);
+}
+
 // Inclusive scan of a 32-bit value over the wave with DPP adds: four shifts
 // inside each row of 16 lanes (a lane whose source falls outside its row adds
 // zero), then lane 15 of rows 0 and 2 into rows 1 and 3, then lane 31 into rows

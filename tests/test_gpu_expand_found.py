@@ -1,6 +1,6 @@
 """Expanding products of smlm_gemm whose workgroups find their tiles without a plan: bit for bit what the same product
-over a finished plan gives, at the edges of its range -- segments up to a thread each, empty and repeated ones, more tiles
-than rows of workgroups, k and columns short of a step and of a chunk, beta and scale, rows no segment covers."""
+over a finished plan gives, at the edges of its range -- segments up to a thread each, empty and repeated ones, more items
+than workgroups, k and columns short of a step and of a chunk, beta and scale, rows no segment covers."""
 import numpy as np
 import pytest
 import torch
@@ -19,12 +19,13 @@ CASES = {
     "k-72": ([3, 50, 31], 2, 72, 1000, 0),
     "k-128": ([1] * 100, 7, 128, 264, 5),
     "decode-256": ([1] * 256, 32, 16, 4096, 0),
-    "rounds": ([1] * 256, 256, 16, 1032, 0),        # a tile a segment: more than the launch has rows of workgroups
+    "rounds": ([1] * 256, 256, 16, 1032, 0),        # a tile a segment: several turns a workgroup
     "planned-257": ([2] * 257, 9, 16, 1032, 0),     # one segment too many: the plan's launch
     "equal-width": ([5, 6], 2, 8, 24, 0),
     "128-wide": ([1] * 128, 40, 16, 12296, 0),
-    "planned-129-wide": ([1] * 129, 40, 16, 12296, 0),  # too many column chunks for so many segments: the plan's launch
-    "planned-256-13-chunks": ([1] * 256, 40, 16, 6152, 0),
+    "129-wide": ([1] * 129, 40, 16, 12296, 0),
+    "256-13-chunks": ([1] * 256, 40, 16, 6152, 0),
+    "70-chunks": ([40] * 30, 30, 16, 35336, 2),         # more column chunks than lists are priced
 }
 
 
@@ -93,7 +94,7 @@ def test_addresses_that_collide_twice(K, gpu_device):
 
 
 def test_many_addresses_take_no_longer_than_the_planned_product(K, gpu_device):
-    """256 one-row segments on as many addresses: more tiles than the launch has rows of workgroups, and as many addresses
+    """256 one-row segments on as many addresses: several items a workgroup, and as many addresses
     as can be to tell apart.  The planned product does the same work plus the plan's launch, so its time is the bound;
     half as much again for what two timings differ by (140 us against 20 with the search done again for every tile)."""
     from loquetier_amd import _lib as lib
