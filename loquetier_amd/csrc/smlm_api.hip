@@ -314,8 +314,12 @@ int launch_shrink_block(int NB, dim3 grid, hipStream_t st, const ShrinkArgs& a) 
 // rounds of chunk rows a CU, within one generation of resident workgroups where that costs nothing, and the most
 // workgroups of those.  us, four / six / twelve lists, three projections of h_in = 4096 at rank 64, k in four: 4096 rows
 // 36.5 / 42.6 / 35.9, 8192 rows 59.4 / 64.4 / 61.7.
-int shrink_lists(int T, int S, int groups, int rows) {
-  const float units = ceil_div(T, kTileRows * kBlkTiles) + 0.5f * (groups > 0 && groups < S ? groups : S);
+// pairs: plans keyed by pairs of addresses, whose table has an entry per segment, so that it says little about how many
+// tile blocks are partly filled (2100 rows of 64 adapters in 256 segments at rank 16: 32.4 us, counting 128 of them, 30.0).
+int shrink_lists(int T, int S, int groups, int rows, bool pairs = false) {
+  float partly = 0.5f * (groups > 0 && groups < S ? groups : S);  // filled tile blocks
+  if (pairs && partly > 32) partly = 32;
+  const float units = ceil_div(T, kTileRows * kBlkTiles) + partly;
   int best = rows;
   float least = units * rows / 256 + 0.4f;
   for (int lists = rows - 1; lists >= 1; --lists) {
@@ -457,7 +461,7 @@ int launch_shrink_self_planned(int dtype, const ShrinkCfg& c, int S, int groups,
     if (a.items.row_start[i + 1] - a.items.row_start[i] > rows) rows = a.items.row_start[i + 1] - a.items.row_start[i];
   dim3 grid((unsigned)rows, (unsigned)sp.units + 1u, (unsigned)a.items.nproj);
   if (block_shrink(c.MT, a)) {
-    const int lists = shrink_lists(a.T, S, groups, a.items.row_start[a.items.nproj]);
+    const int lists = shrink_lists(a.T, S, groups, a.items.row_start[a.items.nproj], pairs);
     sp.builder_rows = ceil_div(kSelfPlanBuilders, S <= kFwdThreads ? lists : ceil_div(lists, 2));
     grid = dim3((unsigned)lists, (unsigned)(sp.units + sp.builder_rows));
   }

@@ -50,6 +50,13 @@ __device__ __attribute__((aligned(16))) uint32_t self_plan_zeros[4];
 // own because what they add costs the others dearly: the arrays below triple the finder's LDS, and their
 // workgroups may take several units in turn (see shrink_self_planned_kernel), a loop around the whole body
 // that takes the tile-block kernel from 68 to 128 registers a lane.
+template <bool PAIRS>
+__device__ __forceinline__ int turn_value(int v) {
+  // what such a loop derives from a thread's place is worked out in every turn: the compiler otherwise keeps all of it
+  // in registers across the products
+  if (PAIRS) asm volatile("" : "+v"(v));
+  return v;
+}
 template <int N, int SLOTS>
 struct FindPairs {
   uint64_t ka[N], kb[N];  // the segments' pairs of addresses
@@ -100,7 +107,7 @@ template <int THREADS, int UT, bool PAIRS, int N, int SLOTS>
 __device__ __forceinline__ FindSeg find_tables(FindLds<THREADS, PAIRS, N, SLOTS>& F, const PlanSortArgs& pa,
                                                const void* const* w_ptrs, const int32_t* w_rank, int NA) {
   constexpr int kEnt = N / THREADS;  // table entries a thread holds: kEnt * tid ...
-  const int tid = threadIdx.x;
+  const int tid = turn_value<PAIRS>(threadIdx.x);
   int key = -1, s0 = 0, len = 0;
   uint64_t pair_a = 0, pair_b = 0;
   if (tid < pa.S) {
@@ -150,7 +157,7 @@ __device__ __forceinline__ FindSeg find_tables(FindLds<THREADS, PAIRS, N, SLOTS>
 template <int THREADS, int UT, bool PAIRS, int N, int SLOTS>
 __device__ __forceinline__ FoundUnit find_unit(FindLds<THREADS, PAIRS, N, SLOTS>& F, int NA, int unit) {
   constexpr int kEnt = N / THREADS;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = turn_value<PAIRS>(threadIdx.x), lane = tid & 63;
   auto units_of = [&](int a) -> uint32_t {
     return a < NA ? (uint32_t)((F.hist[a] + UT * kTileRows - 1) / (UT * kTileRows)) : 0u;
   };
@@ -221,7 +228,7 @@ __device__ __forceinline__ void find_rows(FindLds<THREADS, PAIRS, N, SLOTS>& F, 
   // every segment that reaches into the unit is written out by its whole wave, a lane a row (a long
   // segment fills the unit by itself: one lane writing 64 rows in turn is what this avoids)
   static_assert(UT * kTileRows <= kWaveSize, "a lane per row of the unit");
-  const int lane = threadIdx.x & 63;
+  const int tid = turn_value<PAIRS>(threadIdx.x), lane = tid & 63;
   uint64_t todo = __ballot(q0 < q1);
   while (todo) {  // uniform over the wave
     const int l = __builtin_ctzll(todo);
@@ -230,7 +237,7 @@ __device__ __forceinline__ void find_rows(FindLds<THREADS, PAIRS, N, SLOTS>& F, 
     const int r0 = __builtin_amdgcn_readlane(seg.s0 + (q0 - lo), l);
     if (b0 + lane < b1) {
       F.rows[b0 + lane - q_lo] = r0 + lane;
-      F.rseg[b0 + lane - q_lo] = (int)(threadIdx.x - lane) + l;
+      F.rseg[b0 + lane - q_lo] = (tid - lane) + l;
     }
   }
   __syncthreads();
@@ -263,7 +270,6 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   // x and the weights along the rows (LineTurn), but for sixteen waves a workgroup, two of which fill a CU: q/k/v/o of
   // 900 decoded rows at rank 16 32.4 us in the MFMA's layout, 35.2 along the rows
   constexpr bool kLines = HALVES == 1;
-  const int tid = threadIdx.x;
   if ((int)blockIdx.y == a.units) {  // the extra row of the grid: up to kSelfPlanBuilders workgroups build the plan
     const int part = (int)(blockIdx.z * gridDim.x + blockIdx.x), all = (int)(gridDim.x * gridDim.z);
     if (part < kSelfPlanBuilders) plan_small_body(a.plan, sm.plan, part, all < kSelfPlanBuilders ? all : kSelfPlanBuilders);
@@ -275,6 +281,14 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   if ((int)blockIdx.x * HALVES >= a.sh.items.row_start[pj + 1] - a.sh.items.row_start[pj]) return;
   const ShrinkProj P = a.sh.p[pj];
   FindLds<THREADS, PAIRS>& F = sm.find;
+  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
+
+  // PAIRS: the table has an entry per segment, and a row of workgroups for every tile the batch could have
+  // (one more per table entry) would be mostly idle ones.  The launch has a row for every tile such a batch
+  // usually has -- its rows in whole tiles plus a few dozen part-filled ones -- and a batch with more tiles
+  // sends its workgroups round again.  The other kind has a row per possible tile and takes one turn.
+  for (int tile = blockIdx.y;; tile += a.units) {
+  const int tid = turn_value<PAIRS>(threadIdx.x);
   const int wave_all = tid >> 6, lane = tid & 63;
   const int wave = wave_all % NW;           // wave within its group of eight
   const int yy = (int)blockIdx.x * HALVES + wave_all / NW;
@@ -283,13 +297,6 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   const int n0 = zb * 64;
   const int kbeg = (kz * NW + wave) * P.k_per_wave;
   const int kend = min(kbeg + P.k_per_wave, P.d_in);
-  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
-
-  // PAIRS: the table has an entry per segment, and a row of workgroups for every tile the batch could have
-  // (one more per table entry) would be mostly idle ones.  The launch has a row for every tile such a batch
-  // usually has -- its rows in whole tiles plus a few dozen part-filled ones -- and a batch with more tiles
-  // sends its workgroups round again.  The other kind has a row per possible tile and takes one turn.
-  for (int tile = blockIdx.y;; tile += a.units) {
   FindSeg seg;
   const FoundUnit un =
       find_adapter<THREADS, 1>(F, a.plan, P.w_ptrs, a.sh.plan.w_rank, a.n_weights, tile, &seg);
@@ -713,8 +720,10 @@ union SelfPlanBlockLds {
   char area[THREADS / kFwdThreads][BYTES];  // ... then the product's
 };
 
+// (Keyed by pairs at ranks 17 to 32 three waves a SIMD would spill: 2100 rows in 24 segments at rank 32, 4096 -> 4096,
+// 27.4 us with 136 bytes of spills a lane, 23.6 with 20, 23.1 with none at two waves.)
 template <int DT, int NB, bool WKN, int THREADS, bool PAIRS = false>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB))))
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PAIRS && NB == 2 ? 2 : block_product_waves(NB))))
 void shrink_block_self_planned_kernel(SelfPlanArgs a) {
   static_assert(THREADS == kFwdThreads || THREADS == 2 * kFwdThreads, "one or two groups of four waves");
   typedef BlockProduct<DT, NB, WKN> Product;
@@ -756,7 +765,7 @@ void shrink_block_self_planned_kernel(SelfPlanArgs a) {
     nlim = r8 < nlim ? r8 : nlim;
   }
   // the adapter is known: its first weights are requested while the rows are still being found
-  Product pr(a.sh, tl, wid, nlim, __builtin_amdgcn_readfirstlane(un.tiles), list, lists);
+  Product pr(a.sh, turn_value<PAIRS>(tl), wid, nlim, __builtin_amdgcn_readfirstlane(un.tiles), list, lists);
   typename Product::Stage first;
   if (!pr.exists(list)) pr.r = (int)blockIdx.x * GROUPS;  // (a second group without a row: multiplies, stores nothing)
   pr.open_w(GROUPS > 1 && pr.item(pr.r).pj != pj ? nullptr : W);

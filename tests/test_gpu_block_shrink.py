@@ -14,8 +14,9 @@ CASES = {
     # T, S, NA, widths, r, ranks of the adapters (None: all r)
     "rank8": (2100, 9, 3, [(264, 72), (2048, 64), (72, 136)], 8, None),
     "rank16-ks": (2100, 300, 5, [(1000, 64), (4104, 72)], 16, None),
-    "rank24": (800, 9, 3, [(328, 64), (64, 72), (8, 64)], 24, None),
-    "rank32-packed": (1500, 17, 4, [(1032, 72), (520, 264)], 32, [32, 8, 24, 16]),
+    "rank24": (2100, 9, 3, [(328, 64), (64, 72), (8, 64)], 24, None),
+    "rank24-wide": (800, 9, 3, [(328, 64), (64, 72), (8, 64)], 24, None),  # (too few rows: the other tile-block shrink)
+    "rank32-packed": (2200, 17, 4, [(1032, 72), (520, 264)], 32, [32, 8, 24, 16]),
     "rank40": (3100, 11, 3, [(2056, 64), (136, 72)], 40, None),
     "rank64": (3500, 400, 7, [(576, 64), (2048, 72)], 64, None),
     "rank64-packed": (3100, 40, 12, [(520, 72), (1096, 64)], 64, [8, 64, 40, 16, 24, 56, 32, 48, 8, 8, 64, 16]),
@@ -94,6 +95,35 @@ def test_inf_and_nan_stay_in_their_rows_and_columns(K, gpu_device, r):
     mid[70:3000] = True
     assert v[ok & ~mid].isfinite().all() and not v[~ok].isfinite().any()
     assert v[mid][:, 3].isnan().all() and v[mid][:, [0, 1, 2, 4, 5, 6, 7]].isfinite().all() and not v[mid][:, 8:].any()
+
+
+@pytest.mark.parametrize("S", [9, 300])
+@pytest.mark.parametrize("T,r,d_in", [(2100, 16, 520), (2100, 32, 72), (3100, 64, 520), (3100, 64, 2560)])
+def test_scale_and_beta(K, gpu_device, T, r, d_in, S):
+    """smlm_gemm: products of one slice store what they sum, scaled and added to beta y; the last one's slices are folded.
+    With the plan built in the launch and beforehand; whole numbers, so both are exact."""
+    from loquetier_amd import _lib as lib
+    d, NA = gpu_device, 4
+    g = torch.Generator().manual_seed(T + r)
+    whole = lambda *s: torch.randint(-2, 3, s, generator=g).half()
+    cut = [0] + sorted(int(c) for c in torch.randint(0, T - 5, (S - 1,), generator=g)) + [T - 5]
+    x, y0, W = whole(T, d_in), whole(T, r), [whole(r, d_in) for _ in range(NA)]
+    scale = torch.randint(1, 4, (S,), generator=g).float() / 2
+    want = y0.clone()
+    for i in range(S):
+        q = slice(cut[i], cut[i + 1])
+        want[q] = (0.5 * y0[q].double() + scale[i] * (x[q].double() @ W[i % NA].double().T)).half()
+    xd, Wd, sd = x.to(d), [w.to(d) for w in W], scale.to(d)
+    table, seg = ptrs([Wd[i % NA] for i in range(S)], d), torch.tensor(cut, dtype=torch.int32, device=d)
+    need = lib.size_query("smlm_gemm_workspace_size", T, S, d_in, r)
+    ws, got = torch.empty(need, dtype=torch.uint8, device=d), y0.to(d)
+    rc = lib.load().smlm_gemm(got.data_ptr(), xd.data_ptr(), table.data_ptr(), seg.data_ptr(), ws.data_ptr(), need, T, S,
+                              d_in, r, d_in, 0, lib.SMLM_DTYPE_F16, 0.5, sd.data_ptr(),
+                              torch.cuda.current_stream(d).cuda_stream)
+    assert rc == 0, lib.strerror(rc)
+    planned = y0.to(d)
+    K.smlm_gemm_planned(planned, xd, table, K.SegmentPlan(seg, None, T), seg_scale=sd, beta=0.5)
+    assert torch.equal(got.cpu(), want) and torch.equal(planned.cpu(), want)
 
 
 @pytest.mark.parametrize("S", [200, 300])

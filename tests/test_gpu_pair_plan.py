@@ -31,6 +31,16 @@ CASES = [
     ("tile-blocks-rank-200", [0, 700, 1100, 1101, 1500, 2300], [0, 1, 0, 1, 0], [2, 1, 2, 0, 2], 2048, 320, 200),
     ("tile-blocks-rank-128-300-segments", list(range(0, 1501, 5)), [i % 3 for i in range(300)], [i % 4 for i in range(300)],
      4096, 128, 128),
+    # tile blocks on the block shrink: a group of waves a workgroup and two, with an odd number of chunk rows for them, more
+    # tile blocks than the launch has rows of workgroups
+    ("block-shrink-rank-16", [0, 700, 1100, 1101, 1500, 2300], [0, 1, 0, 1, 0], [2, 1, 2, 0, 2], 2048, 128, 16),
+    ("block-shrink-rank-32-300-segments", list(range(0, 2401, 8)), [i % 3 for i in range(300)],
+     [i % 4 for i in range(300)], 1536, 128, 32),
+    ("block-shrink-rank-16-two-rounds", list(range(0, 2201, 11)), [i % 10 for i in range(200)],
+     [(i // 10) % 10 for i in range(200)], 2048, 128, 16),
+    ("block-shrink-rank-64", [0, 700, 1100, 1101, 1500, 3100], [0, 1, 0, 1, 0], [2, 1, 2, 0, 2], 1096, 64, 64),
+    ("block-shrink-rank-40-300-segments-two-rounds", list(range(0, 3301, 11)), [i % 12 for i in range(300)],
+     [(i // 12) % 11 for i in range(300)], 2560, 64, 40),
     ("1500-segments-two-launch-plan", list(range(1501)), [(i * 7) % 9 for i in range(1500)],
      [(i * 5) % 6 for i in range(1500)], 256, 128, 8),
 ]
