@@ -376,12 +376,27 @@ int launch_shrink(int dtype, const ShrinkCfg& c, int S, int groups, hipStream_t 
              : launch_shrink_dt<SMLM_DTYPE_BF16, false>(c.NB, MT, c.NW, grid, st, a);
 }
 
+// Whether the single-tile shrinks that build their plan request x and the weights along the rows, at up to 32 columns.
+// It pays where the segments are few: 4096 -> 4096, us, in the MFMA's layout / along the rows: one adapter in four
+// segments at rank 32, 64 rows 11.4 / 10.8, 700 rows 14.4 / 13.6; three projections, eight segments, 500 rows at rank 16
+// 18.0 / 17.2, at rank 32 22.9 / 21.1; 32 segments, 300 rows at rank 16 18.5 / 17.9; but 64 one-row segments 18.6 / 20.9,
+// 1400 rows in 256 segments at rank 16, one projection, 19.8 / 21.0.  Keyed by pairs, whose finder holds more registers:
+// one adapter in four segments, 300 rows at rank 32 13.2 / 12.5, 32 segments of 500 rows at rank 16 11.9 / 12.4, 192
+// segments of 700 rows at rank 32 17.8 / 19.0.  Wider shrinks gain at every number of segments; two workgroups of sixteen
+// waves fill a CU and lose (q/k/v/o of 900 decoded rows at rank 16 32.4 / 35.2).
+inline bool shrink_lines(int S, bool pairs) { return S <= (pairs ? 8 : 32); }
+
 template <int DT, int THREADS, bool PAIRS, bool DROP = false>
 int launch_self_planned_nb(int NB, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
   const dim3 block(THREADS);  // U must match shrink_cfg
-  if (NB == 1) return launch(shrink_self_planned_kernel<DT, 1, 4, THREADS, PAIRS, DROP>, grid, block, st, a);
-  if (NB == 2) return launch(shrink_self_planned_kernel<DT, 2, 4, THREADS, PAIRS, DROP>, grid, block, st, a);
-  return launch(shrink_self_planned_kernel<DT, 4, 2, THREADS, PAIRS, DROP>, grid, block, st, a);
+  constexpr bool kMay = THREADS == kSelfPlanThreads;
+  if (kMay && NB <= 2 && shrink_lines(a.plan.S, PAIRS)) {
+    if (NB == 1) return launch(shrink_self_planned_kernel<DT, 1, 4, THREADS, kMay, PAIRS, DROP>, grid, block, st, a);
+    return launch(shrink_self_planned_kernel<DT, 2, 4, THREADS, kMay, PAIRS, DROP>, grid, block, st, a);
+  }
+  if (NB == 1) return launch(shrink_self_planned_kernel<DT, 1, 4, THREADS, false, PAIRS, DROP>, grid, block, st, a);
+  if (NB == 2) return launch(shrink_self_planned_kernel<DT, 2, 4, THREADS, false, PAIRS, DROP>, grid, block, st, a);
+  return launch(shrink_self_planned_kernel<DT, 4, 2, THREADS, kMay, PAIRS, DROP>, grid, block, st, a);
 }
 
 template <int DT, bool WKN, int THREADS, bool PAIRS, bool DROP = false>

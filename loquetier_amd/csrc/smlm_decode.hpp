@@ -260,16 +260,14 @@ union SelfPlanLds {
 };
 
 // DROP (plans keyed by ids): dropout of the training rows of x, as shrink_kernel applies it.
-template <int DT, int NB, int U, int THREADS, bool PAIRS = false, bool DROP = false>
+// LINES: x and the weights are requested along the rows (LineTurn), otherwise as the MFMA wants them; same bits.
+template <int DT, int NB, int U, int THREADS, bool LINES, bool PAIRS = false, bool DROP = false>
 __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanArgs a) {
   static_assert(THREADS == kSelfPlanThreads || THREADS == 2 * kSelfPlanThreads, "one or two groups of eight waves");
   typedef LineTurn<U> Turn;
   __shared__ __attribute__((aligned(16))) SelfPlanLds<NB, U, THREADS, PAIRS> sm;
   constexpr int NW = kSelfPlanThreads / kWaveSize;  // waves that sum one k slice
   constexpr int HALVES = THREADS / kSelfPlanThreads;
-  // x and the weights along the rows (LineTurn), but for sixteen waves a workgroup, two of which fill a CU: q/k/v/o of
-  // 900 decoded rows at rank 16 32.4 us in the MFMA's layout, 35.2 along the rows
-  constexpr bool kLines = HALVES == 1;
   if ((int)blockIdx.y == a.units) {  // the extra row of the grid: up to kSelfPlanBuilders workgroups build the plan
     const int part = (int)(blockIdx.z * gridDim.x + blockIdx.x), all = (int)(gridDim.x * gridDim.z);
     if (part < kSelfPlanBuilders) plan_small_body(a.plan, sm.plan, part, all < kSelfPlanBuilders ? all : kSelfPlanBuilders);
@@ -309,8 +307,8 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
     nlim = r8 < nlim ? r8 : nlim;
   }
   // the adapter is known: its weights are requested while the rows are still being found
-  auto load_row = [&](int i) { return kLines ? Turn::row(lane, i) : c; };  // what load i of a lane brings
-  auto load_k = [&](int i) { return kLines ? 8 * Turn::piece(lane) : 32 * i + 8 * g; };
+  auto load_row = [&](int i) { return LINES ? Turn::row(lane, i) : c; };  // what load i of a lane brings
+  auto load_k = [&](int i) { return LINES ? 8 * Turn::piece(lane) : 32 * i + 8 * g; };
   auto load_w = [&](int k, u32x4 (&wf)[NB][U]) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
@@ -346,7 +344,7 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
       xf[i] = ldg16_or(P.x + (long)lrow[i] * P.d_in + kk, kk < kend && lrow[i] >= 0, zeros);
     }
     if (k != kbeg) load_w(k, wf);  // uniform over the wave (k is usually one batch)
-    if (kLines) {
+    if (LINES) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) Turn::turn(sm.wave[wave_all].turn, lane, wf[nb]);
       Turn::turn(sm.wave[wave_all].turn, lane, xf);
