@@ -112,15 +112,20 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
 
 // Which of the two tile-block shrinks: shrink_block_kernel, whose waves read x and the weights for themselves, or
 // shrink_wide_kernel, whose workgroups stage the weights once for four waves.  Shrink and fold, us, wide / block, h_in =
-// 4096: one projection at rank 16, 2048 rows 13.0 / 11.6, 3000 rows 13.5 / 12.7; three at rank 32, 1000 rows 16.3 / 14.9,
-// 3000 rows 30 / 26.3; at rank 64 1500 rows 21 / 24.0, 2048 rows 23.5 / 25.8, 3000 rows 36 / 36, 7675 rows 68 / 60.
+// 4096: one projection at rank 16, 2048 rows 13.0 / 11.6, 3000 rows 13.5 / 12.7; three at rank 32, 3000 rows 30 / 26.3; at
+// rank 64 1500 rows 21 / 24.0, 2048 rows 23.5 / 25.8, 3000 rows 36 / 36, 7675 rows 68 / 60.
 // Above rank 64 x would be read once for every 64 columns.
-// Below 1024 rows adapters have few rows each, and the block kernel reads 64 rows for however few: 867 rows over 48
-// adapters, three projections at rank 32, forward 15.6 / 19.4, backward (567 rows) 14.0 / 18.0.  Under dropout the
+// Fewer rows belong to adapters of few rows each, and the block kernel reads 64 rows for however few.  What it loses and
+// gains between 1024 and 2048 rows depends on that and on the number of projections, neither of which the rule may look
+// at.  Whole forwards at rank 32, three projections: 1024 rows over 64 adapters 42.5 / 46.0, over 24 32.0 / 34.4, over 4
+// 30.1 / 29.4, 1400 over 64 48.0 / 49.6; one: 1024 rows over 64 25.1 / 23.1, 1400 over 24 22.2 / 21.1; add_lora, 1300
+// rows over 64 28.9 / 34.3.  Backwards, three projections at rank 16, 1024 rows over 64 69.1 / 73.6.  From 2048 rows on,
+// over 4 to 64 adapters, no forward or backward was more than 1 % slower at rank 32 and below, most 2 to 10 % faster.
+// Under dropout the
 // generator keeps the vector units busy and the wide kernel's waves, more of them on a CU, share it better: 2436 rows, two
 // projections at rank 16 21.7 / 28.3.
 inline bool block_shrink(int mt, int T, int d_out, bool drop = false) {
-  return mt > 1 && !drop && T >= (d_out <= 32 ? 1024 : 3072) && d_out <= 64;
+  return mt > 1 && !drop && T >= (d_out <= 32 ? 2048 : 3072) && d_out <= 64;
 }
 // ... of a launch: its weight rows must be within the block kernel's reach too (the slices are the same either way).
 // Whoever decides on the plan's route asks this, as the launch does: the wide kernel needs the splits even where two
