@@ -120,7 +120,11 @@ SMLM_API int smlm_plan_build2(void* plan, size_t plan_bytes, const int32_t* seg_
  * the beta = 0, scale = 1 case.  w_ptrs[i] (device array of S device
  * addresses) is a d_in x d_out matrix: element (k, n) at w[k*w_ld + n] when
  * w_row_major, else at w[n*w_ld + k].  seg_scale: NULL or float [S] (device).
- * Builds its own plan (grouped by weight address) inside `workspace`.
+ * Groups the segments by weight address itself; what it leaves in `workspace`
+ * is for no other call (not every product builds a plan there).
+ * The size does not grow with T throughout (the split of k, and with it the
+ * partial sums, falls where more rows fill the chip): a buffer for several
+ * batch sizes must hold the largest of their sizes.
  * Rows outside every segment are not touched.
  */
 SMLM_API int smlm_gemm_workspace_size(int T, int S, int d_in, int d_out, size_t* bytes);
@@ -137,8 +141,8 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
  * without the workspace, same kernels, same results bit for bit; the plan and the
  * k-split partial sums live in an array of SMLM_STATIC_SCRATCH_BYTES that is part
  * of the library's code object (every GPU the library runs on holds its own copy
- * until the process ends).  Returns SMLM_ERR_SCRATCH when
- * smlm_gemm_workspace_size(T, S, d_in, d_out) exceeds that size.  Calls neither
+ * until the process ends).  Returns SMLM_ERR_SCRATCH when they do not fit (they
+ * do whenever smlm_gemm_workspace_size(T, S, d_in, d_out) does).  Calls neither
  * hipMalloc nor hipFree nor any allocating routine.  The first call on a device
  * looks the array's address up (hipGetSymbolAddress) and should be made outside a
  * capture.  All calls on one GPU share the array: calls that overlap on one GPU

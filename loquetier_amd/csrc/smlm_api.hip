@@ -250,14 +250,15 @@ inline bool shrink_wide(int mt, int d_out, bool w_kn, long wgs) {
   return mt > 1 && d_out > 64 && (w_kn ? wgs > 300 : wgs >= 180);
 }
 
-// most k-split partials a shrink of this shape can leave behind, whichever wave count it runs with
-int fwd_ksplit_bound(int T, int d_in, int d_out, bool plain = false) {
+// most k-split partials a shrink of this shape can leave behind, whichever wave count it runs with (`either`: and
+// whichever of the tile-block shrinks)
+int fwd_ksplit_bound(int T, int d_in, int d_out, bool plain = false, bool either = true) {
   int most = 1;
   for (int solo = 0; solo < 2; ++solo) {
     const int a = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, 1, plain).ksplit;
     const int b = shrink_cfg(T, d_in, d_out, kDecodeWaves, solo != 0, 1, plain).ksplit;
     const int c = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain).ksplit;
-    const int d = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain, !plain).ksplit;
+    const int d = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain, either).ksplit;
     most = a > most ? a : most;
     most = b > most ? b : most;
     most = c > most ? c : most;
@@ -903,15 +904,18 @@ SMLM_API int smlm_plan_build2(void* plan, size_t plan_bytes, const int32_t* seg_
   return plan_build_impl(pv, seg_indptr, seg_key_a, SMLM_KEY_PTR2, S, (hipStream_t)stream, seg_key_b);
 }
 
+// Scratch of one product: what it uses, or (`asked`) what the queries say.  They count both tile-block shrinks: from the
+// row number on at which the block kernel takes over, with fewer slices, a size would otherwise fall to less than half,
+// below what fewer rows use, and a buffer sized for the largest batch alone would be refused for a smaller one.
+static size_t gemm_scratch(int T, int d_in, int d_out, bool asked) {
+  const int ks = d_in >= d_out ? fwd_ksplit_bound(T, d_in, d_out, true, asked) : 1;
+  return ks > 1 ? align_up((size_t)ks * T * d_out * 4, 256) : 256;
+}
+
 SMLM_API int smlm_gemm_planned_workspace_size(int T, int d_in, int d_out, size_t* bytes) {
   if (T < 0 || d_in <= 0 || d_out <= 0 || !bytes) return SMLM_ERR_ARG;
   if (T > (1 << 30)) return SMLM_ERR_LIMIT;
-  size_t n = 256;
-  if (d_in >= d_out) {
-    const int ks = fwd_ksplit_bound(T, d_in, d_out, true);
-    if (ks > 1) n = align_up((size_t)ks * T * d_out * 4, 256);
-  }
-  *bytes = n;
+  *bytes = gemm_scratch(T, d_in, d_out, true);
   return SMLM_OK;
 }
 
@@ -928,10 +932,7 @@ SMLM_API int smlm_gemm_planned(void* y, const void* x, const void* const* w_ptrs
   if (!y || !x || !w_ptrs || !plan || !workspace) return SMLM_ERR_ARG;
   if (!aligned16(y) || !aligned16(x) || !aligned16(workspace) || !aligned16(plan))
     return SMLM_ERR_ALIGN;
-  size_t need = 0;
-  rc = smlm_gemm_planned_workspace_size(T, d_in, d_out, &need);
-  if (rc) return rc;
-  if (workspace_bytes < need) return SMLM_ERR_WORKSPACE;
+  if (workspace_bytes < gemm_scratch(T, d_in, d_out, false)) return SMLM_ERR_WORKSPACE;
 
   hipStream_t st = (hipStream_t)stream;
   PlanView pv;
@@ -988,14 +989,11 @@ SMLM_API int smlm_gemm(void* y, const void* x, const void* const* w_ptrs, const 
   if (T == 0 || S == 0) return SMLM_OK;
   if (!y || !x || !w_ptrs || !seg_indptr || !workspace) return SMLM_ERR_ARG;
   if (!aligned16(y) || !aligned16(x) || !aligned16(workspace)) return SMLM_ERR_ALIGN;
-  size_t need = 0;
-  rc = smlm_gemm_workspace_size(T, S, d_in, d_out, &need);
-  if (rc) return rc;
-  if (workspace_bytes < need) return SMLM_ERR_WORKSPACE;
-
-  hipStream_t st = (hipStream_t)stream;
   PlanView pv;
   const size_t plan_bytes = plan_carve(workspace, T, S, &pv);
+  if (workspace_bytes < plan_bytes + gemm_scratch(T, d_in, d_out, false)) return SMLM_ERR_WORKSPACE;
+
+  hipStream_t st = (hipStream_t)stream;
   // The plan groups the segments by their weight address.  A product that runs on the shrink kernels
   // (d_in >= d_out, weights [n][k]) over few enough segments builds it inside its own launch: every
   // workgroup numbers the addresses by their first occurrence and finds its tile itself, a few more
@@ -1040,9 +1038,8 @@ SMLM_API int smlm_gemm_static(void* y, const void* x, const void* const* w_ptrs,
   int rc = check_common(T, S, dtype);
   if (rc) return rc;
   if (d_in <= 0 || d_out <= 0) return SMLM_ERR_ARG;
-  size_t need = 0;
-  if ((rc = smlm_gemm_workspace_size(T, S, d_in, d_out, &need))) return rc;
-  if (need > SMLM_STATIC_SCRATCH_BYTES) return SMLM_ERR_SCRATCH;
+  if (plan_carve(nullptr, T, S, nullptr) + gemm_scratch(T, d_in, d_out, false) > SMLM_STATIC_SCRATCH_BYTES)
+    return SMLM_ERR_SCRATCH;
   // an empty batch launches nothing (smlm_gemm validates the rest and returns): no device needed
   void* ws = (T == 0 || S == 0) ? nullptr : static_scratch();
   if (!ws && T != 0 && S != 0) return SMLM_ERR_LAUNCH;

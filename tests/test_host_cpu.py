@@ -105,6 +105,15 @@ def test_products_wider_than_64_columns_fit_the_static_scratch(lib, T, d_in, d_o
     assert need <= lib.SMLM_STATIC_SCRATCH_BYTES
 
 
+@pytest.mark.parametrize("d_in,d_out,few,many", [(8192, 16, 2942, 3265), (11008, 8, 2170, 2340), (4096, 64, 2990, 3080),
+                                                 (14336, 32, 2040, 2060)])
+def test_scratch_of_the_larger_batch_serves_the_smaller(lib, d_in, d_out, few, many):
+    """... where the tile-block shrinks of plain products change over, to fewer slices of k."""
+    for query in (("smlm_gemm_workspace_size", 16), ("smlm_gemm_planned_workspace_size",)):
+        size = lambda T: lib.size_query(query[0], T, *query[1:], d_in, d_out)
+        assert size(few) <= size(many)
+
+
 def test_plan_on_first_use_argument_validation(lib):
     """smlm_lora_opts.build_seg_indptr / build_seg_adapter: both or neither, and only with the shrink stage."""
     L = lib.load()
