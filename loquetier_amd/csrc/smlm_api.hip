@@ -145,15 +145,17 @@ inline bool block_shrink(int mt, const ShrinkArgs& a) {
 // piece -- rounds of workgroups over the 256 CUs times (pieces of a slice + what starting one costs), an eighth more where
 // a CU has one workgroup only, the partial sums, and the fold, which costs as much as three pieces.  An uneven last
 // round is what costs most: 4096 rows, h_in = 11008 at rank 64, k in five 44.4 us, in four 30.4, in eight 33.6.
-// us with k in 1 / 2 / 4 / 8 / 16, one projection of h_in = 4096: 1024 rows at rank 64 - / - / - / 13.0 / 13.8; 2048
-// rows - / - / 15.2 / 14.7 / 18.1, at rank 128 - / 19.3 / 17.0 / 19.5 / 24.1; 4096 rows - / 20.0 / 17.3 / 19.1 / 24.6;
+// us with k in 1 / 2 / 4 / 8 / 16, one projection of h_in = 4096 at rank 64: 4096 rows - / 20.0 / 17.3 / 19.1 / 24.6;
 // 8192 rows 27.1 / 29.3 / 27.0 / 30.9, at rank 16 20.2 / 25.3 / 22.1 / 21.5.  From about 7000 rows on slices of up to
 // 4608 fill the chip without being split, and a launch of several projections has no use for more workgroups
-// (8192 rows over 64 adapters, six projections at rank 64: 127 / 142 / 146 us).
+// (8192 rows over 64 adapters, six projections at rank 64: 127 / 142 / 146 us); between 4096 and 8192 rows the line at
+// 112 units (7105 rows) is not measured.  The units are those of full tile blocks; with many adapters there are more, and a
+// split that just fills 256 workgroups runs over: 3200 rows over eight adapters, h_in = 11008 at rank 64, in five 51.7 us,
+// in four 39.8 -- but 4096 rows over 64 adapters in four 67.8, in three 78.0, so the count has no margin.
 // Never more slices than `most`, which what callers' scratch holds was sized for.  `solo`: the backward's products,
 // whose fold leaves by-products behind and is wanted for that.
 int block_pieces(int T, int d_in, int d_out, int most, bool solo) {
-  const int P = ceil_div(d_in, 256), units = ceil_div(T > 0 ? T : 1, kTileRows * kBlkTiles) * ceil_div(d_out, 64);
+  const int P = ceil_div(d_in, 256), units = ceil_div(T > 0 ? T : 1, kTileRows * kBlkTiles);
   if (most > kMaxKsplit) most = kMaxKsplit;
   if (units >= 112 && !solo) {
     const int ks = ceil_div(P, 18);
@@ -334,7 +336,6 @@ int shrink_lists(int T, int S, int groups, int rows, bool pairs = false) {
   }
   return best;
 }
-
 
 template <int DT, bool DIRECT>
 int launch_shrink_dt(int NB, int MT, int NW, dim3 grid, hipStream_t st,

@@ -42,9 +42,6 @@ struct SelfPlanArgs {
   int builder_rows;     // tile blocks up to rank 64: the plan builders are the first rows of the grid (blockIdx.y < builder_rows)
 };
 
-// sixteen zero bytes for predicated-off loads (the other kernels read the plan header's)
-__device__ __attribute__((aligned(16))) uint32_t self_plan_zeros[4];
-
 // ---- finding a unit of work (UT tiles of one adapter) without a plan ------------------------
 // PAIRS: the kernels built for plans keyed by pairs of addresses (SMLM_KEY_PTR2).  They are kernels of their
 // own because what they add costs the others dearly: the arrays below triple the finder's LDS, and their
@@ -279,7 +276,7 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
   if ((int)blockIdx.x * HALVES >= a.sh.items.row_start[pj + 1] - a.sh.items.row_start[pj]) return;
   const ShrinkProj P = a.sh.p[pj];
   FindLds<THREADS, PAIRS>& F = sm.find;
-  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
+  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(product_zeros);
 
   // PAIRS: the table has an entry per segment, and a row of workgroups for every tile the batch could have
   // (one more per table entry) would be mostly idle ones.  The launch has a row for every tile such a batch
@@ -436,7 +433,7 @@ void expand_found_kernel(FoundExpandArgs a) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
   const int mrow = 8 * (c >> 2) + (c & 3);  // column offset of MFMA row c inside a (q,p) block
-  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
+  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(product_zeros);
   constexpr int KSU = KS > 0 ? KS : 1;
 
   const FindSeg seg = find_tables<kFwdThreads, 1>(F, a.plan, P.w_ptrs, nullptr, a.plan.S);
@@ -582,7 +579,7 @@ __global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfP
   const int wave = tl >> 6, lane = threadIdx.x & 63;
   const int yy = (int)blockIdx.x * GROUPS + grp;
   const int c = lane & 15, g = lane >> 4;
-  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(self_plan_zeros);
+  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(product_zeros);
   const int kz = yy % P.ksplit, zb = yy / P.ksplit;
   const int n0 = zb * 16 * NB;  // (several column blocks only where NB = 4 or 8)
   const int kbeg = kz * kFwdWaves * P.k_per_wave;

@@ -210,6 +210,13 @@ struct ShrinkArgs {
   DropArgs drop;              // DROP kernels: dropout of the training rows of x
 };
 
+// a wave's own LDS accesses are served in order; the compiler must keep them in order too
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Sixteen rows of 32 * U of k on their way from memory to the MFMA.  They are requested along the rows, load i of a lane
 // piece `piece` of row `row(i)`, and change layout in an LDS area of the wave's own: afterwards register u of lane (c, g)
 // holds row c, k 32 u + 8 g .. + 7.  Requested in that layout, sixteen rows to sixteen neighbouring lanes, a load occupies
@@ -227,16 +234,10 @@ struct LineTurn {
     u32x4* a = reinterpret_cast<u32x4*>(lds);
 #pragma unroll
     for (int i = 0; i < U; ++i) a[at(row(lane, i), piece(lane))] = v[i];
-    order();
+    lds_order();
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = a[at(lane & 15, 4 * u + (lane >> 4))];
-    order();
-  }
-  // a wave's own LDS accesses are served in order; the compiler must keep them in order too
-  static __device__ __forceinline__ void order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    lds_order();
   }
 };
 
@@ -520,7 +521,8 @@ __global__ __launch_bounds__(kFwdThreads) void shrink_wide_kernel(ShrinkArgs a) 
 //
 // Slots without a row multiply the block's first row and columns at or past the adapter's rank another column's
 // weights: MFMA columns and rows do not mix, the former are not stored and the latter are stored as zeros.
-__device__ __attribute__((aligned(16))) uint32_t product_zeros[4];  // what loads past the end of a slice read
+__device__ __attribute__((aligned(16))) uint32_t product_zeros[4];  // what loads past the end of a slice read, and
+                                                                    // predicated-off ones of kernels without a plan
 
 constexpr int kBlockMaxLd = 1 << 25;  // longest weight row, in elements: a lane's offset in the weights has 32 bits
 
@@ -542,7 +544,7 @@ struct BlockProduct {
     int k0;
   };
   struct Item {  // (all uniform over the four waves)
-    int pj, kz, zb, kbeg, kend, n;  // n: pieces a wave takes
+    int pj, kz, kbeg, kend, n;  // n: pieces a wave takes
   };
 
   const ShrinkArgs& a;
@@ -558,7 +560,7 @@ struct BlockProduct {
   int r, s;
   Item li;
   const uint16_t *wbase, *xbase;
-  int d_in, ldw, ncols;      // ncols: columns of the block that have weights (a multiple of 8, may be 0 or less)
+  int d_in, ldw;
   uint32_t woff;             // the lane's byte offset in the weights (up to 31 rows: ldw <= kBlockMaxLd)
 
   __device__ __forceinline__ BlockProduct(const ShrinkArgs& args, int thread, int wid_, int nlim_, int tiles_, int list,
@@ -586,9 +588,8 @@ struct BlockProduct {
     it.pj = 0;
 #pragma unroll
     for (int i = 1; i < kMaxProj; ++i) it.pj += (i < a.items.nproj && row_ >= a.items.row_start[i]) ? 1 : 0;
-    const int yy = row_ - a.items.row_start[it.pj];
     const ShrinkProj& P = a.p[it.pj];
-    it.kz = yy / P.zblocks, it.zb = yy % P.zblocks;  // (the column blocks of a slice side by side: they read the same x)
+    it.kz = row_ - a.items.row_start[it.pj];
     it.kbeg = it.kz * kFwdWaves * P.k_per_wave;
     it.kend = min(it.kbeg + kFwdWaves * P.k_per_wave, P.d_in);
     it.n = (it.kend - it.kbeg + kFwdWaves * KB - 1) / (kFwdWaves * KB);
@@ -599,15 +600,13 @@ struct BlockProduct {
     li = item(r);
     const ShrinkProj& P = a.p[li.pj];
     if (!W) W = uload_ptr(P.w_ptrs, wid);
-    const int n0 = li.zb * 16 * NB;
     ldw = WKN ? rank_ld(a.plan, P.ldw, nlim) : P.ldw;  // [k][n] weights (B) have the rank contiguous
-    ncols = nlim - n0;
     if (WKN) {
-      wbase = W + n0;
+      wbase = W;
       const int n8 = (lane % (2 * NB)) * 8;
-      woff = ((uint32_t)(lane / (2 * NB)) * (uint32_t)ldw + (uint32_t)(n8 < ncols ? n8 : 0)) * 2u;
+      woff = ((uint32_t)(lane / (2 * NB)) * (uint32_t)ldw + (uint32_t)(n8 < nlim ? n8 : 0)) * 2u;
     } else {
-      wbase = W + (long)n0 * ldw;
+      wbase = W;
       woff = ((uint32_t)(lane >> 3) * (uint32_t)ldw + 8u * (lane & 7)) * 2u;
     }
     s = 0;
@@ -635,7 +634,7 @@ struct BlockProduct {
   __device__ __forceinline__ void load_w(Stage& st) {
     const int k0 = st.k0 = piece_k();
     const uint16_t* zeros = reinterpret_cast<const uint16_t*>(product_zeros);
-    const int kend = ncols > 0 ? li.kend : 0;  // (a block of which no column has weights)
+    const int kend = nlim > 0 ? li.kend : 0;  // (an adapter of rank 0 has no weights)
 #pragma unroll
     for (int j = 0; j < 2 * NB; ++j) {
       if (WKN) {
@@ -644,7 +643,7 @@ struct BlockProduct {
         st.w[j] = ldg16_or(p, kj + lane / (2 * NB) < kend, zeros);
       } else {
         const uint16_t* p = reinterpret_cast<const uint16_t*>(
-            reinterpret_cast<const char*>(wbase + (long)(8 * j < ncols ? 8 * j : 0) * ldw + k0) + woff);
+            reinterpret_cast<const char*>(wbase + (long)(8 * j < nlim ? 8 * j : 0) * ldw + k0) + woff);
         st.w[j] = ldg16_or(p, k0 + 8 * (lane & 7) < kend, zeros);
       }
     }
@@ -684,12 +683,6 @@ struct BlockProduct {
   }
   __device__ __forceinline__ u32x4 get(const char* lds, int u) const {
     return *reinterpret_cast<const u32x4*>(lds + c * (KB * 2) + (((4 * u + g) ^ ((c >> 1) & 7)) << 4));
-  }
-  // a wave's own LDS accesses are served in order; the compiler must keep them in order too
-  static __device__ __forceinline__ void lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   __device__ __forceinline__ void multiply(const Stage& st, char* lds) {
     uint16_t* wl = reinterpret_cast<uint16_t*>(lds);
@@ -741,7 +734,6 @@ struct BlockProduct {
     f32x4(*red)[kBlkTiles][NB][kWaveSize] = reinterpret_cast<f32x4(*)[kBlkTiles][NB][kWaveSize]>(smem);
     const ShrinkProj& P = a.p[it.pj];
     const bool as_partial = P.ksplit > 1 || P.to_partial;
-    const int n0 = it.zb * 16 * NB;
     __syncthreads();  // every wave is done with the area
 #pragma unroll
     for (int t = 0; t < kBlkTiles; ++t)
@@ -760,7 +752,7 @@ struct BlockProduct {
         f32x4 sum = part[0];
 #pragma unroll
         for (int w = 1; w < kFwdWaves; ++w) sum += part[w];
-        const int n = n0 + 16 * nb + 4 * g;  // lane holds columns n .. n+3 of its token
+        const int n = 16 * nb + 4 * g;  // lane holds columns n .. n+3 of its token
         if (n >= P.d_out) continue;
         if (n >= nlim) sum = f32x4{0.f, 0.f, 0.f, 0.f};
         if (as_partial)
@@ -804,7 +796,7 @@ struct BlockProduct {
 };
 
 // Shrink for tile blocks (larger batches, and the backward).  Grid (lists, tile blocks): a workgroup takes the chunk rows
-// (projection, k slice, column block of 16 * NB) blockIdx.x, blockIdx.x + gridDim.x ... of its tile block.
+// (projection, k slice) blockIdx.x, blockIdx.x + gridDim.x ... of its tile block; NB blocks of 16 columns hold the rank.
 template <int DT, int NB, bool WKN>
 __global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB))))
 void shrink_block_kernel(ShrinkArgs a) {
