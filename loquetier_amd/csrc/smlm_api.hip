@@ -163,10 +163,10 @@ int block_pieces(int T, int d_in, int d_out, int most, bool solo) {
   }
   int best = P;
   float least = 0.0f;
-  for (int m = P; m >= 1; --m) {
-    const int ks = ceil_div(P, m);
+  for (int want = 1; want <= most && want <= P; ++want) {
+    const int m = ceil_div(P, want), ks = ceil_div(P, m);
     const long wgs = (long)units * ks;
-    if (ks > most || (ks > 2 && wgs > 512) || (solo && ks == 1 && P > 1 && most > 1)) continue;
+    if ((ks > 2 && wgs > 512) || (solo && ks == 1 && P > 1 && most > 1)) continue;
     const float cost = (wgs + 255) / 256 * (m + 0.3f) * (wgs <= 256 ? 1.12f : 1.0f) + (0.1f + d_out / 160.0f) * ks + (ks > 1 ? 3.0f : 0.0f);
     if (least == 0.0f || cost < least) least = cost, best = m;
   }
@@ -255,16 +255,13 @@ inline bool shrink_wide(int mt, int d_out, bool w_kn, long wgs) {
 // most k-split partials a shrink of this shape can leave behind, whichever wave count it runs with (`either`: and
 // whichever of the tile-block shrinks)
 int fwd_ksplit_bound(int T, int d_in, int d_out, bool plain = false, bool either = true) {
-  int most = 1;
+  const bool two = either && block_shrink(kBlkTiles, T, d_out);
+  int most = shrink_cfg(T, d_in, d_out, kFwdWaves, false, 1, plain).ksplit;
+  auto also = [&](int ks) { most = ks > most ? ks : most; };
+  also(shrink_cfg(T, d_in, d_out, kDecodeWaves, false, 1, plain).ksplit);
   for (int solo = 0; solo < 2; ++solo) {
-    const int a = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, 1, plain).ksplit;
-    const int b = shrink_cfg(T, d_in, d_out, kDecodeWaves, solo != 0, 1, plain).ksplit;
-    const int c = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain).ksplit;
-    const int d = shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain, either).ksplit;
-    most = a > most ? a : most;
-    most = b > most ? b : most;
-    most = c > most ? c : most;
-    most = d > most ? d : most;
+    also(shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain).ksplit);
+    if (two) also(shrink_cfg(T, d_in, d_out, kFwdWaves, solo != 0, kBlkTiles, plain, true).ksplit);
   }
   return most;
 }
