@@ -119,13 +119,14 @@ int shrink_waves(int mt, int nproj, const int* d_in, int d_out) {
 // gains between 1024 and 2048 rows depends on that and on the number of projections, neither of which the rule may look
 // at.  Whole forwards at rank 32, three projections: 1024 rows over 64 adapters 42.5 / 46.0, over 24 32.0 / 34.4, over 4
 // 30.1 / 29.4, 1400 over 64 48.0 / 49.6; one: 1024 rows over 64 25.1 / 23.1, 1400 over 24 22.2 / 21.1; add_lora, 1300
-// rows over 64 28.9 / 34.3.  Backwards, three projections at rank 16, 1024 rows over 64 69.1 / 73.6.  From 2048 rows on,
-// over 4 to 64 adapters, no forward or backward was more than 1 % slower at rank 32 and below, most 2 to 10 % faster.
+// rows over 64 28.9 / 34.3.  Backwards, three projections at rank 16, 1024 rows over 64 69.1 / 73.6.  At ranks 17 to 32 it
+// goes on to 3072 rows: 4096 -> 11008 twice and back, 2112 rows, the whole pass 79.7 / 81.5; two projections, 2048 rows
+// over 100 47.9 / 50.3; 3072 rows over 4 to 64, three projections, 59.9 to 74.3 / 54.2 to 69.2.
 // Under dropout the
 // generator keeps the vector units busy and the wide kernel's waves, more of them on a CU, share it better: 2436 rows, two
 // projections at rank 16 21.7 / 28.3.
 inline bool block_shrink(int mt, int T, int d_out, bool drop = false) {
-  return mt > 1 && !drop && T >= (d_out <= 32 ? 2048 : 3072) && d_out <= 64;
+  return mt > 1 && !drop && T >= (d_out <= 16 ? 2048 : 3072) && d_out <= 64;
 }
 // ... of a launch: its weight rows must be within the block kernel's reach too (the slices are the same either way).
 // Whoever decides on the plan's route asks this, as the launch does: the wide kernel needs the splits even where two

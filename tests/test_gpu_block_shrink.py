@@ -14,9 +14,9 @@ CASES = {
     # T, S, NA, widths, r, ranks of the adapters (None: all r)
     "rank8": (2100, 9, 3, [(264, 72), (2048, 64), (72, 136)], 8, None),
     "rank16-ks": (2100, 300, 5, [(1000, 64), (4104, 72)], 16, None),
-    "rank24": (2100, 9, 3, [(328, 64), (64, 72), (8, 64)], 24, None),
+    "rank24": (3100, 9, 3, [(328, 64), (64, 72), (8, 64)], 24, None),
     "rank24-wide": (800, 9, 3, [(328, 64), (64, 72), (8, 64)], 24, None),  # (too few rows: the other tile-block shrink)
-    "rank32-packed": (2200, 17, 4, [(1032, 72), (520, 264)], 32, [32, 8, 24, 16]),
+    "rank32-packed": (3100, 17, 4, [(1032, 72), (520, 264)], 32, [32, 8, 24, 16]),
     "rank40": (3100, 11, 3, [(2056, 64), (136, 72)], 40, None),
     "rank64": (3500, 400, 7, [(576, 64), (2048, 72)], 64, None),
     "rank64-packed": (3100, 40, 12, [(520, 72), (1096, 64)], 64, [8, 64, 40, 16, 24, 56, 32, 48, 8, 8, 64, 16]),
@@ -98,7 +98,7 @@ def test_inf_and_nan_stay_in_their_rows_and_columns(K, gpu_device, r):
 
 
 @pytest.mark.parametrize("S", [9, 300])
-@pytest.mark.parametrize("T,r,d_in", [(2100, 16, 520), (2100, 32, 72), (3100, 64, 520), (3100, 64, 2560)])
+@pytest.mark.parametrize("T,r,d_in", [(2100, 16, 520), (3100, 32, 72), (3100, 64, 520), (3100, 64, 2560)])
 def test_scale_and_beta(K, gpu_device, T, r, d_in, S):
     """smlm_gemm: products of one slice store what they sum, scaled and added to beta y; the last one's slices are folded.
     With the plan built in the launch and beforehand; whole numbers, so both are exact."""

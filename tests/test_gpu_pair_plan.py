@@ -34,7 +34,7 @@ CASES = [
     # tile blocks on the block shrink: a group of waves a workgroup and two, with an odd number of chunk rows for them, more
     # tile blocks than the launch has rows of workgroups
     ("block-shrink-rank-16", [0, 700, 1100, 1101, 1500, 2300], [0, 1, 0, 1, 0], [2, 1, 2, 0, 2], 2048, 128, 16),
-    ("block-shrink-rank-32-300-segments", list(range(0, 2401, 8)), [i % 3 for i in range(300)],
+    ("block-shrink-rank-32-300-segments", list(range(0, 3301, 11)), [i % 3 for i in range(300)],
      [i % 4 for i in range(300)], 1536, 128, 32),
     ("block-shrink-rank-16-two-rounds", list(range(0, 2201, 11)), [i % 10 for i in range(200)],
      [(i // 10) % 10 for i in range(200)], 2048, 128, 16),
