@@ -423,7 +423,7 @@ template <int DT, bool WKN, bool PAIRS, bool DROP = false>
 int launch_self_planned_block(int NB, int S, dim3 grid, hipStream_t st, const SelfPlanArgs& a) {
   if (S <= kFwdThreads) return launch_self_planned_block_nb<DT, WKN, kFwdThreads, PAIRS, DROP>(NB, grid, st, a);
   // more segments than the four-wave workgroup has threads: two such groups a workgroup, each taking a list of chunk
-  // rows or (ranks above 64) one of two neighbouring k slices (the caller has checked that the splits are even)
+  // rows or (the wide kernel) one of two neighbouring k slices (the caller has checked that the splits are even)
   grid.x = (grid.x + 1) / 2;
   return launch_self_planned_block_nb<DT, WKN, 2 * kFwdThreads, PAIRS, DROP>(NB, grid, st, a);
 }

@@ -39,7 +39,7 @@ struct SelfPlanArgs {
   PlanSortArgs plan;    // what the extra workgroups build; key_kind = SMLM_KEY_I32
   int n_weights;
   int units;            // unit bound; single tiles, wide tile blocks: workgroups with blockIdx.y == units are the plan builders
-  int builder_rows;     // tile blocks up to rank 64: the plan builders are the first rows of the grid (blockIdx.y < builder_rows)
+  int builder_rows;     // block shrinks: the plan builders are the first rows of the grid (blockIdx.y < builder_rows)
 };
 
 // ---- finding a unit of work (UT tiles of one adapter) without a plan ------------------------
@@ -535,7 +535,7 @@ void expand_found_kernel(FoundExpandArgs a) {
   }
 }
 
-// ---- larger batches at ranks above 64: shrink_wide_kernel ----------------------------
+// ---- larger batches: shrink_wide_kernel ------------------------------------------------
 // WKN: the weights are stored [k][n], as B is for the backward's dV = dY B.
 // THREADS = 256: a workgroup is the four waves of shrink_wide_kernel and takes one k slice of its
 // tile block.  THREADS = 512 (more than 256 segments; finder and plan builders hold a segment per
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfP
   }
 }
 
-// ---- larger batches: shrink_block_kernel -------------------------------------------
+// ---- larger batches where block_shrink() says so: shrink_block_kernel ---------------------
 // WKN: the weights are stored [k][n], as B is for the backward's dV = dY B.
 // THREADS = 256: a workgroup is the four waves of shrink_block_kernel and takes one k slice of its
 // tile block.  THREADS = 512 (more than 256 segments; finder and plan builders hold a segment per

@@ -220,7 +220,7 @@ __device__ __forceinline__ void lds_order() {
 // Sixteen rows of 32 * U of k on their way from memory to the MFMA.  They are requested along the rows, load i of a lane
 // piece `piece` of row `row(i)`, and change layout in an LDS area of the wave's own: afterwards register u of lane (c, g)
 // holds row c, k 32 u + 8 g .. + 7.  Requested in that layout, sixteen rows to sixteen neighbouring lanes, a load occupies
-// the CU's address unit for 65 cycles instead of 18.
+// the CU's address unit for 64 cycles instead of 19.
 template <int U>
 struct LineTurn {
   static constexpr int kRow = 4 * U;  // 16-byte pieces of a row
@@ -359,8 +359,8 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
   }
 }
 
-// Shrink for tile blocks (larger batches, and the backward) at ranks above 64.  Work item -> (projection, k
-// slice, column block of 16 * NB, tile block) as above, but here wave w owns tile w of the block
+// Shrink for tile blocks (larger batches, and the backward) where block_shrink() does not choose the other kernel.  Work
+// item -> (projection, k slice, column block of 16 * NB, tile block) as above, but here wave w owns tile w of the block
 // and all four waves walk the whole k slice together: each 32*U-wide batch of the weight
 // rows is staged once in LDS (two buffers in turn, one barrier a batch) and shared by the
 // four tiles, while every wave loads the x fragments of its own tile straight into
@@ -508,7 +508,7 @@ __global__ __launch_bounds__(kFwdThreads) void shrink_wide_kernel(ShrinkArgs a) 
 //
 // x and the weights are requested in full lines, eight lanes to 128 bytes of a row, and change layout through an LDS area
 // of the wave's own.  Requested as the MFMA wants them, sixteen rows to the sixteen neighbouring lanes, a load occupies
-// the CU's address unit for 65 cycles instead of 18 (measured with data out of L2), which alone holds x and the weights
+// the CU's address unit for 64 cycles instead of 19 (measured with data out of L2), which alone holds x and the weights
 // together to 9.4 TB/s.
 //
 // Bound by HBM and by what surrounds it: 7675 rows, three projections 4096 -> 64: 59.4 us with the weights staged for
@@ -795,7 +795,7 @@ struct BlockProduct {
   }
 };
 
-// Shrink for tile blocks (larger batches, and the backward).  Grid (lists, tile blocks): a workgroup takes the chunk rows
+// Shrink for tile blocks where block_shrink() chooses it.  Grid (lists, tile blocks): a workgroup takes the chunk rows
 // (projection, k slice) blockIdx.x, blockIdx.x + gridDim.x ... of its tile block; NB blocks of 16 columns hold the rank.
 template <int DT, int NB, bool WKN>
 __global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(block_product_waves(NB))))
