@@ -42,26 +42,20 @@ struct DropRow {
   bool on;
 };
 
-// threshold and factor of dropout probability p (p <= 0: off)
+// threshold and factor of dropout probability p (p <= 0: off, thresh 0 and factor 1)
 __device__ __forceinline__ DropRow drop_params(float p) {
-  DropRow r{0u, 1.0f, false};
-  if (p > 0.0f) {
-    r.on = true;
-    r.thresh = p >= 1.0f ? 65536u : (uint32_t)(p * 65536.0f);
-    r.scale = p >= 1.0f ? 0.0f : 1.0f / (1.0f - p);
-  }
+  DropRow r;
+  r.on = p > 0.0f;
+  r.thresh = p >= 1.0f ? 65536u : (r.on ? (uint32_t)(p * 65536.0f) : 0u);
+  r.scale = p >= 1.0f ? 0.0f : (r.on ? 1.0f / (1.0f - p) : 1.0f);
   return r;
 }
 
-// the dropout parameters of a row of segment `seg`; only looked up for training rows
-__device__ __forceinline__ DropRow drop_row_of(const DropArgs& d, int row, int seg) {
-  if (row >= 0 && row < d.rows) return drop_params(d.seg_p[seg]);
-  return DropRow{0u, 1.0f, false};
-}
-// the same, with the row's segment in the plan's table
-__device__ __forceinline__ DropRow drop_row(const DropArgs& d, int row, const int32_t* seg_of_slot, int slot) {
-  if (row >= 0 && row < d.rows) return drop_params(d.seg_p[seg_of_slot[slot]]);
-  return DropRow{0u, 1.0f, false};
+// The dropout probability of a row of segment `seg` (either -1: none), 0 for rows that are not training rows.  A load
+// without a branch, so that the loads behind it need not wait for it (zero: readable, holds 0.0f).
+__device__ __forceinline__ float drop_prob(const DropArgs& d, int row, int seg, const uint16_t* zero) {
+  const bool ok = row >= 0 && row < d.rows && seg >= 0;
+  return *(const SMLM_GLOBAL float*)(ok ? d.seg_p + seg : reinterpret_cast<const float*>(zero));
 }
 
 __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
@@ -86,41 +80,33 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
 
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-// The mask of the eight elements at columns 8*colblk .. +7 of a row, two to a word as the elements are: 0xffff in
-// the half of a kept element, 0 in a dropped one's.  Two elements an instruction: thresh - piece, saturating at
-// zero, is nonzero exactly where the piece is below thresh.  A thresh of 65536 (p >= 1) does not fit a half: the
-// caller's last AND, with drop_none_kept, takes what is left.
-// Under dropout the shrink kernels issue six times the vector instructions they issue without it, nearly all of them
-// the generator and the mask.  With a compare and two selects an element and two exclusive ors a generator word:
-// forward + backward of 2786 rows, 2754 of them dropped, two projections 4096 -> 4096 and 1024 at rank 32, 117.1 us;
-// so: 116.0 us.
-__device__ __forceinline__ u32x4 drop_mask8(const DropArgs& d, uint32_t thresh, int row, int colblk) {
+// Which of the eight elements at columns 8*colblk .. +7 of a row are kept, two to a word as the elements are: 1 in the half
+// of a kept element, 0 in a dropped one's.  Two elements an instruction: thresh - piece, saturating at zero, is nonzero
+// exactly where the piece is below thresh.  A thresh of 65536 (p >= 1) does not fit a half: the caller's last AND, with
+// drop_none_kept, takes what is left.
+__device__ __forceinline__ u32x4 drop_keep_pairs(const DropArgs& d, uint32_t thresh, int row, int colblk) {
   uint32_t w[4];
   philox4x32_10((uint32_t)row, (uint32_t)colblk, d.o0, d.o1, d.k0, d.k1, w);
   const uint16_t t16 = (uint16_t)(thresh < 65535u ? thresh : 65535u);
   uint32_t ones = 0x00010001u;
   asm("" : "+s"(ones));  // (knowing the value, the compiler turns this back into compares and selects, an element each)
   const u16x2 t = {t16, t16}, one = __builtin_bit_cast(u16x2, ones);
-  u32x4 m;
+  u32x4 k;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const u16x2 below = __builtin_elementwise_min(__builtin_elementwise_sub_sat(t, __builtin_bit_cast(u16x2, w[e])), one);
-    m[e] = __builtin_bit_cast(uint32_t, (u16x2)(below - one));
-  }
-  return m;
+  for (int e = 0; e < 4; ++e)
+    k[e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(
+                                            one, __builtin_elementwise_sub_sat(t, __builtin_bit_cast(u16x2, w[e]))));
+  return k;
 }
 __device__ __forceinline__ uint32_t drop_none_kept(uint32_t thresh) { return thresh > 65535u ? 0u : ~0u; }
 
-// the same mask as keep bits: bit e = element e is kept
-__device__ __forceinline__ uint32_t mask_bits8(u32x4 m, uint32_t limit) {
-  uint32_t b = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) b |= m[e] & ((1u << (2 * e)) | (2u << (2 * e + 16)));
-  b &= limit;
-  return (b | (b >> 16)) & 0xffu;
+// the same as keep bits: bit e = element e is kept
+__device__ __forceinline__ uint32_t keep_bits8(u32x4 k, uint32_t limit) {
+  const uint32_t b = k[0] | (k[1] << 2) | (k[2] << 4) | (k[3] << 6);
+  return (b | (b >> 15)) & 0xffu & limit;
 }
 __device__ __forceinline__ uint32_t drop_keep8(const DropArgs& d, uint32_t thresh, int row, int colblk) {
-  return mask_bits8(drop_mask8(d, thresh, row, colblk), drop_none_kept(thresh));
+  return keep_bits8(drop_keep_pairs(d, thresh, row, colblk), drop_none_kept(thresh));
 }
 
 // kept elements times the factor (float product, rounded to the 16-bit type), dropped ones +0
@@ -136,23 +122,78 @@ __device__ __forceinline__ u32x4 drop_apply8(u32x4 v, uint32_t keep, float scale
   return o;
 }
 
-// Eight consecutive elements of one row (columns 8*colblk .. +7), packed two to a word.
-// bits_out (may be nullptr): the row's keep bits, one byte per eight columns, are left there
-// for a later pass that reads them instead of running the generator again (write != false
-// selects the lanes that own the byte).
-template <int DT>
-__device__ __forceinline__ u32x4 drop8(u32x4 v, const DropArgs& d, const DropRow& r, int row, int colblk,
-                                       uint8_t* bits_out = nullptr, long bits_pitch = 0, bool write = false) {
-  if (__builtin_amdgcn_ballot_w64(r.on) == 0) return v;  // uniform over the wave
-  const u32x4 m = drop_mask8(d, r.thresh, row, colblk);
-  const uint32_t limit = drop_none_kept(r.thresh);
-  if (bits_out && write && r.on) bits_out[(long)row * bits_pitch + colblk] = (uint8_t)mask_bits8(m, limit);
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = pack2<DT>(Num<DT>::lo(v[e]) * r.scale, Num<DT>::hi(v[e]) * r.scale) & m[e] & limit;
-  return r.on ? o : v;
+// Whether a projection's keep bits can be stored U (2 or 4) bytes at a time: rows and addresses in multiples of U.
+template <int U>
+__device__ __forceinline__ bool drop_words(const uint8_t* bits, long pitch) {
+  return ((reinterpret_cast<uintptr_t>(bits) | (uintptr_t)pitch) & (U - 1)) == 0;
 }
+
+// The masks of U x-fragments of a wave, lane (c, g) holding columns 8 (colblk0 + 4 u + g) .. +7 of row c in fragment u.
+// They need nothing of x: the shrink kernels make them while x is on its way, U generators side by side, whose ten rounds
+// each wait for the one before.  One generator at a time behind x's arrival, a byte stored for each, and so, us: forward
+// of 2786 rows, two projections 4096 -> 4096 at rank 32 50.5 and 47.1, 900 rows 27.1 and 25.9, 8000 rows at rank 16 108.2
+// and 96.6 (without dropout 83).  Most of that is the stores: rows of the mask that only take single bytes gain nothing.
+template <int U>
+struct DropMasks {
+  u32x4 m[U];  // 0xffff in the half of a kept element, 0 in a dropped one's
+
+  // bits_out (may be nullptr): the row's keep bits, one byte per eight columns, are left there for a later pass that reads
+  // them instead of running the generator again; blocks at or past colblk_end are not.  words: drop_words<U> of them; the
+  // bytes of a row then go out U from each of its four lanes instead of one at a time.
+  __device__ __forceinline__ void make(const DropArgs& d, const DropRow& r, int row, int colblk0, int g, uint8_t* bits_out,
+                                       long pitch, int colblk_end, bool words) {
+    const uint32_t limit = drop_none_kept(r.thresh);
+    uint32_t b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const u32x4 k = drop_keep_pairs(d, r.thresh, row, colblk0 + 4 * u + g);
+      b[u] = keep_bits8(k, limit);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t ke = k[e];  // (a vector's element cast in place reads element 0: clang)
+        m[u][e] = __builtin_bit_cast(uint32_t, (u16x2)(u16x2{0, 0} - __builtin_bit_cast(u16x2, ke)));
+      }
+    }
+    if (!bits_out) return;  // uniform over the wave
+    uint8_t* const at = bits_out + (long)row * pitch + colblk0;
+    static_assert(U == 2 || U == 4, "");
+    if (words) {  // uniform over the wave
+      // lane g holds bytes 4 u + g of the row's 4 U and stores bytes U g + j
+      if constexpr (U == 4) {  // halves change places with the lane two groups away, then bytes with the lane next door
+        const uint32_t w = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
+        const auto h = __builtin_amdgcn_permlane32_swap(w, w, false, false);  // the words of groups g & 1 and (g & 1) + 2
+        const uint32_t v = __builtin_amdgcn_perm(h[1], h[0], g & 2 ? 0x07060302u : 0x05040100u);
+        const auto q = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // ... of the even and the odd group
+        const uint32_t o = __builtin_amdgcn_perm(q[1], q[0], g & 1 ? 0x07030501u : 0x06020400u);
+        if (r.on && colblk0 + 4 * g < colblk_end) *(SMLM_GLOBAL uint32_t*)(at + 4 * g) = o;
+      } else {  // the pairs of neighbours together, then the pair and the fragment the lane stores
+        const uint32_t w = b[0] | (b[1] << 8);
+        const auto q = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+        const uint32_t v = __builtin_amdgcn_perm(q[1], q[0], 0x05010400u);
+        const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // of pairs 0 and 1
+        const uint32_t o = (g & 1 ? h[1] : h[0]) >> (g & 2 ? 16 : 0);
+        if (r.on && colblk0 + 2 * g < colblk_end) *(SMLM_GLOBAL uint16_t*)(at + 2 * g) = (uint16_t)o;
+      }
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (r.on && colblk0 + 4 * u + g < colblk_end) *(SMLM_GLOBAL uint8_t*)(at + 4 * u + g) = (uint8_t)b[u];
+  }
+
+  // fragment u of x: kept elements times the factor (float product, rounded to the 16-bit type), dropped ones +0.  Rows
+  // that are not dropped have thresh 0 and factor 1: the product is the element.
+  template <int DT>
+  __device__ __forceinline__ u32x4 apply(u32x4 v, int u, const DropRow& r) const {
+    const uint32_t limit = drop_none_kept(r.thresh);
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = __builtin_amdgcn_bitop3_b32(pack2<DT>(Num<DT>::lo(v[e]) * r.scale, Num<DT>::hi(v[e]) * r.scale), m[u][e],
+                                         limit, 0x80);  // (three-way and)
+    return o;
+  }
+};
 
 // the same from stored keep bits
 template <int DT>
@@ -176,7 +217,7 @@ __global__ __launch_bounds__(256) void drop_bits_kernel(DropBitsArgs a) {
   if (tile >= a.hdr[0]) return;
   const int slot = tile * kTileRows + (threadIdx.x >> 4);
   const int row = a.tile_row[slot];
-  const DropRow r = drop_row(a.drop, row, a.tile_rseg, slot);
+  const DropRow r = drop_params(drop_prob(a.drop, row, a.tile_rseg[slot], reinterpret_cast<const uint16_t*>(a.hdr + kHdrZeros)));
   if (!r.on) return;  // rows that are not dropped never have their byte read
   for (int cb = threadIdx.x & 15; cb < a.drop.bits_pitch; cb += 16)
     a.drop.bits[(long)row * a.drop.bits_pitch + cb] = (uint8_t)drop_keep8(a.drop, r.thresh, row, cb);

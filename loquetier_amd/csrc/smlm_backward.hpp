@@ -184,13 +184,6 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
       }
   };
 
-  DropRow dr{0u, 1.0f, false};  // uniform over the workgroup; .on is set per row below
-  bool drop_on = false;
-  if (DROP && seg0 >= 0) {
-    dr = drop_params(a.drop.seg_p[seg0]);
-    drop_on = dr.on;
-  }
-
   // the first step of the first chunk
   const int32_t row_first = load_rows(wave);  // the rows of the wave's first step: every chunk starts with them
   uint32_t keep[DROP ? 8 : 1];  // bit 8 set: the row is not dropped
@@ -198,6 +191,10 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   load_data(row_first, chunk_first * kWgCols, val, keep);
   load_p(wave, pf);
   int32_t row_next = load_rows(wave + kWgWaves);
+
+  // uniform over the workgroup, whose rows belong to one adapter; .on is set per row below
+  DropRow dr = drop_params(DROP && seg0 >= 0 ? uload(a.drop.seg_p, seg0) : 0.0f);
+  const bool drop_on = dr.on;
 
   f32x4(*red)[4][kWaveSize] = reinterpret_cast<f32x4(*)[4][kWaveSize]>(smem);
   // Store staging.  The MFMA leaves 32-byte pieces per output row; the totals go through LDS once

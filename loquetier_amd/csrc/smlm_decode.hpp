@@ -324,9 +324,12 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
 #pragma unroll
   for (int i = 0; i < U; ++i) lrow[i] = F.rows[load_row(i)];
   __syncthreads();  // every wave holds its rows: the finder's LDS turns into the product's
-  DropRow dr{};
-  DropArgs dp{};
-  if (DROP) dp = drop_proj(a.sh.drop, pj), dr = drop_row_of(dp, row, rseg);
+  const DropArgs dp = DROP ? drop_proj(a.sh.drop, pj) : DropArgs{};
+  // (waited for here: behind x's request it costs the loop registers; 300 rows over 64 adapters at rank 32 27.9 and 30.6 us)
+  const DropRow dr = drop_params(DROP ? drop_prob(dp, row, rseg, zeros) : 0.0f);
+  const bool dropped = DROP && __builtin_amdgcn_ballot_w64(dr.on) != 0;  // uniform over the wave
+  uint8_t* const bits_out = zb == 0 ? P.drop_bits : nullptr;
+  const bool words = drop_words<U>(bits_out, P.d_in >> 3);
 
   // ---- the product, as the eight-wave shrink_kernel does it
   f32x4 acc[NB];
@@ -341,6 +344,11 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
       xf[i] = ldg16_or(P.x + (long)lrow[i] * P.d_in + kk, kk < kend && lrow[i] >= 0, zeros);
     }
     if (k != kbeg) load_w(k, wf);  // uniform over the wave (k is usually one batch)
+    DropMasks<U> dm;
+    if (DROP && dropped) {  // (x is on its way)
+      dm.make(dp, dr, row, k >> 3, g, bits_out, P.d_in >> 3, kend >> 3, words);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (LINES) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) Turn::turn(sm.wave[wave_all].turn, lane, wf[nb]);
@@ -348,10 +356,9 @@ __global__ __launch_bounds__(THREADS) void shrink_self_planned_kernel(SelfPlanAr
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int kk = k + 32 * u + 8 * g;
-      const u32x4 xu = DROP ? drop8<DT>(xf[u], dp, dr, row, kk >> 3, P.drop_bits, P.d_in >> 3, zb == 0 && kk < kend) : xf[u];
+      if (DROP && dropped) xf[u] = dm.template apply<DT>(xf[u], u, dr);
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(wf[nb][u], xu, acc[nb]);
+      for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(wf[nb][u], xf[u], acc[nb]);
     }
   }
 
@@ -641,9 +648,14 @@ __global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfP
   const int row = active ? sm.find.rows[wave * kTileRows + c] : -1;
   const int rseg = active ? sm.find.rseg[wave * kTileRows + c] : -1;
   const uint16_t* xrow = P.x + (long)(row < 0 ? 0 : row) * P.d_in;
+  const DropArgs dp = DROP ? drop_proj(a.sh.drop, pj) : DropArgs{};
+  const float prob = DROP ? drop_prob(dp, row, rseg, zeros) : 0.0f;
   DropRow dr{};
-  DropArgs dp{};
-  if (DROP) dp = drop_proj(a.sh.drop, pj), dr = drop_row_of(dp, row, rseg);
+  bool dropped = false;
+  uint8_t* const bits_out = zb == 0 ? P.drop_bits : nullptr;
+  const bool words = drop_words<U>(bits_out, P.d_in >> 3);
+  DropMasks<U> dm;
+  auto make_masks = [&](int kb) { dm.make(dp, dr, row, kb >> 3, g, bits_out, P.d_in >> 3, kend >> 3, words); };
   auto load_x = [&](int kb, u32x4 (&xf)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -659,6 +671,11 @@ __global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfP
   // ---- the product, as shrink_wide_kernel does it
   u32x4 xf[U];
   load_x(kbeg, xf);
+  if (DROP) {
+    dr = drop_params(prob);
+    dropped = __builtin_amdgcn_ballot_w64(dr.on) != 0;  // (uniform over the wave)
+    if (dropped) make_masks(kbeg);                      // (x is on its way)
+  }
   __syncthreads();  // every wave holds its rows: the finder's LDS turns into the weight staging area
   stage_w(0, wst);
   int buf = 0;
@@ -671,12 +688,12 @@ __global__ __launch_bounds__(THREADS) void shrink_wide_self_planned_kernel(SelfP
     if (active) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int kk = kb + 32 * u + 8 * g;
-        const u32x4 xu = DROP ? drop8<DT>(xf[u], dp, dr, row, kk >> 3, P.drop_bits, P.d_in >> 3, zb == 0 && kk < kend) : xf[u];
+        if (DROP && dropped) xf[u] = dm.template apply<DT>(xf[u], u, dr);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(weight_frag(buf, u, nb), xu, acc[nb]);
+        for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(weight_frag(buf, u, nb), xf[u], acc[nb]);
       }
     }
+    if (DROP && dropped && kb + KB < kend) make_masks(kb + KB);  // (the next batch is on its way)
     stage_w(buf ^ 1, wn);
     buf ^= 1;
 #pragma unroll

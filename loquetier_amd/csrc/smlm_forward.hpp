@@ -274,13 +274,17 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
     for (int i = 0; i < U; ++i) lrow[i] = a.plan.tile_row[tile * kTileRows + Turn::row(lane, i)];
     const uint16_t* W = uload_ptr(P.w_ptrs, wid);
     const int nlim = rank_limit(a.plan, wid, P.d_out);  // weight rows at or past it are zero padding
-    DropRow dr{};
-    DropArgs dp{};
-    if (DROP) dp = drop_proj(a.drop, pj), dr = drop_row(dp, row, a.plan.tile_rseg, slot);
+    const int rseg = DROP ? a.plan.tile_rseg[slot] : -1;
 
     const int kbeg = (kz * NW + wave) * P.k_per_wave;
     const int kend = min(kbeg + P.k_per_wave, P.d_in);
     const uint16_t* zeros = reinterpret_cast<const uint16_t*>(a.plan.hdr + kHdrZeros);
+    const DropArgs dp = DROP ? drop_proj(a.drop, pj) : DropArgs{};
+    const float prob = DROP ? drop_prob(dp, row, rseg, zeros) : 0.0f;
+    uint8_t* const bits_out = zb == 0 ? P.drop_bits : nullptr;
+    const bool words = drop_words<U>(bits_out, P.d_in >> 3);
+    DropRow dr{};
+    bool dropped = false;
 
     f32x4 acc[NB];
 #pragma unroll
@@ -301,21 +305,26 @@ __global__ __launch_bounds__(NW * kWaveSize) void shrink_kernel(ShrinkArgs a) {
         xf[i] = ldg16_or(P.x + (long)lrow[i] * P.d_in + kk, kin && lrow[i] >= 0, zeros);
     };
     auto multiply = [&](int k, u32x4 (&xf)[U], u32x4 (&wf)[NB][U]) {
+      DropMasks<U> dm;
+      if (DROP && dropped) {  // (x is on its way)
+        dm.make(dp, dr, row, k >> 3, g, bits_out, P.d_in >> 3, kend >> 3, words);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) Turn::turn(area[wave], lane, wf[nb]);
       Turn::turn(area[wave], lane, xf);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int kk = k + 32 * u + 8 * g;
-        const u32x4 xu = DROP ? drop8<DT>(xf[u], dp, dr, row, kk >> 3, P.drop_bits, P.d_in >> 3, zb == 0 && kk < kend) : xf[u];
+        if (DROP && dropped) xf[u] = dm.template apply<DT>(xf[u], u, dr);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(wf[nb][u], xu, acc[nb]);
+        for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(wf[nb][u], xf[u], acc[nb]);
       }
     };
     {
       // two load batches in turn: one is on its way while the other is multiplied
       u32x4 xa[U], wa[NB][U], xb[U], wb[NB][U];
       load_batch(kbeg, xa, wa);
+      if (DROP) dr = drop_params(prob), dropped = __builtin_amdgcn_ballot_w64(dr.on) != 0;  // (uniform over the wave)
 #pragma unroll 1
       for (int k = kbeg; k < kend; k += 64 * U) {
         const bool more = k + 32 * U < kend;  // uniform over the wave
@@ -404,9 +413,14 @@ __global__ __launch_bounds__(kFwdThreads) void shrink_wide_kernel(ShrinkArgs a) 
     const int kbeg = kz * kFwdWaves * P.k_per_wave;
     const int kend = min(kbeg + kFwdWaves * P.k_per_wave, P.d_in);
     const uint16_t* xrow = P.x + (long)(row < 0 ? 0 : row) * P.d_in;
+    const DropArgs dp = DROP ? drop_proj(a.drop, pj) : DropArgs{};
+    const float prob = DROP ? drop_prob(dp, row, a.plan.tile_rseg[slot], zeros) : 0.0f;
     DropRow dr{};
-    DropArgs dp{};
-    if (DROP) dp = drop_proj(a.drop, pj), dr = drop_row(dp, row, a.plan.tile_rseg, slot);
+    bool dropped = false;
+    uint8_t* const bits_out = zb == 0 ? P.drop_bits : nullptr;
+    const bool words = drop_words<U>(bits_out, P.d_in >> 3);
+    DropMasks<U> dm;
+    auto make_masks = [&](int kb) { dm.make(dp, dr, row, kb >> 3, g, bits_out, P.d_in >> 3, kend >> 3, words); };
 
     auto load_x = [&](int kb, u32x4 (&xf)[U]) {
 #pragma unroll
@@ -457,6 +471,11 @@ __global__ __launch_bounds__(kFwdThreads) void shrink_wide_kernel(ShrinkArgs a) 
     u32x4 xf[U], wst[kPer];
     load_x(kbeg, xf);
     load_w(kbeg, wst);
+    if (DROP) {
+      dr = drop_params(prob);
+      dropped = __builtin_amdgcn_ballot_w64(dr.on) != 0;  // (uniform over the wave)
+      if (dropped) make_masks(kbeg);                      // (x is on its way)
+    }
     __syncthreads();  // every wave is done with both LDS buffers of the previous item
     stage_w(0, wst);
     int buf = 0;
@@ -470,12 +489,12 @@ __global__ __launch_bounds__(kFwdThreads) void shrink_wide_kernel(ShrinkArgs a) 
       if (active) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int kk = kb + 32 * u + 8 * g;
-          const u32x4 xu = DROP ? drop8<DT>(xf[u], dp, dr, row, kk >> 3, P.drop_bits, P.d_in >> 3, zb == 0 && kk < kend) : xf[u];
+          if (DROP && dropped) xf[u] = dm.template apply<DT>(xf[u], u, dr);
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(weight_frag(buf, u, nb), xu, acc[nb]);
+          for (int nb = 0; nb < NB; ++nb) acc[nb] = Num<DT>::mfma(weight_frag(buf, u, nb), xf[u], acc[nb]);
         }
       }
+      if (DROP && dropped && kb + KB < kend) make_masks(kb + KB);  // (the next batch is on its way)
       stage_w(buf ^ 1, wn);
       buf ^= 1;
 #pragma unroll
@@ -1319,13 +1338,13 @@ void expand_block_kernel(ExpandArgs a) {
     LineLane L;  // rows this lane reads and writes in y
     L.orow = lane >> 3;
     L.ocol = (lane & 7) * 8;
-    int sseg[2];
+    int sseg[2], dseg[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       L.srow[j] = active ? a.plan.tile_row[tslot + L.orow + 8 * j] : -1;
       sseg[j] = (a.seg_scale && active) ? a.plan.tile_rseg[tslot + L.orow + 8 * j] : -1;  // -1 on empty slots
       L.yrow[j] = P.y + (long)(L.srow[j] < 0 ? 0 : L.srow[j]) * P.d_out + ncol0 + L.ocol;
-      if (DROP) L.drop[j] = drop_row(a.drop, L.srow[j], a.plan.tile_rseg, tslot + L.orow + 8 * j);
+      dseg[j] = DROP ? a.plan.tile_rseg[tslot + L.orow + 8 * j] : -1;
     }
     const uint16_t* zeros = reinterpret_cast<const uint16_t*>(a.plan.hdr + kHdrZeros);
 
@@ -1365,6 +1384,9 @@ void expand_block_kernel(ExpandArgs a) {
     load_y_lines<NQ>(yold, L, ncol0, P.d_out, read_y, zeros);
     if (DROP) load_keep_bits<NQ>(L, a.drop, P.drop_bits, P.drop_pitch, ncol0, P.d_out, zeros);
     load_v(0);
+    float prob[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) prob[j] = DROP ? drop_prob(a.drop, L.srow[j], dseg[j], zeros) : 0.0f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) L.scale[j] = (sseg[j] >= 0 && L.srow[j] >= 0) ? a.seg_scale[sseg[j]] : 1.0f;
 
@@ -1413,6 +1435,9 @@ void expand_block_kernel(ExpandArgs a) {
     }
 
     __syncthreads();  // every wave has read its weights: the area is free for the accumulators
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (DROP) L.drop[j] = drop_params(prob[j]);
     if (active) store_y_lines<DT, NQ, DROP>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
     if (P.pt_a && yy == 0 && active) {  // by-products for the backward, when no fold has written them
       const int rseg = a.seg_scale ? a.plan.tile_rseg[slot] : -1;
