@@ -757,6 +757,27 @@ int launch_wgrad(int nbj, bool split, dim3 grid, hipStream_t st, const WgradArgs
   return launch(wgrad_kernel<DT, 4, 1, DROP, false>, grid, bl, st, wa);
 }
 
+// Whether the weight gradients' workgroups are four waves that share an adapter's rows, or one: from how many rows an
+// adapter on.  Four waves take a quarter of the steps but fill a CU sooner (their registers: four workgroups at ranks up
+// to 16, three up to 32, two above, fewer under dropout), so the line rises with the workgroups, one an adapter (and 64
+// ranks) for each 64 columns.  us, one wave / four, two projections 4096 -> 4096 (256 such pieces): one adapter at rank
+// 16, 128 rows 7.3 / 6.8, 512 rows 14.3 / 8.7, 1024 rows 24.4 / 12.3; two of 256 rows 10.2 / 8.6, at rank 32 10.7 / 9.4,
+// at rank 64 12.0 / 10.9, at rank 128 13.1 / 16.1; four of 512 rows at rank 32 22.0 / 21.7, at rank 128 24.2 / 34.8; eight
+// of 512 rows at rank 16 30.9 / 31.4, at rank 32 32.6 / 36.3; sixteen of 512 at rank 128 113 / 132.
+// Under dropout one wave by itself has more to do: two of 256 rows at rank 16 16.8 / 10.6, eight of 512 rows at rank 128,
+// one projection, 61.3 / 42.2, sixteen of 256 rows at rank 32 27.9 / 30.6.
+// A launch of several projections has more pieces and would change over later, of one sooner (four adapters of 384 rows at
+// rank 32: one 14.4 / 10.8, two 18.2 / 19.0; two of 300 rows at rank 64: one 12.5 / 9.4, four 17.4 / 20.2); the rule does
+// not look at their number, so that it gives the bits that launches of one give.
+bool wgrad_split(int rows, int NA, int r, bool drop) {
+  const long m = (long)NA * ceil_div(r, 64);
+  auto least = [](long a, long b) { return a < b ? a : b; };
+  auto most = [](long a, long b) { return a > b ? a : b; };
+  if (r <= 16) return rows >= most(128, least(48 * m, drop ? 256 : 512));
+  if (r <= 32) return rows >= most(128, drop ? least(64 * m, 512) : least(96 * m, most(512, 64 * m)));
+  return rows >= most(192, drop ? least(64 * m, 256) : least(128 * m, most(512, 96 * m)));
+}
+
 struct BwdProjLayout {
   size_t partial, dv16, v16, pt_a, pt_b, bits;
 };
@@ -1454,10 +1475,7 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   wa.grp_id = pv.grp_id;
   wa.tile_row = pv.tile_row;
   wa.nproj = n_proj;
-  // four waves splitting the rows of an adapter pay off when adapters have many rows each (whole backward,
-  // 16 adapters at rank 16 / 64: 1024 rows each 124.7 -> 118.7 / 180.7 -> 175.3 us, 512 rows even, 256 rows
-  // 43.5 -> 44.6 / 62.1 -> 67.3 us, 64 rows 25.7 -> 30.8 / 33.7 -> 46.5 us)
-  const bool split = n_rows / NA >= 512;
+  const bool split = wgrad_split(n_rows / NA, NA, r, drop.seg_p != nullptr);
   // one-wave workgroups take several neighbouring chunks in turn when there are chunks enough to keep the
   // chip busy anyway: about 8192 workgroups are left
   long all_chunks = 0;
