@@ -439,6 +439,16 @@ SMLM_API int smlm_segments_build(const int32_t* req_adapter, const int32_t* req_
                                  int32_t* seg_adapter, int32_t* seg_len, int32_t* seg_indptr,
                                  int32_t* n_seg, void* stream);
 
+/*
+ * Copies `bytes` (a multiple of 4) of host memory to device memory (4-byte aligned) in the
+ * arguments of launches on `stream`, 3584 bytes each: src has been read when the call
+ * returns, and the host waits for nothing.  For the small tables a call needs (row
+ * partitions, adapter numbers, weight addresses), which the reference copies from pageable
+ * memory (src/loquetier_src/models/mixed_lora.py:196-205).  Captured, the words of the capture
+ * are written by every replay.
+ */
+SMLM_API int smlm_put_words(void* dst, const void* src, size_t bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

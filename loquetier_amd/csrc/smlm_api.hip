@@ -3,8 +3,11 @@
 // synchronisation, no state.
 #include <hip/hip_runtime.h>
 
+#include <string.h>
+
 #include <atomic>
 
+#include "put_words.hpp"
 #include "rms_norm.hpp"
 #include "segments.hpp"
 #include "smlm.h"
@@ -1647,6 +1650,36 @@ SMLM_API int smlm_segments_build(const int32_t* req_adapter, const int32_t* req_
   if (R > kMaxSegments) return SMLM_ERR_LIMIT;
   const SegmentsArgs a{req_adapter, req_len, seg_adapter, seg_len, seg_indptr, n_seg, R};
   return launch(segments_kernel, dim3(1), dim3(kPlanThreads), (hipStream_t)stream, a);
+}
+
+SMLM_API int smlm_put_words(void* dst, const void* src, size_t bytes, void* stream) {
+  if (bytes == 0) return SMLM_OK;
+  if (!dst || !src) return SMLM_ERR_ARG;
+  if ((bytes & 3) || (reinterpret_cast<uintptr_t>(dst) & 3)) return SMLM_ERR_ALIGN;
+  uint32_t* d = reinterpret_cast<uint32_t*>(dst);
+  const char* from = reinterpret_cast<const char*>(src);
+  for (size_t words = bytes / 4; words;) {
+    const int n = words < (size_t)kPutLarge ? (int)words : kPutLarge;
+    int rc;
+    if (n <= kPutSmall) {
+      PutArgs<kPutSmall> a;
+      a.dst = d;
+      a.n = n;
+      memcpy(a.words, from, (size_t)n * 4);
+      rc = launch(put_words_kernel<kPutSmall>, dim3(1), dim3(256), (hipStream_t)stream, a);
+    } else {
+      PutArgs<kPutLarge> a;
+      a.dst = d;
+      a.n = n;
+      memcpy(a.words, from, (size_t)n * 4);
+      rc = launch(put_words_kernel<kPutLarge>, dim3(1), dim3(256), (hipStream_t)stream, a);
+    }
+    if (rc) return rc;
+    d += n;
+    from += (size_t)n * 4;
+    words -= n;
+  }
+  return SMLM_OK;
 }
 
 }  // extern "C"

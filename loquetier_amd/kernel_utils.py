@@ -83,10 +83,6 @@ class BatchLenInfo:
         return self._indptr
 
 
-def _ptr_table(tensors: Sequence[torch.Tensor], device: torch.device) -> torch.Tensor:
-    return torch.tensor([t.data_ptr() for t in tensors], dtype=torch.int64, device=device)
-
-
 def _unique_adapters(weight_list: Sequence[torch.Tensor]):
     """Train partitions -> indices into the list of distinct (A, B) pairs."""
     pairs, index, part_adapter = [], {}, []
@@ -112,8 +108,7 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
 
     `step` (mixed_lora.LayerStep or None): the backward's plan, the partitions'
     adapters, the weights' pointer tables and the layout of one buffer for all the
-    gradients, prepared outside the layer loop; without it they are built here
-    (six small host-to-device copies, each of which the host waits for, and a plan launch per call)."""
+    gradients, prepared outside the layer loop; without it they are made here."""
     dev, dt = grad_output.device, grad_output.dtype
     T = grad_output.size(0)
     h_in = x_train.size(1)
@@ -171,12 +166,15 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
         db = [torch.empty_like(wb) for _, wb in pairs]
         if tl > 0:
             g = grad_output if grad_output.is_contiguous() else grad_output.contiguous()
-            part_indptr = torch.tensor(tp, dtype=torch.int32, device=dev)
-            part_ad = torch.tensor(part_adapter, dtype=torch.int32, device=dev)
-            plan = kernel.SegmentPlan(part_indptr, part_ad, tl)
+            # every table of the call in one launch; the plan is built inside the call's own first launch
+            n = len(pairs)
+            tabs, parts = kernel.put_ints(
+                dev, [t.data_ptr() for ts in (da, db, [p[0] for p in pairs], [p[1] for p in pairs]) for t in ts],
+                tp + part_adapter)
+            plan = kernel.SegmentPlan(parts[:n_parts + 1], parts[n_parts + 1:], tl, defer=True)
+            da_tab, db_tab, a_tab, b_tab = tabs.split(n)
             kernel.smlm_lora_backward(
-                grad_x, _ptr_table(da, dev), _ptr_table(db, dev), g, x_train, v_train,
-                _ptr_table([p[0] for p in pairs], dev), _ptr_table([p[1] for p in pairs], dev),
+                grad_x, da_tab, db_tab, g, x_train, v_train, a_tab, b_tab,
                 plan, lora_rank, part_scale, dropout=dropout, adapter_rank=adapter_rank,
                 workspace=None if step is None else step.workspace,
                 packed_ranks=step is not None and step.packed, zero_dx_tail=tail_in_call)

@@ -185,8 +185,8 @@ class MixedLoraContext:
             part_adapter = [order.index(int(i)) for i in self._train_idx[:n_parts]]
             if n_parts == 0 or tp[-1] == 0:
                 return None, part_adapter
-            plan = kernel.SegmentPlan(torch.tensor(tp, dtype=torch.int32, device=device),
-                                      torch.tensor(part_adapter, dtype=torch.int32, device=device), tp[-1],
+            _, parts = kernel.put_ints(device, [], tp + part_adapter)
+            plan = kernel.SegmentPlan(parts[:n_parts + 1], parts[n_parts + 1:], tp[-1],
                                       defer=True)  # built by the step's first backward call
             return plan, part_adapter
         return self.memo(("backward", device), build)
@@ -195,9 +195,12 @@ class MixedLoraContext:
         """Segment that starts every train partition (int64 device indices): the partition's scale
         and dropout probability are those of that segment."""
         def build():
-            n_parts = min(len(self._train_idx), len(self._blen.train_partition) - 1)
-            starts = torch.tensor([int(t) for t in self._blen.train_partition][:n_parts],
-                                  dtype=torch.int32, device=device)
+            bwd_plan, part_adapter = self.backward_tables(device)
+            if bwd_plan is None:   # no partitions, or none with rows
+                n_parts = len(part_adapter)
+                _, starts = kernel.put_ints(device, [], [int(t) for t in self._blen.train_partition][:n_parts])
+            else:
+                starts = bwd_plan.segment[:bwd_plan.S]
             return (torch.searchsorted(plan.segment, starts, right=True) - 1).clamp_(0, max(plan.S - 1, 0))
         return self.memo(("part_segments", device), build)
 

@@ -9,6 +9,7 @@ torch's current stream of that device.  Nothing here computes on the host.
 from __future__ import annotations
 
 import ctypes as C
+import struct
 from typing import Dict, Optional, Tuple
 
 import torch
@@ -207,6 +208,25 @@ def smlm_forward_cutlass_static(y: torch.Tensor, x: torch.Tensor, w_ptr: torch.T
                                           d_out if is_row_major else d_in, int(bool(is_row_major)), code,
                                           float(beta), _ptr(seg_scale), _stream(dev))
     _lib.check(rc, "smlm_forward_cutlass_static")
+
+
+_PUT_BYTES = 4 * 3584  # more words than four launches carry are copied
+
+
+def put_ints(device: torch.device, words64, words32) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Small host tables as device tensors (int64, int32) that share one allocation, without waiting for the device:
+    the words travel in a launch's arguments (smlm_put_words); long tables in one copy."""
+    n64, n32 = len(words64), len(words32)
+    data = struct.pack(f"={n64}q{n32 + (n32 & 1)}i", *words64, *words32, *((0,) * (n32 & 1)))
+    if len(data) > _PUT_BYTES or (data and torch.device(device).type != "cuda"):
+        buf = torch.frombuffer(bytearray(data), dtype=torch.int64).to(device)
+    else:
+        buf = torch.empty(len(data) // 8, dtype=torch.int64, device=device)
+        dev = buf.device
+        with _on(dev):
+            rc = _lib.load().smlm_put_words(buf.data_ptr(), data, len(data), _stream(dev))
+        _lib.check(rc, "put_ints")
+    return buf[:n64], buf[n64:].view(torch.int32)[:n32]
 
 
 class SegmentPlan:
