@@ -6,6 +6,7 @@ operator raises.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -99,6 +100,25 @@ def load() -> C.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+HOST_PATH = os.path.join(_PKG_DIR, "lib", "_smlm_host.so")
+_host = None
+
+
+def host(default_workspace=None):
+    """The native host path (csrc/host_path.cpp), bound to the HIP library; raises RuntimeError when it has not been built."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m loquetier_amd.build`.")
+        lib = load()
+        spec = importlib.util.spec_from_file_location("_smlm_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES}, default_workspace)
+        _host = mod
+    return _host
 
 
 def strerror(code: int) -> str:

@@ -204,6 +204,14 @@ class add_lora(Function):
     trainable weight, written for the layout the forward uses.
     """
 
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if cls is add_lora and not kwargs and not torch._C._are_functorch_transforms_active():
+            out = kernel._host().add_lora(*args)  # (plain calls; None: nothing was done)
+            if out is not None:
+                return out
+        return super().apply(*args, **kwargs)
+
     @staticmethod
     def forward(ctx: FunctionCtx, y_shape, x, wa_ptr, wb_ptr, s, lora_rank, train_len,
                 train_partition, *args):
@@ -245,6 +253,14 @@ class rms_norm(Function):
     (src/loquetier_src/kernel_utils.py:149-176).  x: [rows, cols] fp16/bf16,
     w: [cols].  The backward runs as one fused kernel in float instead of the
     reference's chain of 16-bit tensor expressions."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if cls is rms_norm and not kwargs and not torch._C._are_functorch_transforms_active():
+            out = kernel._host().rms_norm(*args)  # (plain calls; None: nothing was done)
+            if out is not None:
+                return out
+        return super().apply(*args, **kwargs)
 
     @staticmethod
     def forward(ctx: FunctionCtx, x: torch.Tensor, w: torch.Tensor, eps: float = 1e-6):

@@ -280,6 +280,14 @@ class fused_add_lora(Function):
     Gradients: result -> passed through, x -> dX on train rows (zero elsewhere),
     each trainable weight -> its summed gradient (None when not training)."""
 
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if cls is fused_add_lora and not kwargs and not torch._C._are_functorch_transforms_active():
+            out = kernel._host().fused_add_lora(*args)  # (plain training calls; None: nothing was done)
+            if out is not None:
+                return out
+        return super().apply(*args, **kwargs)
+
     @staticmethod
     def forward(ctx: FunctionCtx, result, x, step, *weights):
         wa_table, wb_table, seg_scale, plan, lora_rank = step.wa_table, step.wb_table, step.seg_scale, step.plan, step.rank

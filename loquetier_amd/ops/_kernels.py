@@ -95,6 +95,11 @@ def _workspace(dev: torch.device, nbytes: int, own: Optional[Workspace] = None) 
     return ws.reserve(nbytes)
 
 
+def _host():
+    """The native host path (loaded at the first call that can take it: it needs the built libraries)."""
+    return _lib._host or _lib.host(_workspace)
+
+
 def _check_input(t: torch.Tensor, name: str) -> None:
     # CHECK_INPUT of kernel_src/csrc/loquetier_ops.cc:32-38
     if not t.is_cuda:
@@ -520,6 +525,11 @@ def smlm_lora_forward_multi(ys, xs, a_ptrs, b_ptrs, plan: SegmentPlan, rank: int
     tensors of the same shapes, dtype, device and contiguity and the same tables skip the checks and
     reuse the argument blocks that do not change."""
     n = len(ys)
+    if n == 1 and dropout is None and stages == 3 and dims is None and len(xs) == len(a_ptrs) == len(b_ptrs) == 1 and (
+            v_out is None or len(v_out) == 1) and _host().forward(
+                ys[0], xs[0], a_ptrs[0], b_ptrs[0], plan, rank, seg_scale, beta, None if v_out is None else v_out[0],
+                adapter_rank, workspace, packed_ranks):
+        return  # (one projection, plain: checked and launched by the native host path)
     key = None
     if cache is not None and dropout is None and len(xs) == n:  # (a dropout descriptor is checked call by call)
         scale_list = () if seg_scale is None else (seg_scale,)
