@@ -573,6 +573,25 @@ int launch_expand_dt(bool block, int nq, int KS, dim3 grid, hipStream_t st,
                  : launch_expand_wave<DT, 2, DIRECT>(KS, vfold, grid, st, a);
 }
 
+// the chunk rows of an expand launch, `chunk` columns each
+void expand_rows(ExpandArgs& a, int nproj, int chunk) {
+  a.items.nproj = nproj;
+  a.items.interleave = 0;
+  a.items.row_start[0] = 0;
+  // Workgroups go to the XCDs in turn (workgroup number modulo eight, whatever the XCDs' load).  With an odd
+  // number of chunk rows a tile unit, the workgroups of one column chunk visit all eight XCDs from unit to
+  // unit and each L2 fetches that chunk of an adapter's weights for itself: a launch of one projection gets one
+  // empty row then (8192 rows at rank 64: h_out = 11136, 87 chunks of 128 columns, 83.4 -> 73.3 us; h_out =
+  // 11008, 43 chunks of 256, 87.8 -> 71.7 us).  Launches of several projections are left as they are: empty
+  // workgroups there can fall on the same few XCDs in every unit and leave the others with all the work
+  // (measured on the shrink launch of five and six projections: up to 2.2 x slower).
+  for (int i = 0; i < nproj; ++i) {
+    int rows = ceil_div(a.p[i].d_out, chunk);
+    if (nproj == 1 && rows > 1 && (rows & 1)) rows += 1;
+    a.items.row_start[i + 1] = a.items.row_start[i] + rows;
+  }
+}
+
 // all projections of one launch share the rank (d_in); d_out may differ
 int launch_expand(int dtype, int nq, int MT, int S, int groups, int nproj, int max_d_in,
                   hipStream_t st, ExpandArgs& a) {
@@ -595,21 +614,7 @@ int launch_expand(int dtype, int nq, int MT, int S, int groups, int nproj, int m
     nq = wider && KS <= 2 ? 8 : 4;
   }
   const int chunk = block ? 32 * nq : kFwdWaves * 32 * nq;  // columns per workgroup
-  a.items.nproj = nproj;
-  a.items.interleave = 0;
-  a.items.row_start[0] = 0;
-  // Workgroups go to the XCDs in turn (workgroup number modulo eight, whatever the XCDs' load).  With an odd
-  // number of chunk rows a tile unit, the workgroups of one column chunk visit all eight XCDs from unit to
-  // unit and each L2 fetches that chunk of an adapter's weights for itself: a launch of one projection gets one
-  // empty row then (8192 rows at rank 64: h_out = 11136, 87 chunks of 128 columns, 83.4 -> 73.3 us; h_out =
-  // 11008, 43 chunks of 256, 87.8 -> 71.7 us).  Launches of several projections are left as they are: empty
-  // workgroups there can fall on the same few XCDs in every unit and leave the others with all the work
-  // (measured on the shrink launch of five and six projections: up to 2.2 x slower).
-  for (int i = 0; i < nproj; ++i) {
-    int rows = ceil_div(a.p[i].d_out, chunk);
-    if (nproj == 1 && rows > 1 && (rows & 1)) rows += 1;
-    a.items.row_start[i + 1] = a.items.row_start[i] + rows;
-  }
+  expand_rows(a, nproj, chunk);
   const int units = tile_units_max(a.T, S, groups, block ? kBlkTiles : 1);
   const long items = (long)units * a.items.row_start[nproj];
   bool same_rows = true;
@@ -760,6 +765,23 @@ int launch_wgrad(int nbj, bool split, dim3 grid, hipStream_t st, const WgradArgs
   return launch(wgrad_kernel<DT, 4, 1, DROP, false>, grid, bl, st, wa);
 }
 
+template <int DT, bool DROP, int NW>
+int launch_bwd_tail(int nbj, dim3 grid, hipStream_t st, const BwdTailArgs& a) {
+  const dim3 bl(kFwdThreads);
+  if (a.e.p[0].d_in > 64) return launch(bwd_tail_kernel<DT, 4, NW, DROP, true, 4>, grid, bl, st, a);
+  if constexpr (wgrad_nbj_a(4, NW, DROP) < 4)  // (two dA workgroups a unit)
+    if (a.w.zcount > 1) return launch(bwd_tail_kernel<DT, 4, NW, DROP, true, 2>, grid, bl, st, a);
+  if (nbj == 1) return launch(bwd_tail_kernel<DT, 1, NW, DROP, false, 1>, grid, bl, st, a);
+  if (nbj == 2) return launch(bwd_tail_kernel<DT, 2, NW, DROP, false, 1>, grid, bl, st, a);
+  return launch(bwd_tail_kernel<DT, 4, NW, DROP, false, 2>, grid, bl, st, a);
+}
+template <int DT>
+int launch_bwd_tail_dt(int nbj, bool split, dim3 grid, hipStream_t st, const BwdTailArgs& a) {
+  if (a.w.drop.seg_p)
+    return split ? launch_bwd_tail<DT, true, 4>(nbj, grid, st, a) : launch_bwd_tail<DT, true, 1>(nbj, grid, st, a);
+  return split ? launch_bwd_tail<DT, false, 4>(nbj, grid, st, a) : launch_bwd_tail<DT, false, 1>(nbj, grid, st, a);
+}
+
 // Whether the weight gradients' workgroups are four waves that share an adapter's rows, or one: from how many rows an
 // adapter on.  Four waves take a quarter of the steps but fill a CU sooner (their registers: four workgroups at ranks up
 // to 16, three up to 32, two above, fewer under dropout), so the line rises with the workgroups, one an adapter (and 64
@@ -779,6 +801,27 @@ bool wgrad_split(int rows, int NA, int r, bool drop) {
   if (r <= 16) return rows >= most(128, least(48 * m, drop ? 256 : 512));
   if (r <= 32) return rows >= most(128, drop ? least(64 * m, 512) : least(96 * m, most(512, 64 * m)));
   return rows >= most(192, drop ? least(64 * m, 256) : least(128 * m, most(512, 96 * m)));
+}
+
+// Whether dX and the weight gradients (`waves`: their workgroups, of one wave or four) go out in one launch: while what
+// they move takes little longer than starting and draining two.  Together they hold as many registers and as much LDS as
+// the weight gradients, so fewer of dX's workgroups are resident, which costs where both run at the memory's rate; and
+// workgroups of four one-wave units wait for the longest.  Same bits.  us, two launches / one, h_in = h_out = 4096 (MB: x,
+// dY and dX, then the weights): one adapter of 64 rows at rank 16 (2 + 0) 8.8 / 6.3, of 1024 rows at rank 128 (25 + 6)
+// 19.3 / 14.7; three of 200 rows, four projections at rank 64 (59 + 19) 26.8 / 24.9; two of 1024 rows, two projections at
+// rank 16 (101 + 3) 24.6 / 23.1, four projections (201 + 6) 43.9 / 49.2, at rank 128 (201 + 50) 89.0 / 93.5, two (101 + 25)
+// 43.2 / 40.3; one of 1024 rows, four projections at rank 32 (101 + 3) 26.6 / 27.7; eight of 256 rows, two at rank 32
+// (101 + 13) 27.2 / 28.8; 64 of 32 rows at rank 32 (50 + 50, 8192 waves) 31.2 / 32.8.  Under dropout, two of 1377 rows, two
+// projections at rank 32 (135 + 3) 43.8 / 42.0; eight of 1000 rows (197 + 6) 63.2 / 67.0; 64 of 32 rows at rank 32 35.8 / 40.1.
+bool bwd_one_launch(int n_proj, int n_rows, int NA, int r, const int* h_in, const int* h_out, bool drop, bool split,
+                    long waves) {
+  double rows = 0, weights = 0;  // bytes
+  for (int i = 0; i < n_proj; ++i) {
+    rows += 2.0 * n_rows * (2.0 * h_in[i] + h_out[i]);
+    weights += 2.0 * NA * r * (2.0 * h_in[i] + h_out[i]);
+  }
+  if (r > 64) return rows < 200e6;
+  return (split || waves <= 4096) && rows + weights < (drop ? 140e6 : (n_proj > 2 ? 80e6 : 105e6));
 }
 
 struct BwdProjLayout {
@@ -1467,9 +1510,8 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   }
   ea.w_kn = rm ? 0 : 1;
   ea.drop = drop;  // dX is the gradient with respect to x before its dropout
-  if ((stages & SMLM_BWD_DX) && (rc = launch_expand(dtype, expand_nq(n_rows, widest), mt, P, NA, n_proj, r, st, ea)))
-    return rc;
-  if (!(stages & SMLM_BWD_WGRAD)) return SMLM_OK;
+  auto launch_dx = [&] { return launch_expand(dtype, expand_nq(n_rows, widest), mt, P, NA, n_proj, r, st, ea); };
+  if (!(stages & SMLM_BWD_WGRAD)) return (stages & SMLM_BWD_DX) ? launch_dx() : SMLM_OK;
 
   // 5. dA_a, dB_a for every adapter (zeros when it has no rows)
   WgradArgs wa{};
@@ -1530,6 +1572,27 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   wa.units = units;
   wa.zcount = ceil_div(r, 64) * z_per_64;
   dim3 grid(wa.zcount > 1 ? round_up(units, kWgXcd) * wa.zcount : units, NA);
+  if (stages & SMLM_BWD_DX) {
+    const int dx_units = tile_units_max(n_rows, P, NA, kBlkTiles);
+    ExpandArgs e = ea;
+    expand_rows(e, n_proj, 32 * 4);
+    const long dx_items = (long)dx_units * e.items.row_start[n_proj];
+    // (what passes between the two, dV's by-products, must have been left by the fold; dX of the other weight layout is
+    // another kernel)
+    if (side_in_fold && !rm && dx_items <= kDirectItems &&
+        bwd_one_launch(n_proj, n_rows, NA, r, h_in, h_out, drop.seg_p != nullptr, split, (long)grid.x * NA)) {
+      BwdTailArgs ta;
+      ta.w = wa;
+      ta.e = e;
+      ta.wx = (int)grid.x;
+      ta.wy = NA;
+      ta.wgrad = round_up(ceil_div((int)grid.x * NA, split ? 1 : kFwdWaves), kWgXcd);
+      const dim3 all((unsigned)(ta.wgrad + dx_items));
+      return dtype == SMLM_DTYPE_F16 ? launch_bwd_tail_dt<SMLM_DTYPE_F16>(nbj, split, all, st, ta)
+                                     : launch_bwd_tail_dt<SMLM_DTYPE_BF16>(nbj, split, all, st, ta);
+    }
+    if ((rc = launch_dx())) return rc;
+  }
   if (drop.seg_p)
     return dtype == SMLM_DTYPE_F16 ? launch_wgrad<SMLM_DTYPE_F16, true>(nbj, split, grid, st, wa)
                                    : launch_wgrad<SMLM_DTYPE_BF16, true>(nbj, split, grid, st, wa);

@@ -7,6 +7,7 @@
 #pragma once
 #include "dropout.hpp"
 #include "smlm_common.hpp"
+#include "smlm_forward.hpp"
 
 namespace smlm {
 
@@ -85,13 +86,12 @@ __device__ __forceinline__ int wg_lds_row(int s) {
 // rows are staged; every row of the workgroup belongs to one adapter, whose probability is read
 // once from the group's first segment.
 template <int DT, int NBJ, int NW, bool IS_A, bool DROP, bool ZSPLIT>
-__device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& P, int chunk_first, int n_chunks,
+__device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& P, int ad, int chunk_first, int n_chunks,
                                            int j0, char* smem) {
   constexpr int kWgWaves = NW;
   constexpr int kStageElems = kWgSlots * kWgPitch;
   constexpr int kRedBytes = NW > 1 ? NW * 4 * kWaveSize * 16 : 0;
 
-  const int ad = blockIdx.y;
   // j0: first rank of this workgroup, which takes 16 * NBJ
   constexpr bool is_a = IS_A;
   const int h = is_a ? P.h_in : P.h_out;
@@ -99,7 +99,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   const uint16_t* PT = is_a ? P.pt_a : P.pt_b;
   uint16_t* out = reinterpret_cast<uint16_t*>(is_a ? P.da_ptrs[ad] : P.db_ptrs[ad]);
 
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = NW > 1 ? threadIdx.x >> 6 : 0, lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
 
   // Group of this adapter (ids are distinct and ascending).  When every adapter below this one
@@ -357,19 +357,23 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
 // rank blocks of 16 a dA workgroup takes (a dB workgroup: NBJ)
 constexpr int wgrad_nbj_a(int nbj, int nw, bool drop) { return (drop && nw == 1 && nbj == 4) ? 2 : nbj; }
 
+template <int NW>
+struct WgradLds {
+  static constexpr int kStageBytes = NW * kWgSlots * kWgPitch * 2;
+  static constexpr int kTailBytes = (NW > 1 ? NW * 4 * kWaveSize * 16 : 0) + 16 * (64 + 4) * 4;  // red + store staging
+  static constexpr int kBytes = kStageBytes > kTailBytes ? kStageBytes : kTailBytes;
+};
+
 // ZSPLIT: several workgroups share a unit, each taking other ranks (a.zcount of them: ranks above 64, and those above
 // 32 in the one-wave kernel under dropout, whose dA workgroups take 32 each).  They are
 // numbered eight apart, so that they run at about the same time on one XCD (workgroup number modulo eight) and the
 // rows of x and dY, which all of them read, come out of its L2 for the second (2048 rows, two projections
 // 4096 -> 4096 at rank 128, before the operand came in lines: 40.2 us with the ranks along the grid's z axis, 37.4 eight
 // apart, 32.9 with loads that are not marked non-temporal as well).
+// u: number of the unit and its ranks, ad: adapter; smem: WgradLds of the NW waves
 template <int DT, int NBJ, int NW, bool DROP, bool ZSPLIT>
-// (two waves a SIMD at every rank: the one-wave kernels hide their latencies through occupancy)
-__global__ __launch_bounds__(NW * kWaveSize) __attribute__((amdgpu_waves_per_eu(2))) void wgrad_kernel(WgradArgs a) {
-  constexpr int kStageBytes = NW * kWgSlots * kWgPitch * 2;
-  constexpr int kTailBytes = (NW > 1 ? NW * 4 * kWaveSize * 16 : 0) + 16 * (64 + 4) * 4;  // red + store staging
-  __shared__ __attribute__((aligned(16))) char smem[kStageBytes > kTailBytes ? kStageBytes : kTailBytes];
-  int zi = 0, u = (int)blockIdx.x;
+__device__ __forceinline__ void wgrad_unit(const WgradArgs& a, int u, int ad, char* smem) {
+  int zi = 0;
   if (ZSPLIT) {
     const int per = kWgXcd * a.zcount, in = u % per;
     zi = in / kWgXcd;
@@ -388,13 +392,54 @@ __global__ __launch_bounds__(NW * kWaveSize) __attribute__((amdgpu_waves_per_eu(
   constexpr int NBJ_A = wgrad_nbj_a(NBJ, NW, DROP), ZA = NBJ / NBJ_A;
   if (unit < P.units_a) {  // uniform over the workgroup
     const int first = unit * walk, left = P.chunks_a - first;
-    wgrad_body<DT, NBJ_A, NW, true, DROP, ZSPLIT>(a, P, first, left < walk ? left : walk, 16 * NBJ_A * zi, smem);
+    wgrad_body<DT, NBJ_A, NW, true, DROP, ZSPLIT>(a, P, ad, first, left < walk ? left : walk, 16 * NBJ_A * zi, smem);
   } else {
     if (zi % ZA) return;
     const int chunks_b = (P.h_out + kWgCols - 1) / kWgCols;
     const int first = (unit - P.units_a) * walk, left = chunks_b - first;
-    wgrad_body<DT, NBJ, NW, false, false, ZSPLIT>(a, P, first, left < walk ? left : walk, 16 * NBJ * (zi / ZA), smem);
+    wgrad_body<DT, NBJ, NW, false, false, ZSPLIT>(a, P, ad, first, left < walk ? left : walk, 16 * NBJ * (zi / ZA), smem);
   }
+}
+
+template <int DT, int NBJ, int NW, bool DROP, bool ZSPLIT>
+// (two waves a SIMD at every rank: the one-wave kernels hide their latencies through occupancy)
+__global__ __launch_bounds__(NW * kWaveSize) __attribute__((amdgpu_waves_per_eu(2))) void wgrad_kernel(WgradArgs a) {
+  __shared__ __attribute__((aligned(16))) char smem[WgradLds<NW>::kBytes];
+  wgrad_unit<DT, NBJ, NW, DROP, ZSPLIT>(a, (int)blockIdx.x, (int)blockIdx.y, smem);
+}
+
+// dX and the weight gradients in one launch: its first `wgrad` workgroups are the weight gradients' (of the one-wave kind
+// four to a workgroup, eight numbers apart), the others take dX's items (tile block, column chunk) as
+// expand_block_kernel does.  Neither needs anything of the other once the fold of dV has written what both read.
+struct BwdTailArgs {
+  WgradArgs w;
+  ExpandArgs e;
+  int wgrad, wx, wy;  // workgroups of the weight gradients; units (with their ranks) and adapters
+};
+
+template <int DT, int NBJ, int NW, bool DROP, bool ZSPLIT, int KS>
+__global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(2))) void bwd_tail_kernel(BwdTailArgs a) {
+  constexpr int kW = kFwdWaves / NW * WgradLds<NW>::kBytes, kE = ExpandBlockLds<4, KS, true>::kBytes;
+  __shared__ __attribute__((aligned(16))) char smem[kW > kE ? kW : kE];
+  if ((int)blockIdx.x < a.wgrad) {
+    if (NW > 1) {
+      if ((int)blockIdx.x < a.wx * a.wy)
+        wgrad_unit<DT, NBJ, NW, DROP, ZSPLIT>(a.w, (int)blockIdx.x % a.wx, (int)blockIdx.x / a.wx, smem);
+    } else {
+      const int wave = threadIdx.x >> 6;
+      const int id = __builtin_amdgcn_readfirstlane((int)blockIdx.x / kWgXcd * (kFwdWaves * kWgXcd) + wave * kWgXcd +
+                                                    (int)blockIdx.x % kWgXcd);
+      if (id < a.wx * a.wy)
+        wgrad_unit<DT, NBJ, NW, DROP, ZSPLIT>(a.w, id % a.wx, id / a.wx, smem + wave * WgradLds<NW>::kBytes);
+    }
+    return;
+  }
+  const int d = (int)blockIdx.x - a.wgrad, rows = a.e.items.row_start[a.e.items.nproj];
+  const int cr = d % rows;
+  int pj = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxProj; ++i) pj += (i < a.e.items.nproj && cr >= a.e.items.row_start[i]) ? 1 : 0;
+  expand_block_item<DT, 4, KS, true, DROP>(a.e, pj, cr - a.e.items.row_start[pj], d / rows, smem);
 }
 
 }  // namespace smlm

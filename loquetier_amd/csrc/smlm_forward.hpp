@@ -1292,6 +1292,156 @@ void expand_wave_kernel(ExpandArgs a) {
 // as it lies in memory and read out of LDS with the transposing read.
 // K (= LoRA rank): up to 32*KS in one piece; KS = 4 serves every rank above 64, 128 of k at a time, the
 // next piece on its way while one is multiplied.
+template <int NQ, int KS, bool WKN>
+struct ExpandBlockLds {
+  static constexpr int kPitch = WKN ? 32 * NQ + 8 : 32 * KS + 8;  // LDS row pitch in 16-bit elements
+  // the staged weights and the area the accumulators change layout in share their LDS (the
+  // weights are done with when the accumulators are complete): five workgroups fit a CU at rank 64 too
+  static constexpr int kWBytes = (WKN ? 32 * KS : 32 * NQ) * kPitch * 2;
+  static constexpr int kOBytes = kFwdWaves * kTileRows * kOPitch * 4;
+  static constexpr int kBytes = kWBytes > kOBytes ? kWBytes : kOBytes;
+};
+
+// column chunk yy of projection pj, tile block tb; smem: ExpandBlockLds
+template <int DT, int NQ, int KS, bool WKN, bool DROP>
+__device__ __forceinline__ void expand_block_item(const ExpandArgs& a, int pj, int yy, int tb, char* smem) {
+  static_assert(NQ % 2 == 0, "the output is written 64 columns at a time");
+  constexpr int kPitch = ExpandBlockLds<NQ, KS, WKN>::kPitch;
+  uint16_t* wlds = reinterpret_cast<uint16_t*>(smem);
+  float(*olds)[kTileRows * kOPitch] = reinterpret_cast<float(*)[kTileRows * kOPitch]>(smem);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int c = lane & 15, g = lane >> 4;
+  const int mrow = 8 * (c >> 2) + (c & 3);
+  const ExpandProj P = a.p[pj];
+  if (!P.y) return;  // a projection this call leaves out (uniform over the workgroup)
+  const int ncol0 = yy * 32 * NQ;
+  if (ncol0 >= P.d_out) return;  // a chunk row added to round the count up (uniform over the workgroup)
+  const int packed = uload(a.plan.blk, tb);
+  const int t0 = packed >> 3, cnt = packed & 7;
+  if (cnt == 0) return;  // past the last block (direct mode); uniform over the workgroup
+  const int wid = uload(a.plan.tile_wid, t0);
+  if (!wid_ok(a.plan, wid)) return;  // a negative adapter id (rows that no adapter serves) or one past the tables
+  const uint16_t* W = uload_ptr(P.w_ptrs, wid);
+  const int klim = rank_limit(a.plan, wid, P.d_in);  // k at or past it: zero padding of v and the weights
+  const int ldw = WKN ? P.ldw : rank_ld(a.plan, P.ldw, klim);  // [k][n] weights (A) have whole rows per rank
+  const bool active = wave < cnt;
+  const int tslot = (t0 + (active ? wave : 0)) * kTileRows;
+  const int slot = tslot + c;
+  const int row = active ? a.plan.tile_row[slot] : -1;  // row of the MFMA column this lane feeds
+  LineLane L;  // rows this lane reads and writes in y
+  L.orow = lane >> 3;
+  L.ocol = (lane & 7) * 8;
+  int sseg[2], dseg[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    L.srow[j] = active ? a.plan.tile_row[tslot + L.orow + 8 * j] : -1;
+    sseg[j] = (a.seg_scale && active) ? a.plan.tile_rseg[tslot + L.orow + 8 * j] : -1;  // -1 on empty slots
+    L.yrow[j] = P.y + (long)(L.srow[j] < 0 ? 0 : L.srow[j]) * P.d_out + ncol0 + L.ocol;
+    dseg[j] = DROP ? a.plan.tile_rseg[tslot + L.orow + 8 * j] : -1;
+  }
+  const uint16_t* zeros = reinterpret_cast<const uint16_t*>(a.plan.hdr + kHdrZeros);
+
+  // Every load of the item is issued before anything waits for one (predicated-off loads
+  // read zeros instead of being patched afterwards).
+  // weight chunk -> registers (written to LDS below): 32*NQ rows of 4*KS 16-byte pieces
+  constexpr int kPieces = 32 * NQ * 4 * KS;
+  constexpr int kPer = (kPieces + kFwdThreads - 1) / kFwdThreads;
+  constexpr int kK = 32 * KS;  // k of one piece
+  constexpr bool kLoop = KS > 2;
+  u32x4 stage[kPer], vf[KS];
+  auto load_stage = [&](int k0) {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int idx = threadIdx.x + j * kFwdThreads;
+      if (WKN) {
+        const int kl = k0 + idx / (4 * NQ), n8 = (idx % (4 * NQ)) * 8;
+        stage[j] = ldg16_or(W + (long)kl * ldw + ncol0 + n8,
+                            idx < kPieces && ncol0 + n8 < P.d_out && kl < klim, zeros);
+      } else {
+        const int nl = idx / (4 * KS), k8 = k0 + (idx % (4 * KS)) * 8;
+        stage[j] = ldg16_or(W + (long)(ncol0 + nl) * ldw + k8,
+                            idx < kPieces && ncol0 + nl < P.d_out && k8 < klim, zeros);
+      }
+    }
+  };
+  auto load_v = [&](int k0) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int kk = k0 + 32 * ks + 8 * g;
+      vf[ks] = ldg16_or(P.v + (long)row * P.d_in + kk, kk < klim && row >= 0, zeros);
+    }
+  };
+  load_stage(0);
+  const bool read_y = a.beta != 0.0f;
+  u32x4 yold[NQ / 2][2];
+  load_y_lines<NQ>(yold, L, ncol0, P.d_out, read_y, zeros);
+  if (DROP) load_keep_bits<NQ>(L, a.drop, P.drop_bits, P.drop_pitch, ncol0, P.d_out, zeros);
+  load_v(0);
+  float prob[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) prob[j] = DROP ? drop_prob(a.drop, L.srow[j], dseg[j], zeros) : 0.0f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) L.scale[j] = (sseg[j] >= 0 && L.srow[j] >= 0) ? a.seg_scale[sseg[j]] : 1.0f;
+
+  f32x4 acc[NQ][2];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) acc[q][0] = acc[q][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int k0 = 0;; k0 += kK) {
+    // (opaque: the compiler otherwise keeps an induction register pair for each of a hundred addresses)
+    if (kLoop) asm volatile("" : "+s"(k0));
+    __syncthreads();  // every wave is done reading the previous piece's (or item's) weights
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int idx = threadIdx.x + j * kFwdThreads;
+      const int r_ = WKN ? idx / (4 * NQ) : idx / (4 * KS);
+      const int c_ = WKN ? (idx % (4 * NQ)) * 8 : (idx % (4 * KS)) * 8;
+      if (idx < kPieces) *reinterpret_cast<u32x4*>(&wlds[r_ * kPitch + c_]) = stage[j];
+    }
+    __syncthreads();
+    // (waves without a tile multiply zeros: whole waves only, MFMA runs with every lane, and every
+    // wave reaches the barriers)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          u32x4 wf;
+          if (WKN) {
+            // lane c names k row 32ks + 8g (+4) + c/4 and columns 32q + 4p + 8(c%4) .. +3; it
+            // receives column 32q + 4p + 8(c/4) + c%4 (its MFMA row's column) of four k rows
+            const uint16_t* base = &wlds[(32 * ks + 8 * g + (c >> 2)) * kPitch + 32 * q + 4 * p + 8 * (c & 3)];
+            const u32x2 q0 = lds_read_tr16(base), q1 = lds_read_tr16(base + 4 * kPitch);
+            wf = u32x4{q0[0], q0[1], q1[0], q1[1]};
+          } else {
+            wf = *reinterpret_cast<const u32x4*>(&wlds[(32 * q + 4 * p + mrow) * kPitch + 32 * ks + 8 * g]);
+          }
+          acc[q][p] = Num<DT>::mfma(wf, vf[ks], acc[q][p]);
+        }
+      // (the weight fragments of one k step at a time: all of them at once do not fit the registers)
+      if (kLoop) __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!kLoop || k0 + kK >= P.d_in) break;  // uniform over the workgroup
+    load_stage(k0 + kK);
+    load_v(k0 + kK);
+  }
+
+  __syncthreads();  // every wave has read its weights: the area is free for the accumulators
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (DROP) L.drop[j] = drop_params(prob[j]);
+  if (active) store_y_lines<DT, NQ, DROP>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
+  if (P.pt_a && yy == 0 && active) {  // by-products for the backward, when no fold has written them
+    const int rseg = a.seg_scale ? a.plan.tile_rseg[slot] : -1;
+    const float side_scale = (rseg >= 0 && row >= 0) ? a.seg_scale[rseg] : 1.0f;
+#pragma unroll 1
+    for (int kk = 8 * g; kk < P.d_in; kk += 32)
+      write_side<DT>(a, P, slot, row, kk, ldg16_or(P.v + (long)row * P.d_in + kk, kk < klim && row >= 0, zeros),
+                     side_scale);
+  }
+}
+
 template <int DT, int NQ, int KS, bool DIRECT, bool WKN, bool DROP = false>
 // (five workgroups a CU instead of the four the compiler's own register budget gives: more y
 // lines in flight per CU; worth 2 % on the prefill launch and 6 % on the fine-tune one)
@@ -1301,152 +1451,13 @@ template <int DT, int NQ, int KS, bool DIRECT, bool WKN, bool DROP = false>
 __global__ __launch_bounds__(kFwdThreads)
 __attribute__((amdgpu_waves_per_eu(DIRECT ? ((KS > 2 || NQ > 4) ? 3 : 5) : 1)))
 void expand_block_kernel(ExpandArgs a) {
-  static_assert(NQ % 2 == 0, "the output is written 64 columns at a time");
-  constexpr int kPitch = WKN ? 32 * NQ + 8 : 32 * KS + 8;  // LDS row pitch in 16-bit elements
-  // the staged weights and the area the accumulators change layout in share their LDS (the
-  // weights are done with when the accumulators are complete): five workgroups fit a CU at rank 64 too
-  constexpr int kWBytes = (WKN ? 32 * KS : 32 * NQ) * kPitch * 2;
-  constexpr int kOBytes = kFwdWaves * kTileRows * kOPitch * 4;
-  __shared__ __attribute__((aligned(16))) char smem[kWBytes > kOBytes ? kWBytes : kOBytes];
-  uint16_t* wlds = reinterpret_cast<uint16_t*>(smem);
-  float(*olds)[kTileRows * kOPitch] = reinterpret_cast<float(*)[kTileRows * kOPitch]>(smem);
+  __shared__ __attribute__((aligned(16))) char smem[ExpandBlockLds<NQ, KS, WKN>::kBytes];
   const int units = DIRECT ? 0 : tile_units<kBlkTiles>(a.plan, 0);
   const WorkRange wr = item_range<DIRECT>(a.items, units);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c = lane & 15, g = lane >> 4;
-  const int mrow = 8 * (c >> 2) + (c & 3);
-
   for (int V = wr.first; V < wr.last; V += wr.step) {
     int pj, yy, tb;
     if (!item_get<DIRECT>(a.items, V, units, &pj, &yy, &tb)) break;
-    const ExpandProj P = a.p[pj];
-    if (!P.y) continue;  // a projection this call leaves out (uniform over the workgroup)
-    const int ncol0 = yy * 32 * NQ;
-    if (ncol0 >= P.d_out) continue;  // a chunk row added to round the count up (uniform over the workgroup)
-    const int packed = uload(a.plan.blk, tb);
-    const int t0 = packed >> 3, cnt = packed & 7;
-    if (cnt == 0) continue;  // past the last block (direct mode); uniform over the workgroup
-    const int wid = uload(a.plan.tile_wid, t0);
-    if (!wid_ok(a.plan, wid)) continue;  // a negative adapter id (rows that no adapter serves) or one past the tables
-    const uint16_t* W = uload_ptr(P.w_ptrs, wid);
-    const int klim = rank_limit(a.plan, wid, P.d_in);  // k at or past it: zero padding of v and the weights
-    const int ldw = WKN ? P.ldw : rank_ld(a.plan, P.ldw, klim);  // [k][n] weights (A) have whole rows per rank
-    const bool active = wave < cnt;
-    const int tslot = (t0 + (active ? wave : 0)) * kTileRows;
-    const int slot = tslot + c;
-    const int row = active ? a.plan.tile_row[slot] : -1;  // row of the MFMA column this lane feeds
-    LineLane L;  // rows this lane reads and writes in y
-    L.orow = lane >> 3;
-    L.ocol = (lane & 7) * 8;
-    int sseg[2], dseg[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      L.srow[j] = active ? a.plan.tile_row[tslot + L.orow + 8 * j] : -1;
-      sseg[j] = (a.seg_scale && active) ? a.plan.tile_rseg[tslot + L.orow + 8 * j] : -1;  // -1 on empty slots
-      L.yrow[j] = P.y + (long)(L.srow[j] < 0 ? 0 : L.srow[j]) * P.d_out + ncol0 + L.ocol;
-      dseg[j] = DROP ? a.plan.tile_rseg[tslot + L.orow + 8 * j] : -1;
-    }
-    const uint16_t* zeros = reinterpret_cast<const uint16_t*>(a.plan.hdr + kHdrZeros);
-
-    // Every load of the item is issued before anything waits for one (predicated-off loads
-    // read zeros instead of being patched afterwards).
-    // weight chunk -> registers (written to LDS below): 32*NQ rows of 4*KS 16-byte pieces
-    constexpr int kPieces = 32 * NQ * 4 * KS;
-    constexpr int kPer = (kPieces + kFwdThreads - 1) / kFwdThreads;
-    constexpr int kK = 32 * KS;  // k of one piece
-    constexpr bool kLoop = KS > 2;
-    u32x4 stage[kPer], vf[KS];
-    auto load_stage = [&](int k0) {
-#pragma unroll
-      for (int j = 0; j < kPer; ++j) {
-        const int idx = threadIdx.x + j * kFwdThreads;
-        if (WKN) {
-          const int kl = k0 + idx / (4 * NQ), n8 = (idx % (4 * NQ)) * 8;
-          stage[j] = ldg16_or(W + (long)kl * ldw + ncol0 + n8,
-                              idx < kPieces && ncol0 + n8 < P.d_out && kl < klim, zeros);
-        } else {
-          const int nl = idx / (4 * KS), k8 = k0 + (idx % (4 * KS)) * 8;
-          stage[j] = ldg16_or(W + (long)(ncol0 + nl) * ldw + k8,
-                              idx < kPieces && ncol0 + nl < P.d_out && k8 < klim, zeros);
-        }
-      }
-    };
-    auto load_v = [&](int k0) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int kk = k0 + 32 * ks + 8 * g;
-        vf[ks] = ldg16_or(P.v + (long)row * P.d_in + kk, kk < klim && row >= 0, zeros);
-      }
-    };
-    load_stage(0);
-    const bool read_y = a.beta != 0.0f;
-    u32x4 yold[NQ / 2][2];
-    load_y_lines<NQ>(yold, L, ncol0, P.d_out, read_y, zeros);
-    if (DROP) load_keep_bits<NQ>(L, a.drop, P.drop_bits, P.drop_pitch, ncol0, P.d_out, zeros);
-    load_v(0);
-    float prob[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) prob[j] = DROP ? drop_prob(a.drop, L.srow[j], dseg[j], zeros) : 0.0f;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) L.scale[j] = (sseg[j] >= 0 && L.srow[j] >= 0) ? a.seg_scale[sseg[j]] : 1.0f;
-
-    f32x4 acc[NQ][2];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) acc[q][0] = acc[q][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int k0 = 0;; k0 += kK) {
-      // (opaque: the compiler otherwise keeps an induction register pair for each of a hundred addresses)
-      if (kLoop) asm volatile("" : "+s"(k0));
-      __syncthreads();  // every wave is done reading the previous piece's (or item's) weights
-#pragma unroll
-      for (int j = 0; j < kPer; ++j) {
-        const int idx = threadIdx.x + j * kFwdThreads;
-        const int r_ = WKN ? idx / (4 * NQ) : idx / (4 * KS);
-        const int c_ = WKN ? (idx % (4 * NQ)) * 8 : (idx % (4 * KS)) * 8;
-        if (idx < kPieces) *reinterpret_cast<u32x4*>(&wlds[r_ * kPitch + c_]) = stage[j];
-      }
-      __syncthreads();
-      // (waves without a tile multiply zeros: whole waves only, MFMA runs with every lane, and every
-      // wave reaches the barriers)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-        for (int q = 0; q < NQ; ++q)
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            u32x4 wf;
-            if (WKN) {
-              // lane c names k row 32ks + 8g (+4) + c/4 and columns 32q + 4p + 8(c%4) .. +3; it
-              // receives column 32q + 4p + 8(c/4) + c%4 (its MFMA row's column) of four k rows
-              const uint16_t* base = &wlds[(32 * ks + 8 * g + (c >> 2)) * kPitch + 32 * q + 4 * p + 8 * (c & 3)];
-              const u32x2 q0 = lds_read_tr16(base), q1 = lds_read_tr16(base + 4 * kPitch);
-              wf = u32x4{q0[0], q0[1], q1[0], q1[1]};
-            } else {
-              wf = *reinterpret_cast<const u32x4*>(&wlds[(32 * q + 4 * p + mrow) * kPitch + 32 * ks + 8 * g]);
-            }
-            acc[q][p] = Num<DT>::mfma(wf, vf[ks], acc[q][p]);
-          }
-        // (the weight fragments of one k step at a time: all of them at once do not fit the registers)
-        if (kLoop) __builtin_amdgcn_sched_barrier(0);
-      }
-      if (!kLoop || k0 + kK >= P.d_in) break;  // uniform over the workgroup
-      load_stage(k0 + kK);
-      load_v(k0 + kK);
-    }
-
-    __syncthreads();  // every wave has read its weights: the area is free for the accumulators
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      if (DROP) L.drop[j] = drop_params(prob[j]);
-    if (active) store_y_lines<DT, NQ, DROP>(olds[wave], acc, yold, L, c, g, ncol0, P.d_out, a.beta);
-    if (P.pt_a && yy == 0 && active) {  // by-products for the backward, when no fold has written them
-      const int rseg = a.seg_scale ? a.plan.tile_rseg[slot] : -1;
-      const float side_scale = (rseg >= 0 && row >= 0) ? a.seg_scale[rseg] : 1.0f;
-#pragma unroll 1
-      for (int kk = 8 * g; kk < P.d_in; kk += 32)
-        write_side<DT>(a, P, slot, row, kk, ldg16_or(P.v + (long)row * P.d_in + kk, kk < klim && row >= 0, zeros),
-                       side_scale);
-    }
+    expand_block_item<DT, NQ, KS, WKN, DROP>(a, pj, yy, tb, smem);
   }
 }
 
