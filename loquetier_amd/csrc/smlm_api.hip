@@ -513,12 +513,15 @@ int launch_reduce(int dtype, int S, int groups, hipStream_t st, ReduceArgs& a, b
     const int units = tile_units_max(a.T, S, groups, 1);
     const long items = (long)ceil_div(units, kBlkTiles) * ceil_div(a.d_out, 64) * a.nproj;
     a.units_max = items <= kDirectItems ? units : 0;
-    const int zero_blocks = a.zero.n ? a.zero.first[a.zero.n] : 0;
-    if (zero_blocks && !a.units_max) {  // (a launch that walks its items has no workgroups to spare)
-      const int rc = launch(zero_spans_kernel, dim3((unsigned)zero_blocks), dim3(256), st, a.zero);
+    const int zero_blocks = a.zero.n ? a.zero.first[a.zero.n] : 0, bit_blocks = a.bits.n ? a.bits.first[a.bits.n] : 0;
+    if (!a.units_max) {  // (a launch that walks its items has no workgroups to spare)
+      int rc = SMLM_OK;
+      if (zero_blocks) rc = launch(zero_spans_kernel, dim3((unsigned)zero_blocks), dim3(256), st, a.zero);
+      if (!rc && bit_blocks)
+        rc = launch(tile_bits_kernel, dim3((unsigned)bit_blocks), dim3(256), st, TileBitsArgs{a.bits, a.plan.tile_row});
       if (rc) return rc;
     }
-    const dim3 grid = a.units_max ? dim3((unsigned)(items + ceil_div(zero_blocks, kBlkTiles))) : work_grid(items);
+    const dim3 grid = a.units_max ? dim3((unsigned)(items + ceil_div(zero_blocks + bit_blocks, kBlkTiles))) : work_grid(items);
     return f16 ? launch_side_fold<SMLM_DTYPE_F16>(ks, grid, st, a) : launch_side_fold<SMLM_DTYPE_BF16>(ks, grid, st, a);
   }
   const long fours = ((long)a.T * (a.d_out / 4) + 255) / 256;
@@ -664,6 +667,7 @@ struct SideOut {
   const uint16_t* v2[kMaxProj];
   const float* scale;
   ZeroSpans zero;  // memory the fold's launch is to clear as well (n = 0: none)
+  TileBits bits;   // keep bits it is to turn (n = 0: none)
 };
 
 int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int nproj,
@@ -744,6 +748,7 @@ int run_shrink(int dtype, const PlanView& pv, int T, int S, int groups, int npro
   if (with_side) {
     ra.side_scale = side->scale;
     ra.zero = side->zero;
+    ra.bits = side->bits;
   }
   if (side_done) *side_done = with_side;
   return launch_reduce(dtype, S, groups, st, ra, with_side);
@@ -851,7 +856,7 @@ BwdLayout bwd_layout(int n_proj, int n_rows, int P, int NA, const int* h_in, con
     Q.v16 = take((size_t)n_rows * r * 2);
     Q.pt_a = take(r * slots * 2);
     Q.pt_b = take(r * slots * 2);
-    Q.bits = take((size_t)n_rows * (h_in[i] / 8));  // keep bits of x's dropout mask when the caller has none
+    Q.bits = take(slots * ceil_div(h_in[i], 64) * 8);  // keep bits of x's dropout mask, by tile slot
   }
   L.total = off;
   return L;
@@ -1398,27 +1403,36 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   // (In the row-major layout dV = dY B^T and dX = dV A^T read B [r, h_out] and A [h_in, r] the way the
   // forward reads A [r, h_in] and B [h_out, r], and v = x A reads A as [k][n].)
 
-  // The keep bits of x's dropout mask (projection i: the stream offset + i; the caller's bits of the
-  // projections lie end to end): the forward's when the caller kept them, else made here (same stream,
-  // same bits) so that the kernels below apply a stored mask either way.
-  const uint8_t* bits[kMaxProj] = {};
+  // The keep bits of x's dropout mask by tile slot (projection i: the stream offset + i; the caller's bits of the
+  // projections lie end to end, by row): the forward's when the caller kept them, turned behind the dV shrink, else made
+  // here (same stream, same bits), so that the kernels below apply a stored mask either way.
+  uint8_t* bits[kMaxProj] = {};
+  TileBits turn{};
   if (drop.seg_p) {
     size_t bits_off = 0;
+    const int tiles = tile_units_max(n_rows, P, NA, 1);
     for (int i = 0; i < n_proj; ++i) {
+      bits[i] = reinterpret_cast<uint8_t*>(ws + L.p[i].bits);
       if (drop.bits) {
-        bits[i] = drop.bits + bits_off;
+        turn.rows_bits[i] = drop.bits + bits_off;
+        turn.out[i] = bits[i];
+        turn.pitch[i] = h_in[i] / 8;
+        turn.chunks[i] = ceil_div(h_in[i], 64);
+        const long end = turn.first[i] + (long)tiles * ceil_div(turn.chunks[i], 16);
+        if (end > (1L << 30)) return SMLM_ERR_LIMIT;
+        turn.first[i + 1] = (int)end;
         bits_off += (size_t)drop.rows * (h_in[i] / 8);
       } else {
         DropArgs di = drop;
         const uint64_t off = (((uint64_t)drop.o1 << 32) | drop.o0) + (uint32_t)i;
         di.o0 = (uint32_t)off; di.o1 = (uint32_t)(off >> 32);
-        di.bits = reinterpret_cast<uint8_t*>(ws + L.p[i].bits);
+        di.bits = bits[i];
         di.bits_pitch = h_in[i] / 8;
-        bits[i] = di.bits;
         const DropBitsArgs ba{pv.hdr, pv.tile_row, pv.tile_rseg, di};
         if (products && (rc = launch(drop_bits_kernel, dim3((unsigned)pv.nt_max), dim3(256), st, ba))) return rc;
       }
     }
+    if (drop.bits) turn.n = n_proj, turn.rows = drop.rows < n_rows ? drop.rows : n_rows, turn.tiles = tiles;
   }
 
   float* partial[kMaxProj];
@@ -1476,7 +1490,7 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   }
   // (a function of the shapes and the option: the same in every call of a staged backward)
   const bool side_in_fold = bwd_all_folded(n_proj, n_rows, h_out, r);
-  if (side_in_fold) side.zero = tail;
+  if (side_in_fold) side.zero = tail, side.bits = turn;
   else if (tail.n && products &&
            (rc = launch(zero_spans_kernel, dim3((unsigned)tail.first[tail.n]), dim3(256), st, tail)))
     return rc;
@@ -1486,6 +1500,9 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
                                    self_planned ? &build : nullptr, true, side_in_fold ? &side : nullptr, &side_done)))
     return rc;
   if (products && side_done != side_in_fold) return SMLM_ERR_ARG;  // (cannot happen: both follow shrink_cfg)
+  if (products && turn.n && !side_in_fold &&
+      (rc = launch(tile_bits_kernel, dim3((unsigned)turn.first[turn.n]), dim3(256), st, TileBitsArgs{turn, pv.tile_row})))
+    return rc;
 
   // 4. dX = s dV A, and the slot-ordered transposed s*dV, s*v for step 5
   ExpandArgs ea{};
@@ -1505,7 +1522,6 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
     E.pt_b = side_in_fold ? nullptr : side.pt_b[i];
     E.v2 = side.v2[i];
     E.drop_bits = bits[i];
-    E.drop_pitch = h_in[i] / 8;
     if (h_in[i] > widest) widest = h_in[i];
   }
   ea.w_kn = rm ? 0 : 1;
@@ -1556,7 +1572,6 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
     Q.units_a = ceil_div(Q.chunks_a, walk);
     Q.unit0 = units;
     Q.drop_bits = bits[i];
-    Q.drop_pitch = h_in[i] / 8;
     units += Q.units_a + ceil_div(ceil_div(Q.h_out, kWgCols), walk);
   }
   wa.r = r;

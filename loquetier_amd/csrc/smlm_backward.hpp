@@ -23,8 +23,7 @@ struct WgradProj {
   int h_in, h_out, chunks_a;  // chunks_a = ceil(h_in/64) 64-column chunks of dA (dB: ceil(h_out/64))
   int units_a;                // units (walk chunks each) of dA: the projection's first units_a units work on dA
   int unit0;                  // first unit (blockIdx.x) of this projection; the projections' units lie end to end
-  const uint8_t* drop_bits;   // DROP kernels: keep bits of this projection's mask of x, [rows, drop_pitch]
-  long drop_pitch;
+  const uint8_t* drop_bits;   // DROP kernels: keep bits of this projection's mask of x, by tile slot (tile_bits)
 };
 
 struct WgradArgs {
@@ -82,7 +81,7 @@ __device__ __forceinline__ int wg_lds_row(int s) {
 // 26.5; 2754 rows with dropout at rank 32, two projections 26.0 and 24.6; 4096 rows at rank 16, one 15.2 and 14.2.
 //
 // DROP (dA only): the forward multiplied the dropped x, so dA = dV^T dropout(x).  The keep
-// bits (one byte per eight columns, the projection's drop_bits) travel with the rows and are applied while the
+// bits (one byte per eight columns, the projection's drop_bits) are requested with the rows and applied while the
 // rows are staged; every row of the workgroup belongs to one adapter, whose probability is read
 // once from the group's first segment.
 template <int DT, int NBJ, int NW, bool IS_A, bool DROP, bool ZSPLIT>
@@ -154,7 +153,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   };
   const int slot0 = wg_lds_row(rlow);
   const uint8_t* zero_bytes = reinterpret_cast<const uint8_t*>(zeros);
-  auto load_data = [&](int32_t rows, int n0, u32x4 (&val)[8], uint32_t (&keep)[DROP ? 8 : 1]) {
+  auto load_data = [&](int32_t rows, int step, int n0, u32x4 (&val)[8], uint32_t (&keep)[DROP ? 8 : 1]) {
     const bool col_ok = n0 + lcol < h;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -164,10 +163,12 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
       // reads the same lines for other ranks
       const uint16_t* q = Q + (long)row * h + n0 + lcol;
       val[u] = ZSPLIT ? ldg16_or(q, ok, zeros) : ldg16_or_nt(q, ok, zeros);
-      if (DROP) {  // rows at or past drop.rows keep everything: their byte is never applied
-        const bool dropped = ok && row < a.drop.rows;
-        keep[u] = *(const SMLM_GLOBAL uint8_t*)(dropped ? P.drop_bits + (long)row * P.drop_pitch + ((n0 + lcol) >> 3)
-                                                        : zero_bytes) | (dropped ? 0u : 0x100u);
+      if (DROP) {  // (rows at or past drop.rows keep everything: their byte is never applied)
+        const int tile = t_beg + kStepTiles * step + (u >> 1);
+        const bool in = step < n_steps && tile < t_end;
+        keep[u] = *(const SMLM_GLOBAL uint8_t*)(in ? P.drop_bits + tile_bits(tile, n0 / kWgCols, P.chunks_a, slot0 + 4 * (u & 1)) +
+                                                         (lane & 7)
+                                                   : zero_bytes) | (row < a.drop.rows ? 0u : 0x100u);
       }
     }
   };
@@ -188,7 +189,7 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   const int32_t row_first = load_rows(wave);  // the rows of the wave's first step: every chunk starts with them
   uint32_t keep[DROP ? 8 : 1];  // bit 8 set: the row is not dropped
   u32x4 val[8], pf[NBJ][2];
-  load_data(row_first, chunk_first * kWgCols, val, keep);
+  load_data(row_first, wave, chunk_first * kWgCols, val, keep);
   load_p(wave, pf);
   int32_t row_next = load_rows(wave + kWgWaves);
 
@@ -232,8 +233,8 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
       const bool wrap = last && more_chunks;
       u32x4 val_next[8];
       uint32_t keep_next[DROP ? 8 : 1];
-      if (wrap) load_data(row_first, n0 + kWgCols, val_next, keep_next);
-      else load_data(row_next, n0, val_next, keep_next);
+      if (wrap) load_data(row_first, wave, n0 + kWgCols, val_next, keep_next);
+      else load_data(row_next, step + kWgWaves, n0, val_next, keep_next);
       row_next = load_rows(wrap ? wave + kWgWaves : step + 2 * kWgWaves);
 
       if (DROP && drop_on) {  // uniform over the workgroup

@@ -890,6 +890,7 @@ struct ReduceArgs {
   const float* side_scale;  // SIDE folds: per segment, or null for 1
   ZeroSpans zero;           // SIDE folds, direct mode: memory the launch's last workgroups clear (the rows of dX
                             //   past the backward's own)
+  TileBits bits;            // ... and keep bits they bring into the order of the tiles
 };
 
 // Folds the k-split partial sums of a shrink launch, in split order, into the
@@ -954,7 +955,7 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(ReduceArgs a) {
 // columns, four tiles), a thread per slot and four columns.  The transposed rows go through LDS, so that they are
 // written 128 bytes at a time: two bytes a lane straight from the registers, 268 partitions of 2080 rows, six
 // projections at ranks up to 64: 16.0 us, so 12.0; 2048 rows, two projections at rank 128: 11.3 and 7.5.  The
-// launch's workgroups past its items clear a.zero.
+// launch's workgroups past its items clear a.zero and turn a.bits.
 constexpr int kSideThreads = kBlkTiles * 256;
 template <int DT, int KS>
 __global__ __launch_bounds__(kSideThreads) void side_fold_kernel(ReduceArgs a) {
@@ -965,8 +966,9 @@ __global__ __launch_bounds__(kSideThreads) void side_fold_kernel(ReduceArgs a) {
   const int groups = (tiles + kBlkTiles - 1) / kBlkTiles, cols = (a.d_out + kCols - 1) / kCols;
   const int items = groups * a.nproj * cols;
   if (a.units_max > 0 && (int)blockIdx.x >= items) {  // (uniform over the workgroup)
-    const int block = ((int)blockIdx.x - items) * kBlkTiles + (int)(threadIdx.x >> 8);
-    if (block < a.zero.first[a.zero.n]) zero_span_block(a.zero, block, threadIdx.x & 255);
+    const int block = ((int)blockIdx.x - items) * kBlkTiles + (int)(threadIdx.x >> 8), zeros = a.zero.first[a.zero.n];
+    if (block < zeros) zero_span_block(a.zero, block, threadIdx.x & 255);
+    else if (block - zeros < a.bits.first[a.bits.n]) tile_bits_item(a.bits, a.plan.tile_row, block - zeros, threadIdx.x & 255);
     return;
   }
   const int slot = threadIdx.x >> 4, q = threadIdx.x & 15;
@@ -1029,8 +1031,7 @@ struct ExpandProj {
   uint16_t* pt_a;             // block kernels, optional: scale*v by tile slot, transposed (side_piece)
   uint16_t* pt_b;             // optional: same treatment of v2 (a second [T, d_in] matrix)
   const uint16_t* v2;
-  const uint8_t* drop_bits;   // DROP kernels: keep bits of this projection's mask, [rows, drop_pitch]
-  long drop_pitch;
+  const uint8_t* drop_bits;   // DROP kernels: keep bits of this projection's mask, by tile slot (tile_bits)
 };
 
 constexpr int kMaxVsplit = 4;  // most k-split partials of v the wave kernel folds itself
@@ -1086,18 +1087,19 @@ struct LineLane {
 };
 
 // keep bits of the pieces a lane will store (DROP kernels): requested with the other loads of
-// the item; rows that are not dropped read a zero byte that is never applied
+// the item; what rows that are not dropped find there is never applied
 template <int NQ>
-__device__ __forceinline__ void load_keep_bits(LineLane& L, const DropArgs& d, const uint8_t* bits, long bits_pitch,
-                                               int ncol0, int d_out, const uint16_t* zeros) {
+__device__ __forceinline__ void load_keep_bits(LineLane& L, const uint8_t* bits, int tile, int ncol0, int d_out,
+                                               const uint16_t* zeros) {
+  const int chunks = (d_out + 63) / 64;
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int h = 0; h < NQ / 2; ++h) {
-      const int col = ncol0 + 64 * h + L.ocol;
-      const bool ok = L.srow[j] >= 0 && L.srow[j] < d.rows && col < d_out;  // whatever the row's probability
-      L.keep[h][j] = *(const SMLM_GLOBAL uint8_t*)(ok ? bits + (long)L.srow[j] * bits_pitch + (col >> 3)
-                                                      : reinterpret_cast<const uint8_t*>(zeros));
+      const bool ok = ncol0 + 64 * h < d_out;
+      L.keep[h][j] = *(const SMLM_GLOBAL uint8_t*)(
+          ok ? bits + tile_bits(tile, ncol0 / 64 + h, chunks, L.orow + 8 * j) + (L.ocol >> 3)
+             : reinterpret_cast<const uint8_t*>(zeros));
     }
 }
 
@@ -1375,7 +1377,7 @@ __device__ __forceinline__ void expand_block_item(const ExpandArgs& a, int pj, i
   const bool read_y = a.beta != 0.0f;
   u32x4 yold[NQ / 2][2];
   load_y_lines<NQ>(yold, L, ncol0, P.d_out, read_y, zeros);
-  if (DROP) load_keep_bits<NQ>(L, a.drop, P.drop_bits, P.drop_pitch, ncol0, P.d_out, zeros);
+  if (DROP) load_keep_bits<NQ>(L, P.drop_bits, tslot / kTileRows, ncol0, P.d_out, zeros);
   load_v(0);
   float prob[2];
 #pragma unroll
