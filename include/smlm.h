@@ -440,6 +440,20 @@ SMLM_API int smlm_segments_build(const int32_t* req_adapter, const int32_t* req_
                                  int32_t* n_seg, void* stream);
 
 /*
+ * What the layers of a step share by segment and by train partition, in one launch (the
+ * reference gathers on the host, layer by layer: src/loquetier_src/models/mixed_lora.py:207-216):
+ *   seg_out[s]  = table[seg_adapter[s]]             float [S]; NULL: not wanted
+ *   part_seg[p] = the segment that row starts[p] lies in, within [0, S)   int64 [P]
+ *                 (starts NULL: given instead of written)
+ *   part_out[p] = table[seg_adapter[part_seg[p]]]   float [P]; NULL: not wanted
+ * A negative id counts from the table's end; an id past it (its segment has no adapter) gives 1.
+ * All pointers are device memory; seg_indptr int32 [S + 1] is read with starts.
+ */
+SMLM_API int smlm_segment_scales(const int32_t* seg_adapter, int S, const float* table, int n_table, float* seg_out,
+                                 const int32_t* seg_indptr, const int32_t* starts, int P, int64_t* part_seg,
+                                 float* part_out, void* stream);
+
+/*
  * Copies `bytes` (a multiple of 4) of host memory to device memory (4-byte aligned) in the
  * arguments of launches on `stream`, 3584 bytes each: src has been read when the call
  * returns, and the host waits for nothing.  For the small tables a call needs (row

@@ -73,6 +73,7 @@ SIGNATURES = {
     "smlm_rms_norm_bwd_workspace_size": (_i, [_i, _i, _psz]),
     "smlm_rms_norm_bwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _vp]),
     "smlm_segments_build": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _vp, _vp]),
+    "smlm_segment_scales": (_i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp]),
     "smlm_put_words": (_i, [_vp, _vp, _sz, _vp]),
 }
 

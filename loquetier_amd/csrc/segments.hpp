@@ -73,4 +73,46 @@ __global__ __launch_bounds__(kPlanThreads) void segments_kernel(SegmentsArgs a) 
   for (int i = tid; i < a.R; i += kPlanThreads) a.seg_len[i] = a.seg_indptr[i + 1] - a.seg_indptr[i];
 }
 
+// ---- what a step's layers need by segment and by train partition -----------------------------------------
+// The scale of every segment's adapter, the segment that starts every partition and that segment's scale.  As tensor
+// expressions (widen the ids, index, search, subtract, clamp, index again) these were six launches of 5 us of host time
+// before a fine-tune step's first layer, two before a decode step's.
+struct SegmentScalesArgs {
+  const int32_t* seg_adapter;  // [S]
+  const float* table;          // [n_table], by adapter; seg_out == nullptr: not read
+  float* seg_out;              // [S]
+  const int32_t* seg_indptr;   // [S + 1], with starts
+  const int32_t* starts;       // [P] first rows of the partitions, or nullptr: part_seg is given
+  int64_t* part_seg;           // [P]
+  float* part_out;             // [P], with seg_out
+  int S, n_table, P;
+};
+__global__ __launch_bounds__(256) void segment_scales_kernel(SegmentScalesArgs a) {
+  // (an id counts from the end when it is negative, as indexes of tensors do; segments of ids past the table have no
+  // adapter, and their scale is never applied)
+  auto scale_of = [&](int seg) {
+    int id = a.seg_adapter[seg];
+    if (id < 0) id += a.n_table;
+    return id >= 0 && id < a.n_table ? a.table[id] : 1.0f;
+  };
+  const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (a.seg_out && i < a.S) a.seg_out[i] = scale_of(i);
+  if (i >= a.P) return;
+  int seg;
+  if (a.starts) {  // entries of seg_indptr up to the start, less one
+    const int at = a.starts[i];
+    int lo = 0, hi = a.S + 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if (a.seg_indptr[mid] <= at) lo = mid + 1;
+      else hi = mid;
+    }
+    seg = lo - 1 < 0 ? 0 : (lo - 1 < a.S ? lo - 1 : a.S - 1);
+    a.part_seg[i] = seg;
+  } else {
+    seg = (int)a.part_seg[i];
+  }
+  if (a.part_out) a.part_out[i] = scale_of(seg);
+}
+
 }  // namespace smlm

@@ -1730,6 +1730,19 @@ SMLM_API int smlm_segments_build(const int32_t* req_adapter, const int32_t* req_
   return launch(segments_kernel, dim3(1), dim3(kPlanThreads), (hipStream_t)stream, a);
 }
 
+SMLM_API int smlm_segment_scales(const int32_t* seg_adapter, int S, const float* table, int n_table, float* seg_out,
+                                 const int32_t* seg_indptr, const int32_t* starts, int P, int64_t* part_seg,
+                                 float* part_out, void* stream) {
+  if (S < 0 || P < 0 || n_table < 0) return SMLM_ERR_ARG;
+  if (S > kMaxSegments || P > kMaxSegments) return SMLM_ERR_LIMIT;
+  if (S == 0) return P == 0 ? SMLM_OK : SMLM_ERR_ARG;
+  if (seg_out && (!seg_adapter || !table || n_table == 0)) return SMLM_ERR_ARG;
+  if (P > 0 && (!part_seg || (starts && !seg_indptr) || (part_out && !seg_out))) return SMLM_ERR_ARG;
+  const int n = S > P ? S : P;
+  const SegmentScalesArgs a{seg_adapter, table, seg_out, seg_indptr, starts, part_seg, part_out, S, n_table, P};
+  return launch(segment_scales_kernel, dim3((unsigned)ceil_div(n, 256)), dim3(256), (hipStream_t)stream, a);
+}
+
 SMLM_API int smlm_put_words(void* dst, const void* src, size_t bytes, void* stream) {
   if (bytes == 0) return SMLM_OK;
   if (!dst || !src) return SMLM_ERR_ARG;

@@ -154,7 +154,7 @@ class MixedLoraContext:
             if isinstance(self._lora_ids, torch.Tensor):
                 self._seg_adapter = self._lora_ids.to(device=device, dtype=torch.int32)
             else:
-                self._seg_adapter = torch.tensor(self._lora_ids, dtype=torch.int32, device=device)
+                _, self._seg_adapter = kernel.put_ints(device, [], [int(i) for i in self._lora_ids])
         return self._seg_adapter
 
     def seg_adapter_long(self, device: torch.device) -> torch.Tensor:
@@ -199,10 +199,32 @@ class MixedLoraContext:
             if bwd_plan is None:   # no partitions, or none with rows
                 n_parts = len(part_adapter)
                 _, starts = kernel.put_ints(device, [], [int(t) for t in self._blen.train_partition][:n_parts])
-            else:
-                starts = bwd_plan.segment[:bwd_plan.S]
-            return (torch.searchsorted(plan.segment, starts, right=True) - 1).clamp_(0, max(plan.S - 1, 0))
+                return (torch.searchsorted(plan.segment, starts, right=True) - 1).clamp_(0, max(plan.S - 1, 0))
+            return kernel.segment_scales(self.seg_adapter(device), segment=plan.segment,
+                                         starts=bwd_plan.segment[:bwd_plan.S])[1]
         return self.memo(("part_segments", device), build)
+
+    def seg_scale(self, key, table: torch.Tensor, plan: kernel.SegmentPlan, train: bool) -> torch.Tensor:
+        """table[adapter of every segment], shared by the layers whose adapters have the same scales (`key`).  A training
+        step's partitions get theirs from the same launch, which also finds the segments they start in."""
+        device = table.device
+
+        def build():
+            ids = self.seg_adapter(device)
+            if device.type != "cuda" or not ids.is_contiguous() or ids.dim() != 1 or ids.numel() != plan.S:
+                return table[self.seg_adapter_long(device)]
+            bwd_plan = self.backward_tables(device)[0] if train else None
+            if bwd_plan is None:
+                return kernel.segment_scales(ids, table)[0]
+            known = self._step.get(("part_segments", device))
+            if known is None:
+                scale, known, part = kernel.segment_scales(ids, table, plan.segment, bwd_plan.segment[:bwd_plan.S])
+                self._step[("part_segments", device)] = known
+            else:
+                scale, _, part = kernel.segment_scales(ids, table, part_seg=known)
+            self._step[("gather", id(scale), id(known))] = part   # (what LayerStep.gather would compute)
+            return scale
+        return self.memo(("seg_scale", key, device), build)
 
     def train_bundle(self, device: torch.device, plan: kernel.SegmentPlan):
         """(training adapters in order, backward plan, partition -> training adapter, partition -> segment):
@@ -683,11 +705,6 @@ class MixedLoraLinear(nn.Module):
         if self.fused:
             # per-step tables come from the context (built once for all layers), per-layer ones from
             # the layer (built once per adapter set): nothing is copied from the host in here
-            seg_scale = None
-            if not self.is_scaled:
-                # (layers whose adapters have the same scales share one gather per step)
-                seg_scale = ctx.memo(("seg_scale", self._scaling_key, self.device),
-                                     lambda: self._scaling_f32[ctx.seg_adapter_long(self.device)])
             if result.dtype != self.dtype:
                 result = result.to(self.dtype)
             if not result.is_contiguous():
@@ -697,6 +714,8 @@ class MixedLoraLinear(nn.Module):
             same_dtype = result.dtype == torch_result_dtype
             ctx.check_adapter_ids(len(self.adapters))
             plan = ctx.plan(self.device, x.size(0))
+            seg_scale = None if self.is_scaled else ctx.seg_scale(self._scaling_key, self._scaling_f32, plan,
+                                                                  bool(weights) and blen.tlen > 0)
             if self._group is not None and not self._group[0].suspended and blen.tlen == 0 and not weights and not (
                     torch.is_grad_enabled() and (x.requires_grad or result.requires_grad)):
                 # a serving step: the group's members share one shrink launch

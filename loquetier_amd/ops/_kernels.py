@@ -222,7 +222,10 @@ def put_ints(device: torch.device, words64, words32) -> Tuple[torch.Tensor, torc
     """Small host tables as device tensors (int64, int32) that share one allocation, without waiting for the device:
     the words travel in a launch's arguments (smlm_put_words); long tables in one copy."""
     n64, n32 = len(words64), len(words32)
-    data = struct.pack(f"={n64}q{n32 + (n32 & 1)}i", *words64, *words32, *((0,) * (n32 & 1)))
+    try:
+        data = struct.pack(f"={n64}q{n32 + (n32 & 1)}i", *words64, *words32, *((0,) * (n32 & 1)))
+    except struct.error as e:
+        raise RuntimeError(f"a table entry does not fit its type: {e}") from None
     if len(data) > _PUT_BYTES or (data and torch.device(device).type != "cuda"):
         buf = torch.frombuffer(bytearray(data), dtype=torch.int64).to(device)
     else:
@@ -886,3 +889,32 @@ def segments_build(req_adapter: torch.Tensor, req_len: torch.Tensor):
                                              _stream(dev))
     _lib.check(rc, "segments_build")
     return seg_adapter, seg_len, seg_indptr, n_seg
+
+
+def segment_scales(seg_adapter: torch.Tensor, table: Optional[torch.Tensor] = None,
+                   segment: Optional[torch.Tensor] = None, starts: Optional[torch.Tensor] = None,
+                   part_seg: Optional[torch.Tensor] = None):
+    """(seg_scale, part_seg, part_scale) of a step, in one launch: table[seg_adapter] float32 [S] (None without a
+    table), the segment (int64) each row of `starts` lies in, and that segment's scale.  part_seg: known already, instead
+    of segment and starts; without either there are no partitions and both come back as None."""
+    dev, S = seg_adapter.device, seg_adapter.numel()
+    for t, n, dt in ((seg_adapter, "seg_adapter", torch.int32), (table, "table", torch.float32),
+                     (segment, "segment", torch.int32), (starts, "starts", torch.int32), (part_seg, "part_seg", torch.int64)):
+        if t is not None:
+            _check_input(t, n)
+            _check_dim(1, t, n)
+            if t.dtype != dt or t.device != dev:
+                raise RuntimeError(f"{n} must be {dt} on {dev}")
+    if starts is not None and (segment is None or segment.numel() != S + 1):
+        raise RuntimeError("segment must have one entry more than seg_adapter")
+    seg_out = None if table is None else torch.empty(S, dtype=torch.float32, device=dev)
+    P = starts.numel() if starts is not None else (0 if part_seg is None else part_seg.numel())
+    if starts is not None:
+        part_seg = torch.empty(P, dtype=torch.int64, device=dev)
+    part_out = torch.empty(P, dtype=torch.float32, device=dev) if table is not None and part_seg is not None else None
+    with _on(dev):
+        rc = _lib.load().smlm_segment_scales(_ptr(seg_adapter), S, _ptr(table), 0 if table is None else table.numel(),
+                                             _ptr(seg_out), _ptr(segment), _ptr(starts), P, _ptr(part_seg), _ptr(part_out),
+                                             _stream(dev))
+    _lib.check(rc, "segment_scales")
+    return seg_out, part_seg, part_out
