@@ -197,11 +197,13 @@ __device__ __forceinline__ u32x4 drop8_bits(u32x4 v, const DropRow& r, uint32_t 
   return o;
 }
 
-// Keep bits as dX and the weight gradients read them, by tile slot: [tile][64 columns][16 slots][8 bytes], a line for 64
-// columns of a tile.  (Read by row, the bits of 64 columns are eight bytes of a line a row, fetched by every XCD: under
-// dropout at rank 32 the weight gradients of two adapters of 1024 rows, two projections, took 25.5 us, without 18.9.)
-__device__ __forceinline__ long tile_bits(int tile, int chunk, int chunks, int slot) {
-  return (((long)tile * chunks + chunk) * kTileRows + slot) * 8;
+// Keep bits as dX and the weight gradients read them, by tile slot: [tile][64 columns][8 pairs of slots][8 bytes][2], a
+// line for 64 columns of a tile.  A pair is the slots s and s + 4 that a lane of the weight gradients stages one after the
+// other, so that their two bytes are one load and one register.  (Read by row, the bits of 64 columns are eight bytes of a
+// line a row, fetched by every XCD: under dropout at rank 32 the weight gradients of two adapters of 1024 rows, two
+// projections, took 25.5 us, without 18.9.)
+__device__ __forceinline__ long tile_bits(int tile, int chunk, int chunks, int slot, int byte) {
+  return (((long)tile * chunks + chunk) * 8 + ((slot & 3) | (slot >> 3) << 2)) * 16 + 2 * byte + (slot >> 2 & 1);
 }
 
 // The bits the forward left by row, by tile slot: an item of 256 threads is a tile and 1024 columns.
@@ -216,21 +218,30 @@ __device__ __forceinline__ void tile_bits_item(const TileBits& z, const int32_t*
   int i = 0;
 #pragma unroll
   for (int j = 1; j < 8; ++j) i += (j < z.n && item >= z.first[j]) ? 1 : 0;
-  const int in = item - z.first[i], tile = in % z.tiles, slot = thread >> 4;
+  const int in = item - z.first[i], tile = in % z.tiles;
+  // a wave takes two pairs of slots, the second of each 16 lanes after the first
+  const int pair = thread >> 5, second = thread >> 4 & 1, slot = (pair & 3) + 4 * second + 8 * (pair >> 2);
   const int chunk = in / z.tiles * 16 + (thread & 15);
   const int row = tile_row[tile * kTileRows + slot];
-  if (row < 0 || row >= z.rows || chunk >= z.chunks[i]) return;
-  const uint8_t* from = z.rows_bits[i] + (long)row * z.pitch[i] + 8 * chunk;
+  const bool ok = row >= 0 && row < z.rows && chunk < z.chunks[i];
   u32x2 v = {0u, 0u};
-  if (((reinterpret_cast<uintptr_t>(z.rows_bits[i]) | (uintptr_t)z.pitch[i]) & 7u) == 0) {  // uniform over the workgroup
-    v = *(const SMLM_GLOBAL u32x2*)from;
-  } else {
-    const int left = z.pitch[i] - 8 * chunk;
+  if (ok) {
+    const uint8_t* from = z.rows_bits[i] + (long)row * z.pitch[i] + 8 * chunk;
+    if (((reinterpret_cast<uintptr_t>(z.rows_bits[i]) | (uintptr_t)z.pitch[i]) & 7u) == 0) {  // uniform over the workgroup
+      v = *(const SMLM_GLOBAL u32x2*)from;
+    } else {
+      const int left = z.pitch[i] - 8 * chunk;
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if (e < left) v[e >> 2] |= (uint32_t)*(const SMLM_GLOBAL uint8_t*)(from + e) << (8 * (e & 3));
+      for (int e = 0; e < 8; ++e)
+        if (e < left) v[e >> 2] |= (uint32_t)*(const SMLM_GLOBAL uint8_t*)(from + e) << (8 * (e & 3));
+    }
   }
-  *(SMLM_GLOBAL u32x2*)(z.out[i] + tile_bits(tile, chunk, z.chunks[i], slot)) = v;
+  const bool write = ok | (__shfl_xor((int)ok, 16) != 0);
+  const uint32_t own = second ? v[1] : v[0], got = (uint32_t)__shfl_xor((int)(second ? v[0] : v[1]), 16);
+  const uint32_t lo = second ? got : own, hi = second ? own : got;  // four bytes of the first slot, of the second
+  if (write)
+    *(SMLM_GLOBAL u32x2*)(z.out[i] + tile_bits(tile, chunk, z.chunks[i], slot & ~4, 4 * second)) =
+        u32x2{__builtin_amdgcn_perm(hi, lo, 0x05010400u), __builtin_amdgcn_perm(hi, lo, 0x07030602u)};
 }
 struct TileBitsArgs {
   TileBits bits;
@@ -258,7 +269,7 @@ __global__ __launch_bounds__(256) void drop_bits_kernel(DropBitsArgs a) {
                                           reinterpret_cast<const uint16_t*>(a.hdr + kHdrZeros)));
   if (!r.on) return;  // rows that are not dropped never have their byte applied
   for (int cb = threadIdx.x & 15; cb < a.drop.bits_pitch; cb += 16)
-    a.drop.bits[tile_bits(tile, cb >> 3, chunks, slot) + (cb & 7)] = (uint8_t)drop_keep8(a.drop, r.thresh, row, cb);
+    a.drop.bits[tile_bits(tile, cb >> 3, chunks, slot, cb & 7)] = (uint8_t)drop_keep8(a.drop, r.thresh, row, cb);
 }
 
 }  // namespace smlm

@@ -774,8 +774,6 @@ template <int DT, bool DROP, int NW>
 int launch_bwd_tail(int nbj, dim3 grid, hipStream_t st, const BwdTailArgs& a) {
   const dim3 bl(kFwdThreads);
   if (a.e.p[0].d_in > 64) return launch(bwd_tail_kernel<DT, 4, NW, DROP, true, 4>, grid, bl, st, a);
-  if constexpr (wgrad_nbj_a(4, NW, DROP) < 4)  // (two dA workgroups a unit)
-    if (a.w.zcount > 1) return launch(bwd_tail_kernel<DT, 4, NW, DROP, true, 2>, grid, bl, st, a);
   if (nbj == 1) return launch(bwd_tail_kernel<DT, 1, NW, DROP, false, 1>, grid, bl, st, a);
   if (nbj == 2) return launch(bwd_tail_kernel<DT, 2, NW, DROP, false, 1>, grid, bl, st, a);
   return launch(bwd_tail_kernel<DT, 4, NW, DROP, false, 2>, grid, bl, st, a);
@@ -794,8 +792,11 @@ int launch_bwd_tail_dt(int nbj, bool split, dim3 grid, hipStream_t st, const Bwd
 // 16, 128 rows 7.3 / 6.8, 512 rows 14.3 / 8.7, 1024 rows 24.4 / 12.3; two of 256 rows 10.2 / 8.6, at rank 32 10.7 / 9.4,
 // at rank 64 12.0 / 10.9, at rank 128 13.1 / 16.1; four of 512 rows at rank 32 22.0 / 21.7, at rank 128 24.2 / 34.8; eight
 // of 512 rows at rank 16 30.9 / 31.4, at rank 32 32.6 / 36.3; sixteen of 512 at rank 128 113 / 132.
-// Under dropout one wave by itself has more to do: two of 256 rows at rank 16 16.8 / 10.6, eight of 512 rows at rank 128,
-// one projection, 61.3 / 42.2, sixteen of 256 rows at rank 32 27.9 / 30.6.
+// Under dropout four waves pay sooner, and with adapters of unequal rows sooner still (the longest, alone in a wave, is
+// what the launch waits for).  One projection, then two: four adapters of 256 rows at rank 16 13.2 / 9.5 and 15.1 / 14.6, at
+// rank 64 15.4 / 12.4 and 18.1 / 19.7; eight of 384 at rank 16 20.6 / 19.4 and 27.3 / 29.6, at rank 64 24.3 / 25.1 and 32.9 /
+// 42.8, the longest six times the shortest 38.7 / 24.3 and 43.6 / 42.5; at rank 128, where 64 ranks are a workgroup, 27.5 /
+// 37.4 and 52.5 / 73.6, unequal 38.7 / 37.8 and 52.6 / 74.4, so the line goes on rising there.
 // A launch of several projections has more pieces and would change over later, of one sooner (four adapters of 384 rows at
 // rank 32: one 14.4 / 10.8, two 18.2 / 19.0; two of 300 rows at rank 64: one 12.5 / 9.4, four 17.4 / 20.2); the rule does
 // not look at their number, so that it gives the bits that launches of one give.
@@ -805,7 +806,8 @@ bool wgrad_split(int rows, int NA, int r, bool drop) {
   auto most = [](long a, long b) { return a > b ? a : b; };
   if (r <= 16) return rows >= most(128, least(48 * m, drop ? 256 : 512));
   if (r <= 32) return rows >= most(128, drop ? least(64 * m, 512) : least(96 * m, most(512, 64 * m)));
-  return rows >= most(192, drop ? least(64 * m, 256) : least(128 * m, most(512, 96 * m)));
+  if (drop) return rows >= most(128, r <= 64 ? least(64 * m, 256) : 64 * m);
+  return rows >= most(192, least(128 * m, most(512, 96 * m)));
 }
 
 // Whether dX and the weight gradients (`waves`: their workgroups, of one wave or four) go out in one launch: while what
@@ -1582,10 +1584,8 @@ SMLM_API int smlm_lora_bwd_multi_ex(int n_proj, void* const* dx, void* const* co
   wa.drop = drop;  // dA against the dropped x
   // ranks above 64 are covered 64 at a time by workgroups of their own
   const int nbj = r <= 16 ? 1 : (r <= 32 ? 2 : 4);  // what launch_wgrad has kernels for
-  // (64 ranks a workgroup, or what a dA workgroup of the launched kernel takes when that is less)
-  const int z_per_64 = nbj / wgrad_nbj_a(nbj, split ? 4 : 1, drop.seg_p != nullptr);
   wa.units = units;
-  wa.zcount = ceil_div(r, 64) * z_per_64;
+  wa.zcount = ceil_div(r, 64);
   dim3 grid(wa.zcount > 1 ? round_up(units, kWgXcd) * wa.zcount : units, NA);
   if (stages & SMLM_BWD_DX) {
     const int dx_units = tile_units_max(n_rows, P, NA, kBlkTiles);

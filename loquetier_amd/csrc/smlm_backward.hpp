@@ -59,10 +59,9 @@ __device__ __forceinline__ int wg_lds_row(int s) {
 }
 
 // grid: (sum over the projections of their dA and dB units, NA), block 64*NW; with ZSPLIT several workgroups per unit,
-// one for every 64 ranks -- twice that for the kernel named at wgrad_nbj_a.  A unit is
-// `walk` neighbouring 64-column chunks of one projection's dA or dB.  A workgroup owns the unit's columns (and
-// up to 64 ranks) of one adapter's gradient and walks all of that adapter's tiles once per chunk, 64
-// gathered rows (four tiles, two MFMA k steps) per wave and loop step.  With
+// one for every 64 ranks.  A unit is `walk` neighbouring 64-column chunks of one projection's dA or dB.  A workgroup
+// owns the unit's columns (and up to 64 ranks) of one adapter's gradient and walks all of that adapter's tiles once per
+// chunk, 64 gathered rows (four tiles, two MFMA k steps) per wave and loop step.  With
 // NW = 4 (adapters with many rows each; walk = 1) the waves take steps round-robin and
 // their accumulators are summed through LDS in wave order; with NW = 1 (many
 // adapters with few rows each) a lone wave does it all and more workgroups fit
@@ -81,9 +80,11 @@ __device__ __forceinline__ int wg_lds_row(int s) {
 // 26.5; 2754 rows with dropout at rank 32, two projections 26.0 and 24.6; 4096 rows at rank 16, one 15.2 and 14.2.
 //
 // DROP (dA only): the forward multiplied the dropped x, so dA = dV^T dropout(x).  The keep
-// bits (one byte per eight columns, the projection's drop_bits) are requested with the rows and applied while the
-// rows are staged; every row of the workgroup belongs to one adapter, whose probability is read
-// once from the group's first segment.
+// bits (one byte per eight columns, the projection's drop_bits) are requested with the rows, those of two rows in one
+// load and one register, and applied while the rows are staged; every row of the workgroup belongs to one adapter, whose
+// probability is read once from the group's first segment.  With a register a row the one-wave kernel did not fit 64
+// ranks and took 32 a workgroup, the rows of x twice: 2080 rows in 268 partitions over 64 adapters of ranks up to 64,
+// six projections 225 us, so 141 (without dropout 132).
 template <int DT, int NBJ, int NW, bool IS_A, bool DROP, bool ZSPLIT>
 __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& P, int ad, int chunk_first, int n_chunks,
                                            int j0, char* smem) {
@@ -153,7 +154,8 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   };
   const int slot0 = wg_lds_row(rlow);
   const uint8_t* zero_bytes = reinterpret_cast<const uint8_t*>(zeros);
-  auto load_data = [&](int32_t rows, int step, int n0, u32x4 (&val)[8], uint32_t (&keep)[DROP ? 8 : 1]) {
+  auto load_data = [&](int32_t rows, int step, int n0, u32x4 (&val)[8], uint32_t (&keep)[4], uint32_t& off) {
+    off = 0;
     const bool col_ok = n0 + lcol < h;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -163,12 +165,13 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
       // reads the same lines for other ranks
       const uint16_t* q = Q + (long)row * h + n0 + lcol;
       val[u] = ZSPLIT ? ldg16_or(q, ok, zeros) : ldg16_or_nt(q, ok, zeros);
-      if (DROP) {  // (rows at or past drop.rows keep everything: their byte is never applied)
+      if (DROP) {
+        off |= row < a.drop.rows ? 0u : 1u << u;
+        if (u & 1) continue;
         const int tile = t_beg + kStepTiles * step + (u >> 1);
         const bool in = step < n_steps && tile < t_end;
-        keep[u] = *(const SMLM_GLOBAL uint8_t*)(in ? P.drop_bits + tile_bits(tile, n0 / kWgCols, P.chunks_a, slot0 + 4 * (u & 1)) +
-                                                         (lane & 7)
-                                                   : zero_bytes) | (row < a.drop.rows ? 0u : 0x100u);
+        keep[u >> 1] = *(const SMLM_GLOBAL uint16_t*)(
+            in ? P.drop_bits + tile_bits(tile, n0 / kWgCols, P.chunks_a, slot0, lane & 7) : zero_bytes);
       }
     }
   };
@@ -187,9 +190,9 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
 
   // the first step of the first chunk
   const int32_t row_first = load_rows(wave);  // the rows of the wave's first step: every chunk starts with them
-  uint32_t keep[DROP ? 8 : 1];  // bit 8 set: the row is not dropped
+  uint32_t keep[4], off;  // DROP: keep bits of the rows of `val`, two a register; bit u of `off`: row u is not dropped
   u32x4 val[8], pf[NBJ][2];
-  load_data(row_first, wave, chunk_first * kWgCols, val, keep);
+  load_data(row_first, wave, chunk_first * kWgCols, val, keep, off);
   load_p(wave, pf);
   int32_t row_next = load_rows(wave + kWgWaves);
 
@@ -232,16 +235,16 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
       const bool last = step + kWgWaves >= n_steps;
       const bool wrap = last && more_chunks;
       u32x4 val_next[8];
-      uint32_t keep_next[DROP ? 8 : 1];
-      if (wrap) load_data(row_first, wave, n0 + kWgCols, val_next, keep_next);
-      else load_data(row_next, step + kWgWaves, n0, val_next, keep_next);
+      uint32_t keep_next[4], off_next;
+      if (wrap) load_data(row_first, wave, n0 + kWgCols, val_next, keep_next, off_next);
+      else load_data(row_next, step + kWgWaves, n0, val_next, keep_next, off_next);
       row_next = load_rows(wrap ? wave + kWgWaves : step + 2 * kWgWaves);
 
       if (DROP && drop_on) {  // uniform over the workgroup
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          dr.on = (keep[u] & 0x100u) == 0;
-          val[u] = drop8_bits<DT>(val[u], dr, keep[u]);
+          dr.on = (off >> u & 1u) == 0;
+          val[u] = drop8_bits<DT>(val[u], dr, keep[u >> 1] >> (8 * (u & 1)));
         }
       }
 #pragma unroll
@@ -286,7 +289,8 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
       for (int u = 0; u < 8; ++u) val[u] = val_next[u];
       if (DROP) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) keep[u] = keep_next[u];
+        for (int u = 0; u < 4; ++u) keep[u] = keep_next[u];
+        off = off_next;
       }
     }
     // cross-wave sum in wave order, one rank block at a time; wave 0 ends up with the totals
@@ -355,9 +359,6 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& a, const WgradProj& 
   }
 }
 
-// rank blocks of 16 a dA workgroup takes (a dB workgroup: NBJ)
-constexpr int wgrad_nbj_a(int nbj, int nw, bool drop) { return (drop && nw == 1 && nbj == 4) ? 2 : nbj; }
-
 template <int NW>
 struct WgradLds {
   static constexpr int kStageBytes = NW * kWgSlots * kWgPitch * 2;
@@ -365,8 +366,7 @@ struct WgradLds {
   static constexpr int kBytes = kStageBytes > kTailBytes ? kStageBytes : kTailBytes;
 };
 
-// ZSPLIT: several workgroups share a unit, each taking other ranks (a.zcount of them: ranks above 64, and those above
-// 32 in the one-wave kernel under dropout, whose dA workgroups take 32 each).  They are
+// ZSPLIT (ranks above 64): several workgroups share a unit, each taking 64 other ranks (a.zcount of them).  They are
 // numbered eight apart, so that they run at about the same time on one XCD (workgroup number modulo eight) and the
 // rows of x and dY, which all of them read, come out of its L2 for the second (2048 rows, two projections
 // 4096 -> 4096 at rank 128, before the operand came in lines: 40.2 us with the ranks along the grid's z axis, 37.4 eight
@@ -387,18 +387,13 @@ __device__ __forceinline__ void wgrad_unit(const WgradArgs& a, int u, int ad, ch
   const WgradProj& P = a.p[pj];
   const int unit = u - P.unit0;
   const int walk = NW > 1 ? 1 : a.walk;
-  // The one-wave kernel that applies dropout to 64 ranks at a time does not fit the registers of a lane
-  // (200 bytes of spills, and twice the time of the kernel without dropout): its dA workgroups take 32 ranks
-  // each, two per unit where the others have one; dB, which no dropout touches, keeps 64.
-  constexpr int NBJ_A = wgrad_nbj_a(NBJ, NW, DROP), ZA = NBJ / NBJ_A;
   if (unit < P.units_a) {  // uniform over the workgroup
     const int first = unit * walk, left = P.chunks_a - first;
-    wgrad_body<DT, NBJ_A, NW, true, DROP, ZSPLIT>(a, P, ad, first, left < walk ? left : walk, 16 * NBJ_A * zi, smem);
+    wgrad_body<DT, NBJ, NW, true, DROP, ZSPLIT>(a, P, ad, first, left < walk ? left : walk, 16 * NBJ * zi, smem);
   } else {
-    if (zi % ZA) return;
     const int chunks_b = (P.h_out + kWgCols - 1) / kWgCols;
     const int first = (unit - P.units_a) * walk, left = chunks_b - first;
-    wgrad_body<DT, NBJ, NW, false, false, ZSPLIT>(a, P, ad, first, left < walk ? left : walk, 16 * NBJ * (zi / ZA), smem);
+    wgrad_body<DT, NBJ, NW, false, false, ZSPLIT>(a, P, ad, first, left < walk ? left : walk, 16 * NBJ * zi, smem);
   }
 }
 

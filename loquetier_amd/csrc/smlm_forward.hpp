@@ -1098,7 +1098,7 @@ __device__ __forceinline__ void load_keep_bits(LineLane& L, const uint8_t* bits,
     for (int h = 0; h < NQ / 2; ++h) {
       const bool ok = ncol0 + 64 * h < d_out;
       L.keep[h][j] = *(const SMLM_GLOBAL uint8_t*)(
-          ok ? bits + tile_bits(tile, ncol0 / 64 + h, chunks, L.orow + 8 * j) + (L.ocol >> 3)
+          ok ? bits + tile_bits(tile, ncol0 / 64 + h, chunks, L.orow + 8 * j, L.ocol >> 3)
              : reinterpret_cast<const uint8_t*>(zeros));
     }
 }

@@ -237,8 +237,7 @@ def test_backward_dropout_exact(K, oracle, gpu_device, case, dt, with_v, with_bi
 @pytest.mark.parametrize("tp", [[0, 33, 90], [0, 1100, 2300]], ids=["one-wave", "four-waves"])
 @pytest.mark.parametrize("r", [40, 48, 56])
 def test_backward_dropout_ranks_between_32_and_64(K, oracle, gpu_device, r, tp, packed, dt):
-    """Ranks of three and four blocks of 16: the weight gradient's dA workgroups take 32 ranks each under dropout
-    when an adapter has few rows (one-wave workgroups), 64 when it has many."""
+    """Ranks of three and four blocks of 16, in one-wave workgroups (an adapter has few rows) and in four-wave ones."""
     d = gpu_device
     part_ad, h_in, h_out, n_rows = [0, 1], 192, 136, tp[-1]
     ranks = [r, 8 if r == 48 else 32] if packed else [r, r]
