@@ -227,7 +227,7 @@ def model_step_bench(args, torch, K, finetune=True):
     """The path as the reference drives it (src/loquetier_src/models/mixed_lora.py:173-218, 224 LoRA linears
     per model forward): 32 layers x (q, k, v, o, gate, up, down) of Llama-2-7B through MixedLoraLinear(fused=True)
     with ONE MixedLoraContext.update per step.  The base layers hand back preallocated outputs (their GEMMs
-    are not part of this path).  Reports, per layer call: host time of an eager step (Python + ctypes + launch),
+    are not part of this path).  Reports, per layer call: host time of an eager step (layer code + operator + launch),
     GPU time of the same step replayed from a graph, for the decode batch (forward) and, eager only, for the
     fine-tune + serve batch (forward + backward through autograd)."""
     from loquetier_amd.kernel_utils import BatchLenInfo
@@ -829,8 +829,9 @@ def run_workload(args, cfg, torch, K, probe, brief=False):
                               "bwd_wgrad_bytes_per_launch")]
         gbps = bwd_bytes / (all_us * 1e-6) / 1e9
         backward = dict(algorithmic_bytes=bwd_bytes, us=round(all_us, 3), achieved=round(gbps, 1), unit="GB/s",
-                        frac=round(gbps / HBM_PEAK_GBPS, 4), launches_per_step=4,
-                        note="all projections in one set of launches (smlm_lora_bwd_multi_ex), plan reused; "
+                        frac=round(gbps / HBM_PEAK_GBPS, 4),
+                        note="all projections in one set of four launches (smlm_lora_bwd_multi_ex; three where dX and the "
+                             "weight gradients share one), plan reused; "
                              "algorithmic bytes count dY, x once, dX, A/B and dA/dB of the training adapters, v, dV")
 
     # ---- what plain streaming kernels reach at these launch sizes (loquetier_amd/csrc/stream_probe.hip:

@@ -374,12 +374,13 @@ SMLM_API int smlm_lora_bwd_ex(void* dx, void* const* da_ptrs, void* const* db_pt
 
 /*
  * The backward of up to 8 projections of one batch in one set of launches (one dV product, one
- * fold, one dX product, one weight-gradient launch for all of them): the projections share the
+ * fold, one dX product, one weight-gradient launch for all of them, the last two together where
+ * they are short): the projections share the
  * partition plan, the adapters' indices, the rank and the scale, as q/k/v/o or gate/up/down of
  * a layer do.  dx, da_ptrs, db_ptrs, dy, x, v, a_ptrs, b_ptrs, h_in, h_out are HOST arrays of
  * n_proj entries, each entry what smlm_lora_bwd_ex takes for one projection; v is NULL or
  * names the saved intermediate of every projection.  Results equal n_proj calls of
- * smlm_lora_bwd_ex bit for bit (the kernels and their launch shapes per projection are the same).
+ * smlm_lora_bwd_ex bit for bit (every sum is taken in the same order).
  * With dropout, projection i uses the stream offset + i and the caller's keep bits of the
  * projections lie end to end, as smlm_lora_fwd_multi_ex leaves them.  No counterpart in the
  * reference, whose backward is a Python loop per layer and partition
