@@ -103,6 +103,12 @@ void* stream(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().
 Tensor bytes(size_t n, const Tensor& like) {
   return at::empty({(int64_t)n}, like.options().dtype(at::kByte).requires_grad(false));
 }
+// A saved tensor comes back from whatever hooks its program has set (torch.autograd.graph.saved_tensors_hooks), which torch
+// does not look at: what the kernels take for granted is checked in every backward, with the Python functions' words.
+void check_input(const Tensor& t, const char* name) {
+  TORCH_CHECK(t.is_cuda(), name, " must be a CUDA tensor");
+  TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
+}
 const Tensor* optional(PyObject* o, bool* ok) {
   if (o == Py_None) return nullptr;
   *ok = *ok && plain(o);
@@ -218,6 +224,15 @@ struct RmsNorm : public Function<RmsNorm> {
     const Tensor &x = s[0], &w = s[1], &m = s[2];
     const Tensor g = grads[0].contiguous();
     Tensor dx = at::empty_like(x), dw = at::empty_like(w);
+    check_input(dx, "dx"), check_input(dw, "dw"), check_input(g, "grad_output");
+    check_input(x, "x"), check_input(w, "w"), check_input(m, "rms");
+    TORCH_CHECK(g.sizes() == x.sizes(), "dx / grad_output must match x and dw must match w");
+    TORCH_CHECK(w.dim() == 1 && w.size(0) == x.size(1), "w must have one entry per column of x");
+    TORCH_CHECK(m.scalar_type() == at::kFloat && m.numel() == x.size(0), "rms must be float32 with one entry per row");
+    TORCH_CHECK(x.scalar_type() == g.scalar_type() && w.scalar_type() == g.scalar_type(),
+                "dx, dw, grad_output, x, w must share one dtype");
+    TORCH_CHECK(x.device() == g.device() && w.device() == g.device() && m.device() == g.device(),
+                "dx, dw, grad_output, x, w, rms must share one device");
     const int rows = (int)x.size(0), cols = (int)x.size(1);
     size_t need = 0;
     check(lib.rms_bwd_size(rows, cols, &need), "smlm_rms_norm_bwd_workspace_size");
@@ -233,7 +248,17 @@ struct RmsNorm : public Function<RmsNorm> {
 struct Backward {
   Tensor g, dx;
   int rows, tail;  // rows of the plan; rows of dx when the call is to clear those past the plan's
-  Backward(const Tensor& grad, const Tensor& x, int64_t first, int64_t rows_) : g(grad.contiguous()), rows((int)rows_) {
+  // x, v: as they came back from the forward, where x had h_in columns and v `rank`
+  Backward(const Tensor& grad, const Tensor& x, const Tensor& v, int64_t first, int64_t rows_, int64_t h_in, int64_t rank)
+      : g(grad.contiguous()), rows((int)rows_) {
+    check_input(x, "x");
+    TORCH_CHECK(g.size(0) >= rows && x.dim() == 2 && x.size(0) >= rows, "dy, x and dx need at least plan.T rows");
+    TORCH_CHECK(x.scalar_type() == g.scalar_type() && v.scalar_type() == g.scalar_type(),
+                "dx, dy, x, v must share one dtype");
+    TORCH_CHECK(v.dim() == 2 && v.size(0) >= rows && v.size(1) == rank && v.is_contiguous(),
+                "v must be a contiguous [>=n_rows, rank] tensor (of every projection or of none)");
+    TORCH_CHECK(x.size(1) == h_in, "dx and x must have the same width");
+    TORCH_CHECK(x.device() == g.device() && v.device() == g.device(), "dx, dy, x, v must share one device");
     dx = at::empty({g.size(0), x.size(1)}, g.options());
     if (first > 0) dx.narrow(0, 0, first).zero_();
     tail = rows < g.size(0) ? (int)g.size(0) : 0;
@@ -261,7 +286,7 @@ struct Backward {
 struct AddState : torch::CustomClassHolder {
   PyObject *wa, *wb, *s;  // during the forward only
   std::vector<int64_t> tp;
-  int64_t rank, train_len, h_out;
+  int64_t rank, train_len, h_in, h_out;
 };
 
 struct AddLora : public Function<AddLora> {
@@ -312,7 +337,7 @@ struct AddLora : public Function<AddLora> {
       part_adapter.push_back((int32_t)a);
     }
     const int NA = (int)first.size();
-    const Backward call(grads[0], x, st->tp[0], st->tp[P]);
+    const Backward call(grads[0], x, v, st->tp[0], st->tp[P], st->h_in, rank);
     variable_list out(2 + s.size() - 2);
     out[0] = call.dx;
     // addresses of dA, dB, A and B, then where the partitions start and their adapters
@@ -355,7 +380,7 @@ struct AddLora : public Function<AddLora> {
 // ---- fused_add_lora: the step's tables stay Python's ----
 struct FusedState : torch::CustomClassHolder {
   PyObject* step = nullptr;  // mixed_lora.LayerStep
-  int64_t rank, first;       // first: rows before the first partition
+  int64_t rank, h_in, first;  // first: rows before the first partition
   Tensor part_scale, train_rank;
   std::vector<int64_t> part_adapter;
   std::vector<int64_t> shape_a, shape_b;  // of all dA, all dB: [adapters, ...]
@@ -391,7 +416,7 @@ struct FusedAddLora : public Function<FusedAddLora> {
       THPObjectPtr a_tab = attr(st->step, names.a_tab), b_tab = attr(st->step, names.b_tab);
       THPObjectPtr lay = attr(st->step, names.grad_layout), ws = attr(st->step, names.workspace);
       const Tensor &a = THPVariable_Unpack(a_tab.get()), &b = THPVariable_Unpack(b_tab.get());
-      const Backward call(grads[0], x, st->first, plan.T);
+      const Backward call(grads[0], x, v, st->first, plan.T, st->h_in, st->rank);
       const Tensor ga = at::empty(st->shape_a, call.g.options()), gb = at::empty(st->shape_b, call.g.options());
       // the device tables of the gradients' addresses, kept by address: torch's allocator hands the same blocks out step
       // after step
@@ -525,6 +550,7 @@ PyObject* py_add_lora(PyObject*, PyObject* const* p, Py_ssize_t n) {
       !is(s, at::kInt, 1) || s.size(0) < 2 || !is(wa, at::kLong, 1) || !is(wb, at::kLong, 1) ||
       wa.size(0) != s.size(0) - 1 || wb.size(0) != s.size(0) - 1 || s.device() != x.device())
     Py_RETURN_NONE;
+  st->h_in = x.size(1);
   st->h_out = integer(PyTuple_GET_ITEM(p[0], 1));
   st->rank = integer(p[5]);
   st->train_len = integer(p[6]);
@@ -621,6 +647,7 @@ PyObject* py_fused_add_lora(PyObject*, PyObject* const* p, Py_ssize_t n) {
   // what autograd would refuse is left to the general path, which refuses it before anything is computed
   if (at::GradMode::is_enabled() && (result.requires_grad() && result.is_leaf())) Py_RETURN_NONE;
   if (result.is_inference() || x.is_inference()) Py_RETURN_NONE;
+  st->h_in = x.size(1);
   const Tensor v = at::empty({x.size(0), st->rank}, x.options());
   if (scale) {
     THPObjectPtr g(PyObject_CallMethodObjArgs(step, names.gather, scale_o.get(), segs.get(), nullptr));
