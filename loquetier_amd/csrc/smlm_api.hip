@@ -792,11 +792,15 @@ int launch_bwd_tail_dt(int nbj, bool split, dim3 grid, hipStream_t st, const Bwd
 // 16, 128 rows 7.3 / 6.8, 512 rows 14.3 / 8.7, 1024 rows 24.4 / 12.3; two of 256 rows 10.2 / 8.6, at rank 32 10.7 / 9.4,
 // at rank 64 12.0 / 10.9, at rank 128 13.1 / 16.1; four of 512 rows at rank 32 22.0 / 21.7, at rank 128 24.2 / 34.8; eight
 // of 512 rows at rank 16 30.9 / 31.4, at rank 32 32.6 / 36.3; sixteen of 512 at rank 128 113 / 132.
-// Under dropout four waves pay sooner, and with adapters of unequal rows sooner still (the longest, alone in a wave, is
-// what the launch waits for).  One projection, then two: four adapters of 256 rows at rank 16 13.2 / 9.5 and 15.1 / 14.6, at
-// rank 64 15.4 / 12.4 and 18.1 / 19.7; eight of 384 at rank 16 20.6 / 19.4 and 27.3 / 29.6, at rank 64 24.3 / 25.1 and 32.9 /
-// 42.8, the longest six times the shortest 38.7 / 24.3 and 43.6 / 42.5; at rank 128, where 64 ranks are a workgroup, 27.5 /
-// 37.4 and 52.5 / 73.6, unequal 38.7 / 37.8 and 52.6 / 74.4, so the line goes on rising there.
+// It ends at 512 rows: the rule is given the average, and an adapter of several times that, alone in a wave, is what the
+// launch waits for.  Equal adapters, then the longest four (eight) times the average: eight of 768 rows at rank 64, one
+// projection, 31.7 / 31.2 and 81.8 / 33.4; sixteen of 1024 at rank 32 61.3 / 64.0 and 114 / 66.7 (190 / 77.0), at rank 128
+// 109 / 115 and 142 / 119 (234 / 120), two projections 202 / 214 and 203 / 223 (281 / 234).
+// Under dropout four waves pay sooner, and with adapters of unequal rows sooner still.  One projection, then two: four
+// adapters of 256 rows at rank 16 13.2 / 9.5 and 15.1 / 14.6, at rank 64 15.4 / 12.4 and 18.1 / 19.7; eight of 384 at rank
+// 16 20.6 / 19.4 and 27.3 / 29.6, at rank 64 24.3 / 25.1 and 32.9 / 42.8, the longest six times the shortest 38.7 / 24.3
+// and 43.6 / 42.5; at rank 128, where 64 ranks are a workgroup, 27.5 / 37.4 and 52.5 / 73.6, unequal 38.7 / 37.8 and 52.6 /
+// 74.4, so up to 512 rows the line goes on rising there.
 // A launch of several projections has more pieces and would change over later, of one sooner (four adapters of 384 rows at
 // rank 32: one 14.4 / 10.8, two 18.2 / 19.0; two of 300 rows at rank 64: one 12.5 / 9.4, four 17.4 / 20.2); the rule does
 // not look at their number, so that it gives the bits that launches of one give.
@@ -804,10 +808,11 @@ bool wgrad_split(int rows, int NA, int r, bool drop) {
   const long m = (long)NA * ceil_div(r, 64);
   auto least = [](long a, long b) { return a < b ? a : b; };
   auto most = [](long a, long b) { return a > b ? a : b; };
-  if (r <= 16) return rows >= most(128, least(48 * m, drop ? 256 : 512));
-  if (r <= 32) return rows >= most(128, drop ? least(64 * m, 512) : least(96 * m, most(512, 64 * m)));
-  if (drop) return rows >= most(128, r <= 64 ? least(64 * m, 256) : 64 * m);
-  return rows >= most(192, least(128 * m, most(512, 96 * m)));
+  long line;
+  if (r <= 16) line = drop ? least(48 * m, 256) : 48 * m;
+  else if (r <= 32) line = drop ? 64 * m : 96 * m;
+  else line = drop ? (r <= 64 ? least(64 * m, 256) : 64 * m) : 128 * m;
+  return rows >= most(r > 32 && !drop ? 192 : 128, least(line, 512));
 }
 
 // Whether dX and the weight gradients (`waves`: their workgroups, of one wave or four) go out in one launch: while what
