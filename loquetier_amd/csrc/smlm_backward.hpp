@@ -405,8 +405,14 @@ __global__ __launch_bounds__(NW * kWaveSize) __attribute__((amdgpu_waves_per_eu(
 }
 
 // dX and the weight gradients in one launch: its first `wgrad` workgroups are the weight gradients' (of the one-wave kind
-// four to a workgroup, eight numbers apart), the others take dX's items (tile block, column chunk) as
-// expand_block_kernel does.  Neither needs anything of the other once the fold of dV has written what both read.
+// four to a workgroup), the others take dX's items (tile block, column chunk) as expand_block_kernel does.  Neither needs
+// anything of the other once the fold of dV has written what both read.
+// The four units of a workgroup lie `wgrad` numbers apart, so that the units of a long adapter go to a CU each: eight
+// numbers apart they were of one adapter, and a CU had four of the longest while others had none.  us, whole backward, two
+// launches / one, units eight apart / one, far apart: sixteen adapters averaging 128 rows at rank 16, the longest eight
+// times that, 47.0 / 50.2 / 42.3, four averaging 400 at rank 64, the longest three times that, 57.2 / 60.2 / 53.0, sixteen
+// of 64 rows each at rank 16 25.3 / 23.3 / 23.4.  With ZSPLIT the units that share rows must stay near each other (sixteen
+// averaging 128 rows at rank 128, the longest eight times that, two projections, 107.8 / 104.0 / 111.7).
 struct BwdTailArgs {
   WgradArgs w;
   ExpandArgs e;
@@ -423,8 +429,9 @@ __global__ __launch_bounds__(kFwdThreads) __attribute__((amdgpu_waves_per_eu(2))
         wgrad_unit<DT, NBJ, NW, DROP, ZSPLIT>(a.w, (int)blockIdx.x % a.wx, (int)blockIdx.x / a.wx, smem);
     } else {
       const int wave = threadIdx.x >> 6;
-      const int id = __builtin_amdgcn_readfirstlane((int)blockIdx.x / kWgXcd * (kFwdWaves * kWgXcd) + wave * kWgXcd +
-                                                    (int)blockIdx.x % kWgXcd);
+      const int b = (int)blockIdx.x;  // (either way the unit's number modulo eight is the workgroup's: its XCD)
+      const int id = __builtin_amdgcn_readfirstlane(
+          ZSPLIT ? b / kWgXcd * (kFwdWaves * kWgXcd) + wave * kWgXcd + b % kWgXcd : b + wave * a.wgrad);
       if (id < a.wx * a.wy)
         wgrad_unit<DT, NBJ, NW, DROP, ZSPLIT>(a.w, id % a.wx, id / a.wx, smem + wave * WgradLds<NW>::kBytes);
     }
