@@ -817,14 +817,23 @@ bool wgrad_split(int rows, int NA, int r, bool drop) {
 
 // Whether dX and the weight gradients (`waves`: their workgroups, of one wave or four) go out in one launch: while what
 // they move takes little longer than starting and draining two.  Together they hold as many registers and as much LDS as
-// the weight gradients, so fewer of dX's workgroups are resident, which costs where both run at the memory's rate; and
-// workgroups of four one-wave units wait for the longest.  Same bits.  us, two launches / one, h_in = h_out = 4096 (MB: x,
-// dY and dX, then the weights): one adapter of 64 rows at rank 16 (2 + 0) 8.8 / 6.3, of 1024 rows at rank 128 (25 + 6)
-// 19.3 / 14.7; three of 200 rows, four projections at rank 64 (59 + 19) 26.8 / 24.9; two of 1024 rows, two projections at
-// rank 16 (101 + 3) 24.6 / 23.1, four projections (201 + 6) 43.9 / 49.2, at rank 128 (201 + 50) 89.0 / 93.5, two (101 + 25)
-// 43.2 / 40.3; one of 1024 rows, four projections at rank 32 (101 + 3) 26.6 / 27.7; eight of 256 rows, two at rank 32
-// (101 + 13) 27.2 / 28.8; 64 of 32 rows at rank 32 (50 + 50, 8192 waves) 31.2 / 32.8.  Under dropout, two of 1377 rows, two
-// projections at rank 32 (135 + 3) 43.8 / 42.0; eight of 1000 rows (197 + 6) 63.2 / 67.0; 64 of 32 rows at rank 32 35.8 / 40.1.
+// the weight gradients, so fewer of dX's workgroups are resident, which costs where both run at the memory's rate.  Same
+// bits.  us, whole backward, two launches / one, h_in = h_out = 4096, operands from memory (700 MB of them in turn; the
+// numbers in parentheses: MB of x, dY and dX, then of the weights):
+//   up to rank 64, by the bytes of both: two adapters of 1024 rows at rank 16, two projections (101 + 2) 40.6 / 38.3, one of
+//     646 at rank 32, six (95 + 5) 45.1 / 42.3; sixteen of 128 at rank 32, two (101 + 25) 46.6 / 47.6, four of 512 at rank
+//     64, two (101 + 13) 52.4 / 53.1
+//   ... and where they are workgroups of one wave, by their number (3072 are resident at rank 16, 2048 above; dX's own
+//     kernel keeps five or six waves a SIMD, here three or two): at rank 16 4096 26.4 / 23.9, 16384 47.1 / 48.6; at rank 32
+//     3584 28.2 / 27.9, 4096 28.5 / 29.6, 32768 113 / 132; at rank 64 4096 of few rows 34.2 / 34.7, of 64 rows and the
+//     longest of eight times that 50.0 / 47.7; under dropout 4096 at rank 32 48.2 / 48.4, at rank 64 48.0 / 43.8
+//   above rank 64, where dX's own kernel keeps no more than three waves a SIMD, by the rows alone: one adapter of 1024 rows
+//     at rank 128 (25 + 3) 36.3 / 31.4, two, two projections (101 + 13) 76.3 / 72.6, 64 of 32 rows, two (101 + 403, 32768
+//     workgroups) 173 / 169, unequal ones alike (sixteen averaging 128 rows, the longest eight times that 75.1 / 66.6);
+//     sixteen of 512 rows (201 + 50) 141 / 144, 64 of 128 (201 + 201) 158 / 163
+//   under dropout dX and the gradients have more to do between their loads: two of 1377 rows, two projections at rank 16
+//     (135 + 2) 56.0 / 52.5, at rank 32 62.6 / 63.0, eight of 1000 at rank 32 (197 + 6) 76.2 / 80.6; sixteen of 128, two at
+//     rank 128 (101 + 101) 99.2 / 92.2, 32 of 96 (151 + 201) 168 / 176
 bool bwd_one_launch(int n_proj, int n_rows, int NA, int r, const int* h_in, const int* h_out, bool drop, bool split,
                     long waves) {
   double rows = 0, weights = 0;  // bytes
@@ -832,8 +841,8 @@ bool bwd_one_launch(int n_proj, int n_rows, int NA, int r, const int* h_in, cons
     rows += 2.0 * n_rows * (2.0 * h_in[i] + h_out[i]);
     weights += 2.0 * NA * r * (2.0 * h_in[i] + h_out[i]);
   }
-  if (r > 64) return rows < 200e6;
-  return (split || waves <= 4096) && rows + weights < (drop ? 140e6 : (n_proj > 2 ? 80e6 : 105e6));
+  if (r > 64) return rows < 200e6 && (!drop || rows + weights < 330e6);
+  return (split || waves <= (drop || r <= 16 || r > 32 ? 4096 : 3584)) && rows + weights < (drop ? 140e6 : 105e6);
 }
 
 struct BwdProjLayout {
