@@ -338,6 +338,9 @@ struct AddLora : public Function<AddLora> {
     }
     const int NA = (int)first.size();
     const Backward call(grads[0], x, v, st->tp[0], st->tp[P], st->h_in, rank);
+    for (int p = 0; p < 2 * P; ++p)
+      TORCH_CHECK(s[2 + p].device() == call.g.device() && s[2 + p].scalar_type() == call.g.scalar_type(),
+                  "the weights must share dy's dtype and device");
     variable_list out(2 + s.size() - 2);
     out[0] = call.dx;
     // addresses of dA, dB, A and B, then where the partitions start and their adapters

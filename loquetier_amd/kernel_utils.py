@@ -161,6 +161,8 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
             for b in bufs:
                 b.zero_()
     else:
+        if any(w.device != dev or w.dtype != dt for w in weight_list[: 2 * n_parts]):  # (a saved-tensor hook's doing)
+            raise RuntimeError("the weights must share dy's dtype and device")
         pairs, part_adapter = _unique_adapters(weight_list[: 2 * n_parts])
         da = [torch.empty_like(wa) for wa, _ in pairs]
         db = [torch.empty_like(wb) for _, wb in pairs]

@@ -760,6 +760,8 @@ def smlm_lora_backward_multi(dxs, da_ptrs, db_ptrs, dys, xs, vs, a_ptrs, b_ptrs,
             raise RuntimeError("v must be a contiguous [>=n_rows, rank] tensor (of every projection or of none)")
         if dxs[i].size(1) != xs[i].size(1):
             raise RuntimeError("dx and x must have the same width")
+        if any(t is not None and t.device != dys[0].device for t in (dxs[i], dys[i], xs[i], v)):
+            raise RuntimeError("dx, dy, x, v must share one device")
     code = _dtype_code(dys[0])
     widths_in = tuple(t.size(1) for t in xs)
     widths_out = tuple(t.size(1) for t in dys)

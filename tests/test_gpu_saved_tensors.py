@@ -7,9 +7,9 @@ from test_gpu_host_path import _layer, general, host, table  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
-# (pad: elements apart in memory; wider: more bytes than the kernels would read)
+# (strided: elements apart in memory; wider: more bytes than the kernels would read; elsewhere: on the host)
 FORMS = {"strided": lambda t: t.t().contiguous().t() if t.dim() == 2 and min(t.shape) > 1 else torch.stack([t, t], -1)[..., 0],
-         "wider": lambda t: t.double()}
+         "wider": lambda t: t.double(), "elsewhere": lambda t: t.cpu()}
 
 
 def hooks(which, change):
@@ -68,10 +68,14 @@ def layer_case(d):
 # saves its weight first.)
 CASES = [(rms_case, 0, "strided", "must be contiguous"), (rms_case, 0, "wider", "must share one dtype"),
          (rms_case, 1, "wider", "must share one dtype"), (rms_case, 2, "wider", "float32 with one entry per row"),
+         (rms_case, 2, "elsewhere", "rms must be a CUDA tensor"),
          (add_case, 0, "strided", "x must be contiguous"), (add_case, 0, "wider", "must share one dtype"),
          (add_case, 1, "strided", "v must be a contiguous"), (add_case, 1, "wider", "must share one dtype"),
+         *[(add_case, w, form, "the weights must share dy's dtype and device") for w in (2, 3) for form in ("wider", "elsewhere")],
+         (add_case, 0, "elsewhere", "must be a CUDA tensor"), (add_case, 1, "elsewhere", "must share one device"),
          (layer_case, 1, "strided", "x must be contiguous"), (layer_case, 1, "wider", "must share one dtype"),
-         (layer_case, 2, "strided", "v must be a contiguous"), (layer_case, 2, "wider", "must share one dtype")]
+         (layer_case, 2, "strided", "v must be a contiguous"), (layer_case, 2, "wider", "must share one dtype"),
+         (layer_case, 2, "elsewhere", "must share one device")]
 
 
 @pytest.mark.parametrize("case,which,form,text", CASES, ids=[f"{c[0].__name__}-{c[1]}-{c[2]}" for c in CASES])
