@@ -8,10 +8,12 @@
 // Every function here takes a call only in its plain form (tensors that are exactly torch's, on the current device, of
 // the shapes and types the operator wants; no tracing, no functorch transform, no dispatch mode, no forward-mode
 // tangent) and otherwise hands it back, having done nothing: the Python functions of the same names remain the general
-// path and raise the errors.  Nothing is kept from one call to the next.
+// path and raise the errors.  Nothing is kept from one call to the next but the device tables of the gradients' addresses
+// that the layers' backward keeps in either language (grad_tabs).
 #include <ATen/ATen.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Device.h>
 #include <torch/csrc/Exceptions.h>
@@ -421,8 +423,9 @@ struct FusedAddLora : public Function<FusedAddLora> {
       const Tensor &a = THPVariable_Unpack(a_tab.get()), &b = THPVariable_Unpack(b_tab.get());
       const Backward call(grads[0], x, v, st->first, plan.T, st->h_in, st->rank);
       const Tensor ga = at::empty(st->shape_a, call.g.options()), gb = at::empty(st->shape_b, call.g.options());
-      // the device tables of the gradients' addresses, kept by address: torch's allocator hands the same blocks out step
-      // after step
+      // the device tables of the gradients' addresses, kept by stream and address: torch's allocator hands the same blocks
+      // out step after step.  Not while a graph is recorded: a table made then holds its words from the graph's first
+      // replay on, and one that was kept may be dropped before the graph is.
       auto item = [](PyObject* dict, PyObject* key) {
         PyObject* o = PyDict_GetItemWithError(dict, key);
         if (!o) {
@@ -432,10 +435,12 @@ struct FusedAddLora : public Function<FusedAddLora> {
         return o;
       };
       PyObject* known = item(lay, names.grad_tabs);
-      THPObjectPtr where(Py_BuildValue("(KK)", (unsigned long long)ga.data_ptr(), (unsigned long long)gb.data_ptr()));
+      const bool keep = c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+      THPObjectPtr where(Py_BuildValue("(KKK)", (unsigned long long)ga.data_ptr(), (unsigned long long)gb.data_ptr(),
+                                       (unsigned long long)stream(ga)));
       if (!where) throw python_raised();
       THPObjectPtr tabs;
-      if (PyObject* hit = PyDict_GetItemWithError(known, where)) {
+      if (PyObject* hit = keep ? PyDict_GetItemWithError(known, where) : nullptr) {
         Py_INCREF(hit);
         tabs = THPObjectPtr(hit);
       } else {
@@ -446,8 +451,8 @@ struct FusedAddLora : public Function<FusedAddLora> {
         THPObjectPtr tb(THPVariable_Wrap(at::add(ob, (int64_t)gb.data_ptr())));
         tabs = THPObjectPtr(PyTuple_Pack(2, ta.get(), tb.get()));
         if (!tabs) throw python_raised();
-        if (PyDict_Size(known) >= 64) PyDict_Clear(known);
-        if (PyDict_SetItem(known, where, tabs) < 0) throw python_raised();
+        if (keep && PyDict_Size(known) >= 64) PyDict_Clear(known);
+        if (keep && PyDict_SetItem(known, where, tabs) < 0) throw python_raised();
       }
       const Tensor ta = THPVariable_Unpack(PyTuple_GET_ITEM(tabs.get(), 0));
       const Tensor tb = THPVariable_Unpack(PyTuple_GET_ITEM(tabs.get(), 1));

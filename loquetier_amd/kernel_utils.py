@@ -128,12 +128,16 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
         lay = step.grad_layout
         uniform, known = lay["grad_uniform"], lay["grad_tabs"]
         # addresses of the gradients: device arithmetic, no copy from the host; torch's allocator hands the
-        # same blocks out step after step, so the tables of an address are kept
+        # same blocks out step after step, so the tables of an address (and stream) are kept.  Not while a graph
+        # is recorded: a table made then holds its words from the graph's first replay on, and one that was kept
+        # may be dropped before the graph is.
+        if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            known = {}
         if uniform is not None:   # matrices of one shape: one tensor for the dA, one for the dB
             NA, sa, sb = uniform
             ga, gb = torch.empty((NA,) + sa, dtype=dt, device=dev), torch.empty((NA,) + sb, dtype=dt, device=dev)
             da, db = ga.unbind(0), gb.unbind(0)
-            bufs, where = (ga, gb), (ga.data_ptr(), gb.data_ptr())
+            bufs, where = (ga, gb), (ga.data_ptr(), gb.data_ptr(), kernel._stream(dev))
             tabs = known.get(where)
             if tabs is None:
                 tabs = (lay["grad_offsets_a"] + where[0], lay["grad_offsets_b"] + where[1])
@@ -142,10 +146,10 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
             mats = [buf[o: o + shape[0] * shape[1]].view(shape) for o, shape in lay["grad_shapes"]]
             NA = len(mats) // 2
             da, db = mats[:NA], mats[NA:]
-            bufs, where = (buf,), buf.data_ptr()
+            bufs, where = (buf,), (buf.data_ptr(), kernel._stream(dev))
             tabs = known.get(where)
             if tabs is None:
-                both = lay["grad_offsets"] + where
+                both = lay["grad_offsets"] + where[0]
                 tabs = (both[:NA], both[NA:])
         if where not in known:
             if len(known) >= 64:

@@ -391,7 +391,7 @@ class LayerStep:
         # where the gradients go (MixedLoraLinear._train_tables): byte offsets of dA_0.., dB_0.. inside one buffer
         # (grad_offsets) or inside one buffer for the dA and one for the dB (grad_offsets_a / _b, when the matrices
         # have one shape: grad_uniform), [(offset in elements, shape)] in the same order (grad_shapes, grad_numel),
-        # and the device tables of the gradients' addresses by buffer address (grad_tabs)
+        # and the device tables of the gradients' addresses by buffer address and stream (grad_tabs)
         self.grad_layout = None
 
     def gather(self, table: torch.Tensor, index: torch.Tensor) -> torch.Tensor:

@@ -222,3 +222,45 @@ def test_what_is_refused_stays_refused(host, gpu_device):
         with general(host), pytest.raises(RuntimeError) as python:
             K.smlm_lora_forward(*args, **kw)
         assert str(native.value) == str(python.value)
+
+
+@pytest.mark.parametrize("ranks", [[16, 16], [8, 16]], ids=["one-shape", "two-shapes"])
+@pytest.mark.parametrize("path", ["native", "general"])
+def test_recorded_layer_steps_share_a_pool(host, gpu_device, path, ranks):
+    """Two graphs of one memory pool: the second is recorded over the first one's freed gradients and replayed first, so it
+    must make the tables of their addresses for itself."""
+    from loquetier_amd.kernel_utils import BatchLenInfo
+    d = gpu_device
+    ctx, layer = _layer(d, "bf16", ranks, 16, 512, 384, 5)
+    layer.set_trainable([0, 1])
+    blen = BatchLenInfo([(1, 40), (1, 24)], [], 0, [], d)
+    segment = torch.tensor([0, 40, 64], dtype=torch.int32, device=d)
+    x = torch.randn(64, 512, device=d).to(torch.bfloat16).requires_grad_(True)
+    up = torch.randn(64, 384, device=d).to(torch.bfloat16)
+    params = [p for p in layer.parameters() if p.requires_grad]
+    step = lambda: torch.autograd.grad(layer(x), [x, *params], up)
+    with general(host) if path == "general" else contextlib.nullcontext():
+        ctx.update(blen=blen, lora_ids=[0, 1], lora_len=None, segment=segment, train_idx=[0, 1])
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            for _ in range(2):
+                want = [t.clone() for t in step()]
+            side.synchronize()
+            kept = {k: dict(t["grad_tabs"]) for k, t in layer._train_tabs.items()}
+            first, second = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+            with torch.cuda.graph(first, stream=side):
+                outs = step()
+            del outs
+            with torch.cuda.graph(second, pool=first.pool(), stream=side):
+                outs = step()
+    assert kept and all(t["grad_tabs"].keys() == kept[k].keys() for k, t in layer._train_tabs.items())
+    for _ in range(3):
+        for graph in (second, first, second):
+            for t in outs:
+                t.fill_(7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            if graph is second:
+                same(outs, want)
+        same(step(), want)
