@@ -145,6 +145,14 @@ class MixedLoraContext:
             return True
         self.memo(("ids_ok", n_adapters), check)
 
+    @staticmethod
+    def _ints(device: torch.device, words) -> torch.Tensor:
+        """An int32 table that the step keeps.  Not while a graph is recorded: the words would only arrive with the
+        graph's first replay, and a call outside the graph would find the table there before."""
+        if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("a step's tables cannot be made while a graph is recorded: run the step once before")
+        return kernel.put_ints(device, [], words)[1]
+
     def seg_adapter(self, device: torch.device) -> torch.Tensor:
         """Adapter id of every segment as a device tensor.  `lora_ids` may already be one (int32,
         e.g. from segments.build_segments_device, whose arrays keep the request count as capacity
@@ -154,7 +162,7 @@ class MixedLoraContext:
             if isinstance(self._lora_ids, torch.Tensor):
                 self._seg_adapter = self._lora_ids.to(device=device, dtype=torch.int32)
             else:
-                _, self._seg_adapter = kernel.put_ints(device, [], [int(i) for i in self._lora_ids])
+                self._seg_adapter = self._ints(device, [int(i) for i in self._lora_ids])
         return self._seg_adapter
 
     def seg_adapter_long(self, device: torch.device) -> torch.Tensor:
@@ -185,7 +193,7 @@ class MixedLoraContext:
             part_adapter = [order.index(int(i)) for i in self._train_idx[:n_parts]]
             if n_parts == 0 or tp[-1] == 0:
                 return None, part_adapter
-            _, parts = kernel.put_ints(device, [], tp + part_adapter)
+            parts = self._ints(device, tp + part_adapter)
             plan = kernel.SegmentPlan(parts[:n_parts + 1], parts[n_parts + 1:], tp[-1],
                                       defer=True)  # built by the step's first backward call
             return plan, part_adapter
@@ -198,7 +206,7 @@ class MixedLoraContext:
             bwd_plan, part_adapter = self.backward_tables(device)
             if bwd_plan is None:   # no partitions, or none with rows
                 n_parts = len(part_adapter)
-                _, starts = kernel.put_ints(device, [], [int(t) for t in self._blen.train_partition][:n_parts])
+                starts = self._ints(device, [int(t) for t in self._blen.train_partition][:n_parts])
                 return (torch.searchsorted(plan.segment, starts, right=True) - 1).clamp_(0, max(plan.S - 1, 0))
             return kernel.segment_scales(self.seg_adapter(device), segment=plan.segment,
                                          starts=bwd_plan.segment[:bwd_plan.S])[1]

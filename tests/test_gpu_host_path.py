@@ -243,6 +243,11 @@ def test_recorded_layer_steps_share_a_pool(host, gpu_device, path, ranks):
         ctx.update(blen=blen, lora_ids=[0, 1], lora_len=None, segment=segment, train_idx=[0, 1])
         side = torch.cuda.Stream()
         with torch.cuda.stream(side):
+            layer.base_layer(x)
+            side.synchronize()
+            with pytest.raises(RuntimeError, match="run the step once before"):
+                with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=side):
+                    layer(x)
             for _ in range(2):
                 want = [t.clone() for t in step()]
             side.synchronize()
