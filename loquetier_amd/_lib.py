@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes as C
 import importlib.util
 import os
+import warnings
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "lib", "libsmlm_hip.so")
@@ -107,17 +108,30 @@ HOST_PATH = os.path.join(_PKG_DIR, "lib", "_smlm_host.so")
 _host = None
 
 
+class _NoHost:
+    """In the native host path's place where it cannot be loaded: declines every call, and the Python functions take it."""
+    forward = staticmethod(lambda *args: False)
+    rms_norm = add_lora = fused_add_lora = staticmethod(lambda *args: None)
+
+
 def host(default_workspace=None):
-    """The native host path (csrc/host_path.cpp), bound to the HIP library; raises RuntimeError when it has not been built."""
+    """The native host path (csrc/host_path.cpp), bound to the HIP library.  It is built against one torch: where there is
+    none for this one, the Python functions do its work, slower on the host, and a warning says so."""
     global _host
     if _host is None:
-        if not os.path.exists(HOST_PATH):
-            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m loquetier_amd.build`.")
+        import torch
         lib = load()
-        spec = importlib.util.spec_from_file_location("_smlm_host", HOST_PATH)
-        mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)
-        mod.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES}, default_workspace)
+        try:
+            spec = importlib.util.spec_from_file_location("_smlm_host", HOST_PATH)
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            if not torch.__version__.startswith(mod.torch_version):
+                raise ImportError(f"built for torch {mod.torch_version}, this is {torch.__version__}")
+            mod.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES}, default_workspace)
+        except (ImportError, OSError) as e:
+            warnings.warn(f"{HOST_PATH} cannot be used ({e}): build it with `python -m loquetier_amd.build`.",
+                          RuntimeWarning, stacklevel=3)
+            mod = _NoHost
         _host = mod
     return _host
 

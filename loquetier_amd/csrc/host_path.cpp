@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/object_ptr.h>
+#include <torch/version.h>
 
 #include <string.h>
 
@@ -718,5 +719,7 @@ PyMODINIT_FUNC PyInit__smlm_host(void) {
            s("train_len"), s("train_partition"), s("dropout"), s("adapter_rank"), s("part_segments"), s("bwd_plan"),
            s("part_adapter"), s("a_tab"), s("b_tab"), s("grad_layout"), s("gather"), s("grad_uniform"), s("grad_tabs"),
            s("grad_offsets_a"), s("grad_offsets_b")};
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
 }

@@ -41,6 +41,23 @@ def test_missing_library_fails_loudly(lib, monkeypatch):
         lib.load()
 
 
+@pytest.mark.parametrize("why", ["missing", "another torch"])
+def test_without_the_native_host_path_the_python_functions_serve(lib, monkeypatch, tmp_path, why):
+    monkeypatch.setattr(lib, "_host", None)
+    if why == "missing":
+        monkeypatch.setattr(lib, "HOST_PATH", str(tmp_path / "_smlm_host.so"))
+    else:
+        monkeypatch.setattr(torch, "__version__", "1.0.0")
+    with pytest.warns(RuntimeWarning, match="cannot be used"):
+        host = lib.host()
+    assert lib.host() is host   # (and warns once)
+    assert host.forward(*range(12)) is False
+    assert host.rms_norm(1, 2) is host.add_lora(*range(10)) is host.fused_add_lora(*range(5)) is None
+    monkeypatch.undo()
+    from loquetier_amd.ops import _kernels
+    assert torch.__version__.startswith(_kernels._host().torch_version)
+
+
 def test_size_queries(lib):
     assert lib.size_query("smlm_tmp_size", 0) == 0
     assert lib.size_query("smlm_tmp_size", 256) == 64 * 256
