@@ -1,5 +1,6 @@
 """The native host path against the Python functions it stands before: the same bits, the same refusals, and the forms of
 a call it must leave to them (hooks on saved tensors, functorch transforms, forward-mode tangents, tracing, subclasses)."""
+import concurrent.futures
 import contextlib
 
 import pytest
@@ -39,9 +40,26 @@ def same(a, b):
             assert p.dtype == q.dtype and p.shape == q.shape and torch.equal(p, q)
 
 
-def both(host, run):
-    """run() natively and through the general path; the native function must have taken it."""
-    native = run()
+@contextlib.contextmanager
+def taken(host, by):
+    """The native function `by` takes every call it is given within the block, and is given one."""
+    native, answers = getattr(host, by), []
+
+    def watched(*args):
+        answers.append(native(*args))
+        return answers[-1]
+    setattr(host, by, watched)
+    try:
+        yield
+    finally:
+        setattr(host, by, native)
+    assert answers and not any(a is None or a is False for a in answers)
+
+
+def both(host, run, by):
+    """run() natively, where the function `by` must take its calls, and through the general path."""
+    with taken(host, by):
+        native = run()
     with general(host):
         same(native, run())
     return native
@@ -65,7 +83,7 @@ def test_rms_norm(host, gpu_device, dt, rows, cols, need):
         o = rms_norm.apply(x, w, 1e-5)
         o.backward(up[:, ::2])       # (a gradient that is not contiguous)
         return o.detach(), x.grad, w.grad
-    want = both(host, run)
+    want = both(host, run, "rms_norm")
     for mode in (torch.no_grad, torch.inference_mode):
         with mode():
             same([rms_norm.apply(x, w, 1e-5)], want[:1])
@@ -137,7 +155,7 @@ def test_add_lora(host, gpu_device, dt, tp, ids, tail):
         y = add_lora.apply((T, h_out), x, wa, wb, s, r, tp[-1], tp, *weights)
         grads = torch.autograd.grad(y, [x] + [w for i in sorted(set(ids)) for w in (A[i], B[i])], up)
         return [y.detach(), *grads]
-    want = both(host, run)
+    want = both(host, run, "add_lora")
     with torch.no_grad():
         same([add_lora.apply((T, h_out), x, wa, wb, s, r, tp[-1], tp, *weights)], want[:1])
     packed = []
@@ -191,7 +209,8 @@ def test_layers(host, gpu_device, dt, ranks, lens, train, tail):
             y = layer(x)
         y.backward(up)
         return [y.detach().clone(), x.grad, *[p.grad for p in params]]
-    want = both(host, run)
+    # (gradients of two shapes are Python's; the forward below it is not)
+    want = both(host, run, "fused_add_lora" if len({ranks[i] for i in train}) == 1 else "forward")
     assert all(g is not None for g in want)
     for _ in range(3):   # the tables of the gradients' addresses are kept: other blocks, the same values
         same(run(), want)
@@ -201,6 +220,38 @@ def test_layers(host, gpu_device, dt, ranks, lens, train, tail):
     with torch.no_grad():
         ctx.update(blen=blen, lora_ids=ids, lora_len=lens_t, segment=segment, train_idx=train)
         same([layer(x)], want[:1])
+
+
+def test_streams_and_threads_at_once(host, gpu_device):
+    """Four threads, a stream each, against the same calls one after the other."""
+    from loquetier_amd.kernel_utils import add_lora, rms_norm
+    d, r, T = gpu_device, 16, 300
+    s = torch.tensor([0, 180, T], dtype=torch.int32, device=d)
+
+    def inputs(seed):
+        g = torch.Generator(d).manual_seed(seed)
+        rand = lambda *n: torch.randn(*n, generator=g, device=d).to(torch.bfloat16)
+        A, B = [rand(r, 1024).requires_grad_(True) for _ in range(2)], [rand(512, r).requires_grad_(True) for _ in range(2)]
+        return rand(T, 1024).requires_grad_(True), rand(1024).requires_grad_(True), A, B, table(A, d), table(B, d), rand(T, 512)
+    cases = [inputs(i) for i in range(4)]
+
+    def run(case):
+        x, w, A, B, wa, wb, up = case
+        y = add_lora.apply((T, 512), rms_norm.apply(x, w, 1e-5), wa, wb, s, r, T, [0, 180, T], A[0], B[0], A[1], B[1])
+        return [y.detach(), *torch.autograd.grad(y, [x, w, *A, *B], up)]
+    want = [run(c) for c in cases]
+    torch.cuda.synchronize()
+
+    def work(case):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            outs = [run(case) for _ in range(8)]
+        stream.synchronize()
+        return outs
+    with taken(host, "add_lora"), taken(host, "rms_norm"), concurrent.futures.ThreadPoolExecutor(4) as pool:
+        for outs, ref in zip(pool.map(work, cases), want):
+            for o in outs:
+                same(o, ref)
 
 
 def test_what_is_refused_stays_refused(host, gpu_device):

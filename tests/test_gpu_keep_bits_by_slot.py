@@ -16,8 +16,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("h_in", [8, 192, 200, 584])   # mask rows of 1, 24, 25 and 73 bytes
 @pytest.mark.parametrize("r", [16, 64, 72])
 @pytest.mark.parametrize("tp", [[0, 1, 6, 19, 42, 97], [0, 3, 300, 305, 318, 640]], ids=["one-wave", "four-waves"])
-def test_backward_keep_bits(K, oracle, gpu_device, tp, r, h_in, shift):  # noqa: F811
-    d, dt, h_out, n_rows = gpu_device, "bf16", 72, tp[-1]
+# (1032 columns of dY are summed in two: the fold of dV then turns the bits, and dX shares the gradients' launch)
+@pytest.mark.parametrize("h_out", [72, 1032], ids=["turned-alone", "turned-in-fold"])
+def test_backward_keep_bits(K, oracle, gpu_device, h_out, tp, r, h_in, shift):  # noqa: F811
+    d, dt, n_rows = gpu_device, "bf16", tp[-1]
     part_ad, ad_p = [2, 0, 1, 2, 0], [0.5, 0.5, 0.0]
     rows = n_rows - 5   # the last five keep everything
     rng = np.random.default_rng(n_rows + h_in)
