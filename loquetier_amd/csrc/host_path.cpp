@@ -285,10 +285,23 @@ struct Backward {
   }
 };
 
+// the places of a tensor's elements (the stride of a dimension of one names none)
+struct Layout {
+  c10::DimVector sizes, strides;
+  explicit Layout(const Tensor& t) : sizes(t.sizes()), strides(t.strides()) {}
+  bool of(const Tensor& t) const {
+    if (t.sizes() != c10::IntArrayRef(sizes)) return false;
+    for (size_t i = 0; i < sizes.size(); ++i)
+      if (sizes[i] != 1 && t.stride((int64_t)i) != strides[i]) return false;
+    return true;
+  }
+};
+
 // ---- add_lora: everything a backward needs besides the saved tensors ----
 struct AddState : torch::CustomClassHolder {
   PyObject *wa, *wb, *s;  // during the forward only
   std::vector<int64_t> tp;
+  std::vector<Layout> layouts;  // of the weights
   int64_t rank, train_len, h_in, h_out;
 };
 
@@ -341,9 +354,11 @@ struct AddLora : public Function<AddLora> {
     }
     const int NA = (int)first.size();
     const Backward call(grads[0], x, v, st->tp[0], st->tp[P], st->h_in, rank);
-    for (int p = 0; p < 2 * P; ++p)
+    for (int p = 0; p < 2 * P; ++p) {
       TORCH_CHECK(s[2 + p].device() == call.g.device() && s[2 + p].scalar_type() == call.g.scalar_type(),
                   "the weights must share dy's dtype and device");
+      TORCH_CHECK(st->layouts[p].of(s[2 + p]), "the weights must come back laid out as they were saved");
+    }
     variable_list out(2 + s.size() - 2);
     out[0] = call.dx;
     // addresses of dA, dB, A and B, then where the partitions start and their adapters
@@ -574,6 +589,8 @@ PyObject* py_add_lora(PyObject*, PyObject* const* p, Py_ssize_t n) {
   if (parts < 1 || st->tp[parts] <= 0 || st->tp[parts] > st->train_len) Py_RETURN_NONE;
   for (const Tensor& w : weights)
     if (w.device() != x.device() || w.scalar_type() != x.scalar_type()) Py_RETURN_NONE;
+  st->layouts.reserve(2 * parts);
+  for (Py_ssize_t i = 0; i < 2 * parts; ++i) st->layouts.emplace_back(weights[i]);
   st->wa = p[2], st->wb = p[3], st->s = p[4];
   Tensor y;
   {

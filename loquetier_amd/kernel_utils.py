@@ -95,10 +95,16 @@ def _unique_adapters(weight_list: Sequence[torch.Tensor]):
     return pairs, part_adapter
 
 
+def _layouts(tensors: Sequence[torch.Tensor]):
+    """Where the tensors' elements lie: shapes, and strides (0 for a dimension of one, whose stride names nothing)."""
+    return [t if t is None else (tuple(t.shape), tuple(0 if n == 1 else s for n, s in zip(t.shape, t.stride())))
+            for t in tensors]
+
+
 def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Optional[torch.Tensor],
                   weight_list: Sequence[torch.Tensor], tp: Sequence[int], lora_rank: int,
                   part_scale: Optional[torch.Tensor] = None, dropout=None,
-                  adapter_rank: Optional[torch.Tensor] = None, step=None):
+                  adapter_rank: Optional[torch.Tensor] = None, step=None, layouts=None):
     """Shared backward: returns (grad_x [T, h_in], [grad per weight occurrence]).
 
     Partitions that train the same adapter contribute to one summed gradient,
@@ -108,7 +114,8 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
 
     `step` (mixed_lora.LayerStep or None): the backward's plan, the partitions'
     adapters, the weights' pointer tables and the layout of one buffer for all the
-    gradients, prepared outside the layer loop; without it they are made here."""
+    gradients, prepared outside the layer loop; without it they are made here.
+    `layouts` (_layouts or None): the weights' in the forward, which the kernels read them in."""
     dev, dt = grad_output.device, grad_output.dtype
     T = grad_output.size(0)
     h_in = x_train.size(1)
@@ -165,8 +172,11 @@ def lora_backward(grad_output: torch.Tensor, x_train: torch.Tensor, v_train: Opt
             for b in bufs:
                 b.zero_()
     else:
-        if any(w.device != dev or w.dtype != dt for w in weight_list[: 2 * n_parts]):  # (a saved-tensor hook's doing)
-            raise RuntimeError("the weights must share dy's dtype and device")
+        if tl > 0:  # (what a saved-tensor hook hands back is as it likes)
+            if any(w.device != dev or w.dtype != dt for w in weight_list[: 2 * n_parts]):
+                raise RuntimeError("the weights must share dy's dtype and device")
+            if layouts is not None and _layouts(weight_list[: 2 * n_parts]) != layouts[: 2 * n_parts]:
+                raise RuntimeError("the weights must come back laid out as they were saved")
         pairs, part_adapter = _unique_adapters(weight_list[: 2 * n_parts])
         da = [torch.empty_like(wa) for wa, _ in pairs]
         db = [torch.empty_like(wb) for _, wb in pairs]
@@ -233,6 +243,7 @@ class add_lora(Function):
         ctx.tp = train_partition
         ctx.rank = lora_rank
         ctx.has_v = v is not None
+        ctx.layouts = _layouts(args)
         if v is not None:
             ctx.save_for_backward(x[:train_len, ...], v[:train_len, ...], *args)
         else:
@@ -249,7 +260,7 @@ class add_lora(Function):
         if len(weight_list) == 0:
             return None, None, None, None, None, None, None, None
         assert len(weight_list) % 2 == 0
-        grad_x, grads = lora_backward(grad_output, x, v, weight_list, ctx.tp, ctx.rank)
+        grad_x, grads = lora_backward(grad_output, x, v, weight_list, ctx.tp, ctx.rank, layouts=ctx.layouts)
         return (None, grad_x, None, None, None, None, None, None, *grads)
 
 

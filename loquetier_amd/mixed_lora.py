@@ -19,7 +19,7 @@ import torch
 from torch import nn
 from torch.autograd.function import Function, FunctionCtx
 
-from .kernel_utils import BatchLenInfo, add_lora, lora_backward
+from .kernel_utils import BatchLenInfo, _layouts, add_lora, lora_backward
 from .ops import _kernels as kernel
 
 
@@ -358,6 +358,8 @@ class fused_add_lora(Function):
             if dropout is not None:  # the same stream, probabilities by train partition
                 ctx.part_drop = kernel.DropoutSpec(gather(dropout.seg_p), train_len,
                                                    dropout.seed, dropout.offset, dropout.mask_bits)
+        # (the backward reads the weights through the step's tables where those are prepared)
+        ctx.layouts = None if step.bwd_plan is not None and step.grad_layout is not None else _layouts(weights)
         if need_v:
             ctx.save_for_backward(x, v, *weights)  # (whole: the backward reads the plan's rows of them)
         return result
@@ -370,7 +372,7 @@ class fused_add_lora(Function):
         x, v, *weight_list = ctx.saved_tensors
         grad_x, grads = lora_backward(grad_output, x, v, weight_list, ctx.tp, ctx.rank,
                                       part_scale=ctx.part_scale, dropout=ctx.part_drop,
-                                      adapter_rank=ctx.train_rank, step=ctx.step)
+                                      adapter_rank=ctx.train_rank, step=ctx.step, layouts=ctx.layouts)
         return (grad_output, grad_x) + (None,) * (n_fixed - 2) + tuple(grads)
 
 

@@ -72,6 +72,7 @@ CASES = [(rms_case, 0, "strided", "must be contiguous"), (rms_case, 0, "wider", 
          (add_case, 0, "strided", "x must be contiguous"), (add_case, 0, "wider", "must share one dtype"),
          (add_case, 1, "strided", "v must be a contiguous"), (add_case, 1, "wider", "must share one dtype"),
          *[(add_case, w, form, "the weights must share dy's dtype and device") for w in (2, 3) for form in ("wider", "elsewhere")],
+         *[(add_case, w, "strided", "laid out as they were saved") for w in (2, 3)],
          (add_case, 0, "elsewhere", "must be a CUDA tensor"), (add_case, 1, "elsewhere", "must share one device"),
          (layer_case, 1, "strided", "x must be contiguous"), (layer_case, 1, "wider", "must share one dtype"),
          (layer_case, 2, "strided", "v must be a contiguous"), (layer_case, 2, "wider", "must share one dtype"),
