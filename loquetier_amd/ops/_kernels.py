@@ -526,7 +526,8 @@ def smlm_lora_forward_multi(ys, xs, a_ptrs, b_ptrs, plan: SegmentPlan, rank: int
     AT their true rank rounded up to 8 (A_a [r_a, h_in], B_a [h_out, r_a]) instead of padded.
     cache: a dict the caller keeps (one per layer): after a call has been checked, later calls with
     tensors of the same shapes, dtype, device and contiguity and the same tables skip the checks and
-    reuse the argument blocks that do not change."""
+    reuse the argument blocks that do not change.  Not for calls with dropout, nor for those of one
+    projection that the native host path takes: it checks every call."""
     n = len(ys)
     if n == 1 and dropout is None and stages == 3 and dims is None and len(xs) == len(a_ptrs) == len(b_ptrs) == 1 and (
             v_out is None or len(v_out) == 1) and _host().forward(
