@@ -26,7 +26,7 @@ def _cfg1_inputs(oracle, dt, exact):
         x = dyadic(rng, (T, h), 16, 8)
         A = [dyadic(rng, (r, h), 8, 64) for _ in range(NA)]
         B = [dyadic(rng, (h, r), 8, 8) for _ in range(NA)]
-    else:  # x ~ N(0,1), A ~ N(0, 1/4096), B ~ N(0, 1/16), as BASELINE.json states them
+    else:  # x ~ N(0,1), A ~ N(0, 1/4096), B ~ N(0, 1/16), the distributions this workload is stated with
         x = oracle.round_to(rng.standard_normal((T, h)), dt)
         A = [oracle.round_to(rng.standard_normal((r, h)) / 64.0, dt) for _ in range(NA)]
         B = [oracle.round_to(rng.standard_normal((h, r)) / 4.0, dt) for _ in range(NA)]
@@ -67,7 +67,7 @@ def test_baseline_config1_dyadic_bit_exact(K, oracle, gpu_device, dt, route):
 
 @pytest.mark.parametrize("dt", ["fp16", "bf16"])
 def test_baseline_config1_gaussian(K, oracle, gpu_device, dt):
-    """The inputs BASELINE.json states: the intermediate v within rtol 1e-2 / atol 1e-3 of the fp32 oracle,
+    """Inputs of the stated distributions: the intermediate v within rtol 1e-2 / atol 1e-3 of the fp32 oracle,
     y within that tolerance of the oracle fed with the kernel's own v (one 16-bit step of a v element
     moves a whole row of y by more than atol), and y end to end within the error budget of the exact
     result: no worse than the reference's own semantics (v rounded to the I/O type)."""
